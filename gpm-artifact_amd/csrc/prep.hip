@@ -19,6 +19,7 @@
 #include <vector>
 
 #include <rocprim/device/device_radix_sort.hpp>
+#include <rocprim/device/device_scan.hpp>
 #include <rocprim/device/device_select.hpp>
 
 #include "graph_dev.hpp"
@@ -121,6 +122,59 @@ __global__ void relabel_keys_kernel(const uint32_t* __restrict__ off, const uint
     const unsigned long long hi = (unsigned long long)new_id[u] << 32;
     for (uint32_t i = off[u] + lane_id(); i < off[u + 1]; i += kWave) keys[i] = hi | new_id[adj[i]];
   }
+}
+
+// Topological relabel of a DAG (topo_relabel_device).  deg[v] = out-degree
+// plus in-degree: the out-degrees first, then one increment per entry.
+__global__ void out_degree_kernel(const uint32_t* __restrict__ off, uint32_t n,
+                                  uint32_t* __restrict__ deg, uint32_t* __restrict__ ids) {
+  for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x) {
+    deg[v] = off[v + 1] - off[v];
+    ids[v] = v;
+  }
+}
+
+__global__ void in_degree_kernel(const uint32_t* __restrict__ adj, uint64_t m,
+                                 uint32_t* __restrict__ deg) {
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m;
+       i += (uint64_t)gridDim.x * blockDim.x)
+    atomicAdd(&deg[adj[i]], 1u);
+}
+
+// Keys rank(u) << bits | rank(x) of every entry, one wave per u;
+// *descent is set when some edge does not go up in rank.
+__global__ void topo_keys_kernel(const uint32_t* __restrict__ off, const uint32_t* __restrict__ adj,
+                                 const uint32_t* __restrict__ rank, uint32_t n, uint32_t bits,
+                                 unsigned long long* __restrict__ keys,
+                                 unsigned int* __restrict__ descent) {
+  const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
+  const uint32_t nwaves = gridDim.x * blockDim.x / kWave;
+  bool down = false;
+  for (uint32_t u = wave; u < n; u += nwaves) {
+    const uint32_t ru = rank[u];
+    for (uint32_t i = off[u] + lane_id(); i < off[u + 1]; i += kWave) {
+      const uint32_t rx = rank[adj[i]];
+      down |= rx <= ru;
+      keys[i] = (unsigned long long)ru << bits | rx;
+    }
+  }
+  if (down) *descent = 1u;
+}
+
+// Out-degrees in rank order (entry n = 0, so the scan ends with m).
+__global__ void ranked_degree_kernel(const uint32_t* __restrict__ off,
+                                     const uint32_t* __restrict__ order, uint32_t n,
+                                     uint32_t* __restrict__ out) {
+  for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r <= n; r += gridDim.x * blockDim.x)
+    out[r] = r < n ? off[order[r] + 1] - off[order[r]] : 0u;
+}
+
+__global__ void key_targets_kernel(const unsigned long long* __restrict__ keys, uint64_t m,
+                                   uint32_t bits, uint32_t* __restrict__ out) {
+  const uint32_t mask = bits >= 32 ? 0xFFFFFFFFu : (1u << bits) - 1u;
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m;
+       i += (uint64_t)gridDim.x * blockDim.x)
+    out[i] = (uint32_t)keys[i] & mask;
 }
 
 // Device buffers of one preparation call, freed on every exit path unless
@@ -374,6 +428,75 @@ int relabel(gpm_graph* g, gpm_graph** out, uint32_t** perm) {
 }
 
 }  // namespace
+
+namespace gpm {
+
+int topo_relabel_device(gpm_graph* g, uint32_t** toff, uint32_t** tadj, std::vector<uint32_t>* rank,
+                        bool* ordered) {
+  const uint32_t n = g->n;
+  const uint64_t m = g->m;
+  const int cus = device_cus(g);
+  *ordered = false;
+  if (!n || !m) return GPM_OK;
+  struct Drain {  // the buffers below are freed only once the stream is done with them
+    hipStream_t s;
+    ~Drain() { (void)hipStreamSynchronize(s); }
+  };
+  Bufs b;
+  Drain drain{g->stream};
+  int st;
+  const unsigned bits = (unsigned)bits_for(std::max(n, 1u) - 1u);
+  uint32_t *deg = nullptr, *ids = nullptr, *sdeg = nullptr, *order = nullptr, *new_id = nullptr;
+  unsigned int* descent = nullptr;
+  unsigned long long *keys = nullptr, *sorted = nullptr;
+  if ((st = b.alloc(&deg, n)) != GPM_OK || (st = b.alloc(&ids, n)) != GPM_OK ||
+      (st = b.alloc(&sdeg, (uint64_t)n + 1)) != GPM_OK || (st = b.alloc(&order, n)) != GPM_OK ||
+      (st = b.alloc(&new_id, n)) != GPM_OK || (st = b.alloc(&descent, 1)) != GPM_OK ||
+      (st = b.alloc(&keys, m)) != GPM_OK || (st = b.alloc(&sorted, m)) != GPM_OK ||
+      (st = b.alloc(toff, (uint64_t)n + 1)) != GPM_OK || (st = b.alloc(tadj, m)) != GPM_OK)
+    return st;
+  const dim3 block(kBlock);
+  const dim3 per_vertex(grid_for_items((uint64_t)n + 1, cus));
+  size_t sort_ids = 0, sort_keys = 0, scan = 0;
+  GPM_HIP(rocprim::radix_sort_pairs(nullptr, sort_ids, deg, sdeg, ids, order, n, 0u, 32u,
+                                    g->stream));
+  GPM_HIP(rocprim::radix_sort_keys(nullptr, sort_keys, keys, sorted, m, 0u, 2 * bits, g->stream));
+  GPM_HIP(rocprim::exclusive_scan(nullptr, scan, sdeg, *toff, 0u, (size_t)n + 1,
+                                  rocprim::plus<uint32_t>(), g->stream));
+  char* temp = nullptr;
+  if ((st = b.alloc(&temp, std::max(std::max(sort_ids, sort_keys), scan))) != GPM_OK) return st;
+  hipLaunchKernelGGL(out_degree_kernel, per_vertex, block, 0, g->stream, g->off, n, deg, ids);
+  hipLaunchKernelGGL(in_degree_kernel, dim3(grid_for_items(m, cus)), block, 0, g->stream, g->adj,
+                     m, deg);
+  GPM_HIP(hipGetLastError());
+  GPM_HIP(rocprim::radix_sort_pairs(temp, sort_ids, deg, sdeg, ids, order, n, 0u, 32u, g->stream));
+  hipLaunchKernelGGL(scatter_rank_kernel, per_vertex, block, 0, g->stream, order, n, new_id);
+  hipLaunchKernelGGL(ranked_degree_kernel, per_vertex, block, 0, g->stream, g->off, order, n, sdeg);
+  GPM_HIP(hipGetLastError());
+  GPM_HIP(rocprim::exclusive_scan(temp, scan, sdeg, *toff, 0u, (size_t)n + 1,
+                                  rocprim::plus<uint32_t>(), g->stream));
+  const unsigned int zero = 0;
+  if ((st = h2d(g, descent, &zero, sizeof(zero))) != GPM_OK) return st;
+  hipLaunchKernelGGL(topo_keys_kernel, dim3(grid_for_items((uint64_t)n * kWave, cus)), block, 0,
+                     g->stream, g->off, g->adj, new_id, n, bits, keys, descent);
+  GPM_HIP(hipGetLastError());
+  GPM_HIP(rocprim::radix_sort_keys(temp, sort_keys, keys, sorted, m, 0u, 2 * bits, g->stream));
+  hipLaunchKernelGGL(key_targets_kernel, dim3(grid_for_items(m, cus)), block, 0, g->stream, sorted,
+                     m, bits, *tadj);
+  GPM_HIP(hipGetLastError());
+  unsigned int down = 0;
+  rank->resize(n);
+  GPM_HIP(hipMemcpyAsync(&down, descent, sizeof(down), hipMemcpyDeviceToHost, g->stream));
+  GPM_HIP(hipMemcpyAsync(rank->data(), new_id, (size_t)n * 4, hipMemcpyDeviceToHost, g->stream));
+  GPM_HIP(hipStreamSynchronize(g->stream));
+  if (down) return GPM_OK;
+  *ordered = true;
+  b.release(*toff);
+  b.release(*tadj);
+  return GPM_OK;
+}
+
+}  // namespace gpm
 
 extern "C" {
 
