@@ -11,21 +11,21 @@
 //     k=4: sum_i sum_{j in row_i} |row_i & row_j|
 //     k=5: sum_i sum_{j in row_i} sum_{l in row_i & row_j} |row_i & row_j & row_l|
 // Row i equals the reference's W1 for the edge (v0, S[i]); row_i & row_j is its
-// W2.  Rows are built by streaming the lists N+(S[i]) through an LDS hash of S
-// (a flattened walk: all lanes read consecutive entries, whatever the list
-// lengths), or, for lists much longer than S, by binary-searching each S[j]
-// in N+(S[i]) and taking the 64-bit ballot as the row word.
+// W2.  Rows are built by streaming the lists N+(S[i]) past a bitmap (block
+// tiers) or a hash table (wave tier) of S in LDS, or, for lists much longer than
+// S, by binary-searching each S[j] in N+(S[i]).  In the block tiers the k = 5
+// sum is a masked product of 0/1 matrices on the matrix cores (count5_row).
 //
 // The kernels read the DAG relabelled in a topological order (gpm_graph's
 // toff/tadj, built once per handle), so S = N+(v0) is sorted topologically
 // and every row is upper triangular: row i only holds positions > i.  For
-// k=5 the popcount of row_i & row_j & row_l then starts at l's word, which
-// skips about half to two thirds of the words.  Counts do not depend on ids.
+// k=5 the product for l then starts at l's 128-position chunk.  Counts do not
+// depend on ids.
 //
 // Three tiers by |S| (tiers.hpp): one wave per root with rows in registers
-// (|S| <= 64, one 64-bit word per row, lane i owns row i); one 256-thread
-// block per root with rows in LDS (|S| <= 512); one block per root with rows
-// in a per-block HBM region (larger |S|).
+// (|S| <= 64, one 64-bit word per row, lane i owns row i); one 512-thread
+// block per root with rows in LDS (|S| <= 1024, in two tiers); one block per
+// root with rows in a per-block HBM region (larger |S|).
 //
 // MODE selects what is accumulated: kCount (the clique count), kBytes (the
 // algorithmic bytes of the reference's edge-rooted plan, see gpm.h), kWork
@@ -45,13 +45,23 @@ constexpr int kWavesPerBlock = kBlock / kWave;
 constexpr uint32_t kWaveTable = 128;
 constexpr uint32_t kBlockCap = 512;
 // Threads per block of the block tiers.  Rows are shared by the whole block,
-// so wider blocks raise the waves per SIMD that hide LDS latency without
-// more LDS: the wide tier fits one block per CU, the LDS tier three.
+// so wider blocks raise the waves per SIMD that hide latency without more LDS.
+// The k = 5 count keeps 128 registers and more: two blocks of the LDS tier fit
+// a CU (three of 256 threads were slower, 11.6 against 10.3 ms a launch on
+// R-MAT scale 20: too few waves for the row build), and one of the wide tier.
 constexpr int kLdsBlock = 512;
-constexpr int kWideBlock = 1024;
+constexpr int kWideBlock = 512;
 constexpr int kHbmBlock = 1024;
-// Consecutive list entries one thread streams in the row build.
+// Consecutive list entries one thread streams in the row build of the HBM
+// tier.
 constexpr uint32_t kSeg = 8;
+// Row build of the LDS tiers: the ids of [n - kIdBits, n) have one bit each in
+// LDS.  The relabelled DAG gives the most linked vertices the highest ids, so
+// on R-MAT scale 20 nine in ten list entries fall into the top 32768.
+constexpr uint32_t kIdBits = 32768;
+constexpr uint32_t kIdWords = kIdBits / 32;
+// 64-entry windows of a list one wave has in flight in that build.
+constexpr uint32_t kListWindows = 4;
 enum { kCount = 0, kBytes = 1, kWork = 2, kAll = 3 };
 // kAll (with K = 5): the 3-, 4- and 5-clique counts of every root from one
 // build of its rows; out[0..2] receive them.
@@ -59,9 +69,11 @@ enum { kCount = 0, kBytes = 1, kWork = 2, kAll = 3 };
 // A list N+(S[i]) much longer than S is not streamed: each S[t] is looked up
 // in it by binary search instead (d searches of log2(len) steps against len
 // streamed entries).  Thresholds measured on R-MAT scale 20: lists longer
-// than max(64, 2d) for the wave tier and max(64, 4d) for the block tiers.
+// than max(64, 2d) for the wave tier; for the block tiers, whose bitmap makes
+// a streamed entry cheap, longer than 16d (the 3-clique count of the LDS tier
+// took 3.5 ms with 4d, 3.0 ms with 16d).
 __device__ __forceinline__ bool use_probe(uint32_t len, uint32_t d) {
-  return len > max(64u, 4u * d);
+  return len > max(64u, 16u * d);
 }
 __device__ __forceinline__ bool use_probe_wave(uint32_t len, uint32_t d) {
   return len > max(64u, 2u * d);
@@ -441,14 +453,283 @@ __device__ __forceinline__ uint64_t count_rows(const unsigned long long* rows, u
   return c;
 }
 
-// Block per root.  LDS_ROWS: rows, S, lens, begins and the hash table live in
+// Rows of one root in LDS: bit idx of row i is set when S[idx] is in N+(S[i]).
+// One wave per list, 64 consecutive entries per load; an entry x >= id_base is
+// looked up in the bitmap of S (one LDS word: in S or not), and its position in
+// S is the word's prefix plus the set bits below x.  Entries below id_base only
+// matter when S has some there (*s_low of them, at its front): those are
+// binary-searched.  Lists much longer than S are left to the probing pass
+// (*s_any_probe).  A bitmap word answers an entry in a fixed few instructions,
+// where an open-addressed table of S made the 64 lanes wait for the longest
+// probe sequence among them: the 3-clique count of the LDS tier on R-MAT scale
+// 20, nearly all row build, fell from 7.2 to 3.0 ms (2.3e9 entries).
+template <int BS>
+__device__ __forceinline__ void build_rows(const uint32_t* __restrict__ adj,
+                                           unsigned long long* rows, uint32_t RS, uint32_t d,
+                                           const uint32_t* lens, const uint32_t* begs,
+                                           const uint32_t* sids, uint32_t* bits, uint16_t* pre,
+                                           uint32_t id_base, uint32_t* s_wsum, uint32_t* s_low,
+                                           int* s_any_probe) {
+  constexpr uint32_t kPer = kIdWords / BS;  // consecutive bitmap words per thread
+  static_assert(kPer * BS == kIdWords, "whole words per thread");
+  const uint32_t lane = lane_id();
+  uint32_t low = 0;
+  for (uint32_t i = threadIdx.x; i < d; i += BS) {
+    const uint32_t t = sids[i] - id_base;
+    if (sids[i] < id_base)
+      ++low;
+    else
+      atomicOr(&bits[t >> 5], 1u << (t & 31));
+  }
+  if (low) atomicAdd(s_low, low);
+  __syncthreads();
+  const uint32_t nlow = uniform(*s_low);
+  {
+    uint32_t c[kPer], sum = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k) sum += c[k] = (uint32_t)__popc(bits[kPer * threadIdx.x + k]);
+    uint32_t at = nlow + block_incl_scan(sum, s_wsum) - sum;
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k) {
+      pre[kPer * threadIdx.x + k] = (uint16_t)at;
+      at += c[k];
+    }
+  }
+  __syncthreads();
+  // The next kListWindows windows of a wave's lists are loaded before the last
+  // ones are looked up, so a wave always has a batch of loads in flight.
+  uint32_t* rows32 = reinterpret_cast<uint32_t*>(rows);
+  struct Batch {
+    uint32_t row, len, t0;  // entries [t0, t0 + kListWindows * kWave) of list `row`
+    const uint32_t* list;
+    uint32_t x[kListWindows];
+  };
+  // Moves to the wave's list i or the next one that is streamed.
+  auto open = [&](Batch& b, uint32_t i) {
+    b.t0 = 0;
+    for (; i < d; i += BS / kWave) {
+      b.len = uniform(lens[i]);
+      if (!use_probe(b.len, d) && b.len) break;
+      if (b.len && lane == 0) *s_any_probe = 1;
+    }
+    b.row = i;
+    b.list = adj + (i < d ? uniform(begs[i]) : 0u);
+  };
+  auto load = [&](Batch& b) {
+#pragma unroll
+    for (uint32_t q = 0; q < kListWindows; ++q) {
+      const uint32_t p = b.t0 + q * kWave + lane;
+      b.x[q] = p < b.len ? b.list[p] : kEmpty;  // kEmpty: past every id and bitmap word
+    }
+  };
+  Batch cur;
+  open(cur, uniform(threadIdx.x / kWave));
+  if (cur.row < d) load(cur);
+  while (cur.row < d) {
+    Batch next = cur;
+    next.t0 += kListWindows * kWave;
+    if (next.t0 >= next.len) open(next, cur.row + BS / kWave);
+    if (next.row < d) load(next);
+    uint32_t* row = rows32 + 2 * cur.row * RS;
+#pragma unroll
+    for (uint32_t q = 0; q < kListWindows; ++q) {
+      if (cur.t0 + q * kWave >= cur.len) break;
+      const uint32_t t = cur.x[q] - id_base;
+      if (t < kIdBits) {
+        const uint32_t w = bits[t >> 5], below = (1u << (t & 31)) - 1u;
+        if ((w >> (t & 31)) & 1u) {
+          const uint32_t idx = pre[t >> 5] + (uint32_t)__popc(w & below);
+          atomicOr(&row[idx >> 5], 1u << (idx & 31));
+        }
+      } else if (nlow && cur.x[q] < id_base) {
+        const uint32_t p = upper_index(sids, nlow, cur.x[q]);
+        if (p > 0 && sids[p - 1] == cur.x[q]) atomicOr(&row[(p - 1) >> 5], 1u << ((p - 1) & 31));
+      }
+    }
+    cur = next;
+  }
+  __syncthreads();
+}
+
+typedef int intx4 __attribute__((ext_vector_type(4)));
+typedef int intx8 __attribute__((ext_vector_type(8)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+// 32 bits -> 32 FP4 (E2M1) values, eight to a register, register r holding bits
+// r, r + 4, ...: a set bit becomes the value whose code it already is in place
+// (0b0001 = 0.5, 0b0010 = 1, 0b0100 = 2; the bit at the sign's place moves down,
+// 2) on the one side of a product, and the reciprocal on the other, so that two
+// set bits make 1.  The side that is expanded more often takes the in-place codes.
+__device__ __forceinline__ intx4 fp4_in_place(uint32_t w) {
+  return intx4{(int)(w & 0x11111111u), (int)(w & 0x22222222u), (int)(w & 0x44444444u),
+               (int)((w >> 1) & 0x44444444u)};
+}
+__device__ __forceinline__ intx4 fp4_reciprocal(uint32_t w) {
+  return intx4{(int)((w << 2) & 0x44444444u), (int)(w & 0x22222222u),
+               (int)((w >> 2) & 0x11111111u), (int)((w >> 3) & 0x11111111u)};
+}
+
+// c + A B^T over 128 positions: A, B = 16 rows of FP4 values, lane l holding
+// 32 positions (4 of the 128-position chunk's 32-bit words: word l / 16) of row
+// l % 16.
+__device__ __forceinline__ floatx4 mfma_fp4(intx4 a, intx4 b, floatx4 c) {
+  constexpr int kFp4 = 4, kOne = 127;  // operand format; block scale 2^0
+  const intx8 a8 = __builtin_shufflevector(a, a, 0, 1, 2, 3, -1, -1, -1, -1);
+  const intx8 b8 = __builtin_shufflevector(b, b, 0, 1, 2, 3, -1, -1, -1, -1);
+  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a8, b8, c, kFp4, kFp4, 0, kOne, 0, kOne);
+}
+
+// Column blocks lb, lb + 1, ... whose first position lies in chunk C0 (of 128
+// positions), against the row blocks in a; adds to sum.  Rows l hold positions
+// > l only, so the sizes start at chunk C0, and the adjacency of a column block
+// sits in the chunks of its positions.  Then the same for the chunks after C0.
+template <int NC, int J, int C0>
+__device__ __forceinline__ void count5_columns(const uint32_t* rows32, uint32_t RS32,
+                                               const intx4 (&a)[J][NC], const uint16_t* list,
+                                               uint32_t nt, uint32_t lb, floatx4& sum) {
+  const uint32_t lane = lane_id(), r16 = lane & 15, g = lane >> 4;
+  const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+  for (; lb < nt; ++lb) {
+    const uint32_t l = list[16 * lb + r16];
+    if (C0 + 1 < NC && uniform(l) >= 128 * (C0 + 1)) break;
+    const uint32_t last = __builtin_amdgcn_readlane(l, 15) / 128;
+    const uint32_t* rl = rows32 + __umul24(l, RS32) + g;
+    const uint32_t lw = (l >> 5) - g;  // word of l's own bit, from this lane's first
+    const uint32_t lbit = 1u << (l & 31);
+    floatx4 both[J], adj[J];
+    const intx4 b0 = fp4_in_place(rl[4 * C0]);
+    const intx4 e0 = fp4_in_place(lw == 4 * C0 ? lbit : 0u);
+#pragma unroll
+    for (int q = 0; q < J; ++q) {
+      both[q] = mfma_fp4(a[q][C0], b0, zero);
+      adj[q] = mfma_fp4(a[q][C0], e0, zero);
+    }
+#pragma unroll
+    for (int c = C0 + 1; c < NC; ++c) {
+      const intx4 b = fp4_in_place(rl[4 * c]);
+#pragma unroll
+      for (int q = 0; q < J; ++q) both[q] = mfma_fp4(a[q][c], b, both[q]);
+      if ((uint32_t)c <= last) {
+        const intx4 e = fp4_in_place(lw == 4 * c ? lbit : 0u);
+#pragma unroll
+        for (int q = 0; q < J; ++q) adj[q] = mfma_fp4(a[q][c], e, adj[q]);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < J; ++q)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sum[r] = __builtin_fmaf(both[q][r], adj[q][r], sum[r]);
+  }
+  if constexpr (C0 + 1 < NC) count5_columns<NC, J, C0 + 1>(rows32, RS32, a, list, nt, lb, sum);
+}
+
+// Row blocks jg .. jg + J - 1 (16 positions of N_i each) of the k = 5 count of
+// row i, see count5_row.
+template <int NC, int J, bool ALL>
+__device__ __forceinline__ float count5_blocks(const uint32_t* rows32, uint32_t RS32,
+                                               const uint32_t (&ri)[NC], const uint16_t* list,
+                                               uint32_t nt, uint32_t jg, uint32_t& c4) {
+  const uint32_t lane = lane_id(), r16 = lane & 15, g = lane >> 4;
+  intx4 a[J][NC];
+#pragma unroll
+  for (int q = 0; q < J; ++q) {
+    const uint32_t* rj = rows32 + __umul24(list[16 * (jg + q) + r16], RS32) + g;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const uint32_t w = rj[4 * c] & ri[c];
+      if (ALL) c4 += (uint32_t)__popc(w);
+      a[q][c] = fp4_reciprocal(w);
+    }
+  }
+  floatx4 sum = {0.f, 0.f, 0.f, 0.f};
+  count5_columns<NC, J, 0>(rows32, RS32, a, list, nt, jg, sum);
+  return (sum[0] + sum[1]) + (sum[2] + sum[3]);
+}
+
+// One row i of the k = 5 count, by one wave: with N_i the set bits of row i,
+//     sum over j, l in N_i, l in row j, of |row_i & row_j & row_l|.
+// The sizes are a product of 0/1 matrices (rows j masked by row i, times rows
+// l), which the matrix cores evaluate in FP4 with FP32 sums, 16 x 16 pairs and
+// 128 positions per instruction; the rows of N_i are gathered from LDS and
+// expanded in registers.  The pairs that are adjacent are picked by a second
+// product, of the same rows j with the unit vectors of l, which leaves the 0/1
+// adjacency of the pair in the register and lane of its size: one fused
+// multiply-add then sums.  Every value is a whole number below 2^24 (a lane
+// sums at most 1024^2 / 64 pairs of at most 1024), so FP32 is exact.
+// The pairs within a hub's out-list are dense (30 - 45 % of all pairs on R-MAT
+// scale 20), so a dense product does less work than AND + popcount over the
+// set bits one by one, which ran at 95 % of the VALU issue rate with 54 % of the
+// lanes in use.  On R-MAT scale 20 the k = 5 launch of the LDS tier went from
+// 19.7 to 9.6 ms (with the row build above) and the wide tier's from 7.2 to
+// 2.9 ms.  VALU issue still bounds it: expanding and gathering take about 20
+// instructions per 16 x 16 pairs.  The kernel must not spill inside the count:
+// matrix instructions read every lane's register, whatever the active lanes.
+// The list of N_i is filled up with d, the index of a row of zeros.
+template <int NC, bool ALL>
+__device__ __forceinline__ uint32_t count5_row(const uint32_t* rows32, uint32_t RS32, uint32_t d,
+                                               uint32_t W, uint32_t i, uint16_t* list,
+                                               uint32_t& c3, uint32_t& c4) {
+  const uint32_t lane = lane_id(), g = lane >> 4;
+  const uint32_t* row = rows32 + i * RS32;
+  uint32_t ni = 0;
+  for (uint32_t w = 0; w < W; ++w) {
+    const uint64_t word = (uint64_t)uniform(row[2 * w + 1]) << 32 | uniform(row[2 * w]);
+    const bool in = (word >> lane) & 1ull;
+    if (in) list[ni + lanes_below(word)] = (uint16_t)(64 * w + lane);
+    if (ALL) c3 += in ? 1u : 0u;
+    ni += (uint32_t)__popcll(word);
+  }
+  list[ni + lane] = (uint16_t)d;
+  __builtin_amdgcn_wave_barrier();
+  if (ni < 2) return 0;  // no pair j, l
+  uint32_t ri[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) ri[c] = 4 * c + g < 2 * W ? row[4 * c + g] : 0u;
+  float s = 0.f;
+  const uint32_t nt = (ni + 15) / 16;
+  if (nt == 1) {
+    s = count5_blocks<NC, 1, ALL>(rows32, RS32, ri, list, nt, 0, c4);
+  } else if (nt == 2) {
+    s = count5_blocks<NC, 2, ALL>(rows32, RS32, ri, list, nt, 0, c4);
+  } else {
+    constexpr int J = NC <= 2 ? 4 : NC <= 4 ? 2 : 2;
+    for (uint32_t jg = 0; jg < nt; jg += J)
+      s += count5_blocks<NC, J, ALL>(rows32, RS32, ri, list, nt, jg, c4);
+  }
+  __builtin_amdgcn_wave_barrier();
+  return (uint32_t)s;
+}
+
+// The k = 5 count of the rows part, part + n_parts, ... of a root: the block's
+// waves take them in turn (the rows' costs fall slowly with their index, so
+// the waves end together).  Rows are MAXW words at most; words past W are
+// masked out by row i's.  A lane's sums over one root fit 32 bits (at most
+// C(1024, 4) 4-cliques over the block's lanes).
+template <int NC, bool ALL, int BS>
+__device__ __forceinline__ uint32_t count5_rows(const unsigned long long* rows, uint32_t d,
+                                                uint32_t W, uint32_t RS, uint32_t part,
+                                                uint32_t n_parts, uint16_t* list, uint32_t& c3,
+                                                uint32_t& c4) {
+  uint32_t c = 0;
+  for (uint32_t i = part + uniform(threadIdx.x / kWave) * n_parts; i < d; i += BS / kWave * n_parts)
+    c += count5_row<NC, ALL>(reinterpret_cast<const uint32_t*>(rows), 2 * RS, d, W, i, list, c3, c4);
+  return c;
+}
+
+// Block per root.  LDS_ROWS: rows, S, lens, begins and the bitmap of S live in
 // dynamic LDS (|S| <= cap, W <= MAXW words per row).  Otherwise rows live in this block's
 // HBM region `grows` (cap*W words) and membership in S is a binary search.
+// Waves per SIMD the registers have to leave room for: as many as the LDS of
+// two resident blocks (k = 5, 8-word rows) needs.
+constexpr int block_waves(int k, int mode, bool lds_rows, int maxw) {
+  return k == 5 && (mode == kCount || mode == kAll) && lds_rows && maxw == 8 ? 4 : 1;
+}
+
 template <int K, int MODE, bool LDS_ROWS, int MAXW, int BS>
-__global__ __launch_bounds__(BS) void clique_block_kernel(
+__global__ __launch_bounds__(BS, block_waves(K, MODE, LDS_ROWS, MAXW)) void clique_block_kernel(
     const uint32_t* __restrict__ off, const uint32_t* __restrict__ adj,
-    const uint32_t* __restrict__ roots, const uint32_t* __restrict__ parts, uint32_t n_roots,
-    uint32_t cap, uint32_t table, unsigned int* __restrict__ queue,
+    uint32_t n, const uint32_t* __restrict__ roots, const uint32_t* __restrict__ parts,
+    uint32_t n_roots, uint32_t cap, unsigned int* __restrict__ queue,
     unsigned long long* __restrict__ grows, uint32_t* __restrict__ gmeta,
     unsigned long long* __restrict__ out, unsigned long long* __restrict__ work) {
   extern __shared__ unsigned long long s_dyn[];
@@ -457,7 +738,9 @@ __global__ __launch_bounds__(BS) void clique_block_kernel(
   __shared__ uint32_t s_root;
   __shared__ uint32_t s_np;
   __shared__ int s_any_probe;
+  __shared__ uint32_t s_low;   // entries of S below id_base
   __shared__ unsigned long long s_red[(BS / kWave)];
+  __shared__ unsigned long long s_tot[BS / kWave][3];  // k = 5: counts for k = 5, 3, 4
   const uint32_t Wcap = (cap + 63) / 64;
   // LDS rows of the 8-word tier are padded to an odd stride (in 8-byte words):
   // the rows read together sit at data-dependent indices, and an even stride
@@ -465,23 +748,28 @@ __global__ __launch_bounds__(BS) void clique_block_kernel(
   constexpr bool kPad = LDS_ROWS && MAXW == 8;
   const uint32_t RScap = kPad ? (Wcap | 1u) : Wcap;
   unsigned long long* rows;
-  uint32_t *lens, *begs, *keys;
-  uint32_t* vals;
+  uint32_t *lens, *begs;
+  uint32_t* sids = nullptr;   // S itself
+  uint32_t* bits = nullptr;   // kIdWords words: the ids of S from id_base on
+  uint16_t* pre = nullptr;    // position in S of the first id of each word
+  uint16_t* lists = nullptr;  // cap + 64 entries per wave (k = 5), over lens .. pre
   if (LDS_ROWS) {
     rows = s_dyn;
-    lens = reinterpret_cast<uint32_t*>(rows + (size_t)cap * RScap);
+    lens = reinterpret_cast<uint32_t*>(rows + (size_t)(cap + 1) * RScap);
     begs = lens + cap;
-    keys = begs + cap;
-    vals = keys + table;
+    sids = begs + cap;
+    bits = sids + cap;
+    pre = reinterpret_cast<uint16_t*>(bits + kIdWords);
+    lists = reinterpret_cast<uint16_t*>(lens) + (threadIdx.x / kWave) * (cap + kWave);
   } else {
     rows = grows + (size_t)blockIdx.x * cap * Wcap;
     lens = gmeta + (size_t)blockIdx.x * 2 * cap;
     begs = lens + cap;
-    keys = nullptr;
-    vals = nullptr;
   }
-  const uint32_t hmask = table - 1;
+  const uint32_t id_base = n > kIdBits ? n - kIdBits : 0u;
+  constexpr bool kCount5 = LDS_ROWS && K == 5 && (MODE == kCount || MODE == kAll);
   uint64_t acc = 0, acc3 = 0, acc4 = 0;
+  if (kCount5 && threadIdx.x < BS / kWave * 3) (&s_tot[0][0])[threadIdx.x] = 0ull;
   while (true) {
     if (threadIdx.x == 0) s_root = atomicAdd(queue, 1u);
     __syncthreads();
@@ -495,24 +783,29 @@ __global__ __launch_bounds__(BS) void clique_block_kernel(
     const uint32_t* S = adj + sb;
     const uint32_t W = (d + 63) / 64;
     const uint32_t RS = kPad ? (W | 1u) : W;
-    if (threadIdx.x == 0) s_any_probe = 0;
+    if (threadIdx.x == 0) {
+      s_any_probe = 0;
+      s_low = 0;
+    }
     for (uint32_t i = threadIdx.x; i < d; i += BS) {
       const uint32_t v = S[i];
       const uint32_t b = off[v];
       const uint32_t len = off[v + 1] - b;
       lens[i] = len;
       begs[i] = b;
+      if (LDS_ROWS) sids[i] = v;
     }
-    for (uint32_t i = threadIdx.x; i < d * RS; i += BS) rows[i] = 0ull;
+    // LDS rows: row d stays empty.
+    for (uint32_t i = threadIdx.x; i < (LDS_ROWS ? d + 1 : d) * RS; i += BS) rows[i] = 0ull;
     if (LDS_ROWS)
-      for (uint32_t i = threadIdx.x; i < table; i += BS) keys[i] = kEmpty;
+      for (uint32_t i = threadIdx.x; i < kIdWords; i += BS) bits[i] = 0u;
     __syncthreads();
     // HBM rows: drop stale L1 lines of the previous root before reading.
     if (!LDS_ROWS) __threadfence();
-    if (LDS_ROWS)
-      for (uint32_t i = threadIdx.x; i < d; i += BS)
-        lds_hash_insert(keys, vals, hmask, S[i], i);
-    __syncthreads();
+    if constexpr (LDS_ROWS) {
+      build_rows<BS>(adj, rows, RS, d, lens, begs, sids, bits, pre, id_base, s_wsum, &s_low,
+                     &s_any_probe);
+    } else
     // Flattened walk over the lists that are streamed.
     for (uint32_t c0 = 0; c0 < d; c0 += BS) {
       const uint32_t i = c0 + threadIdx.x;
@@ -544,14 +837,9 @@ __global__ __launch_bounds__(BS) void clique_block_kernel(
           }
           const uint32_t row_i = c0 + j;
           const uint32_t x = adj[begs[row_i] + (f - excl)];
-          int idx;
-          if (LDS_ROWS) {
-            idx = lds_hash_find(keys, vals, hmask, x);
-          } else {
-            const uint32_t p = upper_index(S, d, x);
-            idx = (p > 0 && S[p - 1] == x) ? (int)(p - 1) : -1;
-          }
-          // Rows are this block's alone (LDS, or its slice of HBM scratch).
+          const uint32_t p = upper_index(S, d, x);
+          const int idx = (p > 0 && S[p - 1] == x) ? (int)(p - 1) : -1;
+          // The rows are this block's slice of HBM scratch.
           if (idx >= 0) wg_atomic_or(&rows[(size_t)row_i * RS + (idx >> 6)], 1ull << (idx & 63));
         }
       }
@@ -581,8 +869,39 @@ __global__ __launch_bounds__(BS) void clique_block_kernel(
     }
     __syncthreads();
     if (!LDS_ROWS) __threadfence();
-    uint64_t c;
-    if ((MODE == kCount || MODE == kAll) && K >= 4) {
+    uint64_t c = 0;
+    if constexpr (kCount5) {
+      constexpr bool ALL = MODE == kAll;
+      uint32_t r3 = 0, r4 = 0, c = 0;
+#define GPM_ROWS(NC) count5_rows<NC, ALL, BS>(rows, d, W, RS, part, n_parts, lists, r3, r4)
+      if (MAXW == 8) {
+        switch ((W + 1) / 2) {
+          case 0: case 1: c = GPM_ROWS(1); break;
+          case 2: c = GPM_ROWS(2); break;
+          case 3: c = GPM_ROWS(3); break;
+          default: c = GPM_ROWS(4); break;
+        }
+      } else {
+        switch ((W + 1) / 2) {
+          case 0: case 1: case 2: case 3: case 4: case 5: c = GPM_ROWS(5); break;
+          case 6: c = GPM_ROWS(6); break;
+          case 7: c = GPM_ROWS(7); break;
+          default: c = GPM_ROWS(8); break;
+        }
+      }
+#undef GPM_ROWS
+      // The totals stay in LDS: the count needs the registers.
+      const uint64_t w5 = wave_sum_u64(c), w3 = ALL ? wave_sum_u64(r3) : 0,
+                     w4 = ALL ? wave_sum_u64(r4) : 0;
+      if (lane_id() == 0) {
+        unsigned long long* t = s_tot[threadIdx.x / kWave];
+        t[0] += w5;
+        if (ALL) {
+          t[1] += w3;
+          t[2] += w4;
+        }
+      }
+    } else if ((MODE == kCount || MODE == kAll) && K >= 4) {
       // Narrowest register width that holds this root's rows.
       constexpr bool ALL = MODE == kAll;
       // One instantiation per word count: the k = 5 loop reads MAXW words
@@ -634,6 +953,11 @@ __global__ __launch_bounds__(BS) void clique_block_kernel(
     }
     __syncthreads();
   }
+  if (kCount5 && lane_id() == 0) {
+    acc = s_tot[threadIdx.x / kWave][0];
+    acc3 = s_tot[threadIdx.x / kWave][1];
+    acc4 = s_tot[threadIdx.x / kWave][2];
+  }
   if (MODE == kAll) {
     acc3 = wave_sum_u64(acc3);
     acc4 = wave_sum_u64(acc4);
@@ -654,16 +978,13 @@ __global__ void zero_u32_kernel(unsigned int* p, int count) {
   if (i < count) p[i] = 0u;
 }
 
-// LDS hash slots for a tier of this cap (a power of two, >= 2 cap).
-uint32_t table_for(uint32_t cap) {
-  uint32_t table = 1;
-  while (table < 2 * cap) table <<= 1;
-  return table;
-}
-
-size_t block_lds_bytes(uint32_t cap, uint32_t table, bool pad) {
+// Dynamic LDS of a block of `waves` waves: rows and an empty row; then S with
+// its list bounds and the bitmap of S with its prefixes, whose place the k = 5
+// count's position lists take over.
+size_t block_lds_bytes(uint32_t cap, uint32_t waves, bool pad) {
   const uint32_t W = (cap + 63) / 64;
-  return (size_t)cap * (pad ? (W | 1u) : W) * 8 + (size_t)cap * 8 + (size_t)table * 8;
+  return (size_t)(cap + 1) * (pad ? (W | 1u) : W) * 8 +
+         std::max<size_t>((size_t)cap * 12 + kIdWords * 6, (size_t)waves * (cap + kWave) * 2);
 }
 
 // Largest out-degree whose rows fit one block's LDS on this device (at most
@@ -678,7 +999,7 @@ uint32_t lds_wide_cap() {
       limit = prop.sharedMemPerBlock;
     uint32_t cap = kBlockCap;
     for (uint32_t c = 1024; c > kBlockCap; c -= 64) {
-      if (block_lds_bytes(c, table_for(c), false) + 4096 <= limit) {
+      if (block_lds_bytes(c, kWideBlock / kWave, false) + 4096 <= limit) {
         cap = c;
         break;
       }
@@ -691,7 +1012,7 @@ uint32_t lds_wide_cap() {
 // Blocks of an LDS-rows tier of this cap resident per CU: limited by LDS
 // (160 KiB per CU) and by 32 waves per CU.
 int lds_blocks_per_cu(uint32_t cap, int block_threads, bool pad) {
-  const size_t lds = block_lds_bytes(cap, table_for(cap), pad);
+  const size_t lds = block_lds_bytes(cap, block_threads / kWave, pad);
   const int by_waves = std::max(1, 32 / (block_threads / kWave));
   return std::min(by_waves, std::max<int>(1, (int)(160 * 1024 / (lds + 2048))));
 }
@@ -703,16 +1024,15 @@ int launch_lds_tier(gpm_graph* g, hipStream_t stream, const uint32_t* roots,
                     unsigned int* queue, unsigned long long* out, unsigned long long* work,
                     const char* name) {
   const int cus = device_cus(g);
-  const uint32_t table = table_for(cap);
-  const size_t lds = block_lds_bytes(cap, table, MAXW == 8);
+  const size_t lds = block_lds_bytes(cap, BS / kWave, MAXW == 8);
   auto kern = clique_block_kernel<K, MODE, true, MAXW, BS>;
   if (lds > 48 * 1024)
     GPM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   const unsigned blocks =
       (unsigned)std::min<uint64_t>(n_roots, (uint64_t)cus * lds_blocks_per_cu(cap, BS, MAXW == 8));
-  hipLaunchKernelGGL(kern, dim3(blocks), dim3(BS), lds, stream, g->toff, g->tadj, roots,
-                     parts, n_roots, cap, table, queue, nullptr, nullptr, out, work);
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(BS), lds, stream, g->toff, g->tadj, g->n,
+                     roots, parts, n_roots, cap, queue, nullptr, nullptr, out, work);
   GPM_HIP(hipGetLastError());
   if ((MODE == kCount || MODE == kAll) && stream == g->stream) timing_mark(g, name);
   return GPM_OK;
@@ -756,8 +1076,8 @@ int launch_tiers(gpm_graph* g, const RootTiers* t, unsigned long long* out,
     unsigned long long* grows = static_cast<unsigned long long*>(g->scratch);
     uint32_t* gmeta = reinterpret_cast<uint32_t*>(static_cast<char*>(g->scratch) + row_bytes);
     hipLaunchKernelGGL((clique_block_kernel<K, MODE, false, 0, kHbmBlock>), dim3(blocks),
-                       dim3(kHbmBlock), 0, g->stream, g->toff, g->tadj, t->d_big, t->d_big_parts,
-                       t->n_big, cap, 0u, q + 2, grows, gmeta, out, work);
+                       dim3(kHbmBlock), 0, g->stream, g->toff, g->tadj, g->n, t->d_big,
+                       t->d_big_parts, t->n_big, cap, q + 2, grows, gmeta, out, work);
     GPM_HIP(hipGetLastError());
     if (MODE == kCount || MODE == kAll) timing_mark(g, "clique_hbm_block");
   }
