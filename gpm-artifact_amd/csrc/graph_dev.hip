@@ -243,6 +243,7 @@ void release(gpm_graph* g) {
   (void)hipFree(g->toff);
   (void)hipFree(g->tadj);
   (void)hipFree(g->bmask);
+  (void)hipFree(g->nbits);
   hipFree(g->scratch);
   hipFree(g->counters);
   (void)hipFree(g->tc_partial);

@@ -1,6 +1,10 @@
 // Fixed-pattern counting on a symmetric graph (replaces G2MinerSolver and
 // PatternSolver, src/G2MinerSolver.cuh and src/PatternSolver.cuh).
 //
+// The kernels here work on sorted lists.  Graphs of up to 16384 vertices whose
+// lists are not short are counted on adjacency bit matrices instead
+// (pattern_bits.hip), with the same results.
+//
 // Direct formulation (GPM_FORM_G2MINER): one wave per directed edge
 // (v0, v1), fetched from a work queue in chunks; the nested set operations
 // of src/gpu_kernels/G2Miner_kernels.cuh run as wave64 filters (setops.hpp)
@@ -544,15 +548,20 @@ extern "C" int gpm_pattern(gpm_graph* g, int pattern_id, int formulation, uint64
       else
         h[0] = pattern_id == GPM_P1 ? m4[0] : m4[1];
     } else {
+      // The matrix path counts the same pairs whether a block mask would have
+      // ruled them out or not.
+      bool bits = false;
+      if ((st = prepare_pattern_bits(g, &bits)) != GPM_OK) return st;
       BlockMask blk{nullptr, 0};
-      if (prefilter) {
+      if (prefilter && !bits) {
         if ((st = ensure_block_mask(g)) != GPM_OK) return st;
         blk = BlockMask{g->bmask, g->bmask_shift};
       }
       if ((st = timing_begin(g)) != GPM_OK) return st;
-      if ((st = zero_counters(g, 8)) != GPM_OK) return st;
-      st = counting ? launch_pid<GPM_FORM_PATTERN>(g, pattern_id, blk, g->counters)
-                    : launch_pid<GPM_FORM_G2MINER>(g, pattern_id, blk, g->counters);
+      if ((st = zero_counters(g, 16)) != GPM_OK) return st;
+      st = bits ? launch_pattern_bits(g, pattern_id, counting, g->counters + 8, g->counters)
+           : counting ? launch_pid<GPM_FORM_PATTERN>(g, pattern_id, blk, g->counters)
+                      : launch_pid<GPM_FORM_G2MINER>(g, pattern_id, blk, g->counters);
       if (st != GPM_OK) return st;
       if ((st = timing_end(g)) != GPM_OK) return st;
       unsigned long long hh[6];

@@ -1,0 +1,499 @@
+// Fixed patterns on the adjacency bit matrix (both formulations of
+// gpm_pattern, see pattern.hip for what each counts).
+//
+// The nested set operations of the patterns walk sets of vertices and, for
+// each, intersect or subtract its neighbours from another set.  As lists those
+// are a binary search per entry; here sets and neighbourhoods are rows of bits,
+// and the two inner loops of a pattern become one masked product per edge:
+//     sum over a in R1, b in R2 with Q(a, b) of |C & X[a] & Y[b]|
+// with X, Y one of the matrices below.  16 x 16 pairs (a, b) and 128 columns
+// are one FP4 matrix instruction (fp4_bits.hpp).  Q is always "b is in X[a]" or
+// its opposite, so it is the product of the same rows of a with the unit
+// vectors of b, and lands in the lanes that hold the sizes.
+//
+//   D01 = N(v0) \ N(v1), D10 = N(v1) \ N(v0), I = N(v0) & N(v1)
+//         R1   R2   C    X    direct: Y, Q       counting: Y, Q
+//   P2    D10  D01  D01  !N   below, !N   in     above, !N   not in
+//   P3    D01  D01  D01  below, !N  below, !N in  above, !N  not in
+//   P5    I    D01  D10  !N   !N          in     the same
+//   P6    I    I    D10  !N   !N          in     the same
+//   P7    I    I    I    below, !N  below, !N in  above, !N  not in
+//   P8    D10  I    I    !N   below, N    in     above, N    not in
+// (the opposite: an a and b that are adjacent; where X and Y leave no column
+// between them the size is 0 whatever Q says).  P1, P4 and the direct Motif4
+// have one inner loop: |C & X[a]| summed over a.
+//
+// A row has n / 128 chunks to multiply, whatever the lists' lengths, so this
+// path is for graphs of at most kBitsMaxN vertices and not for sparse large
+// ones (bits_pay).
+#include <algorithm>
+#include <cmath>
+
+#include "fp4_bits.hpp"
+#include "graph_dev.hpp"
+
+using namespace gpm;
+
+namespace {
+
+constexpr int kBlock = 256;
+constexpr int kWaves = kBlock / kWave;
+constexpr uint32_t kBitsMaxN = 16384;
+// A segment: the 2048 ids whose bits are one word per lane.
+constexpr uint32_t kSegWords = kWave, kSegIds = 32 * kSegWords;
+// Entries of a list: a segment's ids, filled up with the empty row's index.
+constexpr uint32_t kListLen = kSegIds + kWave;
+enum Matrix { kN, kNotN, kBelowNotN, kAboveNotN, kBelowN, kAboveN, kMatrices };
+
+struct Bits {
+  const uint32_t* base;  // kMatrices matrices of n + 1 rows of rw words; row n is empty
+  uint32_t n, rw;
+  __device__ const uint32_t* row(int matrix, uint32_t v) const {
+    return base + ((size_t)matrix * (n + 1) + v) * rw;
+  }
+};
+
+// Bits of word w below / above id v.
+__device__ __forceinline__ uint32_t bits_below(uint32_t w, uint32_t v) {
+  return w < v / 32 ? 0xFFFFFFFFu : w == v / 32 ? (1u << (v & 31)) - 1u : 0u;
+}
+__device__ __forceinline__ uint32_t bits_above(uint32_t w, uint32_t v) {
+  return w > v / 32 ? 0xFFFFFFFFu : w == v / 32 ? ~((2u << (v & 31)) - 1u) : 0u;
+}
+
+// ------------------------------------------------------------- the matrices
+
+// Sets the neighbour bits of every vertex (N zeroed before); one wave per v.
+__global__ __launch_bounds__(kBlock) void neighbour_bits_kernel(const uint32_t* __restrict__ off,
+                                                                const uint32_t* __restrict__ adj,
+                                                                uint32_t n, uint32_t rw,
+                                                                uint32_t* __restrict__ bits) {
+  const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
+  const uint32_t nwaves = gridDim.x * blockDim.x / kWave;
+  for (uint32_t v = wave; v < n; v += nwaves)
+    for (uint32_t i = off[v] + lane_id(); i < off[v + 1]; i += kWave)
+      atomicOr(&bits[(size_t)v * rw + adj[i] / 32], 1u << (adj[i] & 31));
+}
+
+__global__ __launch_bounds__(kBlock) void zero_words_kernel(uint32_t* p, uint64_t count) {
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count;
+       i += (uint64_t)gridDim.x * blockDim.x)
+    p[i] = 0u;
+}
+
+// The other matrices from N, and the number of bits of N.
+__global__ __launch_bounds__(kBlock) void derived_bits_kernel(uint32_t* __restrict__ base,
+                                                              uint32_t n, uint32_t rw,
+                                                              unsigned long long* __restrict__ total) {
+  const uint64_t words = (uint64_t)(n + 1) * rw;
+  uint64_t set = 0;
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < words;
+       i += (uint64_t)gridDim.x * blockDim.x) {
+    const uint32_t v = (uint32_t)(i / rw), w = (uint32_t)(i % rw);
+    const uint32_t m = base[i];
+    const uint32_t ids = v < n ? bits_below(w, n) : 0u;  // row n stays empty
+    const uint32_t lo = ids & bits_below(w, v), hi = ids & bits_above(w, v);
+    base[kNotN * words + i] = ~m & ids;
+    base[kBelowNotN * words + i] = ~m & lo;
+    base[kAboveNotN * words + i] = ~m & hi;
+    base[kBelowN * words + i] = m & lo;
+    base[kAboveN * words + i] = m & hi;
+    set += (uint32_t)__popc(m);
+  }
+  set = wave_sum_u64(set);
+  if (lane_id() == 0 && set) atomicAdd(total, (unsigned long long)set);
+}
+
+// ---------------------------------------------------------------- the count
+
+// The set bits of a segment (one word per lane) as ascending ids into list,
+// filled up with `none` to a multiple of 64; returns how many there are.
+__device__ __forceinline__ uint32_t list_bits(uint32_t word, uint32_t seg, uint32_t none,
+                                              uint16_t* list) {
+  const uint32_t incl = wave_incl_scan((uint32_t)__popc(word));
+  const uint32_t total = uniform(wave_bcast(incl, kWave - 1));
+  uint32_t at = incl - (uint32_t)__popc(word);
+  const uint32_t id0 = seg * kSegIds + 32 * lane_id();
+  __builtin_amdgcn_wave_barrier();
+  for (; word; word &= word - 1) list[at++] = (uint16_t)(id0 + __builtin_ctz(word));
+  list[total + lane_id()] = (uint16_t)none;
+  __builtin_amdgcn_wave_barrier();
+  return total;
+}
+
+struct Product {
+  const uint32_t *x, *y;   // matrices of a's and b's rows
+  const uint32_t *ca, *cb; // column sets of X[a] (with R2's ids for Q) and of Y[b], in LDS
+  uint32_t rw, chunks;
+  bool in;                 // Q: b in X[a], or not
+};
+
+// Blocks ja .. ja + J - 1 of R1 (list a) against blocks lb .. lb + L - 1 of R2.
+// The sizes of all J x L tiles accumulate over the chunks; the adjacency of one
+// block of b at a time then masks its column of tiles.  A lane's sum stays
+// below 2^24: 4 J L sizes of at most kBitsMaxN.
+template <int J, int L>
+__device__ __forceinline__ uint32_t product_tiles(const Product& p, const uint16_t* a,
+                                                  const uint16_t* b, uint32_t ja, uint32_t lb) {
+  static_assert(4ull * J * L * kBitsMaxN < (1ull << 24), "sums must be exact");
+  const uint32_t lane = lane_id(), r16 = lane & 15, g = lane >> 4;
+  uint32_t ra[J], rb[L], ib[L];
+#pragma unroll
+  for (int q = 0; q < J; ++q) ra[q] = a[16 * (ja + q) + r16] * p.rw + g;
+#pragma unroll
+  for (int q = 0; q < L; ++q) {
+    ib[q] = b[16 * (lb + q) + r16];
+    rb[q] = ib[q] * p.rw + g;
+  }
+  floatx4 both[J][L];
+#pragma unroll
+  for (int q = 0; q < J; ++q)
+#pragma unroll
+    for (int t = 0; t < L; ++t) both[q][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (uint32_t c = 0; c < p.chunks; ++c) {
+    const uint32_t ca = p.ca[4 * c + g], cb = p.cb[4 * c + g];
+    if (wave_ballot(cb != 0u) == 0ull) continue;
+    uint32_t wa[J], wb[L];
+#pragma unroll
+    for (int q = 0; q < J; ++q) wa[q] = p.x[ra[q] + 4 * c];
+#pragma unroll
+    for (int t = 0; t < L; ++t) wb[t] = p.y[rb[t] + 4 * c];
+    intx4 fb[L];
+#pragma unroll
+    for (int t = 0; t < L; ++t) fb[t] = fp4_in_place(wb[t] & cb);
+#pragma unroll
+    for (int q = 0; q < J; ++q) {
+      const intx4 fa = fp4_reciprocal(wa[q] & ca);
+#pragma unroll
+      for (int t = 0; t < L; ++t) both[q][t] = mfma_fp4(fa, fb[t], both[q][t]);
+    }
+  }
+  float sum = 0.f;
+#pragma unroll
+  for (int t = 0; t < L; ++t) {
+    floatx4 adj[J];
+#pragma unroll
+    for (int q = 0; q < J; ++q) adj[q] = floatx4{0.f, 0.f, 0.f, 0.f};
+    // b's ascend, the empty row (index n) last: it has no column.
+    const uint32_t first = uniform(ib[t]) / 128;
+    const uint32_t last = min(__builtin_amdgcn_readlane(ib[t], 15) / 128, p.chunks - 1);
+    for (uint32_t c = first; c <= last; ++c) {
+      const uint32_t ca = p.ca[4 * c + g];
+      const intx4 e = fp4_in_place(ib[t] / 32 == 4 * c + g ? 1u << (ib[t] & 31) : 0u);
+#pragma unroll
+      for (int q = 0; q < J; ++q) adj[q] = mfma_fp4(fp4_reciprocal(p.x[ra[q] + 4 * c] & ca), e, adj[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < J; ++q)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        sum = __builtin_fmaf(both[q][t][r], p.in ? adj[q][r] : 1.f - adj[q][r], sum);
+  }
+  return (uint32_t)sum;
+}
+
+// Every pair of the lists a (na entries) and b (nb); triangular: only pairs with
+// b's block up to a's count (lists of one set, X or Y leave nothing beyond).
+__device__ __forceinline__ uint64_t product(const Product& p, const uint16_t* a, uint32_t na,
+                                            const uint16_t* b, uint32_t nb, bool triangular) {
+  const uint32_t ta = (na + 15) / 16, tb = (nb + 15) / 16;
+  uint64_t sum = 0;
+  uint32_t ja = 0;
+  while (ja < ta) {
+    const uint32_t left = ta - ja, step = left >= 3 ? 4 : left;
+    const uint32_t end = triangular ? min(tb, ja + step) : tb;
+    for (uint32_t lb = 0; lb < end; lb += 4) {
+      if (step == 4)
+        sum += end - lb == 1 ? product_tiles<4, 1>(p, a, b, ja, lb) : product_tiles<4, 4>(p, a, b, ja, lb);
+      else if (step == 2)
+        sum += end - lb == 1 ? product_tiles<2, 1>(p, a, b, ja, lb) : product_tiles<2, 4>(p, a, b, ja, lb);
+      else
+        sum += end - lb == 1 ? product_tiles<1, 1>(p, a, b, ja, lb) : product_tiles<1, 4>(p, a, b, ja, lb);
+    }
+    ja += step;
+  }
+  return sum;
+}
+
+// sum over the ids v of the list of |C & X[v]|, this lane's share; the set in
+// LDS, four rows at a time.
+__device__ __forceinline__ uint64_t sum_rows(const uint32_t* x, const uint32_t* set, uint32_t rw,
+                                             uint32_t words, const uint16_t* list, uint32_t n) {
+  uint64_t sum = 0;
+  for (uint32_t t = 0; t < n; t += 4) {
+    // The list is filled up with the empty row.
+    const uint32_t* r0 = x + uniform(list[t]) * (size_t)rw;
+    const uint32_t* r1 = x + uniform(list[t + 1]) * (size_t)rw;
+    const uint32_t* r2 = x + uniform(list[t + 2]) * (size_t)rw;
+    const uint32_t* r3 = x + uniform(list[t + 3]) * (size_t)rw;
+    uint32_t c = 0;
+    for (uint32_t w = lane_id(); w < words; w += kWave) {
+      const uint32_t s = set[w];
+      c += (uint32_t)__popc(r0[w] & s) + (uint32_t)__popc(r1[w] & s) +
+           (uint32_t)__popc(r2[w] & s) + (uint32_t)__popc(r3[w] & s);
+    }
+    sum += c;
+  }
+  return sum;
+}
+
+// sum over the ids v of the list of |S & X[v]| |T & Y[v]| (one lane's share):
+// the two sizes are summed over the wave in the halves of one word.
+__device__ __forceinline__ uint64_t sum_products(const uint32_t* x, const uint32_t* s,
+                                                 const uint32_t* y, const uint32_t* t, uint32_t rw,
+                                                 uint32_t words, const uint16_t* list, uint32_t n) {
+  static_assert(kBitsMaxN < (1u << 16), "two sizes in a word");
+  uint64_t sum = 0;
+  for (uint32_t k = 0; k < n; k += 4) {
+    uint32_t c[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const size_t r = uniform(list[k + q]) * (size_t)rw;
+      c[q] = 0;
+      for (uint32_t w = lane_id(); w < words; w += kWave)
+        c[q] += (uint32_t)__popc(x[r + w] & s[w]) | (uint32_t)__popc(y[r + w] & t[w]) << 16;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) c[q] = wave_sum_u32(c[q]);
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (lane_id() == (uint32_t)q) sum += (uint64_t)(c[q] & 0xFFFFu) * (c[q] >> 16);
+  }
+  return sum;
+}
+
+// One wave per directed edge, in chunks from a queue.  LDS per wave: two lists
+// and two sets of rw words.  PRODUCTS: P2, P3, P5 - P8 (16 tiles of sizes and
+// their operands: 210 registers, 2 waves per SIMD; bounds that make it spill are
+// not safe, as matrix instructions read every lane's register); otherwise P1,
+// P4 and Motif4.  R-MAT, 16 edges a vertex, all of P1 - P8 and Motif4: n = 512
+// direct 362 ms on lists, 1.7 ms here; n = 2048 counting 982 ms, 13.8 ms, half
+// of it P3 (3.2 M blocks of 16 x 16 pairs, 16 chunks each): latency of the row
+// loads bounds it, at two waves per SIMD.
+template <bool PRODUCTS>
+__global__ __launch_bounds__(kBlock, PRODUCTS ? 2 : 4) void pattern_bits_kernel(
+    const uint32_t* __restrict__ adj, const uint32_t* __restrict__ src, uint64_t m, Bits g,
+    int pid, bool counting, uint32_t chunk, unsigned long long* __restrict__ queue,
+    unsigned long long* __restrict__ out) {
+  extern __shared__ uint32_t s_words[];
+  const uint32_t lane = lane_id(), wave = threadIdx.x / kWave;
+  const uint32_t per_wave = 2 * g.rw + kListLen;  // words: two sets, two lists of halves
+  uint32_t* s0 = s_words + wave * per_wave;
+  uint32_t* s1 = s0 + g.rw;
+  uint16_t* l0 = reinterpret_cast<uint16_t*>(s1 + g.rw);
+  uint16_t* l1 = l0 + kListLen;
+  const uint32_t segs = g.rw / kSegWords, words = (g.n + 31) / 32, chunks = (g.n + 127) / 128;
+  const uint32_t none = g.n;
+  uint64_t c[6] = {0, 0, 0, 0, 0, 0};
+  while (true) {
+    unsigned long long base = 0;
+    if (lane == 0) base = atomicAdd(queue, (unsigned long long)chunk);
+    base = __shfl(base, 0, kWave);
+    if (base >= m) break;
+    const uint64_t stop = min((unsigned long long)m, base + chunk);
+    for (uint64_t e = base; e < stop; ++e) {
+      const uint32_t v0 = uniform(src[e]), v1 = uniform(adj[e]);
+      if (v0 == v1 || (pid == 4 && v1 >= v0)) continue;
+      const uint32_t *n0 = g.row(kN, v0), *n1 = g.row(kN, v1);
+      // Word w of the sets of the edge.
+      auto d01 = [&](uint32_t w) { return n0[w] & ~n1[w]; };
+      auto d10 = [&](uint32_t w) { return n1[w] & ~n0[w]; };
+      auto both = [&](uint32_t w) { return n0[w] & n1[w]; };
+      auto fill = [&](uint32_t* set, auto f) {
+        __builtin_amdgcn_wave_barrier();
+        for (uint32_t w = lane; w < g.rw; w += kWave) set[w] = f(w);
+        __builtin_amdgcn_wave_barrier();
+      };
+      // sum over a in R of |set & X[a]|
+      auto sums = [&](auto r, int x, const uint32_t* set) {
+        uint64_t t = 0;
+        for (uint32_t k = 0; k < segs; ++k) {
+          const uint32_t na = list_bits(r(k * kSegWords + lane), k, none, l0);
+          t += sum_rows(g.row(x, 0), set, g.rw, words, l0, na);
+        }
+        return t;
+      };
+      if (!PRODUCTS && pid == 1) {
+        auto r = [&](uint32_t w) { return d01(w) & bits_below(w, v1); };
+        fill(s0, r);
+        c[0] += sums(r, kBelowNotN, s0);
+      } else if (!PRODUCTS && pid == 4) {
+        fill(s0, d10);
+        const uint64_t t = sums(d01, kNotN, s0);
+        (counting ? c[1] : c[0]) += t;
+      } else if (!PRODUCTS) {
+        auto star = [&](uint32_t w) { return d01(w) & bits_below(w, v1); };
+        fill(s0, star);
+        c[0] += sums(star, kBelowNotN, s0);
+        if (v1 > v0) continue;
+        fill(s0, both);
+        fill(s1, [&](uint32_t w) { return ~n0[w] & ~n1[w]; });
+        c[4] += sums(both, kBelowNotN, s0);
+        c[2] += sums(both, kN, s1);
+        auto top = [&](uint32_t w) { return both(w) & bits_below(w, v1); };
+        fill(s0, top);
+        c[5] += sums(top, kBelowN, s0);
+        fill(s0, d10);
+        c[1] += sums(d01, kNotN, s0);
+        fill(s0, [&](uint32_t w) { return d10(w) & bits_below(w, v0); });
+        c[3] += sums([&](uint32_t w) { return d01(w) & bits_below(w, v1); }, kN, s0);
+      } else {
+        const bool wedge = pid == 3 || pid == 7, pairs = pid == 5 || pid == 6;
+        const bool i1 = pairs || pid == 7, i2 = pid >= 6;
+        auto r1 = [&](uint32_t w) { return i1 ? both(w) : wedge ? d01(w) : d10(w); };
+        auto r2 = [&](uint32_t w) { return i2 ? both(w) : d01(w); };
+        // Edges without a common neighbour, or whose ends share all of them,
+        // often have nothing to count.
+        uint32_t any1 = 0, any2 = 0;
+        for (uint32_t w = lane; w < g.rw; w += kWave) {
+          any1 |= r1(w);
+          any2 |= r2(w);
+        }
+        if (wave_ballot(any2 != 0u) == 0ull) continue;
+        if (wave_ballot(any1 != 0u) == 0ull && (!counting || pairs)) continue;
+        if (pairs) {
+          fill(s0, [&](uint32_t w) { return r2(w) | d10(w); });
+          fill(s1, d10);
+        } else {
+          fill(s0, r2);
+        }
+        Product p;
+        p.x = g.row(wedge ? kBelowNotN : kNotN, 0);
+        p.y = g.row(pairs ? kNotN
+                    : pid == 8 ? (counting ? kAboveN : kBelowN)
+                               : (counting ? kAboveNotN : kBelowNotN), 0);
+        p.ca = s0;
+        p.cb = pairs ? s1 : s0;
+        p.rw = g.rw;
+        p.chunks = chunks;
+        p.in = pairs || !counting;
+        uint64_t t = 0;
+        for (uint32_t k = 0; k < segs; ++k) {
+          const uint32_t na = list_bits(r1(k * kSegWords + lane), k, none, l0);
+          if (!na) continue;
+          for (uint32_t k2 = 0; k2 < (wedge ? k + 1 : segs); ++k2) {
+            const uint32_t nb = list_bits(r2(k2 * kSegWords + lane), k2, none, l1);
+            if (nb) t += product(p, l0, na, l1, nb, wedge && k2 == k);
+          }
+        }
+        if (!counting) {
+          c[0] += t;
+        } else if (pairs) {
+          c[1] += t;
+        } else {
+          c[2] += t;
+          // Frequency times count per v in R2 (s0): P2, P8: non-neighbours in
+          // D10 times the entries of R2 below v; P3, P7: non-neighbours in R2
+          // below times above.
+          if (!wedge) fill(s1, d10);
+          const uint32_t* x = g.row(wedge ? kAboveNotN : kNotN, 0);
+          const uint32_t* y = g.row(pid == 8 ? kBelowN : kBelowNotN, 0);
+          for (uint32_t k = 0; k < segs; ++k) {
+            const uint32_t nb = list_bits(r2(k * kSegWords + lane), k, none, l1);
+            c[1] += sum_products(x, wedge ? s0 : s1, y, s0, g.rw, words, l1, nb);
+          }
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < (PRODUCTS ? 3 : 6); ++i) {
+    c[i] = wave_sum_u64(c[i]);
+    if (lane == 0 && c[i]) atomicAdd(&out[i], (unsigned long long)c[i]);
+  }
+}
+
+unsigned grid_of(const gpm_graph* g, uint64_t threads) {
+  return (unsigned)std::max<uint64_t>(
+      1, std::min<uint64_t>((threads + kBlock - 1) / kBlock, (uint64_t)device_cus(g) * 16));
+}
+
+// Whether the matrix path is the faster one.  It costs every edge n / 2048
+// segments of set work and every 16 x 16 pairs n / 128 chunks; lists cost an edge
+// the pairs of its sets, each at least a window and a search.  So it is taken
+// up to one segment, and beyond where the degree an edge meets, dw = sum d^2 /
+// sum d, is large.  P2, P3, P6, P8 (both formulations) and P4, ms in all, matrix
+// against lists: Erdos-Renyi n = 1500, dw = 17: 2.0 against 6.7; n = 4096, dw = 9:
+// 3.8, 3.7; dw = 17: 8.4, 13; n = 16384, dw = 17: 532, 44; R-MAT n = 1500, dw = 48:
+// 2.0, 143; n = 8192, dw = 63: 30, 881; n = 16384, dw = 83: 226, 2994.
+bool bits_pay(const gpm_graph* g) {
+  if (g->n > kBitsMaxN || !g->m) return false;
+  if (g->n <= kSegIds) return true;
+  double d2 = 0.0;
+  for (uint32_t v = 0; v < g->n; ++v) {
+    const double d = g->h_off[v + 1] - g->h_off[v];
+    d2 += d * d;
+  }
+  return d2 / (double)g->m >= 16.0 * std::sqrt((double)g->n / kSegIds);
+}
+
+// Builds g->nbits if missing; *ok is false where the lists hold an entry twice
+// (a bit cannot) or the matrices do not fit.
+int ensure_bits(gpm_graph* g, bool* ok) {
+  *ok = g->nbits != nullptr;
+  if (g->nbits || g->nbits_off) return GPM_OK;
+  const uint32_t rw = (g->n + kSegIds - 1) / kSegIds * kSegWords;
+  const uint64_t words = (uint64_t)(g->n + 1) * rw;
+  uint32_t* bits = nullptr;
+  if (hipMalloc(&bits, kMatrices * words * 4) != hipSuccess) {
+    (void)hipGetLastError();
+    g->nbits_off = true;
+    return GPM_OK;
+  }
+  unsigned long long set = 0;
+  int st = zero_counters(g, 1);
+  if (st == GPM_OK) {
+    hipLaunchKernelGGL(zero_words_kernel, dim3(grid_of(g, words)), dim3(kBlock), 0, g->stream, bits,
+                       words);
+    hipLaunchKernelGGL(neighbour_bits_kernel, dim3(grid_of(g, (uint64_t)g->n * kWave)), dim3(kBlock),
+                       0, g->stream, g->off, g->adj, g->n, rw, bits);
+    hipLaunchKernelGGL(derived_bits_kernel, dim3(grid_of(g, words)), dim3(kBlock), 0, g->stream,
+                       bits, g->n, rw, g->counters);
+    if (hipGetLastError() != hipSuccess ||
+        hipMemcpyAsync(&set, g->counters, sizeof(set), hipMemcpyDeviceToHost, g->stream) !=
+            hipSuccess ||
+        hipStreamSynchronize(g->stream) != hipSuccess)
+      st = fail(GPM_EHIP, "adjacency bit matrices");
+  }
+  if (st != GPM_OK || set != g->m) {
+    (void)hipStreamSynchronize(g->stream);
+    (void)hipFree(bits);
+    g->nbits_off = st == GPM_OK;
+    return st;
+  }
+  g->nbits = bits;
+  *ok = true;
+  return GPM_OK;
+}
+
+}  // namespace
+
+namespace gpm {
+
+int prepare_pattern_bits(gpm_graph* g, bool* ok) {
+  *ok = false;
+  if (!bits_pay(g)) return GPM_OK;
+  const int st = ensure_bits(g, ok);
+  return st != GPM_OK || !*ok ? st : ensure_src(g);
+}
+
+int launch_pattern_bits(gpm_graph* g, int pid, bool counting, unsigned long long* queue,
+                        unsigned long long* out) {
+  Bits b;
+  b.base = g->nbits;
+  b.n = g->n;
+  b.rw = (g->n + kSegIds - 1) / kSegIds * kSegWords;
+  const size_t lds = (size_t)kWaves * (2 * b.rw + kListLen) * 4;
+  const unsigned per_cu = (unsigned)std::min<size_t>(3, 160 * 1024 / (lds + 1024));
+  const uint32_t chunk = 2;
+  const unsigned blocks = (unsigned)std::min<uint64_t>(
+      (g->m + (uint64_t)chunk * kWaves - 1) / (chunk * kWaves), (uint64_t)device_cus(g) * per_cu);
+  const bool products = pid != GPM_P1 && pid != GPM_P4 && pid != GPM_MOTIF4;
+  hipLaunchKernelGGL(products ? pattern_bits_kernel<true> : pattern_bits_kernel<false>, dim3(blocks), dim3(kBlock), lds, g->stream, g->adj,
+                     g->src, g->m, b, pid, counting, chunk, queue, out);
+  GPM_HIP(hipGetLastError());
+  timing_mark(g, counting ? "pattern_counting" : "pattern_direct");
+  return GPM_OK;
+}
+
+}  // namespace gpm
