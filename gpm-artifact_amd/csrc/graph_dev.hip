@@ -95,6 +95,18 @@ int device_cus(const gpm_graph* g) {
   return cached_cus;
 }
 
+double mean_met_degree(gpm_graph* g) {
+  if (g->met_degree < 0.0) {
+    double d2 = 0.0;
+    for (uint32_t v = 0; v < g->n; ++v) {
+      const double d = g->h_off[v + 1] - g->h_off[v];
+      d2 += d * d;
+    }
+    g->met_degree = g->m ? d2 / (double)g->m : 0.0;
+  }
+  return g->met_degree;
+}
+
 int h2d(gpm_graph* g, void* dst, const void* src, size_t bytes) {
   if (!bytes) return GPM_OK;
   GPM_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, g->stream));
@@ -102,29 +114,37 @@ int h2d(gpm_graph* g, void* dst, const void* src, size_t bytes) {
   return GPM_OK;
 }
 
-int ensure_topo(gpm_graph* g) {
-  if (g->toff) return GPM_OK;
-  // The order by (out + in degree, id) costs a few radix sort passes on the
-  // device; it is topological for every degree-oriented graph.  Other DAGs,
-  // and graphs whose sort buffers do not fit, take Kahn's algorithm on the
-  // host.  R-MAT scale 20 (15.7 M edges): what the first clique count of a
-  // handle takes beyond a later one fell from 136 ms to 25 ms.
-  {
-    uint32_t *doff = nullptr, *dadj = nullptr;
-    std::vector<uint32_t> drank;
-    bool ordered = false;
-    const int st = topo_relabel_device(g, &doff, &dadj, &drank, &ordered);
-    if (st != GPM_OK && st != GPM_ENOMEM) return st;
-    if (st == GPM_ENOMEM) {
-      (void)hipGetLastError();
-      clear_error();
-    } else if (ordered) {
-      g->toff = doff;
-      g->tadj = dadj;
-      g->h_rank.swap(drank);
-      return GPM_OK;
-    }
+// The order by (out + in degree, id) costs a few radix sort passes on the
+// device; it is topological for every degree-oriented graph.  R-MAT scale 20
+// (15.7 M edges): what the first clique count of a handle takes beyond a later
+// one fell from 136 ms to 25 ms.
+int try_topo(gpm_graph* g) {
+  if (g->toff || g->unranked) return GPM_OK;
+  uint32_t *toff = nullptr, *tadj = nullptr;
+  std::vector<uint32_t> rank;
+  bool ordered = false;
+  const int st = topo_relabel_device(g, &toff, &tadj, &rank, &ordered);
+  if (st == GPM_ENOMEM) {
+    (void)hipGetLastError();
+    clear_error();
+    return GPM_OK;
   }
+  if (st != GPM_OK) return st;
+  if (!ordered) {
+    g->unranked = true;
+    return GPM_OK;
+  }
+  g->toff = toff;
+  g->tadj = tadj;
+  g->h_rank.swap(rank);
+  return GPM_OK;
+}
+
+int ensure_topo(gpm_graph* g) {
+  const int ranked = try_topo(g);
+  if (ranked != GPM_OK || g->toff) return ranked;
+  // Other DAGs, and graphs whose sort buffers do not fit: Kahn's algorithm on
+  // the host.
   std::vector<uint32_t> h_adj(std::max<uint64_t>(g->m, 1));
   if (g->m) {
     GPM_HIP(hipMemcpyAsync(h_adj.data(), g->adj, g->m * 4, hipMemcpyDeviceToHost, g->stream));

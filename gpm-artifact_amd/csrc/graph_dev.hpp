@@ -41,6 +41,7 @@ struct gpm_graph {
   // when L > 1024.  Feeds the matcher's cost estimates.
   std::vector<double> h_lpair;
   std::vector<uint32_t> h_off;
+  double met_degree = -1.0;  // see mean_met_degree
   std::vector<uint32_t> h_labels;
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -80,6 +81,7 @@ struct gpm_graph {
   // ids), else in the order of Kahn's algorithm.
   uint32_t* toff = nullptr;
   uint32_t* tadj = nullptr;
+  bool unranked = false;  // total degree gives no topological order
   std::vector<uint32_t> h_rank;
   // SYMMETRIC graphs: block mask of the counting formulation's prefilter,
   // bmask[v] bit b set when v has a neighbour w with (w >> bmask_shift) == b,
@@ -112,10 +114,15 @@ int timing_begin(gpm_graph* g);
 // Records an event after the kernel just launched; `name` must be static.
 int timing_mark(gpm_graph* g, const char* name);
 int timing_end(gpm_graph* g);
+// Mean list length an adjacency entry meets, sum d^2 / sum d (kept on the handle).
+double mean_met_degree(gpm_graph* g);
 // Number of compute units of the handle's device.
 int device_cus(const gpm_graph* g);
 // Builds g->toff/tadj/h_rank if missing; GPM_EINVAL if the graph has a cycle.
 int ensure_topo(gpm_graph* g);
+// The same where the order by total degree is topological; otherwise (and where
+// its buffers do not fit) g->toff stays null and the status is GPM_OK.
+int try_topo(gpm_graph* g);
 // Relabels the ORIENTED graph g by (out-degree + in-degree, id) on the device
 // (prep.hip).  Where every edge goes up in that order -- gpm_graph_orient and
 // gpm_csr_orient give such graphs -- *ordered is set and *toff / *tadj /

@@ -416,15 +416,10 @@ unsigned grid_of(const gpm_graph* g, uint64_t threads) {
 // against lists: Erdos-Renyi n = 1500, dw = 17: 2.0 against 6.7; n = 4096, dw = 9:
 // 3.8, 3.7; dw = 17: 8.4, 13; n = 16384, dw = 17: 532, 44; R-MAT n = 1500, dw = 48:
 // 2.0, 143; n = 8192, dw = 63: 30, 881; n = 16384, dw = 83: 226, 2994.
-bool bits_pay(const gpm_graph* g) {
+bool bits_pay(gpm_graph* g) {
   if (g->n > kBitsMaxN || !g->m) return false;
   if (g->n <= kSegIds) return true;
-  double d2 = 0.0;
-  for (uint32_t v = 0; v < g->n; ++v) {
-    const double d = g->h_off[v + 1] - g->h_off[v];
-    d2 += d * d;
-  }
-  return d2 / (double)g->m >= 16.0 * std::sqrt((double)g->n / kSegIds);
+  return mean_met_degree(g) >= 16.0 * std::sqrt((double)g->n / kSegIds);
 }
 
 // Builds g->nbits if missing; *ok is false where the lists hold an entry twice

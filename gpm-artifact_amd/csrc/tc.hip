@@ -9,13 +9,14 @@
 //                low-degree graphs keep all 64 lanes busy.  Blocks store
 //                partial sums that a one-block kernel adds up.
 //  GPM_TC_VERTEX (v_centric, TCSolver.cuh:64-113, tc_hi_warp_vertex.cuh):
-//                one wave per root u with |N+(u)| <= 256 (roots interleaved
-//                statically over the waves), one 256-thread block per larger
-//                root.  N+(u) goes into an LDS hash table;
-//                the lists N+(v), v in N+(u), are walked as one flattened
-//                range so that every lane reads one entry per step
-//                (coalesced, no idle lanes on short lists).  Roots above the
-//                LDS capacity probe N+(u) by binary search instead.
+//                on the DAG relabelled by total degree (gpm_graph's
+//                toff/tadj): one wave per root u with |N+(u)| <= 64 searches
+//                the pairs of N+(u) in each other's lists; one 256-thread block
+//                per larger root streams the lists N+(v), v in N+(u), past an
+//                LDS bitmap of N+(u).  Graphs of near-uniform degrees, and
+//                ORIENTED graphs that this order is not topological for (gpm_tc
+//                asks for no acyclic graph), keep the hash kernels: N+(u) in an
+//                LDS table, the lists walked as one flattened range.
 //  Count = sum over oriented edges (u, v) of |N+(u) & N+(v)|.
 #include <algorithm>
 #include <mutex>
@@ -44,7 +45,8 @@ static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 namespace {
 
 constexpr int kBlock = 256;
-constexpr uint32_t kTcWaveCap = 256;     // roots served by one wave
+constexpr uint32_t kTcPairsCap = 16;    // roots served by part of a wave, relabelled DAG
+constexpr uint32_t kTcWaveCap = 256;     // roots served by one wave, hash kernels
 constexpr uint32_t kTcWaveTable = 512;   // LDS keys per wave
 constexpr uint32_t kTcBlockTableMax = 8192;  // 32 KiB of keys per block
 constexpr uint64_t kTcFusedEdgesPerGroup = 4;  // edges per group, fused repeat
@@ -311,6 +313,199 @@ __global__ __launch_bounds__(kBlock) void tc_vertex_block_kernel(
   if (lane_id() == 0 && cnt) atomicAdd(out, (unsigned long long)cnt);
 }
 
+// The two kernels below read the DAG relabelled by total degree: every list
+// N+(s) holds ids above s, and the ids that most lists hold are the highest.
+
+// Lists a search runs in at once per lane: a search is a chain of dependent
+// loads, and the waves alone do not hide it.
+constexpr int kTcSearches = 4;
+
+// G lanes per root u with d = |N+(u)| <= G, lane i holding S[i] and the bounds of
+// its list: every pair of S, at distance k around the circle of S, is one search
+// of the higher id in the lower one's list.  Roots are interleaved statically
+// (ordered by degree).  A root of more than 16 ids is streamed: on R-MAT scale 20
+// the searches of the roots up to 32 or 64 ids, 64 cache lines a step, took longer
+// than their lists' stream (all roots: 3.2 ms with 8 or 16, 3.4 with 32, 4.6 with
+// 64; the roots up to 16: 0.53 ms, bound by the chain of dependent loads).
+template <int G>
+__global__ __launch_bounds__(kBlock) void tc_pairs_kernel(const uint32_t* __restrict__ off,
+                                                          const uint32_t* __restrict__ adj,
+                                                          const uint32_t* __restrict__ roots,
+                                                          uint32_t n_roots,
+                                                          unsigned long long* __restrict__ out) {
+  __shared__ unsigned long long s_sum[kBlock / kWave];
+  const uint32_t sub = threadIdx.x & (G - 1);
+  const uint32_t ngrp = gridDim.x * (kBlock / G);
+  uint64_t cnt = 0;
+  // Waves run the loop together: a group past the last root holds an empty one.
+  for (uint32_t r0 = (blockIdx.x * kBlock + threadIdx.x) / G; wave_ballot(r0 < n_roots) != 0ull;
+       r0 += ngrp) {
+    const uint32_t u = r0 < n_roots ? roots[r0] : kEmpty;
+    const uint32_t sb = u != kEmpty ? off[u] : 0u, d = u != kEmpty ? off[u + 1] - sb : 0u;
+    const bool act = sub < d;
+    const uint32_t s = act ? adj[sb + sub] : 0u;
+    const uint32_t b = act ? off[s] : 0u, len = act ? off[s + 1] - b : 0u;
+    // Distances 1 .. (d - 1) / 2, and d / 2 from the first half when d is even.
+    for (uint32_t k0 = 1; wave_ballot(k0 <= d / 2) != 0ull; k0 += kTcSearches) {
+      uint32_t lo[kTcSearches], n[kTcSearches], key[kTcSearches];
+      bool any = false;
+#pragma unroll
+      for (int q = 0; q < kTcSearches; ++q) {
+        const uint32_t k = k0 + q;
+        uint32_t j = sub + k;
+        if (j >= d) j -= d;
+        const uint32_t sj = __shfl(s, (int)j, G), bj = __shfl(b, (int)j, G),
+                       nj = __shfl(len, (int)j, G);
+        const bool pair = act && (2 * k < d || (2 * k == d && sub < k));
+        const bool up = s < sj;  // this lane's list is the one searched
+        key[q] = up ? sj : s;
+        lo[q] = up ? b : bj;
+        n[q] = pair ? (up ? len : nj) : 0u;
+        any |= n[q] > 1;
+      }
+      // Lower bounds of the keys, all searches of the lane side by side.
+      while (wave_ballot(any) != 0ull) {
+        any = false;
+#pragma unroll
+        for (int q = 0; q < kTcSearches; ++q) {
+          const uint32_t half = n[q] >> 1;
+          const uint32_t at = n[q] > 1 ? adj[lo[q] + half] : kEmpty;
+          lo[q] += at <= key[q] ? half : 0u;
+          n[q] -= n[q] > 1 ? half : 0u;
+          any |= n[q] > 1;
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < kTcSearches; ++q) cnt += n[q] && adj[lo[q]] == key[q] ? 1u : 0u;
+    }
+  }
+  cnt = wave_sum_u64(cnt);
+  if (lane_id() == 0) s_sum[threadIdx.x / kWave] = cnt;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned long long total = 0;
+    for (int i = 0; i < kBlock / kWave; ++i) total += s_sum[i];
+    if (total) atomicAdd(out, total);
+  }
+}
+
+// Ids with a bit in LDS: the top 65536 hold 97 % of the list entries on R-MAT
+// scale 20, and 8 KiB leave the CU's wave slots full.
+constexpr uint32_t kTcIdBits = 65536;
+// 64-entry windows of a list in flight per wave.
+constexpr uint32_t kTcWindows = 4;
+
+// Block per root u with |N+(u)| > kTcPairsCap (statically interleaved, ordered by degree:
+// a queue's same-address atomics would cost as much as the small roots).  The
+// block's S = N+(u) has its bits in LDS; each wave streams every fourth list
+// N+(S[i]), the next windows loaded before the last are looked up.  Lists much
+// longer than S are searched for S's later ids instead.  Ids below the bitmap
+// count only where S has such ids (s_low of them, its first).  On R-MAT scale
+// 20 (157 000 such roots, 3.9e9 entries streamed) 2.65 ms, 5.9 TB/s of L2 and
+// last-level cache reads; the hash kernels took 31 ms for all roots, in the owner
+// search of every entry and the table's probe sequences.
+__global__ __launch_bounds__(kBlock) void tc_stream_kernel(const uint32_t* __restrict__ off,
+                                                           const uint32_t* __restrict__ adj,
+                                                           uint32_t n,
+                                                           const uint32_t* __restrict__ roots,
+                                                           uint32_t n_roots,
+                                                           unsigned long long* __restrict__ out) {
+  constexpr uint32_t kWaves = kBlock / kWave;
+  __shared__ uint32_t s_bits[kTcIdBits / 32];
+  __shared__ uint32_t s_low;
+  __shared__ unsigned long long s_sum[kWaves];
+  const uint32_t lane = lane_id(), w = uniform(threadIdx.x / kWave);
+  const uint32_t id_base = n > kTcIdBits ? n - kTcIdBits : 0u;
+  for (uint32_t i = threadIdx.x; i < kTcIdBits / 32; i += kBlock) s_bits[i] = 0u;
+  uint64_t cnt = 0;
+  for (uint32_t r = blockIdx.x; r < n_roots; r += gridDim.x) {
+    const uint32_t u = uniform(roots[r]);
+    const uint32_t sb = uniform(off[u]), d = uniform(off[u + 1]) - sb;
+    const uint32_t* S = adj + sb;
+    if (threadIdx.x == 0) s_low = 0;
+    __syncthreads();
+    uint32_t low = 0;
+    for (uint32_t i = threadIdx.x; i < d; i += kBlock) {
+      const uint32_t t = S[i] - id_base;
+      if (S[i] < id_base)
+        ++low;
+      else
+        atomicOr(&s_bits[t >> 5], 1u << (t & 31));
+    }
+    if (low) atomicAdd(&s_low, low);
+    __syncthreads();
+    const uint32_t nlow = uniform(s_low);
+    // The last list has no later id of S to meet.
+    for (uint32_t c0 = 0; c0 + 1 < d; c0 += kBlock) {
+      // Lane l holds the bounds of list c0 + kWaves l + w.
+      const uint32_t mine = c0 + kWaves * lane + w;
+      uint32_t b = 0, len = 0;
+      if (mine + 1 < d) {
+        const uint32_t v = S[mine];
+        b = off[v];
+        len = off[v + 1] - b;
+      }
+      const bool longer = len > 16 * d;
+      for (uint64_t m = wave_ballot(longer); m; m &= m - 1) {
+        const uint32_t j = (uint32_t)__builtin_ctzll(m);
+        const uint32_t lb = __builtin_amdgcn_readlane(b, j), ln = __builtin_amdgcn_readlane(len, j);
+        for (uint32_t t = c0 + kWaves * j + w + 1 + lane; t < d; t += kWave)
+          cnt += sorted_contains(adj + lb, ln, S[t]) ? 1u : 0u;
+      }
+      uint64_t todo = wave_ballot(len && !longer);
+      // Batches of kTcWindows windows: list j's entries [t0, t0 + 64 kTcWindows).
+      uint32_t cb = 0, cn = 0, ct = 0, x[kTcWindows];
+      auto next = [&]() {  // moves on to the next batch; false after the last
+        ct += kTcWindows * kWave;
+        if (ct < cn) return true;
+        if (!todo) return false;
+        const uint32_t j = (uint32_t)__builtin_ctzll(todo);
+        todo &= todo - 1;
+        cb = __builtin_amdgcn_readlane(b, j);
+        cn = __builtin_amdgcn_readlane(len, j);
+        ct = 0;
+        return true;
+      };
+      auto load = [&](uint32_t (&y)[kTcWindows]) {
+#pragma unroll
+        for (uint32_t q = 0; q < kTcWindows; ++q) {
+          const uint32_t p = ct + q * kWave + lane;
+          y[q] = p < cn ? adj[cb + p] : kEmpty;  // past every id and bitmap word
+        }
+      };
+      bool more = next();
+      if (more) load(x);
+      while (more) {
+        uint32_t y[kTcWindows];
+        more = next();
+        if (more) load(y);
+#pragma unroll
+        for (uint32_t q = 0; q < kTcWindows; ++q) {
+          const uint32_t t = x[q] - id_base;
+          if (t < kTcIdBits) {
+            cnt += (s_bits[t >> 5] >> (t & 31)) & 1u;
+          } else if (nlow && x[q] < id_base) {
+            cnt += sorted_contains(S, nlow, x[q]) ? 1u : 0u;
+          }
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < kTcWindows; ++q) x[q] = y[q];
+      }
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < d; i += kBlock)
+      if (S[i] >= id_base) s_bits[(S[i] - id_base) >> 5] = 0u;
+  }
+  cnt = wave_sum_u64(cnt);
+  if (lane == 0) s_sum[w] = cnt;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned long long total = 0;
+    for (uint32_t i = 0; i < kWaves; ++i) total += s_sum[i];
+    if (total) atomicAdd(out, total);
+  }
+}
+
 // src[e] = u for every e in [off[u], off[u+1]) with e < m; one wave per
 // vertex, grid-stride.  Entries past m are never written, whatever the
 // offsets hold.
@@ -378,6 +573,25 @@ int ensure_tc_partial(gpm_graph* g) {
   return GPM_OK;
 }
 
+// Root tiers of the vertex-centric count and whether they are on the relabelled
+// DAG.  Lists of one length have no hubs for the bitmap to gather, and every root
+// is a middling one: there the flattened walk of the hash kernels keeps more
+// lanes in use.  Hash against relabelled kernels, ms: Erdos-Renyi n = 900 000, 16
+// edges a vertex (mean met degree 1.2 times the mean) 1.12, 3.2; 8 edges 0.43,
+// 0.47; 5 edges, n = 100 000, 0.048, 0.030; R-MAT n = 100 000, 3 edges a vertex (6
+// times) 0.41, 0.07; R-MAT scale 20 (10 times) 31.0, 3.2.
+int vertex_tiers(gpm_graph* g, const RootTiers** t, bool* ranked) {
+  const double met = mean_met_degree(g);
+  *ranked = met < 8.0 || met >= 2.0 * (double)g->m / std::max(g->n, 1u);
+  if (*ranked) {
+    const int st = try_topo(g);
+    if (st != GPM_OK) return st;
+    *ranked = g->toff != nullptr;
+  }
+  return *ranked ? get_tc_tiers(g, kTcPairsCap, g->h_rank.data(), t)
+                 : get_tc_tiers(g, kTcWaveCap, nullptr, t);
+}
+
 // Enqueues one triangle count (counter reset + kernels) on g's stream; the
 // count lands in g->counters[0].  mark: record per-kernel timing marks.
 int enqueue_tc(gpm_graph* g, int variant, bool mark) {
@@ -397,8 +611,33 @@ int enqueue_tc(gpm_graph* g, int variant, bool mark) {
     return GPM_OK;
   }
   const RootTiers* t = nullptr;
-  if ((st = get_tc_tiers(g, kTcWaveCap, &t)) != GPM_OK) return st;
+  bool ranked = false;
+  if ((st = vertex_tiers(g, &t, &ranked)) != GPM_OK) return st;
   if ((st = zero_counters(g, 1)) != GPM_OK) return st;
+  if (ranked) {
+    if (t->n_block) {
+      const unsigned blocks = (unsigned)std::min<uint64_t>(t->n_block, (uint64_t)cus * 8);
+      hipLaunchKernelGGL(tc_stream_kernel, dim3(blocks), dim3(kBlock), 0, g->stream, g->toff,
+                         g->tadj, g->n, t->d_block, t->n_block, g->counters);
+      GPM_HIP(hipGetLastError());
+      if (mark) timing_mark(g, "tc_vertex_block");
+    }
+    // The roots are in decreasing degree: those above 16, above 8 and the rest.
+    const uint32_t cuts[] = {0, t->n_wave_above[1], t->n_wave_above[0], t->n_wave};
+    for (int c = 0; c < 3; ++c) {
+      const uint32_t count = cuts[c + 1] - cuts[c];
+      if (!count) continue;
+      const int G = c == 0 ? 32 : c == 1 ? 16 : 8;
+      const uint64_t blocks = ((uint64_t)count * G + kBlock - 1) / kBlock;
+      auto kern = c == 0 ? tc_pairs_kernel<32> : c == 1 ? tc_pairs_kernel<16> : tc_pairs_kernel<8>;
+      hipLaunchKernelGGL(kern, dim3((unsigned)std::min<uint64_t>(blocks, (uint64_t)cus * 8)),
+                         dim3(kBlock), 0, g->stream, g->toff, g->tadj, t->d_wave + cuts[c], count,
+                         g->counters);
+      GPM_HIP(hipGetLastError());
+    }
+    if (t->n_wave && mark) timing_mark(g, "tc_vertex_wave");
+    return GPM_OK;
+  }
   unsigned int* q = t->queues;
   hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, g->stream, q, 4);
   if (t->n_wave) {
@@ -526,7 +765,8 @@ int tc_run(gpm_graph* g, int variant, int reps, uint64_t* out) {
   if (variant == GPM_TC_EDGE && (st = ensure_src(g)) != GPM_OK) return st;
   if (variant == GPM_TC_VERTEX) {
     const RootTiers* t = nullptr;  // build (and cache) the tiers before timing
-    if ((st = get_tc_tiers(g, kTcWaveCap, &t)) != GPM_OK) return st;
+    bool ranked = false;
+    if ((st = vertex_tiers(g, &t, &ranked)) != GPM_OK) return st;
   }
   const bool graph = variant == GPM_TC_EDGE && reps > 1;
   if (graph && (st = ensure_tc_graph(g)) != GPM_OK) return st;

@@ -157,6 +157,11 @@ int get_tiers(gpm_graph* g, const TierRequest& req, const RootTiers** out) {
   }
   RootTiers t;
   t.n_wave = (uint32_t)wave.size();
+  for (const uint32_t v : wave) {
+    const uint32_t d = g->h_off[v + 1] - g->h_off[v];
+    t.n_wave_above[0] += d > 8;
+    t.n_wave_above[1] += d > 16;
+  }
   t.n_block = (uint32_t)block.size();
   t.n_big = (uint32_t)big.size();
   t.max_block_deg = maxb;
@@ -197,11 +202,12 @@ int get_tiers(gpm_graph* g, const TierRequest& req, const RootTiers** out) {
   return GPM_OK;
 }
 
-int get_tc_tiers(gpm_graph* g, uint32_t wave_cap, const RootTiers** out) {
+int get_tc_tiers(gpm_graph* g, uint32_t wave_cap, const uint32_t* rank, const RootTiers** out) {
   TierRequest r;
   r.min_deg = 2;
   r.wave_cap = wave_cap;
   r.block_cap = 0xFFFFFFFFu;
+  r.rank = rank;
   return get_tiers(g, r, out);
 }
 

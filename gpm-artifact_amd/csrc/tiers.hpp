@@ -17,6 +17,7 @@ namespace gpm {
 struct RootTiers {
   uint32_t* d_wave = nullptr;   // roots served by one wave
   uint32_t n_wave = 0;
+  uint32_t n_wave_above[2] = {0, 0};  // ... of out-degree above 8, above 16
   uint32_t* d_block = nullptr;  // roots served by one block, rows in LDS
   uint32_t n_block = 0;
   uint32_t max_block_deg = 0;
@@ -72,8 +73,8 @@ constexpr uint32_t kMinRowsPerPart = 8;
 // Returns cached tiers for (graph, request); builds and uploads on a miss.
 int get_tiers(gpm_graph* g, const TierRequest& req, const RootTiers** out);
 // Tiers for vertex-centric triangle counting (min_deg 2, wave_cap as given,
-// everything above goes to the block kernel).
-int get_tc_tiers(gpm_graph* g, uint32_t wave_cap, const RootTiers** out);
+// everything above goes to the block kernel); rank as in TierRequest.
+int get_tc_tiers(gpm_graph* g, uint32_t wave_cap, const uint32_t* rank, const RootTiers** out);
 void free_tiers(gpm_graph* g);
 
 }  // namespace gpm
