@@ -264,6 +264,8 @@ void release(gpm_graph* g) {
   (void)hipFree(g->tadj);
   (void)hipFree(g->bmask);
   (void)hipFree(g->nbits);
+  for (void* p : {(void*)g->motif.below, g->motif.heavy, g->motif.light, g->motif.triangles})
+    (void)hipFree(p);
   hipFree(g->scratch);
   hipFree(g->counters);
   (void)hipFree(g->tc_partial);

@@ -67,6 +67,16 @@ struct gpm_graph {
   uint32_t* rk_off = nullptr;
   uint32_t* rk_adj = nullptr;
   gpm_graph* dag = nullptr;
+  // Motif counters (motif_count.hip), built on first use: host offsets and
+  // lower-neighbour counts of rk_off / rk_adj, and the task lists of the 4-cycle
+  // kernels (hbm: some heavy task counts in HBM) and the triangle kernel.
+  struct {
+    std::vector<uint32_t> h_off;
+    uint32_t* below = nullptr;
+    void *heavy = nullptr, *light = nullptr, *triangles = nullptr;
+    uint32_t n_heavy = 0, n_light = 0, n_triangles = 0;
+    bool hbm = false, built = false;
+  } motif;
   // Last prepared matching batch (match.hip), replayed on identical calls.
   void* match_cache = nullptr;
   // Instantiated hipGraph of repeated edge-parallel triangle counts, and the

@@ -8,9 +8,8 @@
 //   N_cycle   = 4-cycles, counted per max-rank corner (below)
 //   N_diamond = sum_{edges e} C(c_e, 2)        (c_e = triangles on e)
 //   N_K4      = 4-cliques of the degree-oriented DAG
-// The edge sums take every undirected edge once (the DAG's edges); c_e
-// comes from listing every triangle once on the DAG (its first edge and apex)
-// and adding one to each of its three edges.
+// The edge sums take every undirected edge once, at its lower-ranked end; c_e
+// comes from streaming the neighbours' lists past each vertex's (below).
 // and the induced counts by inclusion-exclusion over how many copies of
 // each shape a larger shape holds:
 //   I_K4 = N_K4
@@ -23,12 +22,10 @@
 // 4-cycles: with rank = position in (degree, id) order, every 4-cycle has a
 // unique top corner u of maximal rank; its wedges u-v-w with v, w below u
 // land on the opposite corner w.  The walk runs on the graph relabelled by
-// rank with sorted lists, so "below u" is a prefix of each list (one binary
-// search, no rank lookups).  For each root u a block counts, for every w,
-// the wedges reaching it in a block-private counter array in HBM; each
-// increment adds the counter's previous value, which sums to
-// sum_w C(cnt_w, 2).  The first increment of a counter also appends w to a
-// block-private list, and only the listed counters are cleared afterwards.
+// rank with sorted lists, so the ends w in a range of ranks are a part of each
+// list (binary search, no rank lookups).  For each root u and band of ranks a
+// block counts, for every w of the band, the wedges reaching it in LDS, and sums
+// C(cnt_w, 2) over the band (cycles_kernel); roots of few wedges use a hash table.
 #include <algorithm>
 #include <numeric>
 #include <vector>
@@ -42,20 +39,29 @@ using namespace gpm;
 namespace {
 
 constexpr int kBlock = 256;
-// 4-cycle corners: threads per block and blocks per CU (the best of the
-// shapes measured at the launch).
-constexpr int kCycBlock = 256;
-constexpr int kCycBlocksPerCu = 1;
-constexpr uint32_t kWedgesInFlight = 8;
-// Counters of the wedge endpoints ranked just below the root, [u - kCycBand,
-// u), live in LDS rather than in the block's HBM array.  On R-MAT scale 22,
-// 32768 ranks below the root hold 43.6 % of the wedges of the top 1 % of
-// roots (hubs link to hubs).  The walk took 1.39 s with every counter in
-// HBM; with the band (words, wedges in flight): 32768 x 4 1.08 s,
-// 32768 x 8 1.07 s, 40000 x 4 1.05 s, 40000 x 8 1.04 s.  40000 words with
-// the walk's other arrays use 158 KB of the CU's 160 KB of LDS; the kernel
-// runs one block per CU.
-constexpr uint32_t kCycBand = 40000;
+// 4-cycle corners, roots of kCycHeavy wedges and more: one block per CU whose
+// LDS holds the counters of a band of ranks, 16-bit ones where the root has less
+// than 65536 lower neighbours (no counter can pass that).
+constexpr int kCycBlock = 1024;
+constexpr uint32_t kCycWords = 39936;  // 156 KiB of counters
+constexpr uint32_t kCycHeavy = 2048;
+// A root's last task covers every rank below its other tasks: a band in LDS and
+// the ranks further down in HBM.  Roots of so many wedges have their first band
+// (89 % of the wedges on R-MAT scale 19), and their second (another 8 %), as tasks
+// of their own before it.
+constexpr uint64_t kCycBand1 = 1u << 14, kCycBand2 = 1u << 17;
+// Lighter roots: a hash table of their wedges' ends.
+constexpr int kLightBlock = 256;
+constexpr uint32_t kLightSlots = 4096;
+static_assert(kLightSlots >= 2 * kCycHeavy, "load factor at most 1/2");
+// 64-entry windows of a list in flight per wave.
+constexpr uint32_t kCycWindows = 4;
+
+// The wedges u - v - x with lo <= x < hi (hi <= u), v one of the n_below first
+// neighbours of u.  Ranks from band on have their counters in LDS.
+struct CycleTask {
+  uint32_t u, n_below, lo, hi, band;
+};
 
 // Blocks of 256 threads for `threads` threads, at most 32 per CU (the
 // kernels stride over the rest).
@@ -64,80 +70,240 @@ unsigned grid_of(const gpm_graph* g, uint64_t threads) {
   return (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(want, (uint64_t)device_cus(g) * 32));
 }
 
-// Triangles per DAG edge (c_e = |N(u) & N(v)| for the undirected edge of e):
-// every triangle is found once, from its first DAG edge (u, v) and its apex
-// w in N+(u) & N+(v) -- G lanes per edge, each taking entries of the shorter
-// list and searching the longer (on R-MAT scale 22, 14 % fewer search steps
-// than always taking N+(u)) -- and adds one to each of its three edges:
-// (u, w) and (v, w) by their positions in the DAG lists, (u, v) once per
-// edge with the group's total.  tri must be zero on entry; m_dag entries.
-template <int G>
-__global__ __launch_bounds__(kBlock) void edge_triangles_kernel(
-    const uint32_t* __restrict__ doff, const uint32_t* __restrict__ dadj,
-    const uint32_t* __restrict__ dsrc, uint64_t m, uint32_t* __restrict__ tri) {
-  const uint64_t tid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint32_t sub = threadIdx.x & (G - 1);
-  const uint64_t ngrp = (uint64_t)gridDim.x * blockDim.x / G;
-  for (uint64_t e = tid / G; e < m; e += ngrp) {
-    const uint32_t u = dsrc[e], v = dadj[e];
-    const uint32_t ub = doff[u], nu = doff[u + 1] - ub;
-    const uint32_t vb = doff[v], nv = doff[v + 1] - vb;
-    // a = the list walked, b = the list searched
-    const bool swap = nu > nv;
-    const uint32_t ab = swap ? vb : ub, na = swap ? nv : nu;
-    const uint32_t bb = swap ? ub : vb, nb = swap ? nu : nv;
-    uint32_t cnt = 0;
-    for (uint32_t i = sub; i < na; i += G) {
-      const uint32_t w = dadj[ab + i];
-      // position of w in list b (lower bound), if present
-      uint32_t lo = 0, len = nb;
-      while (len > 1) {
-        const uint32_t half = len >> 1;
-        lo = dadj[bb + lo + half] <= w ? lo + half : lo;
-        len -= half;
-      }
-      if (nb && dadj[bb + lo] == w) {
-        atomicAdd(&tri[ab + i], 1u);
-        atomicAdd(&tri[bb + lo], 1u);
-        ++cnt;
+// ---------------------------------------------------- triangles per edge
+//
+// tri[e] of the entry e = (v, x), x > v, of the rank-relabelled graph is c_e.  A
+// triangle u < v < x lies on three entries.  A block that holds N+(v) as bits and
+// a counter per position counts both (v, .) entries of the triangles v is the
+// lowest of, from the lists of its higher neighbours, and the (v, x) entry of
+// those it is the middle of, from the lists of its lower ones: all in LDS.  (One
+// global atomic per entry and triangle, three in all, had bound this: about 50
+// per ns on the chip.)  Triangles whose lowest vertex has kTriPairs higher
+// neighbours or fewer are found by searching its pairs, with atomics.
+
+constexpr uint32_t kTriPairs = 16;
+// Ids with a bit in LDS, counters in LDS (N+ longer than that: global atomics),
+// and neighbours of v whose lists one task streams.
+constexpr uint32_t kTriIdBits = 65536, kTriIdWords = kTriIdBits / 32;
+constexpr uint32_t kTriCounters = 1024;
+constexpr uint32_t kTriLists = 1024;
+
+// Entries [begin, end) of v's list: the lists of these neighbours.
+struct TriangleTask {
+  uint32_t v, begin, end;
+};
+
+// Block per task (statically interleaved, in decreasing degree).  R-MAT scale
+// 19: the edge sums take 5.3 ms, 11.6 ms with three global atomics a triangle.
+__global__ __launch_bounds__(kBlock) void stream_triangles_kernel(
+    const uint32_t* __restrict__ off, const uint32_t* __restrict__ adj,
+    const uint32_t* __restrict__ below, uint32_t n, const TriangleTask* __restrict__ tasks,
+    uint32_t n_tasks, uint32_t* __restrict__ tri) {
+  constexpr uint32_t kWaves = kBlock / kWave, kPer = kTriIdWords / kBlock;
+  __shared__ uint32_t s_bits[kTriIdWords];
+  __shared__ uint16_t s_pre[kTriIdWords];
+  __shared__ uint32_t s_cnt[kTriCounters];
+  __shared__ uint32_t s_low, s_wsum[kWaves];
+  const uint32_t lane = lane_id(), w = uniform(threadIdx.x / kWave);
+  const uint32_t id_base = n > kTriIdBits ? n - kTriIdBits : 0u;
+  for (uint32_t i = threadIdx.x; i < kTriIdWords; i += kBlock) s_bits[i] = 0u;
+  for (uint32_t i = threadIdx.x; i < kTriCounters; i += kBlock) s_cnt[i] = 0u;
+  for (uint32_t q = blockIdx.x; q < n_tasks; q += gridDim.x) {
+    const uint32_t v = uniform(tasks[q].v), begin = uniform(tasks[q].begin),
+                   end = uniform(tasks[q].end);
+    const uint32_t vb = uniform(off[v]), sb = vb + uniform(below[v]);
+    const uint32_t d = uniform(off[v + 1]) - sb;
+    const uint32_t* S = adj + sb;
+    if (threadIdx.x == 0) s_low = 0;
+    __syncthreads();
+    uint32_t low = 0;
+    for (uint32_t i = threadIdx.x; i < d; i += kBlock) {
+      const uint32_t t = S[i] - id_base;
+      if (S[i] < id_base)
+        ++low;
+      else
+        atomicOr(&s_bits[t >> 5], 1u << (t & 31));
+    }
+    if (low) atomicAdd(&s_low, low);
+    __syncthreads();
+    const uint32_t nlow = uniform(s_low);
+    {
+      // Ids of S before every bitmap word (at most kTriIdBits - 32: 16 bits hold it).
+      uint32_t c[kPer], sum = 0;
+#pragma unroll
+      for (uint32_t k = 0; k < kPer; ++k) sum += c[k] = (uint32_t)__popc(s_bits[kPer * threadIdx.x + k]);
+      const uint32_t incl = wave_incl_scan(sum);
+      if (lane == kWave - 1) s_wsum[w] = incl;
+      __syncthreads();
+      uint32_t at = incl - sum;
+      for (uint32_t k = 0; k < w; ++k) at += s_wsum[k];
+#pragma unroll
+      for (uint32_t k = 0; k < kPer; ++k) {
+        s_pre[kPer * threadIdx.x + k] = (uint16_t)at;
+        at += c[k];
       }
     }
+    __syncthreads();
+    auto count = [&](uint32_t pos) {  // one triangle on entry `pos` of S
+      if (pos < kTriCounters)
+        atomicAdd(&s_cnt[pos], 1u);
+      else
+        atomicAdd(&tri[sb + pos], 1u);
+    };
+    for (uint32_t c0 = begin; c0 < end; c0 += kBlock) {
+      // Lane l holds the list of neighbour c0 + kWaves l + w.
+      const uint32_t mine = c0 + kWaves * lane + w;
+      uint32_t b = 0, len = 0;
+      if (mine < end) {
+        const uint32_t y = adj[vb + mine];
+        b = off[y] + below[y];
+        len = off[y + 1] - b;
+        // Lower neighbours with few higher ones search their pairs.
+        if (y < v && len <= kTriPairs) len = 0;
+      }
+      uint64_t todo = wave_ballot(len != 0u);
+      uint32_t cb = 0, cn = 0, ct = 0, ci = 0, x[kCycWindows];
+      auto next = [&]() {  // moves on to the next batch of windows; false after the last
+        ct += kCycWindows * kWave;
+        if (ct < cn) return true;
+        if (!todo) return false;
+        const uint32_t j = (uint32_t)__builtin_ctzll(todo);
+        todo &= todo - 1;
+        cb = __builtin_amdgcn_readlane(b, j);
+        cn = __builtin_amdgcn_readlane(len, j);
+        ci = c0 + kWaves * j + w;
+        ct = 0;
+        return true;
+      };
+      auto load = [&](uint32_t (&y)[kCycWindows]) {
 #pragma unroll
-    for (int o = G / 2; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o, kWave);
-    if (sub == 0 && cnt) atomicAdd(&tri[e], cnt);
+        for (uint32_t k = 0; k < kCycWindows; ++k) {
+          const uint32_t p = ct + k * kWave + lane;
+          y[k] = p < cn ? adj[cb + p] : kEmpty;  // past every id and bitmap word
+        }
+      };
+      bool more = next();
+      if (more) load(x);
+      while (more) {
+        uint32_t y[kCycWindows];
+        const uint32_t entry = vb + ci;  // of v's list: the neighbour being streamed
+        more = next();
+        if (more) load(y);
+#pragma unroll
+        for (uint32_t k = 0; k < kCycWindows; ++k) {
+          const uint32_t t = x[k] - id_base;
+          uint32_t pos = kEmpty;
+          if (t < kTriIdBits) {
+            const uint32_t word = s_bits[t >> 5];
+            if ((word >> (t & 31)) & 1u)
+              pos = nlow + s_pre[t >> 5] + (uint32_t)__popc(word & ((1u << (t & 31)) - 1u));
+          } else if (nlow && x[k] < id_base) {
+            const uint32_t p = upper_index(S, nlow, x[k]);
+            if (p > 0 && S[p - 1] == x[k]) pos = p - 1;
+          }
+          if (pos != kEmpty) {
+            count(pos);
+            if (entry >= sb) count(entry - sb);
+          }
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kCycWindows; ++k) x[k] = y[k];
+      }
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < d; i += kBlock) {
+      if (S[i] >= id_base) s_bits[(S[i] - id_base) >> 5] = 0u;
+      if (i < kTriCounters && s_cnt[i]) {
+        atomicAdd(&tri[sb + i], s_cnt[i]);
+        s_cnt[i] = 0u;
+      }
+    }
   }
 }
 
-// Edge sums over the undirected edges {u, v} (each once: the DAG's edges),
-// from the per-edge triangle counts c and the symmetric degrees:
+// 16 lanes per vertex v with 2 <= |N+(v)| <= kTriPairs: the pairs of N+(v), at
+// distance k around the circle of its ids, searched in the lower one's list.
+__global__ __launch_bounds__(kBlock) void pair_triangles_kernel(
+    const uint32_t* __restrict__ off, const uint32_t* __restrict__ adj,
+    const uint32_t* __restrict__ below, uint32_t n, uint32_t* __restrict__ tri) {
+  constexpr int G = kTriPairs;
+  const uint32_t sub = threadIdx.x & (G - 1);
+  const uint32_t ngrp = gridDim.x * (kBlock / G);
+  for (uint32_t v = (blockIdx.x * kBlock + threadIdx.x) / G; wave_ballot(v < n) != 0ull; v += ngrp) {
+    const uint32_t sb = v < n ? off[v] + below[v] : 0u;
+    uint32_t d = v < n ? off[v + 1] - sb : 0u;
+    if (d > kTriPairs) d = 0;
+    if (wave_ballot(d >= 2) == 0ull) continue;
+    const bool act = sub < d;
+    const uint32_t s = act ? adj[sb + sub] : 0u;
+    const uint32_t b = act ? off[s] + below[s] : 0u, len = act ? off[s + 1] - b : 0u;
+    for (uint32_t k = 1; wave_ballot(k <= d / 2) != 0ull; ++k) {
+      uint32_t j = sub + k;
+      if (j >= d) j -= d;
+      const uint32_t sj = __shfl(s, (int)j, G), bj = __shfl(b, (int)j, G), nj = __shfl(len, (int)j, G);
+      const bool pair = act && (2 * k < d || (2 * k == d && sub < k));
+      const bool up = s < sj;  // this lane's list is the one searched
+      const uint32_t key = up ? sj : s;
+      uint32_t lo = up ? b : bj, m = pair ? (up ? len : nj) : 0u;
+      const bool any = m != 0u;
+      while (m > 1) {
+        const uint32_t half = m >> 1;
+        lo = adj[lo + half] <= key ? lo + half : lo;
+        m -= half;
+      }
+      if (any && adj[lo] == key) {
+        atomicAdd(&tri[sb + sub], 1u);
+        atomicAdd(&tri[sb + j], 1u);
+        atomicAdd(&tri[lo], 1u);
+      }
+    }
+  }
+}
+
+// Adds the threads' values to *out with one atomic per block of kBlock threads:
+// atomics to one address serialise (about 10 ns each), and four per wave of a
+// full launch took 1.5 ms.
+__device__ __forceinline__ void block_add(unsigned long long* out, uint64_t value) {
+  __shared__ unsigned long long s_part[kBlock / kWave];
+  value = wave_sum_u64(value);
+  __syncthreads();  // an earlier call's parts have been read
+  if (lane_id() == 0) s_part[threadIdx.x / kWave] = value;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned long long t = 0;
+    for (int i = 0; i < kBlock / kWave; ++i) t += s_part[i];
+    if (t) atomicAdd(out, t);
+  }
+}
+
+// Edge sums over the undirected edges {v, x} (each once: x > v), from the per-edge
+// triangle counts c and the degrees; one wave per v:
 //   out[0] += 2c                      (sum: 6T)
-//   out[2] += c (d_u + d_v - 4)       (sum: 2 N_paw)
+//   out[2] += c (d_v + d_x - 4)       (sum: 2 N_paw)
 //   out[3] += c (c - 1)               (sum: 2 N_diamond)
-//   out[4] += 2 (d_u - 1)(d_v - 1)    (sum: 2 x the path edge sum)
+//   out[4] += 2 (d_v - 1)(d_x - 1)    (sum: 2 x the path edge sum)
 __global__ __launch_bounds__(kBlock) void edge_stats_kernel(
-    const uint32_t* __restrict__ off, const uint32_t* __restrict__ dsrc,
-    const uint32_t* __restrict__ dadj, const uint32_t* __restrict__ tri, uint64_t m,
+    const uint32_t* __restrict__ off, const uint32_t* __restrict__ adj,
+    const uint32_t* __restrict__ below, const uint32_t* __restrict__ tri, uint32_t n,
     unsigned long long* __restrict__ out) {
   uint64_t s6t = 0, spaw = 0, sdia = 0, spath = 0;
-  for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < m;
-       e += (uint64_t)gridDim.x * blockDim.x) {
-    const uint32_t u = dsrc[e], v = dadj[e];
-    const uint64_t c = tri[e], da = off[u + 1] - off[u], db = off[v + 1] - off[v];
-    s6t += 2 * c;
-    spaw += c ? c * (da + db - 4) : 0;
-    sdia += c * (c - (c ? 1 : 0));
-    spath += 2 * (da - 1) * (db - 1);
+  const uint32_t nw = gridDim.x * blockDim.x / kWave;
+  for (uint32_t v = (blockIdx.x * blockDim.x + threadIdx.x) / kWave; v < n; v += nw) {
+    const uint32_t b = off[v], end = off[v + 1];
+    const uint64_t da = end - b;
+    for (uint32_t e = b + below[v] + lane_id(); e < end; e += kWave) {
+      const uint32_t x = adj[e];
+      const uint64_t c = tri[e], db = off[x + 1] - off[x];
+      s6t += 2 * c;
+      spaw += c ? c * (da + db - 4) : 0;
+      sdia += c * (c - (c ? 1 : 0));
+      spath += 2 * (da - 1) * (db - 1);
+    }
   }
-  s6t = wave_sum_u64(s6t);
-  spaw = wave_sum_u64(spaw);
-  sdia = wave_sum_u64(sdia);
-  spath = wave_sum_u64(spath);
-  if (lane_id() == 0) {
-    atomicAdd(&out[0], (unsigned long long)s6t);
-    atomicAdd(&out[2], (unsigned long long)spaw);
-    atomicAdd(&out[3], (unsigned long long)sdia);
-    atomicAdd(&out[4], (unsigned long long)spath);
-  }
+  block_add(&out[0], s6t);
+  block_add(&out[2], spaw);
+  block_add(&out[3], sdia);
+  block_add(&out[4], spath);
 }
 
 // out[1] += sum_v C(d_v, 3).
@@ -149,8 +315,7 @@ __global__ __launch_bounds__(kBlock) void star_sum_kernel(const uint32_t* __rest
     const uint64_t d = off[v + 1] - off[v];
     acc += d >= 3 ? d * (d - 1) * (d - 2) / 6 : 0;
   }
-  acc = wave_sum_u64(acc);
-  if (lane_id() == 0 && acc) atomicAdd(&out[1], (unsigned long long)acc);
+  block_add(&out[1], acc);
 }
 
 // Entries of the sorted list a[0..n) below key.
@@ -167,125 +332,200 @@ __device__ __forceinline__ uint32_t count_below(const uint32_t* __restrict__ a, 
   return lo;
 }
 
-// 4-cycle walk of root u over the rank-relabelled graph (ids = rank, lists
-// sorted): the wedges u - v - x with v, x < u are the prefixes below u of
-// N(u) and of every such N(v).  Atomic increments whose previous values sum
-// to sum_x C(cnt_x, 2); every x seen first is appended to `touched`
-// (*s_nt entries).
-template <int BS>
-__device__ __forceinline__ void cycle_walk(const uint32_t* __restrict__ off,
-                                           const uint32_t* __restrict__ adj, uint32_t u,
-                                           uint32_t* __restrict__ cnt,
-                                           uint32_t* __restrict__ touched, uint32_t* s_nt,
-                                           uint64_t* acc, uint32_t* s_pre, uint32_t* s_beg,
-                                           uint32_t* s_wsum, uint32_t* s_band) {
-  const uint32_t band_lo = u > kCycBand ? u - kCycBand : 0u;
-  const uint32_t b = uniform(off[u]);
-  const uint32_t dl = uniform(count_below(adj + b, uniform(off[u + 1]) - b, u));
-  for (uint32_t c0 = 0; c0 < dl; c0 += BS) {
-    const uint32_t i = c0 + threadIdx.x;
-    uint32_t len = 0, vb = 0;
-    if (i < dl) {
-      const uint32_t v = adj[b + i];
-      vb = off[v];
-      len = count_below(adj + vb, off[v + 1] - vb, u);
+// Number of a's first n entries (sorted) below each of two keys, side by side.
+__device__ __forceinline__ void count_below2(const uint32_t* __restrict__ a, uint32_t n,
+                                             uint32_t key0, uint32_t key1, uint32_t* below0,
+                                             uint32_t* below1) {
+  uint32_t lo0 = 0, lo1 = 0, hi0 = n, hi1 = n;
+  while (lo0 < hi0 || lo1 < hi1) {
+    const uint32_t m0 = (lo0 + hi0) >> 1, m1 = (lo1 + hi1) >> 1;
+    const uint32_t x0 = lo0 < hi0 ? a[m0] : 0u, x1 = lo1 < hi1 ? a[m1] : 0u;
+    if (lo0 < hi0) (x0 < key0 ? lo0 : hi0) = x0 < key0 ? m0 + 1 : m0;
+    if (lo1 < hi1) (x1 < key1 ? lo1 : hi1) = x1 < key1 ? m1 + 1 : m1;
+  }
+  *below0 = lo0;
+  *below1 = lo1;
+}
+
+// Calls f(x) for every wedge end x of the task, the middle vertices dealt out
+// over the block's waves one by one (whole groups of 64 left most waves idle on
+// roots of a few hundred): the lanes find the bounds of their lists' parts, then
+// the wave streams one part after another, 64 consecutive entries a load and the
+// next windows loaded before the last are handled.
+template <int BS, typename F>
+__device__ __forceinline__ void for_wedges(const uint32_t* __restrict__ off,
+                                           const uint32_t* __restrict__ adj, const CycleTask& t,
+                                           F&& f) {
+  const uint32_t lane = lane_id(), w = uniform(threadIdx.x / kWave);
+  const uint32_t* mid = adj + uniform(off[t.u]);
+  for (uint32_t c0 = 0; c0 < t.n_below; c0 += BS) {
+    const uint32_t mine = c0 + BS / kWave * lane + w;
+    uint32_t b = 0, len = 0;
+    if (mine < t.n_below) {
+      const uint32_t v = mid[mine];
+      b = off[v];
+      uint32_t first, end;
+      count_below2(adj + b, off[v + 1] - b, t.lo, t.hi, &first, &end);
+      b += first;
+      len = end - first;
     }
-    // Block scan of the prefix lengths.
-    const uint32_t lane = lane_id(), w = threadIdx.x / kWave;
-    const uint32_t incl0 = wave_incl_scan(len);
-    if (lane == kWave - 1) s_wsum[w] = incl0;
-    __syncthreads();
-    uint32_t add = 0;
-    for (uint32_t k = 0; k < w; ++k) add += s_wsum[k];
-    s_pre[threadIdx.x] = incl0 + add;
-    s_beg[threadIdx.x] = vb;
-    __syncthreads();
-    const uint32_t total = uniform(s_pre[BS - 1]);
-    // kWedgesInFlight wedges per thread per step: their endpoint loads and
-    // counter atomics are independent, so their latencies overlap (the walk
-    // runs few waves per CU: one block per CU holds the counters).  On R-MAT
-    // scale 22, before the LDS band (device-scope fences per root): 1 in
-    // flight 1.96 s, 4 1.85 s, 8 1.88 s; with workgroup-scope atomics and
-    // fences 1.39 s.  With the band, 8 in flight beat 4.  Aggregating a
-    // root's increments in an LDS hash table first (4.5 wedges per distinct
-    // endpoint on the heaviest roots) measured 3.01 s: the table's inserts
-    // and the barriers of its flushes cost more than the atomics saved.
-    for (uint32_t f0 = threadIdx.x; f0 < total; f0 += BS * kWedgesInFlight) {
-      uint32_t x[kWedgesInFlight], old[kWedgesInFlight];
+    uint64_t todo = wave_ballot(len != 0u);
+    uint32_t cb = 0, cn = 0, ct = 0, x[kCycWindows];
+    auto next = [&]() {  // moves on to the next batch of windows; false after the last
+      ct += kCycWindows * kWave;
+      if (ct < cn) return true;
+      if (!todo) return false;
+      const uint32_t j = (uint32_t)__builtin_ctzll(todo);
+      todo &= todo - 1;
+      cb = __builtin_amdgcn_readlane(b, j);
+      cn = __builtin_amdgcn_readlane(len, j);
+      ct = 0;
+      return true;
+    };
+    auto load = [&](uint32_t (&y)[kCycWindows]) {
 #pragma unroll
-      for (uint32_t k = 0; k < kWedgesInFlight; ++k) {
-        const uint32_t f = f0 + k * BS;
-        x[k] = kEmpty;
-        if (f < total) {
-          const uint32_t j = upper_index(s_pre, BS, f);
-          const uint32_t excl = j ? s_pre[j - 1] : 0u;
-          x[k] = adj[s_beg[j] + (f - excl)];
-        }
+      for (uint32_t q = 0; q < kCycWindows; ++q) {
+        const uint32_t p = ct + q * kWave + lane;
+        y[q] = p < cn ? adj[cb + p] : kEmpty;
       }
+    };
+    bool more = next();
+    if (more) load(x);
+    while (more) {
+      uint32_t y[kCycWindows];
+      more = next();
+      if (more) load(y);
 #pragma unroll
-      for (uint32_t k = 0; k < kWedgesInFlight; ++k)
-        old[k] = x[k] == kEmpty ? 1u
-                 : x[k] >= band_lo ? wg_atomic_add(&s_band[x[k] - band_lo], 1u)
-                                   : wg_atomic_add(&cnt[x[k]], 1u);
+      for (uint32_t q = 0; q < kCycWindows; ++q)
+        if (x[q] != kEmpty) f(x[q]);
 #pragma unroll
-      for (uint32_t k = 0; k < kWedgesInFlight; ++k) {
-        if (x[k] == kEmpty) continue;
-        *acc += old[k];
-        if (old[k] == 0u) touched[atomicAdd(s_nt, 1u)] = x[k];
-      }
+      for (uint32_t q = 0; q < kCycWindows; ++q) x[q] = y[q];
     }
-    __syncthreads();
   }
 }
 
-// Block per root, highest rank first (dynamic queue).  Each block owns
-// 2 n words at counters + blockIdx.x * stride: n counters, then the list of
-// the counters the current root touched.
-template <int BS>
-__global__ __launch_bounds__(BS) void cycles_kernel(
+// One task per block at a time (queue, heaviest roots first): increments the LDS
+// counters of the task's ranks from t.band on, then sums C(count, 2) over them and
+// clears them on the way.  Lower ranks count in HBM (the block's n counters at
+// `counters`): the increments' previous values sum to C(count, 2) there, and a
+// second walk clears them.  R-MAT scale 19 (2.2e9 wedges, 98 % of them below 7100
+// roots): 7.0 ms with the light roots, against 42.7 ms for one 256-thread block
+// per CU that searched the owner of every wedge, kept 40000 32-bit counters in
+// LDS and listed the touched ones.  What is left is latency: a group's list
+// bounds are some 20 dependent loads, and 16 waves share the CU.  Cutting the
+// heaviest roots into narrower bands lost (7.3 - 9.4 ms): the queue's order ends
+// evenly without it.
+__global__ __launch_bounds__(kCycBlock) void cycles_kernel(
     const uint32_t* __restrict__ off, const uint32_t* __restrict__ adj, uint32_t n,
-    unsigned int* __restrict__ queue, uint32_t* __restrict__ counters, uint64_t stride,
-    unsigned long long* __restrict__ out) {
-  __shared__ uint32_t s_pre[BS];
-  __shared__ uint32_t s_beg[BS];
-  __shared__ uint32_t s_wsum[BS / kWave];
-  __shared__ uint32_t s_root;
-  __shared__ uint32_t s_nt;
-  __shared__ uint32_t s_band[kCycBand];
-  uint32_t* cnt = counters + (uint64_t)blockIdx.x * stride;
-  uint32_t* touched = cnt + n;
+    const CycleTask* __restrict__ tasks, uint32_t n_tasks, unsigned int* __restrict__ queue,
+    uint32_t* __restrict__ counters, unsigned long long* __restrict__ out) {
+  __shared__ __align__(16) uint32_t s_cnt[kCycWords];
+  __shared__ uint32_t s_task;
   uint64_t acc = 0;
-  if (threadIdx.x == 0) s_nt = 0u;
-  for (uint32_t i = threadIdx.x; i < kCycBand; i += BS) s_band[i] = 0u;
+  for (uint32_t i = threadIdx.x; i < kCycWords; i += kCycBlock) s_cnt[i] = 0u;
   while (true) {
-    if (threadIdx.x == 0) s_root = atomicAdd(queue, 1u);
+    if (threadIdx.x == 0) s_task = atomicAdd(queue, 1u);
     __syncthreads();
-    const uint32_t q = uniform(s_root);
+    const uint32_t q = uniform(s_task);
     __syncthreads();
-    if (q >= n) break;
-    const uint32_t u = n - 1 - q;
-    cycle_walk<BS>(off, adj, u, cnt, touched, &s_nt, &acc, s_pre, s_beg, s_wsum, s_band);
-    // Counter updates and list appends of this root must be complete before
-    // the listed counters are cleared, and the clears before the next root's
-    // increments; the counters are this block's alone, so workgroup-scope
-    // fences order them.
-    __threadfence_block();
-    __syncthreads();
-    const uint32_t nt = uniform(s_nt);
-    const uint32_t band_lo = u > kCycBand ? u - kCycBand : 0u;
-    for (uint32_t i = threadIdx.x; i < nt; i += BS) {
-      const uint32_t x = touched[i];
-      if (x >= band_lo)
-        s_band[x - band_lo] = 0u;
-      else
-        cnt[x] = 0u;
+    if (q >= n_tasks) break;
+    CycleTask t = tasks[q];
+    t.u = uniform(t.u);
+    t.n_below = uniform(t.n_below);
+    t.lo = uniform(t.lo);
+    t.hi = uniform(t.hi);
+    t.band = uniform(t.band);
+    const uint32_t half = t.n_below < 65536u ? 1u : 0u;  // counters of 16 bits
+    const uint32_t words = (t.hi - t.band + half) >> half;
+    uint32_t* cnt = counters + (uint64_t)blockIdx.x * n;
+    if (t.lo == t.band) {
+      for_wedges<kCycBlock>(off, adj, t, [&](uint32_t x) {
+        const uint32_t i = x - t.band;
+        atomicAdd(&s_cnt[i >> half], 1u << (half & i) * 16);
+      });
+    } else {
+      for_wedges<kCycBlock>(off, adj, t, [&](uint32_t x) {
+        const uint32_t i = x - t.band;
+        if (x >= t.band)
+          atomicAdd(&s_cnt[i >> half], 1u << (half & i) * 16);
+        else
+          acc += wg_atomic_add(&cnt[x], 1u);
+      });
+      __threadfence_block();
     }
-    __threadfence_block();
     __syncthreads();
-    if (threadIdx.x == 0) s_nt = 0u;
+    uint4* v = reinterpret_cast<uint4*>(s_cnt);
+    for (uint32_t i = threadIdx.x; 4 * i < words; i += kCycBlock) {
+      const uint4 c = v[i];
+      if (c.x | c.y | c.z | c.w) {
+        v[i] = make_uint4(0u, 0u, 0u, 0u);
+        for (uint32_t k : {c.x, c.y, c.z, c.w}) {
+          const uint64_t lo = half ? k & 0xFFFFu : k, hi = half ? k >> 16 : 0u;
+          acc += lo * (lo - (lo != 0)) / 2 + hi * (hi - (hi != 0)) / 2;
+        }
+      }
+    }
+    if (t.lo < t.band) {
+      CycleTask low = t;
+      low.hi = t.band;
+      for_wedges<kCycBlock>(off, adj, low, [&](uint32_t x) { cnt[x] = 0u; });
+      __threadfence_block();
+    }
+    __syncthreads();
   }
   acc = wave_sum_u64(acc);
   if (lane_id() == 0 && acc) atomicAdd(out, (unsigned long long)acc);
+}
+
+// Block per root of fewer than kCycHeavy wedges (statically interleaved).
+__global__ __launch_bounds__(kLightBlock) void light_cycles_kernel(
+    const uint32_t* __restrict__ off, const uint32_t* __restrict__ adj,
+    const CycleTask* __restrict__ tasks, uint32_t n_tasks, unsigned long long* __restrict__ out) {
+  __shared__ uint32_t s_key[kLightSlots];
+  __shared__ uint32_t s_cnt[kLightSlots];
+  constexpr uint32_t mask = kLightSlots - 1;
+  uint64_t acc = 0;
+  for (uint32_t q = blockIdx.x; q < n_tasks; q += gridDim.x) {
+    CycleTask t = tasks[q];
+    t.u = uniform(t.u);
+    t.n_below = uniform(t.n_below);
+    t.lo = uniform(t.lo);
+    t.hi = uniform(t.hi);
+    for (uint32_t i = threadIdx.x; i < kLightSlots; i += kLightBlock) {
+      s_key[i] = kEmpty;
+      s_cnt[i] = 0u;
+    }
+    __syncthreads();
+    for_wedges<kLightBlock>(off, adj, t, [&](uint32_t x) {
+      uint32_t h = hslot(x, mask);
+      while (true) {
+        const uint32_t old = atomicCAS(&s_key[h], kEmpty, x);
+        if (old == kEmpty || old == x) break;
+        h = (h + 1) & mask;
+      }
+      acc += atomicAdd(&s_cnt[h], 1u);
+    });
+    __syncthreads();
+  }
+  acc = wave_sum_u64(acc);
+  if (lane_id() == 0 && acc) atomicAdd(out, (unsigned long long)acc);
+}
+
+// below[u] = neighbours of u of lower rank; wedges[u] = sum over them of their
+// neighbours below u (zero on entry): the entry (v, u) of v's list adds its
+// position, as many entries as v has below u.  One wave per v.
+__global__ __launch_bounds__(kBlock) void wedge_totals_kernel(
+    const uint32_t* __restrict__ off, const uint32_t* __restrict__ adj, uint32_t n,
+    uint32_t* __restrict__ below, unsigned long long* __restrict__ wedges) {
+  const uint32_t lane = lane_id();
+  const uint32_t nw = gridDim.x * blockDim.x / kWave;
+  for (uint32_t v = (blockIdx.x * blockDim.x + threadIdx.x) / kWave; v < n; v += nw) {
+    const uint32_t b = off[v], len = off[v + 1] - b;
+    const uint32_t first = count_below(adj + b, len, v);
+    if (lane == 0) below[v] = first;
+    for (uint32_t p = first + lane; p < len; p += kWave)
+      if (p) atomicAdd(&wedges[adj[b + p]], (unsigned long long)p);
+  }
 }
 
 __global__ void zero_u32_kernel(unsigned int* p, uint64_t count) {
@@ -376,6 +616,94 @@ int ensure_rank_csr(gpm_graph* g) {
   if (hipStreamSynchronize(g->stream) != hipSuccess)
     return fail_all(fail(GPM_EHIP, "building the rank-relabelled graph"));
   cleanup();
+  g->motif.h_off.swap(rk_off);
+  return GPM_OK;
+}
+
+// Degree of the vertex of rank v.
+uint32_t rk_degree(const gpm_graph* g, uint32_t v) {
+  return g->motif.h_off[v + 1] - g->motif.h_off[v];
+}
+
+// The tasks of the motif counters (g->motif), built once per handle from every
+// vertex's lower neighbours and wedge total.
+int ensure_motif_tasks(gpm_graph* g) {
+  if (g->motif.built) return GPM_OK;
+  const uint32_t n = g->n;
+  int st = ensure_scratch(g, (size_t)n * 8 + 64);
+  if (st != GPM_OK) return st;
+  unsigned long long* d_wedges = static_cast<unsigned long long*>(g->scratch);
+  if (!g->motif.below && hipMalloc(&g->motif.below, (size_t)std::max(n, 1u) * 4) != hipSuccess) {
+    g->motif.below = nullptr;
+    (void)hipGetLastError();
+    return fail(GPM_ENOMEM, "lower-neighbour counts (%u)", n);
+  }
+  uint32_t* d_below = g->motif.below;
+  std::vector<unsigned long long> wedges(n);
+  std::vector<uint32_t> below(n);
+  if (n) {
+    hipLaunchKernelGGL(zero_u32_kernel, dim3(grid_of(g, 2ull * n)), dim3(256), 0, g->stream,
+                       reinterpret_cast<unsigned int*>(d_wedges), 2ull * n);
+    hipLaunchKernelGGL(wedge_totals_kernel, dim3(grid_of(g, (uint64_t)n * kWave)), dim3(kBlock), 0,
+                       g->stream, g->rk_off, g->rk_adj, n, d_below, d_wedges);
+    GPM_HIP(hipGetLastError());
+    GPM_HIP(hipMemcpyAsync(wedges.data(), d_wedges, (size_t)n * 8, hipMemcpyDeviceToHost,
+                           g->stream));
+    GPM_HIP(hipMemcpyAsync(below.data(), d_below, (size_t)n * 4, hipMemcpyDeviceToHost,
+                           g->stream));
+    GPM_HIP(hipStreamSynchronize(g->stream));
+  }
+  std::vector<uint32_t> roots;
+  std::vector<CycleTask> heavy, light;
+  for (uint32_t u = n; u-- > 0;) {
+    if (wedges[u] >= kCycHeavy)
+      roots.push_back(u);
+    else if (wedges[u] >= 2)
+      light.push_back({u, below[u], 0u, u, 0u});
+  }
+  std::stable_sort(roots.begin(), roots.end(),
+                   [&](uint32_t a, uint32_t b) { return wedges[a] > wedges[b]; });
+  bool hbm = false;
+  for (const uint32_t u : roots) {
+    const uint32_t band = below[u] < 65536u ? 2 * kCycWords : kCycWords;
+    uint32_t hi = u;
+    auto task_to = [&](uint32_t lo) {
+      heavy.push_back({u, below[u], lo, hi, hi - lo > band ? hi - band : lo});
+      hi = lo;
+    };
+    const uint32_t first = u > band ? u - band : 0u;
+    if (wedges[u] >= kCycBand1 && first) task_to(first);
+    if (wedges[u] >= kCycBand2 && hi > band) task_to(hi - band);
+    hbm |= hi > band;
+    if (hi) task_to(0u);
+  }
+  // Triangle tasks, in decreasing degree (rank).
+  std::vector<TriangleTask> tri;
+  for (uint32_t v = n; v-- > 0;) {
+    const uint32_t deg = rk_degree(g, v), high = deg - below[v];
+    if (deg <= kTriPairs) break;  // so have all vertices of lower rank
+    if (!high) continue;
+    // Higher neighbours only where v's pairs are not searched.
+    const uint32_t end = high > kTriPairs ? deg : below[v];
+    for (uint32_t c = 0; c < end; c += kTriLists) tri.push_back({v, c, std::min(end, c + kTriLists)});
+  }
+  auto put = [&](const auto& list, void** d) -> int {
+    if (list.empty()) return GPM_OK;
+    if (hipMalloc(d, list.size() * sizeof(list[0])) != hipSuccess) {
+      *d = nullptr;
+      (void)hipGetLastError();
+      return fail(GPM_ENOMEM, "motif tasks (%zu)", list.size());
+    }
+    return h2d(g, *d, list.data(), list.size() * sizeof(list[0]));
+  };
+  if ((st = put(heavy, &g->motif.heavy)) != GPM_OK || (st = put(light, &g->motif.light)) != GPM_OK ||
+      (st = put(tri, &g->motif.triangles)) != GPM_OK)
+    return st;
+  g->motif.n_heavy = (uint32_t)heavy.size();
+  g->motif.n_light = (uint32_t)light.size();
+  g->motif.n_triangles = (uint32_t)tri.size();
+  g->motif.hbm = hbm;
+  g->motif.built = true;
   return GPM_OK;
 }
 
@@ -387,22 +715,17 @@ int motif4_by_identities(gpm_graph* g, uint64_t out[6]) {
   int st;
   if ((st = ensure_rank_csr(g)) != GPM_OK) return st;
   if (!g->dag && (st = gpm_graph_orient(g, &g->dag)) != GPM_OK) return st;
-  if ((st = ensure_src(g->dag)) != GPM_OK) return st;
+  if ((st = ensure_motif_tasks(g)) != GPM_OK) return st;
   const int cus = device_cus(g);
-  // Scratch: per block, n 4-cycle counters and a list of up to n touched
-  // counters; kCycBlocksPerCu blocks of kCycBlock threads per CU, within
-  // 8 GiB (fewer blocks when that much is not free).  The wedge increments
-  // are random atomics into these arrays: more or wider blocks keep more of
-  // them in flight but spread them over more memory.  4-cycle corners on
-  // R-MAT scale 22 (blocks x threads): 256 x 256 1.96 s, 128 x 256 2.62 s,
-  // 512 x 256 2.24 s, 1024 x 256 2.91 s, 2048 x 256 2.97 s, 256 x 512 2.47 s,
-  // 256 x 1024 3.64 s, 128 x 1024 3.44 s.
-  const uint64_t stride = 2 * (uint64_t)std::max<uint32_t>(g->n, 1);
-  unsigned blocks_c = (unsigned)std::min<uint64_t>((uint64_t)cus * kCycBlocksPerCu, std::max(g->n, 1u));
+  const auto& tk = g->motif;
+  // Scratch: where some root's ranks pass its LDS bands, n 4-cycle counters per
+  // block, within 8 GiB (fewer blocks when that much is not free).
+  const uint64_t stride = tk.hbm ? g->n : 0;
+  unsigned blocks_c = (unsigned)std::min<uint64_t>(cus, std::max(tk.n_heavy, 1u));
   while (blocks_c > 16 && (uint64_t)blocks_c * stride * 4 > (8ull << 30)) blocks_c /= 2;
-  // The per-edge triangle counts (one uint32 per DAG edge) use the same
+  // The per-edge triangle counts (one uint32 per adjacency entry) use the same
   // scratch before the 4-cycle counters do.
-  const uint64_t tri_bytes = std::max<uint64_t>(g->dag->m, 1) * 4;
+  const uint64_t tri_bytes = std::max<uint64_t>(g->m, 1) * 4;
   while (true) {
     const uint64_t want = std::max((uint64_t)blocks_c * stride * 4, tri_bytes) + 256;
     if ((st = ensure_scratch(g, want)) == GPM_OK) break;
@@ -413,29 +736,44 @@ int motif4_by_identities(gpm_graph* g, uint64_t out[6]) {
   const uint64_t cyc_bytes = (uint64_t)blocks_c * stride * 4;
   uint32_t* tri = static_cast<uint32_t*>(g->scratch);
   uint32_t* ccnt = static_cast<uint32_t*>(g->scratch);
+  // Kernels that end in a sum over all blocks: at most 8 blocks per CU.
+  auto sum_grid = [&](uint64_t threads) {
+    return (unsigned)std::min<uint64_t>(grid_of(g, threads), (uint64_t)cus * 8);
+  };
   if ((st = timing_begin(g)) != GPM_OK) return st;
   if ((st = zero_counters(g, 16)) != GPM_OK) return st;
   unsigned int* queue = reinterpret_cast<unsigned int*>(g->counters + 8);
-  const uint64_t me = g->dag->m;
-  if (me) {
-    hipLaunchKernelGGL(zero_u32_kernel, dim3(grid_of(g, me)), dim3(256), 0, g->stream, tri, me);
-    hipLaunchKernelGGL(edge_triangles_kernel<8>, dim3(grid_of(g, me * 8)), dim3(kBlock), 0,
-                       g->stream, g->dag->off, g->dag->adj, g->dag->src, me, tri);
-    hipLaunchKernelGGL(edge_stats_kernel, dim3(grid_of(g, me)), dim3(kBlock), 0, g->stream,
-                       g->off, g->dag->src, g->dag->adj, tri, me, g->counters);
+  if (g->m) {
+    hipLaunchKernelGGL(zero_u32_kernel, dim3(grid_of(g, g->m)), dim3(256), 0, g->stream, tri, g->m);
+    if (tk.n_triangles)
+      hipLaunchKernelGGL(stream_triangles_kernel,
+                         dim3((unsigned)std::min<uint64_t>(tk.n_triangles, (uint64_t)cus * 8)),
+                         dim3(kBlock), 0, g->stream, g->rk_off, g->rk_adj, tk.below, g->n,
+                         static_cast<const TriangleTask*>(tk.triangles), tk.n_triangles, tri);
+    hipLaunchKernelGGL(pair_triangles_kernel, dim3(grid_of(g, (uint64_t)g->n * kTriPairs)),
+                       dim3(kBlock), 0, g->stream, g->rk_off, g->rk_adj, tk.below, g->n, tri);
+    hipLaunchKernelGGL(edge_stats_kernel, dim3(sum_grid((uint64_t)g->n * kWave)), dim3(kBlock), 0,
+                       g->stream, g->rk_off, g->rk_adj, tk.below, tri, g->n, g->counters);
     GPM_HIP(hipGetLastError());
   }
   timing_mark(g, "motif_edge_sums");
-  hipLaunchKernelGGL(star_sum_kernel, dim3(grid_of(g, g->n)), dim3(kBlock), 0, g->stream, g->off,
+  hipLaunchKernelGGL(star_sum_kernel, dim3(sum_grid(g->n)), dim3(kBlock), 0, g->stream, g->off,
                      g->n, g->counters);
   GPM_HIP(hipGetLastError());
   timing_mark(g, "motif_star_sum");
   // The 4-cycle counters start at zero (the triangle counts lived here).
-  const uint64_t zero_n = cyc_bytes / 4;
-  hipLaunchKernelGGL(zero_u32_kernel, dim3(grid_of(g, zero_n)), dim3(256), 0, g->stream, ccnt,
-                     zero_n);
-  hipLaunchKernelGGL(cycles_kernel<kCycBlock>, dim3(blocks_c), dim3(kCycBlock), 0, g->stream,
-                     g->rk_off, g->rk_adj, g->n, queue, ccnt, stride, g->counters + 5);
+  if (cyc_bytes)
+    hipLaunchKernelGGL(zero_u32_kernel, dim3(grid_of(g, cyc_bytes / 4)), dim3(256), 0, g->stream,
+                       ccnt, cyc_bytes / 4);
+  if (tk.n_heavy)
+    hipLaunchKernelGGL(cycles_kernel, dim3(blocks_c), dim3(kCycBlock), 0, g->stream, g->rk_off,
+                       g->rk_adj, g->n, static_cast<const CycleTask*>(tk.heavy), tk.n_heavy, queue,
+                       ccnt, g->counters + 5);
+  if (tk.n_light)
+    hipLaunchKernelGGL(light_cycles_kernel,
+                       dim3((unsigned)std::min<uint64_t>(tk.n_light, (uint64_t)cus * 5)),
+                       dim3(kLightBlock), 0, g->stream, g->rk_off, g->rk_adj,
+                       static_cast<const CycleTask*>(tk.light), tk.n_light, g->counters + 5);
   GPM_HIP(hipGetLastError());
   timing_mark(g, "motif_cycles");
   if ((st = timing_end(g)) != GPM_OK) return st;
