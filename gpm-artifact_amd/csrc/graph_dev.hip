@@ -259,6 +259,8 @@ void release(gpm_graph* g) {
   hipFree(g->ladj);
   hipFree(g->loff);
   hipFree(g->lverts);
+  (void)hipFree(g->lpos);
+  (void)hipFree(g->lloc);
   (void)hipFree(g->sig);
   (void)hipFree(g->toff);
   (void)hipFree(g->tadj);

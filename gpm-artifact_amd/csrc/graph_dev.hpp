@@ -34,6 +34,10 @@ struct gpm_graph {
   // per label l, min(15, neighbours of label l) in bits 4l..4l+3 -- the
   // matcher's degree and neighbour-label filter in one load.
   unsigned long long* sig = nullptr;
+  // Position of every vertex in lverts within its label, and of every ladj entry's
+  // vertex, built on first use by the matcher.
+  uint32_t* lpos = nullptr;
+  uint32_t* lloc = nullptr;
   // Vertices grouped by label: lverts[h_lvoff[l] .. h_lvoff[l+1]) have label l.
   uint32_t* lverts = nullptr;
   std::vector<uint32_t> h_lvoff;

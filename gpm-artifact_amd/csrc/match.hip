@@ -39,6 +39,7 @@
 //  * With a fixed chunk, the launch (counter reset + enumeration) can be
 //    built once as a two-node hipGraph and replayed.
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <numeric>
 #include <queue>
@@ -711,6 +712,196 @@ __global__ __launch_bounds__(kBlock) void match_kernel(
   }
 }
 
+// ------------------------------------------------------------------ squares
+//
+// A 4-cycle's plan: depths 1 and 2 (a, b) both hang on the root alone, and depth
+// 3 (x) on a and b.  The DFS would intersect the lists of every pair (a, b) of
+// the root's neighbours; the pairs are not needed.  With A(x) the number of a
+// that x is a neighbour of, the root's count is
+//     sum over b, x in N(b) of A(x), less 1 where b is itself one of the a
+// (b stands for a different vertex than a), over the x that pass depth 3's
+// filter and are not the root: linear in the lists instead of quadratic.  A
+// block keeps A(x) in LDS, 16 bits (32 where a root has more than 65535 a) per vertex of x's label in the order of lverts,
+// a band of them at a time where a label has more vertices than fit.  Bound by the
+// latency of the list loads and the LDS atomics behind them; the three walks
+// (count, look up, clear) read lists that the L2 holds.  R-MAT scale 18 ef 16
+// with 8 labels: 30.8 ms of DFS -> 0.29 ms; scale 14 with 2: 32.3 -> 0.35.
+constexpr int kSquareBlock = 512;
+constexpr uint32_t kSquareWords = 18432;  // of counters: 72 KiB, two blocks per CU
+constexpr uint32_t kSquareWindows = 2;   // 64-entry windows in flight per wave
+constexpr uint32_t kSquareSingles = 2048;  // roots fetched one by one, then 8 at a time
+
+// lpos[v] = position of v among the vertices of its label (lverts order).
+__global__ __launch_bounds__(kBlock) void label_positions_kernel(
+    const uint32_t* __restrict__ lverts, const uint32_t* __restrict__ lvoff, uint32_t L,
+    uint32_t* __restrict__ lpos) {
+  for (uint32_t l = blockIdx.y; l < L; l += gridDim.y)
+    for (uint32_t i = lvoff[l] + blockIdx.x * blockDim.x + threadIdx.x; i < lvoff[l + 1];
+         i += gridDim.x * blockDim.x)
+      lpos[lverts[i]] = i - lvoff[l];
+}
+
+// out[i] = lpos[ladj[i]].
+__global__ __launch_bounds__(kBlock) void label_entries_kernel(const uint32_t* __restrict__ ladj,
+                                                               const uint32_t* __restrict__ lpos,
+                                                               uint64_t m, uint32_t* __restrict__ out) {
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m;
+       i += (uint64_t)gridDim.x * blockDim.x)
+    out[i] = lpos[ladj[i]];
+}
+
+// Bit i of valid: the i-th vertex of depth 3's label passes its filter; one word
+// per thread.
+__global__ __launch_bounds__(kBlock) void square_valid_kernel(DevGraph g, QPlan p,
+                                                              const uint32_t* __restrict__ verts,
+                                                              uint32_t count,
+                                                              uint32_t* __restrict__ valid) {
+  for (uint32_t w = blockIdx.x * blockDim.x + threadIdx.x; w < (count + 31) / 32;
+       w += gridDim.x * blockDim.x) {
+    uint32_t bits = 0;
+    for (uint32_t k = 0; k < 32 && 32 * w + k < count; ++k)
+      bits |= (nlf_ok(g, p, 3, verts[32 * w + k]) ? 1u : 0u) << k;
+    valid[w] = bits;
+  }
+}
+
+// Calls f(i, same) for every entry of the depth-3 slices of the vertices y =
+// ladj[begin .. begin + count) that pass depth `depth`'s filter, i its position
+// among its label in [lo, hi); same: y passes depth 1's filter too and has
+// its label.  The block's waves take the y in turn.
+template <typename F>
+__device__ __forceinline__ void square_walk(const DevGraph& g, const QPlan& p,
+                                            const uint32_t* __restrict__ lloc, uint32_t begin,
+                                            uint32_t count, uint32_t depth, uint32_t lo,
+                                            uint32_t hi, bool whole, F&& f) {
+  const uint32_t lane = lane_id(), w = uniform(threadIdx.x / kWave);
+  for (uint32_t c0 = 0; c0 < count; c0 += kSquareBlock) {
+    const uint32_t mine = c0 + kSquareBlock / kWave * lane + w;
+    uint32_t b = 0, len = 0;
+    bool same = false;
+    if (mine < count) {
+      const uint32_t y = g.ladj[begin + mine];
+      if (nlf_ok(g, p, depth, y)) {
+        same = depth != 1 && p.label[1] == p.label[depth] && nlf_ok(g, p, 1, y);
+        label_slice(g, y, p.label[3], &b, &len);
+        if (!whole) {  // the slice's part in [lo, hi)
+          uint32_t e = len;
+          if (lo) {
+            const uint32_t first = upper_index(lloc + b, len, lo - 1);
+            b += first;
+            e -= first;
+          }
+          len = hi ? upper_index(lloc + b, e, hi - 1) : 0u;
+        }
+      }
+    }
+    const uint64_t sames = wave_ballot(same);
+    uint64_t todo = wave_ballot(len != 0u);
+    uint32_t cb = 0, cn = 0, ct = 0, cs = 0, x[kSquareWindows];
+    auto next = [&]() {  // moves on to the next batch of windows; false after the last
+      ct += kSquareWindows * kWave;
+      if (ct < cn) return true;
+      if (!todo) return false;
+      const uint32_t j = (uint32_t)__builtin_ctzll(todo);
+      todo &= todo - 1;
+      cb = __builtin_amdgcn_readlane(b, j);
+      cn = __builtin_amdgcn_readlane(len, j);
+      cs = (uint32_t)(sames >> j) & 1u;
+      ct = 0;
+      return true;
+    };
+    auto load = [&](uint32_t (&v)[kSquareWindows]) {
+#pragma unroll
+      for (uint32_t q = 0; q < kSquareWindows; ++q) {
+        const uint32_t at = ct + q * kWave + lane;
+        v[q] = at < cn ? lloc[cb + at] : kEmpty;
+      }
+    };
+    bool more = next();
+    if (more) load(x);
+    while (more) {
+      uint32_t y[kSquareWindows];
+      const uint32_t s = cs;
+      more = next();
+      if (more) load(y);
+#pragma unroll
+      for (uint32_t q = 0; q < kSquareWindows; ++q)
+        if (x[q] != kEmpty) f(x[q], s);
+#pragma unroll
+      for (uint32_t q = 0; q < kSquareWindows; ++q) x[q] = y[q];
+    }
+  }
+}
+
+// The roots of one square plan, heaviest first, a block per root.  `classes`:
+// vertices of depth 3's label; band: counters in LDS.
+template <bool kWide>
+__global__ __launch_bounds__(kSquareBlock) void square_kernel(
+    DevGraph g, QPlan p, const uint32_t* __restrict__ lloc, const uint32_t* __restrict__ lpos,
+    const uint32_t* __restrict__ roots, uint32_t n_roots, const uint32_t* __restrict__ valid,
+    uint32_t classes, uint32_t band, unsigned int* __restrict__ queue,
+    unsigned long long* __restrict__ count) {
+  extern __shared__ uint32_t s_square[];  // counters (two per word), valid bits of the band
+  __shared__ uint32_t s_ticket;
+  const uint32_t words = kWide ? band : (band + 1) / 2;
+  uint32_t* s_valid = s_square + words;
+  const bool whole = classes <= band;
+  uint64_t acc = 0;
+  for (uint32_t i = threadIdx.x; i < words; i += kSquareBlock) s_square[i] = 0u;
+  if (whole)
+    for (uint32_t i = threadIdx.x; i < (classes + 31) / 32; i += kSquareBlock) s_valid[i] = valid[i];
+  while (true) {
+    if (threadIdx.x == 0) s_ticket = atomicAdd(queue, 1u);
+    __syncthreads();
+    const uint32_t t = uniform(s_ticket);
+    __syncthreads();
+    const uint32_t r0 = t < kSquareSingles ? t : kSquareSingles + 8 * (t - kSquareSingles);
+    if (r0 >= n_roots) break;
+    const uint32_t r1 = min(n_roots, t < kSquareSingles ? r0 + 1 : r0 + 8);
+    for (uint32_t r = r0; r < r1; ++r) {
+      const uint32_t v0 = uniform(roots[r]);
+      uint32_t ab, an, bb, bn;
+      label_slice(g, v0, p.label[1], &ab, &an);
+      label_slice(g, v0, p.label[2], &bb, &bn);
+      ab = uniform(ab);
+      an = uniform(an);
+      bb = uniform(bb);
+      bn = uniform(bn);
+      if (!an || !bn) continue;
+      const uint32_t self = p.label[3] == p.label[0] ? uniform(lpos[v0]) : kEmpty;
+      for (uint32_t lo = 0; lo < classes; lo += band) {
+        const uint32_t hi = min(classes, lo + band);
+        if (!whole)  // band is a multiple of 32 then
+          for (uint32_t i = threadIdx.x; i < (hi - lo + 31) / 32; i += kSquareBlock)
+            s_valid[i] = valid[lo / 32 + i];
+        square_walk(g, p, lloc, ab, an, 1, lo, hi, whole, [&](uint32_t x, uint32_t) {
+          const uint32_t i = x - lo;
+          if (kWide)
+            atomicAdd(&s_square[i], 1u);
+          else
+            atomicAdd(&s_square[i >> 1], 1u << (i & 1) * 16);
+        });
+        __syncthreads();
+        square_walk(g, p, lloc, bb, bn, 2, lo, hi, whole, [&](uint32_t x, uint32_t same) {
+          const uint32_t i = x - lo;
+          if (x != self && (s_valid[i >> 5] >> (i & 31)) & 1u)
+            acc += (kWide ? s_square[i] : (s_square[i >> 1] >> (i & 1) * 16) & 0xFFFFu) - same;
+        });
+        __syncthreads();
+        square_walk(g, p, lloc, ab, an, 1, lo, hi, whole, [&](uint32_t x, uint32_t) {
+          if (kWide)
+            s_square[x - lo] = 0u;
+          else
+            reinterpret_cast<uint16_t*>(s_square)[x - lo] = 0;
+        });
+        __syncthreads();
+      }
+    }
+  }
+  acc = wave_sum_u64(acc);
+  if (lane_id() == 0 && acc) atomicAdd(count, (unsigned long long)acc);
+}
+
 __global__ void zero_f32_kernel(float* a, uint64_t n) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (uint64_t)gridDim.x * blockDim.x)
@@ -1065,6 +1256,18 @@ struct MatchBatch {
   size_t pass_cap = 0;
   unsigned int* d_abort = nullptr;    // own allocation: count, then indices
   size_t abort_cap = 0;
+  // Square plans, counted apart from the tasks: their plans, and in d_square (own
+  // allocation) their roots, valid bits, queues and, per query, counts.
+  struct Square {
+    QPlan plan;
+    const uint32_t *roots, *valid;
+    uint32_t n_roots, classes;
+    bool wide;
+  };
+  std::vector<Square> squares;
+  uint32_t* d_square = nullptr;
+  unsigned int* d_square_queue = nullptr;
+  unsigned long long* d_square_counts = nullptr;
   uint32_t n_heavy = 0, split_len = 0;
   uint32_t nq = 0, n_tasks = 0;
   int n_queries = 0;
@@ -1084,6 +1287,7 @@ void free_batch(void* p) {
   (void)hipFree(b->d_log);
   (void)hipFree(b->d_pass);
   (void)hipFree(b->d_abort);
+  (void)hipFree(b->d_square);
   delete b;
 }
 
@@ -1427,6 +1631,155 @@ int predict_root_costs(gpm_graph* g, const DevGraph& dg, const QPlan* d_plans, u
   return GPM_OK;
 }
 
+// Counters of a band.
+uint32_t square_band(bool wide) { return wide ? kSquareWords : 2 * kSquareWords; }
+
+// Whether plan p is a 4-cycle's; then *sq is p with both neighbours of the root
+// before the vertex opposite (see square_kernel).
+bool square_plan(const QPlan& p, QPlan* sq) {
+  if (p.n != 4 || p.bn[1] != 1u) return false;
+  *sq = p;
+  if (p.bn[2] == 1u && p.bn[3] == 6u) return true;
+  if (p.bn[2] != 2u || p.bn[3] != 5u) return false;
+  std::swap(sq->label[2], sq->label[3]);
+  std::swap(sq->qdeg[2], sq->qdeg[3]);
+  std::swap(sq->nlf_n[2], sq->nlf_n[3]);
+  std::swap(sq->nlf_label[2], sq->nlf_label[3]);
+  std::swap(sq->nlf_count[2], sq->nlf_count[3]);
+  return true;
+}
+
+// Builds g->lpos and g->lloc if missing.
+int ensure_label_positions(gpm_graph* g, const uint32_t* d_lvoff) {
+  if (g->lloc) return GPM_OK;
+  uint32_t *lpos = nullptr, *lloc = nullptr;
+  if (hipMalloc(&lpos, (size_t)std::max(g->n, 1u) * 4) != hipSuccess ||
+      hipMalloc(&lloc, std::max<uint64_t>(g->m, 1) * 4) != hipSuccess) {
+    (void)hipFree(lpos);
+    (void)hipGetLastError();
+    return fail(GPM_ENOMEM, "label positions");
+  }
+  const unsigned cus = (unsigned)device_cus(g);
+  hipLaunchKernelGGL(label_positions_kernel, dim3(cus, std::min(g->n_labels, 64u)), dim3(kBlock), 0,
+                     g->stream, g->lverts, d_lvoff, g->n_labels, lpos);
+  hipLaunchKernelGGL(label_entries_kernel, dim3(cus * 8), dim3(kBlock), 0, g->stream, g->ladj, lpos,
+                     g->m, lloc);
+  if (hipGetLastError() != hipSuccess || hipStreamSynchronize(g->stream) != hipSuccess) {
+    (void)hipFree(lpos);
+    (void)hipFree(lloc);
+    return fail(GPM_EHIP, "label positions");
+  }
+  g->lpos = lpos;
+  g->lloc = lloc;
+  return GPM_OK;
+}
+
+// Moves the roots of the square plans (which: their indexes in plans) that the
+// square kernel takes out of the batch's tasks: the lists in b->d_roots, b->d_rlen
+// and rlen are sorted by length and the plans keep the shorter end.  GPM_ENOMEM
+// changes nothing.
+int build_squares(gpm_graph* g, std::vector<QPlan>& plans, const std::vector<uint32_t>& which,
+                  std::vector<uint32_t>& rlen, const uint32_t* d_lvoff, int n_counters,
+                  MatchBatch* b) {
+  if (which.empty()) return GPM_OK;
+  int st = ensure_label_positions(g, d_lvoff);
+  if (st != GPM_OK) return st;
+  std::vector<uint32_t> roots;
+  size_t valid_words = 0;
+  std::vector<size_t> root_at, valid_at;
+  std::vector<uint32_t> taken;
+  for (const uint32_t i : which) {
+    QPlan p;
+    (void)square_plan(plans[i], &p);
+    std::vector<uint32_t> mine(p.n_roots), order(p.n_roots);
+    GPM_HIP(hipMemcpyAsync(mine.data(), b->d_roots + p.root_off, (size_t)p.n_roots * 4,
+                           hipMemcpyDeviceToHost, g->stream));
+    GPM_HIP(hipStreamSynchronize(g->stream));
+    std::iota(order.begin(), order.end(), 0u);
+    std::sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) {
+      const uint32_t lx = rlen[p.root_off + x], ly = rlen[p.root_off + y];
+      return lx > ly || (lx == ly && mine[x] < mine[y]);
+    });
+    root_at.push_back(roots.size());
+    const uint32_t classes = g->h_lvoff[p.label[3] + 1] - g->h_lvoff[p.label[3]];
+    // One band: every root with a depth-1 entry (4 labels, ER n=200k m=1M: 0.76 ms
+    // with all roots here, 0.91 with those of 16 entries and more, 0.87 all DFS).
+    // More: a pair of the DFS costs a CU 0.29 us, a band 2.9 us on light roots
+    // (no labels, same graph, 6 bands: 13.4 ms here, 20.5 from 16 entries on, 22.4
+    // all DFS; R-MAT scale 18 ef 4, 8 bands: 17.6, 16.3, 1260), so from
+    // sqrt(10 bands) entries on.
+    const bool wide = rlen[p.root_off + order[0]] > 65535u;
+    const uint32_t bands = (classes + square_band(wide) - 1) / square_band(wide);
+    const uint32_t least = bands <= 1 ? 1u : (uint32_t)std::ceil(std::sqrt(10.0 * bands));
+    uint32_t take = 0;
+    std::vector<uint32_t> lens(p.n_roots);
+    for (uint32_t k = 0; k < p.n_roots; ++k) {
+      lens[k] = rlen[p.root_off + order[k]];
+      take += lens[k] >= least;
+    }
+    std::copy(lens.begin(), lens.end(), rlen.begin() + p.root_off);
+    for (const uint32_t r : order) roots.push_back(mine[r]);
+    taken.push_back(take);
+    valid_at.push_back(valid_words);
+    valid_words += (classes + 31) / 32;
+  }
+  const size_t counts = ((size_t)n_counters + 1) * 2;  // words
+  const size_t words = counts + which.size() + valid_words;
+  if (hipMalloc(&b->d_square, words * 4) != hipSuccess) {
+    b->d_square = nullptr;
+    (void)hipGetLastError();
+    return fail(GPM_ENOMEM, "square plans (%zu words)", words);
+  }
+  b->d_square_counts = reinterpret_cast<unsigned long long*>(b->d_square);
+  b->d_square_queue = b->d_square + counts;
+  uint32_t* d_valid = b->d_square + counts + which.size();
+  for (size_t k = 0; k < which.size(); ++k) {
+    QPlan sq;
+    (void)square_plan(plans[which[k]], &sq);
+    QPlan& p = plans[which[k]];
+    if ((st = h2d(g, b->d_roots + p.root_off, roots.data() + root_at[k], (size_t)p.n_roots * 4)) != GPM_OK ||
+        (st = h2d(g, b->d_rlen + p.root_off, rlen.data() + p.root_off, (size_t)p.n_roots * 4)) != GPM_OK)
+      return st;
+    const uint32_t first = g->h_lvoff[sq.label[3]], count = g->h_lvoff[sq.label[3] + 1] - first;
+    hipLaunchKernelGGL(square_valid_kernel,
+                       dim3(std::max(1u, std::min((count + 32 * kBlock - 1) / (32 * kBlock), 1024u))),
+                       dim3(kBlock), 0, g->stream, b->dg, sq, g->lverts + first, count,
+                       d_valid + valid_at[k]);
+    GPM_HIP(hipGetLastError());
+    b->squares.push_back({sq, b->d_roots + p.root_off, d_valid + valid_at[k], taken[k], count,
+                          rlen[p.root_off] > 65535u});
+    p.root_off += taken[k];
+    p.n_roots -= taken[k];
+  }
+  return GPM_OK;
+}
+
+// Enqueues the square plans' counts of a prepared batch.
+int launch_squares(gpm_graph* g, MatchBatch* b, int n_queries) {
+  if (b->squares.empty()) return GPM_OK;
+  hipLaunchKernelGGL(zero_kernel, dim3((std::max<int>(n_queries, b->squares.size()) + 63) / 64),
+                     dim3(64), 0, g->stream, b->d_square_counts, n_queries, b->d_square_queue,
+                     (int)b->squares.size());
+  for (size_t k = 0; k < b->squares.size(); ++k) {
+    const MatchBatch::Square& q = b->squares[k];
+    if (!q.n_roots || !q.classes) continue;
+    auto* kernel = q.wide ? &square_kernel<true> : &square_kernel<false>;
+    const uint32_t band = std::min(q.classes, square_band(q.wide));
+    const size_t lds = ((q.wide ? band : (size_t)(band + 1) / 2) + (band + 31) / 32) * 4;
+    GPM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)(kSquareWords + 2 * kSquareWords / 32) * 4));
+    const unsigned per_cu = (unsigned)std::min<size_t>(4, 160 * 1024 / (lds + 1024));
+    hipLaunchKernelGGL(kernel,
+                       dim3((unsigned)std::min<uint64_t>(q.n_roots, (uint64_t)device_cus(g) * per_cu)),
+                       dim3(kSquareBlock), lds, g->stream, b->dg, q.plan, g->lloc, g->lpos, q.roots,
+                       q.n_roots, q.valid, q.classes, band, b->d_square_queue + k,
+                       b->d_square_counts + q.plan.qid);
+    GPM_HIP(hipGetLastError());
+  }
+  return GPM_OK;
+}
+
 // Lays out a batch of `plans` (plan.qid = index of its counter; n_counters
 // counters): device buffers, root candidates, chunks (roots per task) and
 // the parts of heavy roots.
@@ -1442,7 +1795,7 @@ int predict_root_costs(gpm_graph* g, const DevGraph& dg, const QPlan* d_plans, u
 // hubs represented without running them whole.
 int build_batch(gpm_graph* g, std::vector<QPlan> plans, int n_counters, const gpm_tuning& tun,
                 MatchBatch* b, std::vector<double>* scale, const float* model = nullptr,
-                bool log_roots = false) {
+                bool log_roots = false, bool squares = false) {
   const bool trial = scale != nullptr;
   const uint32_t nq0 = (uint32_t)plans.size();
   uint64_t root_total = 0;
@@ -1591,6 +1944,19 @@ int build_batch(gpm_graph* g, std::vector<QPlan> plans, int n_counters, const gp
       for (uint32_t r = 0; r < plans[i].n_roots; ++r) sum += rcost[plans[i].root_off + r];
       cost_per_root[i] = std::max(1.0, plans[i].n_roots ? sum / plans[i].n_roots : 1.0);
     }
+  }
+  // Square plans leave the tasks.  (A model sizes tasks by predicted root costs,
+  // and a hipGraph replays one launch: both keep the DFS.)
+  if (squares && !learned && !tun.use_graph) {
+    std::vector<uint32_t> which;
+    QPlan sq;
+    for (uint32_t i = 0; i < nq; ++i)
+      if (plans[i].n_roots && square_plan(plans[i], &sq)) which.push_back(i);
+    st = build_squares(g, plans, which, rlen, d_lvoff, n_counters, b);
+    if (st == GPM_ENOMEM)
+      clear_error();  // the DFS takes them
+    else if (st != GPM_OK)
+      return st;
   }
   // Chunks (roots per task) and layout, heaviest queries first when tuned.
   // A tuned chunk gives a task about kTaskWork estimated entries, but no
@@ -1941,7 +2307,7 @@ int prepare_batch(gpm_graph* g, const gpm_query* queries, int n_queries, const g
   int st = plan_queries(g, queries, n_queries, tun, &plans);
   if (st != GPM_OK) return st;
   return build_batch(g, std::move(plans), n_queries, tun, b, nullptr,
-                     tun.policy == GPM_SCHED_LEARNED ? tun.root_model : nullptr);
+                     tun.policy == GPM_SCHED_LEARNED ? tun.root_model : nullptr, false, true);
 }
 
 }  // namespace
@@ -2136,6 +2502,7 @@ extern "C" int gpm_match_batch(gpm_graph* g, const gpm_query* queries, int n_que
     if (b->pass_auto)
       passes = b->pass_ms[1] < 0.0 || (b->pass_ms[0] >= 0.0 && b->pass_ms[1] <= b->pass_ms[0]);
     if ((st = timing_begin(g)) != GPM_OK) return st;
+    if ((st = launch_squares(g, b, n_queries)) != GPM_OK) return st;
     if ((st = passes ? run_passes(g, b) : launch_batch(g, b)) != GPM_OK) return st;
     timing_mark(g, "match_batch");
     if ((st = timing_end(g)) != GPM_OK) return st;
@@ -2143,11 +2510,15 @@ extern "C" int gpm_match_batch(gpm_graph* g, const gpm_query* queries, int n_que
       double& best = b->pass_ms[passes ? 1 : 0];
       best = best < 0.0 ? g->last_ms : std::min(best, g->last_ms);
     }
-    std::vector<unsigned long long> cnt(n_queries);
-    GPM_HIP(hipMemcpyAsync(cnt.data(), b->d_counts, (size_t)n_queries * 8, hipMemcpyDeviceToHost,
-                           g->stream));
+    std::vector<unsigned long long> cnt(n_queries, 0ull), square(n_queries, 0ull);
+    if (b->n_tasks)
+      GPM_HIP(hipMemcpyAsync(cnt.data(), b->d_counts, (size_t)n_queries * 8, hipMemcpyDeviceToHost,
+                             g->stream));
+    if (!b->squares.empty())
+      GPM_HIP(hipMemcpyAsync(square.data(), b->d_square_counts, (size_t)n_queries * 8,
+                             hipMemcpyDeviceToHost, g->stream));
     GPM_HIP(hipStreamSynchronize(g->stream));
-    for (int i = 0; i < n_queries; ++i) per_query[i] = cnt[i];
+    for (int i = 0; i < n_queries; ++i) per_query[i] = cnt[i] + square[i];
     return GPM_OK;
   });
 }
