@@ -26,53 +26,6 @@ __global__ void build_src_kernel(const uint32_t* __restrict__ off,
   }
 }
 
-// Orientation pass 1: out-degree under the rule of graph.h:128-129.
-__global__ void orient_count_kernel(const uint32_t* __restrict__ off,
-                                    const uint32_t* __restrict__ adj,
-                                    uint32_t n, uint32_t* __restrict__ cnt) {
-  const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-  const uint32_t nwaves = gridDim.x * blockDim.x / kWave;
-  const uint32_t lane = lane_id();
-  for (uint32_t u = wave; u < n; u += nwaves) {
-    const uint32_t b = off[u], e = off[u + 1], du = e - b;
-    uint32_t c = 0;
-    for (uint32_t i = b + lane; i < e; i += kWave) {
-      const uint32_t v = adj[i];
-      const uint32_t dv = off[v + 1] - off[v];
-      c += (dv > du || (dv == du && v > u)) ? 1u : 0u;
-    }
-    c = wave_sum_u32(c);
-    if (lane == 0) cnt[u] = c;
-  }
-}
-
-// Orientation pass 2: stable compaction of each list (order kept).
-__global__ void orient_fill_kernel(const uint32_t* __restrict__ off,
-                                   const uint32_t* __restrict__ adj, uint32_t n,
-                                   const uint32_t* __restrict__ new_off,
-                                   uint32_t* __restrict__ new_adj) {
-  const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-  const uint32_t nwaves = gridDim.x * blockDim.x / kWave;
-  const uint32_t lane = lane_id();
-  for (uint32_t u = wave; u < n; u += nwaves) {
-    const uint32_t b = off[u], e = off[u + 1], du = e - b;
-    uint32_t pos = new_off[u];
-    for (uint32_t i0 = b; i0 < e; i0 += kWave) {
-      const uint32_t i = i0 + lane;
-      bool keep = false;
-      uint32_t v = 0;
-      if (i < e) {
-        v = adj[i];
-        const uint32_t dv = off[v + 1] - off[v];
-        keep = dv > du || (dv == du && v > u);
-      }
-      const uint64_t mask = wave_ballot(keep);
-      if (keep) new_adj[pos + lanes_below(mask)] = v;
-      pos += (uint32_t)__popcll(mask);
-    }
-  }
-}
-
 int grid_for(const gpm_graph* g, uint64_t items, int block) {
   int cus = device_cus(g);
   uint64_t want = (items + block - 1) / block;
@@ -514,65 +467,27 @@ int gpm_graph_orient(gpm_graph* sym, gpm_graph** dag) {
     clear_error();
     GPM_CHECK_ARG(sym && dag, "null pointer");
     GPM_CHECK_ARG(sym->flags & GPM_GRAPH_SYMMETRIC, "graph is not SYMMETRIC");
-    const uint32_t n = sym->n;
-    uint32_t* cnt = nullptr;
-    GPM_HIP(hipMalloc(&cnt, (size_t)(n + 1) * 4));
-    const int grid = grid_for(sym, (uint64_t)n * kWave, 256);
     int st = timing_begin(sym);
-    if (st != GPM_OK) {
-      hipFree(cnt);
-      return st;
-    }
-    hipLaunchKernelGGL(orient_count_kernel, dim3(grid), dim3(256), 0, sym->stream, sym->off,
-                       sym->adj, n, cnt);
-    std::vector<uint32_t> h_cnt(n + 1, 0);
-    if (hipMemcpyAsync(h_cnt.data(), cnt, (size_t)n * 4, hipMemcpyDeviceToHost, sym->stream) !=
-            hipSuccess ||
-        hipStreamSynchronize(sym->stream) != hipSuccess) {
-      hipFree(cnt);
-      return fail(GPM_EHIP, "orientation count pass failed");
-    }
-    // Exclusive scan on the host (n+1 entries); the list pass is on the GPU.
-    std::vector<uint32_t> h_new(n + 1, 0);
-    uint32_t maxd = 0;
-    for (uint32_t v = 0; v < n; ++v) {
-      h_new[v + 1] = h_new[v] + h_cnt[v];
-      maxd = std::max(maxd, h_cnt[v]);
-    }
-    const uint64_t m2 = h_new[n];
+    if (st != GPM_OK) return st;
+    uint32_t *off = nullptr, *adj = nullptr;
+    std::vector<uint32_t> h_off;
+    if ((st = orient_device(sym, &off, &adj, &h_off)) != GPM_OK) return st;
     gpm_graph* g = new gpm_graph();
     g->device = sym->device;
-    g->n = n;
-    g->m = m2;
-    g->max_deg = maxd;
+    g->n = sym->n;
+    g->m = h_off.back();
     g->flags = GPM_GRAPH_ORIENTED;
-    g->h_off = h_new;
-    do {
-      if (hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking) != hipSuccess ||
-          hipEventCreate(&g->ev0) != hipSuccess || hipEventCreate(&g->ev1) != hipSuccess) {
-        st = fail(GPM_EHIP, "stream/event creation failed");
-        break;
-      }
-      if (hipMalloc(&g->off, (size_t)(n + 1) * 4) != hipSuccess ||
-          hipMalloc(&g->adj, std::max<uint64_t>(m2, 1) * 4) != hipSuccess ||
-          hipMalloc(&g->counters, 64 * sizeof(unsigned long long)) != hipSuccess) {
-        st = fail(GPM_ENOMEM, "device CSR allocation");
-        break;
-      }
-      if (hipMemcpyAsync(g->off, h_new.data(), (size_t)(n + 1) * 4, hipMemcpyHostToDevice,
-                         sym->stream) != hipSuccess) {
-        st = fail(GPM_EHIP, "H2D of offsets failed");
-        break;
-      }
-      hipLaunchKernelGGL(orient_fill_kernel, dim3(grid), dim3(256), 0, sym->stream, sym->off,
-                         sym->adj, n, g->off, g->adj);
-      if (hipGetLastError() != hipSuccess) {
-        st = fail(GPM_EHIP, "orientation fill launch failed");
-        break;
-      }
+    g->off = off;
+    g->adj = adj;
+    for (uint32_t v = 0; v < g->n; ++v) g->max_deg = std::max(g->max_deg, h_off[v + 1] - h_off[v]);
+    g->h_off = std::move(h_off);
+    if (hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking) != hipSuccess ||
+        hipEventCreate(&g->ev0) != hipSuccess || hipEventCreate(&g->ev1) != hipSuccess)
+      st = fail(GPM_EHIP, "stream/event creation failed");
+    else if (hipMalloc(&g->counters, 64 * sizeof(unsigned long long)) != hipSuccess)
+      st = fail(GPM_ENOMEM, "device counters");
+    else
       st = timing_end(sym);
-    } while (0);
-    hipFree(cnt);
     if (st != GPM_OK) {
       release(g);
       return st;

@@ -137,6 +137,9 @@ int ensure_topo(gpm_graph* g);
 // The same where the order by total degree is topological; otherwise (and where
 // its buffers do not fit) g->toff stays null and the status is GPM_OK.
 int try_topo(gpm_graph* g);
+// Orients the SYMMETRIC graph by (degree, id) (prep.hip): CSR in new device buffers
+// *d_off, *d_adj, the caller's, and the offsets on the host; lists keep their order.
+int orient_device(gpm_graph* sym, uint32_t** d_off, uint32_t** d_adj, std::vector<uint32_t>* h_off);
 // Relabels the ORIENTED graph g by (out-degree + in-degree, id) on the device
 // (prep.hip).  Where every edge goes up in that order -- gpm_graph_orient and
 // gpm_csr_orient give such graphs -- *ordered is set and *toff / *tadj /

@@ -41,11 +41,33 @@ int bits_for(uint64_t max_value) {
   return b;
 }
 
+__global__ void zero_words_kernel(uint32_t* a, uint32_t n) {
+  for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) a[i] = 0u;
+}
+
+// What a pass over the edges found: checks[0] endpoints outside the graph,
+// checks[2..3] self loops (64 bits; one addition per block, since additions to one
+// address take about 10 ns each).
+__device__ __forceinline__ void add_checks(bool bad, uint32_t loops, uint32_t* checks) {
+  __shared__ uint32_t s_loops;
+  if (threadIdx.x == 0) s_loops = 0u;
+  __syncthreads();
+  if (wave_ballot(bad) && lane_id() == 0) checks[0] = 1u;
+  loops = wave_sum_u32(loops);
+  if (lane_id() == 0 && loops) atomicAdd(&s_loops, loops);
+  __syncthreads();
+  if (threadIdx.x == 0 && s_loops)
+    atomicAdd(reinterpret_cast<unsigned long long*>(checks + 2), (unsigned long long)s_loops);
+}
+
 // Records of edge i: (u, v) and, when symmetrising, (v, u) right after it.
 __global__ void emit_keys_kernel(const uint32_t* __restrict__ src, const uint32_t* __restrict__ dst,
                                  uint64_t n_edges, uint32_t n, bool sym, bool drop_self,
-                                 unsigned long long* __restrict__ keys) {
+                                 unsigned long long* __restrict__ keys,
+                                 uint32_t* __restrict__ checks) {
   const uint32_t per = sym ? 2u : 1u;
+  bool bad = false;
+  uint32_t loops = 0;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_edges;
        i += (uint64_t)gridDim.x * blockDim.x) {
     const uint32_t u = src[i], v = dst[i];
@@ -53,14 +75,20 @@ __global__ void emit_keys_kernel(const uint32_t* __restrict__ src, const uint32_
     const unsigned long long sentinel = (unsigned long long)n << 32;
     keys[per * i] = drop ? sentinel : ((unsigned long long)u << 32 | v);
     if (sym) keys[per * i + 1] = drop ? sentinel : ((unsigned long long)v << 32 | u);
+    bad |= u >= n || v >= n;
+    loops += u == v;
   }
+  add_checks(bad, loops, checks);
 }
 
 // Input-order mode: source keys (n for dropped records) and target values.
 __global__ void emit_pairs_kernel(const uint32_t* __restrict__ src, const uint32_t* __restrict__ dst,
                                   uint64_t n_edges, uint32_t n, bool sym, bool drop_self,
-                                  uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
+                                  uint32_t* __restrict__ keys, uint32_t* __restrict__ vals,
+                                  uint32_t* __restrict__ checks) {
   const uint32_t per = sym ? 2u : 1u;
+  bool bad = false;
+  uint32_t loops = 0;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_edges;
        i += (uint64_t)gridDim.x * blockDim.x) {
     const uint32_t u = src[i], v = dst[i];
@@ -71,7 +99,10 @@ __global__ void emit_pairs_kernel(const uint32_t* __restrict__ src, const uint32
       keys[per * i + 1] = drop ? n : v;
       vals[per * i + 1] = u;
     }
+    bad |= u >= n || v >= n;
+    loops += u == v;
   }
+  add_checks(bad, loops, checks);
 }
 
 __global__ void split_keys_kernel(const unsigned long long* __restrict__ keys, uint64_t m,
@@ -124,8 +155,84 @@ __global__ void relabel_keys_kernel(const uint32_t* __restrict__ off, const uint
   }
 }
 
+// Orientation of a symmetric CSR, by entries: every list has a hub's length or a
+// leaf's, so a wave or block per list leaves the hubs for last.  Pass 1 decides each
+// entry (u, v) -- kept when (deg, id) of v is above u's (graph.h:128-129) -- and writes one bit per
+// entry and a count per 64; after a scan of the counts, pass 2 compacts the
+// entries and a pass over the vertices reads the new offsets off the bits.  Pass 1 is
+// bound by the gathers of off[v]; the other two stream.  R-MAT scale 17 ef 16 (3.7 M
+// entries): the two passes of a wave per list took 336 + 380 us, the three take
+// 37 + 9 + 4 us.
+constexpr uint32_t kOrientEntries = 2048;  // per block and step of pass 1
+constexpr uint32_t kOrientOffsets = 1024;  // offsets kept in LDS, where that covers them
+
+__global__ __launch_bounds__(kBlock) void orient_bits_kernel(
+    const uint32_t* __restrict__ off, const uint32_t* __restrict__ adj, uint32_t n, uint64_t m,
+    unsigned long long* __restrict__ bits, uint32_t* __restrict__ count) {
+  __shared__ uint32_t s_off[kOrientOffsets + 2];
+  for (uint64_t base = (uint64_t)blockIdx.x * kOrientEntries; base < m;
+       base += (uint64_t)gridDim.x * kOrientEntries) {
+    // Owners of the step's first and last entry: the last vertices whose offset is
+    // not past them.
+    const uint32_t last_entry = (uint32_t)(min(base + kOrientEntries, m) - 1);
+    const uint32_t first = upper_index(off, n + 1, (uint32_t)base) - 1;
+    const uint32_t last = upper_index(off, n + 1, last_entry) - 1;
+    const uint32_t span = last - first + 1;
+    const bool local = span <= kOrientOffsets;
+    __syncthreads();  // the last step's readers are done
+    if (local)
+      for (uint32_t i = threadIdx.x; i <= span; i += kBlock) s_off[i] = off[first + i];
+    __syncthreads();
+    for (uint32_t i0 = 0; i0 < kOrientEntries; i0 += kBlock) {
+      const uint64_t i = base + i0 + threadIdx.x;
+      bool keep = false;
+      if (i < m) {
+        uint32_t u, du;
+        if (local) {
+          const uint32_t k = upper_index(s_off, span, (uint32_t)i) - 1;
+          u = first + k;
+          du = s_off[k + 1] - s_off[k];
+        } else {
+          u = first + upper_index(off + first, span, (uint32_t)i) - 1;
+          du = off[u + 1] - off[u];
+        }
+        const uint32_t v = adj[i], dv = off[v + 1] - off[v];
+        keep = dv > du || (dv == du && v > u);
+      }
+      const uint64_t mask = wave_ballot(keep);
+      if (lane_id() == 0 && i < m) {
+        bits[i / kWave] = mask;
+        count[i / kWave] = (uint32_t)__popcll(mask);
+      }
+    }
+  }
+}
+
+// adj[i] of every set bit, packed; before[w]: set bits below word w.
+__global__ __launch_bounds__(kBlock) void orient_pack_kernel(
+    const uint32_t* __restrict__ adj, uint64_t m, const unsigned long long* __restrict__ bits,
+    const uint32_t* __restrict__ before, uint32_t* __restrict__ new_adj) {
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m;
+       i += (uint64_t)gridDim.x * blockDim.x) {
+    const uint64_t mask = bits[i / kWave];
+    if ((mask >> (i % kWave)) & 1u) new_adj[before[i / kWave] + lanes_below(mask)] = adj[i];
+  }
+}
+
+// New offset of every vertex (and of the end): the set bits below its old one.
+__global__ __launch_bounds__(kBlock) void orient_offsets_kernel(
+    const uint32_t* __restrict__ off, uint32_t n, uint64_t m,
+    const unsigned long long* __restrict__ bits, const uint32_t* __restrict__ before,
+    uint32_t* __restrict__ new_off) {
+  for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v <= n;
+       v += (uint64_t)gridDim.x * blockDim.x) {
+    const uint32_t o = off[v], w = o / kWave;
+    new_off[v] = before[w] + (o % kWave ? (uint32_t)__popcll(bits[w] << (kWave - o % kWave)) : 0u);
+  }
+}
+
 // Topological relabel of a DAG (topo_relabel_device).  deg[v] = out-degree
-// plus in-degree: the out-degrees first, then one increment per entry.
+// plus in-degree: the out-degrees first, then the
 __global__ void out_degree_kernel(const uint32_t* __restrict__ off, uint32_t n,
                                   uint32_t* __restrict__ deg, uint32_t* __restrict__ ids) {
   for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x) {
@@ -134,11 +241,17 @@ __global__ void out_degree_kernel(const uint32_t* __restrict__ off, uint32_t n,
   }
 }
 
-__global__ void in_degree_kernel(const uint32_t* __restrict__ adj, uint64_t m,
+// in-degrees off the sorted targets: x's run [b, e) adds e - b.  (An increment per
+// entry serialises on the hubs: 1.44 ms on R-MAT scale 19 ef 16; at scale 20, twice
+// the entries, this takes 30 us behind three sort passes of about 60.)
+__global__ void in_degree_kernel(const uint32_t* __restrict__ targets, uint64_t m,
                                  uint32_t* __restrict__ deg) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m;
-       i += (uint64_t)gridDim.x * blockDim.x)
-    atomicAdd(&deg[adj[i]], 1u);
+       i += (uint64_t)gridDim.x * blockDim.x) {
+    const uint32_t x = targets[i];
+    if (i == 0 || targets[i - 1] != x) atomicSub(&deg[x], (uint32_t)i);
+    if (i + 1 == m || targets[i + 1] != x) atomicAdd(&deg[x], (uint32_t)i + 1u);
+  }
 }
 
 // Keys rank(u) << bits | rank(x) of every entry, one wave per u;
@@ -198,14 +311,15 @@ struct Bufs {
   }
 };
 
+uint64_t aligned(uint64_t bytes) { return (bytes + 255) & ~255ull; }
+
 // Sorted 64-bit keys (u << 32 | v, the m_kept first valid) -> CSR in new
-// buffers *d_off, *d_adj (owned by `b` until released).
+// buffers *d_off, *d_adj (owned by `b` until released).  d_src: room for m sources,
+// apart from the keys.
 int keys_to_csr(Bufs& b, const unsigned long long* keys, uint64_t m, uint32_t n, int cus,
-                hipStream_t stream, uint32_t** d_off, uint32_t** d_adj) {
+                hipStream_t stream, uint32_t* d_src, uint32_t** d_off, uint32_t** d_adj) {
   int st;
-  uint32_t* d_src = nullptr;
-  if ((st = b.alloc(&d_src, m)) != GPM_OK || (st = b.alloc(d_adj, m)) != GPM_OK ||
-      (st = b.alloc(d_off, (uint64_t)n + 1)) != GPM_OK)
+  if ((st = b.alloc(d_adj, m)) != GPM_OK || (st = b.alloc(d_off, (uint64_t)n + 1)) != GPM_OK)
     return st;
   if (m)
     hipLaunchKernelGGL(split_keys_kernel, dim3(grid_for_items(m, cus)), dim3(kBlock), 0, stream,
@@ -222,11 +336,6 @@ int build(uint32_t n, const uint32_t* src, const uint32_t* dst, uint64_t n_edges
   GPM_CHECK_ARG(n_edges == 0 || (src && dst), "null edge arrays");
   GPM_CHECK_ARG(n < 0xFFFFFFFFu, "n must be < 2^32 - 1");
   GPM_CHECK_ARG(!labels || (n_labels >= 1 && n_labels <= 4096), "n_labels must be in [1, 4096]");
-  uint64_t self_loops = 0;
-  for (uint64_t i = 0; i < n_edges; ++i) {
-    if (src[i] >= n || dst[i] >= n) return fail(GPM_EINVAL, "edge endpoint >= n (%u)", n);
-    self_loops += src[i] == dst[i];
-  }
   if (labels)
     for (uint32_t v = 0; v < n; ++v)
       if (labels[v] >= n_labels) return fail(GPM_EINVAL, "label of %u >= n_labels", v);
@@ -235,8 +344,6 @@ int build(uint32_t n, const uint32_t* src, const uint32_t* dst, uint64_t n_edges
   const bool drop_self = csr_flags & GPM_CSR_DROP_SELF;
   const bool sorted = (csr_flags & GPM_CSR_SORT) || dedup;
   const uint64_t records = n_edges * (sym ? 2 : 1);
-  // Dropped self loops become sentinel records that sort past the real ones.
-  const uint64_t dropped = drop_self ? self_loops * (sym ? 2 : 1) : 0;
   GPM_CHECK_ARG(records < (1ull << 32), "too many adjacency records (%llu)",
                 (unsigned long long)records);
   int dev = 0, cus = 256;
@@ -255,71 +362,86 @@ int build(uint32_t n, const uint32_t* src, const uint32_t* dst, uint64_t n_edges
   } guard{&stream};
   Bufs b;
   int st;
-  uint32_t *d_src = nullptr, *d_dst = nullptr;
-  if ((st = b.alloc(&d_src, n_edges)) != GPM_OK || (st = b.alloc(&d_dst, n_edges)) != GPM_OK)
-    return st;
+  // One workspace: the records as emitted (later the unique keys), the sorted
+  // records, whose room first holds the edges, temporary storage, the checks and
+  // the number of unique keys.
+  const int vbits = bits_for(n);  // source keys go up to n (the drop sentinel)
+  const unsigned end_bit = 32u + (unsigned)vbits;
+  size_t sort_bytes = 0, unique_bytes = 0;
+  unsigned long long *keys = nullptr, *sorted_keys = nullptr, *d_count = nullptr;
+  uint32_t *keys32 = nullptr, *vals = nullptr, *skeys = nullptr;
+  uint32_t *d_off = nullptr, *d_adj = nullptr;
+  if (records && sorted) {
+    GPM_HIP(rocprim::radix_sort_keys(nullptr, sort_bytes, keys, sorted_keys, records, 0u, end_bit,
+                                     stream));
+    if (dedup)
+      GPM_HIP(rocprim::unique(nullptr, unique_bytes, sorted_keys, keys, d_count, records,
+                              rocprim::equal_to<unsigned long long>(), stream));
+  } else if (records) {
+    GPM_HIP(rocprim::radix_sort_pairs(nullptr, sort_bytes, keys32, skeys, vals, d_adj, records, 0u,
+                                      (unsigned)vbits, stream));
+  }
+  const uint64_t edge_at = aligned(std::max(sort_bytes, unique_bytes));
+  const uint64_t key_at = edge_at + aligned(std::max(n_edges, records) * 8);
+  const uint64_t small_at = key_at + aligned(records * 8);
+  char* temp = nullptr;
+  if ((st = b.alloc(&temp, small_at + 24)) != GPM_OK) return st;
+  uint32_t* d_src = reinterpret_cast<uint32_t*>(temp + edge_at);
+  uint32_t* d_dst = d_src + n_edges;
+  uint32_t* checks = reinterpret_cast<uint32_t*>(temp + small_at);
+  d_count = reinterpret_cast<unsigned long long*>(checks + 4);
+  hipLaunchKernelGGL(zero_words_kernel, dim3(1), dim3(64), 0, stream, checks, 6u);
   if (n_edges) {
     GPM_HIP(hipMemcpyAsync(d_src, src, n_edges * 4, hipMemcpyHostToDevice, stream));
     GPM_HIP(hipMemcpyAsync(d_dst, dst, n_edges * 4, hipMemcpyHostToDevice, stream));
   }
-  const int vbits = bits_for(n);  // source keys go up to n (the drop sentinel)
-  uint32_t *d_off = nullptr, *d_adj = nullptr;
-  uint64_t m = 0;
-  void* temp = nullptr;
-  size_t temp_bytes = 0;
+  const unsigned emit_grid = std::min(grid_for_items(n_edges, cus), (unsigned)cus * 8);
   if (sorted) {
-    unsigned long long *keys = nullptr, *sorted_keys = nullptr;
-    if ((st = b.alloc(&keys, records)) != GPM_OK || (st = b.alloc(&sorted_keys, records)) != GPM_OK)
-      return st;
+    keys = reinterpret_cast<unsigned long long*>(temp + key_at);
+    sorted_keys = reinterpret_cast<unsigned long long*>(d_src);
     if (records) {
-      hipLaunchKernelGGL(emit_keys_kernel, dim3(grid_for_items(n_edges, cus)), dim3(kBlock), 0,
-                         stream, d_src, d_dst, n_edges, n, sym, drop_self, keys);
+      hipLaunchKernelGGL(emit_keys_kernel, dim3(emit_grid), dim3(kBlock), 0,
+                         stream, d_src, d_dst, n_edges, n, sym, drop_self, keys, checks);
       GPM_HIP(hipGetLastError());
-      const unsigned end_bit = 32u + (unsigned)vbits;
-      GPM_HIP(rocprim::radix_sort_keys(nullptr, temp_bytes, keys, sorted_keys, records, 0u,
-                                       end_bit, stream));
-      if ((st = b.alloc(reinterpret_cast<char**>(&temp), temp_bytes)) != GPM_OK) return st;
-      GPM_HIP(rocprim::radix_sort_keys(temp, temp_bytes, keys, sorted_keys, records, 0u, end_bit,
+      GPM_HIP(rocprim::radix_sort_keys(temp, sort_bytes, keys, sorted_keys, records, 0u, end_bit,
                                        stream));
+      if (dedup)  // unique keys into `keys`, which the sort is done with
+        GPM_HIP(rocprim::unique(temp, unique_bytes, sorted_keys, keys, d_count, records,
+                                rocprim::equal_to<unsigned long long>(), stream));
     }
-    unsigned long long* final_keys = sorted_keys;
-    uint64_t kept = records;
-    if (dedup && records) {
-      // Unique keys into `keys` (reused), count on the device.
-      unsigned long long* d_count = nullptr;
-      if ((st = b.alloc(&d_count, 1)) != GPM_OK) return st;
-      size_t ubytes = 0;
-      GPM_HIP(rocprim::unique(nullptr, ubytes, sorted_keys, keys, d_count, records,
-                              rocprim::equal_to<unsigned long long>(), stream));
-      void* utemp = nullptr;
-      if ((st = b.alloc(reinterpret_cast<char**>(&utemp), ubytes)) != GPM_OK) return st;
-      GPM_HIP(rocprim::unique(utemp, ubytes, sorted_keys, keys, d_count, records,
-                              rocprim::equal_to<unsigned long long>(), stream));
-      unsigned long long h_count = 0;
-      GPM_HIP(hipMemcpyAsync(&h_count, d_count, 8, hipMemcpyDeviceToHost, stream));
-      GPM_HIP(hipStreamSynchronize(stream));
-      kept = h_count;
-      final_keys = keys;
-    }
-    // Dedup keeps one sentinel record when any was dropped.
-    m = dedup ? kept - (dropped ? 1 : 0) : records - dropped;
-    if ((st = keys_to_csr(b, final_keys, m, n, cus, stream, &d_off, &d_adj)) != GPM_OK) return st;
   } else {
-    uint32_t *keys = nullptr, *vals = nullptr, *skeys = nullptr;
-    if ((st = b.alloc(&keys, records)) != GPM_OK || (st = b.alloc(&vals, records)) != GPM_OK ||
-        (st = b.alloc(&skeys, records)) != GPM_OK || (st = b.alloc(&d_adj, records)) != GPM_OK)
-      return st;
+    keys32 = reinterpret_cast<uint32_t*>(temp + key_at);
+    vals = keys32 + records;
+    skeys = d_src;
+    if ((st = b.alloc(&d_adj, records)) != GPM_OK) return st;
     if (records) {
-      hipLaunchKernelGGL(emit_pairs_kernel, dim3(grid_for_items(n_edges, cus)), dim3(kBlock), 0,
-                         stream, d_src, d_dst, n_edges, n, sym, drop_self, keys, vals);
+      hipLaunchKernelGGL(emit_pairs_kernel, dim3(emit_grid), dim3(kBlock), 0,
+                         stream, d_src, d_dst, n_edges, n, sym, drop_self, keys32, vals, checks);
       GPM_HIP(hipGetLastError());
-      GPM_HIP(rocprim::radix_sort_pairs(nullptr, temp_bytes, keys, skeys, vals, d_adj, records, 0u,
-                                        (unsigned)vbits, stream));
-      if ((st = b.alloc(reinterpret_cast<char**>(&temp), temp_bytes)) != GPM_OK) return st;
-      GPM_HIP(rocprim::radix_sort_pairs(temp, temp_bytes, keys, skeys, vals, d_adj, records, 0u,
+      GPM_HIP(rocprim::radix_sort_pairs(temp, sort_bytes, keys32, skeys, vals, d_adj, records, 0u,
                                         (unsigned)vbits, stream));
     }
-    m = records - dropped;
+  }
+  // The edges are checked where they are read; nothing below indexes by a vertex
+  // before this.
+  uint32_t found[6];
+  GPM_HIP(hipMemcpyAsync(found, checks, sizeof(found), hipMemcpyDeviceToHost, stream));
+  GPM_HIP(hipStreamSynchronize(stream));
+  if (found[0]) return fail(GPM_EINVAL, "edge endpoint >= n (%u)", n);
+  // Dropped self loops became sentinel records that sort past the real ones; dedup
+  // keeps one of them.
+  const uint64_t self_loops = (uint64_t)found[3] << 32 | found[2];
+  const uint64_t dropped = drop_self ? self_loops * (sym ? 2 : 1) : 0;
+  const uint64_t unique = (uint64_t)found[5] << 32 | found[4];
+  const uint64_t m = dedup ? unique - (dropped ? 1 : 0) : records - dropped;
+  if (sorted) {
+    // The keys are in `keys` after dedup, else where the sort put them; the other
+    // buffer holds the sources.
+    if ((st = keys_to_csr(b, dedup ? keys : sorted_keys, m, n, cus, stream,
+                          reinterpret_cast<uint32_t*>(dedup ? sorted_keys : keys), &d_off, &d_adj)) !=
+        GPM_OK)
+      return st;
+  } else {
     if ((st = b.alloc(&d_off, (uint64_t)n + 1)) != GPM_OK) return st;
     hipLaunchKernelGGL(offsets_kernel, dim3(grid_for_items(m + 1, cus)), dim3(kBlock), 0, stream,
                        skeys, m, n, d_off);
@@ -397,7 +519,9 @@ int relabel(gpm_graph* g, gpm_graph** out, uint32_t** perm) {
     GPM_HIP(rocprim::radix_sort_keys(t2, tb, keys, sorted_keys, m, 0u, end_bit, stream));
   }
   uint32_t *d_off = nullptr, *d_adj = nullptr;
-  if ((st = keys_to_csr(b, sorted_keys, m, n, cus, stream, &d_off, &d_adj)) != GPM_OK) return st;
+  if ((st = keys_to_csr(b, sorted_keys, m, n, cus, stream, reinterpret_cast<uint32_t*>(keys), &d_off,
+                        &d_adj)) != GPM_OK)
+    return st;
   std::vector<uint32_t> h_off((size_t)n + 1), h_new(std::max(n, 1u));
   GPM_HIP(hipMemcpyAsync(h_off.data(), d_off, ((size_t)n + 1) * 4, hipMemcpyDeviceToHost, stream));
   if (n) GPM_HIP(hipMemcpyAsync(h_new.data(), new_id, (size_t)n * 4, hipMemcpyDeviceToHost, stream));
@@ -431,6 +555,60 @@ int relabel(gpm_graph* g, gpm_graph** out, uint32_t** perm) {
 
 namespace gpm {
 
+int orient_device(gpm_graph* sym, uint32_t** d_off, uint32_t** d_adj, std::vector<uint32_t>* h_off) {
+  const uint32_t n = sym->n;
+  const uint64_t m = sym->m;
+  const uint64_t words = (m + kWave - 1) / kWave;
+  const int cus = device_cus(sym);
+  struct Drain {  // the buffers below are freed only once the stream is done with them
+    hipStream_t s;
+    ~Drain() { (void)hipStreamSynchronize(s); }
+  };
+  Bufs b;
+  Drain drain{sym->stream};
+  int st;
+  // One workspace: bits, counts and their scan (one word more each, so that the
+  // scan ends with the total), temporary storage.
+  size_t scan = 0;
+  GPM_HIP(rocprim::exclusive_scan(nullptr, scan, (uint32_t*)nullptr, (uint32_t*)nullptr, 0u,
+                                  (size_t)words + 1, rocprim::plus<uint32_t>(), sym->stream));
+  const uint64_t flags_at = aligned(scan), count_at = flags_at + aligned(words * 8);
+  const uint64_t before_at = count_at + aligned((words + 1) * 4);
+  char* temp = nullptr;
+  if ((st = b.alloc(&temp, before_at + (words + 1) * 4)) != GPM_OK ||
+      (st = b.alloc(d_off, (uint64_t)n + 1)) != GPM_OK)
+    return st;
+  auto* bits = reinterpret_cast<unsigned long long*>(temp + flags_at);
+  auto* count = reinterpret_cast<uint32_t*>(temp + count_at);
+  auto* before = reinterpret_cast<uint32_t*>(temp + before_at);
+  const dim3 block(kBlock);
+  hipLaunchKernelGGL(zero_words_kernel, dim3(1), dim3(1), 0, sym->stream, count + words, 1u);
+  if (m)
+    hipLaunchKernelGGL(orient_bits_kernel,
+                       dim3((unsigned)std::min<uint64_t>((m + kOrientEntries - 1) / kOrientEntries,
+                                                         (uint64_t)cus * 32)),
+                       block, 0, sym->stream, sym->off, sym->adj, n, m, bits, count);
+  GPM_HIP(hipGetLastError());
+  GPM_HIP(rocprim::exclusive_scan(temp, scan, count, before, 0u, (size_t)words + 1,
+                                  rocprim::plus<uint32_t>(), sym->stream));
+  hipLaunchKernelGGL(orient_offsets_kernel, dim3(grid_for_items((uint64_t)n + 1, cus)), block, 0,
+                     sym->stream, sym->off, n, m, bits, before, *d_off);
+  GPM_HIP(hipGetLastError());
+  h_off->resize((size_t)n + 1);
+  GPM_HIP(hipMemcpyAsync(h_off->data(), *d_off, ((size_t)n + 1) * 4, hipMemcpyDeviceToHost,
+                         sym->stream));
+  GPM_HIP(hipStreamSynchronize(sym->stream));
+  if ((st = b.alloc(d_adj, h_off->back())) != GPM_OK) return st;
+  if (m)
+    hipLaunchKernelGGL(orient_pack_kernel, dim3(grid_for_items(m, cus)), block, 0, sym->stream,
+                       sym->adj, m, bits, before, *d_adj);
+  GPM_HIP(hipGetLastError());
+  GPM_HIP(hipStreamSynchronize(sym->stream));
+  b.release(*d_off);
+  b.release(*d_adj);
+  return GPM_OK;
+}
+
 int topo_relabel_device(gpm_graph* g, uint32_t** toff, uint32_t** tadj, std::vector<uint32_t>* rank,
                         bool* ordered) {
   const uint32_t n = g->n;
@@ -457,16 +635,19 @@ int topo_relabel_device(gpm_graph* g, uint32_t** toff, uint32_t** tadj, std::vec
     return st;
   const dim3 block(kBlock);
   const dim3 per_vertex(grid_for_items((uint64_t)n + 1, cus));
-  size_t sort_ids = 0, sort_keys = 0, scan = 0;
+  size_t sort_ids = 0, sort_keys = 0, sort_targets = 0, scan = 0;
+  uint32_t* targets = reinterpret_cast<uint32_t*>(sorted);  // until the keys are sorted
   GPM_HIP(rocprim::radix_sort_pairs(nullptr, sort_ids, deg, sdeg, ids, order, n, 0u, 32u,
                                     g->stream));
   GPM_HIP(rocprim::radix_sort_keys(nullptr, sort_keys, keys, sorted, m, 0u, 2 * bits, g->stream));
+  GPM_HIP(rocprim::radix_sort_keys(nullptr, sort_targets, g->adj, targets, m, 0u, bits, g->stream));
   GPM_HIP(rocprim::exclusive_scan(nullptr, scan, sdeg, *toff, 0u, (size_t)n + 1,
                                   rocprim::plus<uint32_t>(), g->stream));
   char* temp = nullptr;
-  if ((st = b.alloc(&temp, std::max(std::max(sort_ids, sort_keys), scan))) != GPM_OK) return st;
+  if ((st = b.alloc(&temp, std::max(std::max(sort_ids, sort_keys), std::max(sort_targets, scan)))) != GPM_OK) return st;
   hipLaunchKernelGGL(out_degree_kernel, per_vertex, block, 0, g->stream, g->off, n, deg, ids);
-  hipLaunchKernelGGL(in_degree_kernel, dim3(grid_for_items(m, cus)), block, 0, g->stream, g->adj,
+  GPM_HIP(rocprim::radix_sort_keys(temp, sort_targets, g->adj, targets, m, 0u, bits, g->stream));
+  hipLaunchKernelGGL(in_degree_kernel, dim3(grid_for_items(m, cus)), block, 0, g->stream, targets,
                      m, deg);
   GPM_HIP(hipGetLastError());
   GPM_HIP(rocprim::radix_sort_pairs(temp, sort_ids, deg, sdeg, ids, order, n, 0u, 32u, g->stream));
