@@ -1,7 +1,9 @@
 // Device graph handle: creation (H2D of the CSR, label index), destruction,
 // device-side orientation, timing and scratch management.
 #include <algorithm>
+#include <mutex>
 #include <numeric>
+#include <utility>
 
 #include "graph_dev.hpp"
 
@@ -58,6 +60,44 @@ double mean_met_degree(gpm_graph* g) {
     g->met_degree = g->m ? d2 / (double)g->m : 0.0;
   }
   return g->met_degree;
+}
+
+// A stream's hardware queue is set up when it is first used: creation, the first copy
+// and destruction of one took 2 ms of a 2.2 ms call beside other streams.  A few idle
+// ones are therefore kept for the next call or handle, each with one owner at a time.
+namespace {
+constexpr size_t kIdleStreams = 4;
+std::mutex idle_mutex;
+std::vector<std::pair<int, hipStream_t>>& idle_streams() {
+  static auto* streams = new std::vector<std::pair<int, hipStream_t>>();  // outlives every handle
+  return *streams;
+}
+}  // namespace
+
+hipError_t stream_take(int device, hipStream_t* stream) {
+  {
+    std::lock_guard<std::mutex> lock(idle_mutex);
+    auto& idle = idle_streams();
+    for (size_t i = idle.size(); i-- > 0;)
+      if (idle[i].first == device) {
+        *stream = idle[i].second;
+        idle.erase(idle.begin() + i);
+        return hipSuccess;
+      }
+  }
+  return hipStreamCreateWithFlags(stream, hipStreamNonBlocking);
+}
+
+void stream_give(int device, hipStream_t stream) {
+  if (!stream) return;
+  if (hipStreamSynchronize(stream) == hipSuccess) {
+    std::lock_guard<std::mutex> lock(idle_mutex);
+    if (idle_streams().size() < kIdleStreams) {
+      idle_streams().emplace_back(device, stream);
+      return;
+    }
+  }
+  (void)hipStreamDestroy(stream);
 }
 
 int h2d(gpm_graph* g, void* dst, const void* src, size_t bytes) {
@@ -228,7 +268,7 @@ void release(gpm_graph* g) {
     if (e) (void)hipEventDestroy(e);
   if (g->ev0) hipEventDestroy(g->ev0);
   if (g->ev1) hipEventDestroy(g->ev1);
-  if (g->stream) hipStreamDestroy(g->stream);
+  stream_give(g->device, g->stream);
   delete g;
 }
 
@@ -374,7 +414,7 @@ int gpm_graph_create(const uint32_t* offsets, uint32_t n, const uint32_t* adj,
     if (labels) g->h_labels.assign(labels, labels + n);
     int st = GPM_OK;
     do {
-      if (hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking) != hipSuccess ||
+      if (stream_take(g->device, &g->stream) != hipSuccess ||
           hipEventCreate(&g->ev0) != hipSuccess || hipEventCreate(&g->ev1) != hipSuccess) {
         st = fail(GPM_EHIP, "stream/event creation failed");
         break;
@@ -481,7 +521,7 @@ int gpm_graph_orient(gpm_graph* sym, gpm_graph** dag) {
     g->adj = adj;
     for (uint32_t v = 0; v < g->n; ++v) g->max_deg = std::max(g->max_deg, h_off[v + 1] - h_off[v]);
     g->h_off = std::move(h_off);
-    if (hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking) != hipSuccess ||
+    if (stream_take(g->device, &g->stream) != hipSuccess ||
         hipEventCreate(&g->ev0) != hipSuccess || hipEventCreate(&g->ev1) != hipSuccess)
       st = fail(GPM_EHIP, "stream/event creation failed");
     else if (hipMalloc(&g->counters, 64 * sizeof(unsigned long long)) != hipSuccess)
