@@ -12,8 +12,8 @@
 //     k=5: sum_i sum_{j in row_i} sum_{l in row_i & row_j} |row_i & row_j & row_l|
 // Row i equals the reference's W1 for the edge (v0, S[i]); row_i & row_j is its
 // W2.  Rows are built by streaming the lists N+(S[i]) past a bitmap (block
-// tiers) or a hash table (wave tier) of S in LDS, or, for lists much longer than
-// S, by binary-searching each S[j] in N+(S[i]).  In the block tiers the k = 5
+// tiers) of S in LDS, or, for lists much longer than S and in the wave tier, by
+// binary-searching each S[j] in N+(S[i]).  In the block tiers the k = 5
 // sum is a masked product of 0/1 matrices on the matrix cores (count5_row).
 //
 // The kernels read the DAG relabelled in a topological order (gpm_graph's
@@ -41,9 +41,6 @@ using namespace gpm;
 
 namespace {
 
-constexpr int kBlock = 256;
-constexpr int kWavesPerBlock = kBlock / kWave;
-constexpr uint32_t kWaveTable = 128;
 constexpr uint32_t kBlockCap = 512;
 // Threads per block of the block tiers.  Rows are shared by the whole block,
 // so wider blocks raise the waves per SIMD that hide latency without more LDS.
@@ -69,16 +66,16 @@ enum { kCount = 0, kBytes = 1, kWork = 2, kAll = 3 };
 
 // A list N+(S[i]) much longer than S is not streamed: each S[t] is looked up
 // in it by binary search instead (d searches of log2(len) steps against len
-// streamed entries).  Thresholds measured on R-MAT scale 20: lists longer
-// than max(64, 2d) for the wave tier; for the block tiers, whose bitmap makes
-// a streamed entry cheap, longer than 16d (the 3-clique count of the LDS tier
-// took 3.5 ms with 4d, 3.0 ms with 16d).
+// streamed entries).  In the block tiers, whose bitmap makes a streamed entry
+// cheap, that are lists longer than 16d (R-MAT scale 20: the 3-clique count of
+// the LDS tier took 3.5 ms with 4d, 3.0 ms with 16d).
 __device__ __forceinline__ bool use_probe(uint32_t len, uint32_t d) {
   return len > max(64u, 16u * d);
 }
-__device__ __forceinline__ bool use_probe_wave(uint32_t len, uint32_t d) {
-  return len > max(64u, 2u * d);
-}
+// Threads per block of the wave tier: a root per wave, and one addition to the count
+// per block.
+constexpr int kTierBlock = 512;
+constexpr int kTierWaves = kTierBlock / kWave;
 
 __device__ __forceinline__ uint32_t ctz64(uint64_t x) { return (uint32_t)__builtin_ctzll(x); }
 
@@ -99,33 +96,49 @@ __device__ __forceinline__ uint32_t select_bit(uint64_t x, uint32_t k) {
 }
 
 // ------------------------------------------------------------ wave tier
+// Rows by searches alone, bound by their scattered loads (about 7 a pair): lists are
+// some 80 to 170 entries on R-MAT graphs, so even at |S| = 64 streaming them past a
+// hash table, or through LDS with the searches there, was no faster.  4-cliques of
+// R-MAT n = 100 k, 1.1 M samples: 200 us with a hash table and an addition to the
+// count per wave, 84 us with searches and one per block; 5-cliques of scale 18 488 ->
+// 350 us, 3- to 5-cliques of scale 20 1455 -> 1060 us.
+// Pair first + lane of the pairs (i, t), i < t < d, in the order of i, t: row i gets
+// bit t where S[t] is in S[i]'s list.
+__device__ __forceinline__ void pair_search(const uint32_t* __restrict__ adj, const uint32_t* beg,
+                                            const uint32_t* lens, const uint32_t* svals, uint32_t d,
+                                            uint32_t first, unsigned long long* rows) {
+  const uint32_t pairs = d * (d - 1) / 2, f = first + lane_id();
+  if (f >= pairs) return;
+  // Counted from the last pair, row d - 2 - k begins at k (k + 1) / 2: exact in FP32
+  // for at most 64 rows.
+  const uint32_t back = pairs - 1 - f;
+  const uint32_t k = (uint32_t)((sqrtf((float)(8 * back + 1)) - 1.f) * 0.5f);
+  const uint32_t i = d - 2 - k, t = d - 1 - (back - k * (k + 1) / 2);
+  if (sorted_contains(adj + beg[i], lens[i], svals[t])) atomicOr(&rows[i], 1ull << t);
+}
+
 // Wave w takes the chunks of `chunk` roots w, w + waves, ... of the tier's
 // list (ordered by degree or predicted cost, so the interleave evens the
 // waves' loads out).  No task queue: a queue fetch is an atomic on one
 // address, and those serialise (about 10 ns each), which bounded this tier
 // at ~1 M roots per fused pass.
 template <int K, int MODE>
-__global__ __launch_bounds__(kBlock) void clique_wave_kernel(
+__global__ __launch_bounds__(kTierBlock) void clique_wave_kernel(
     const uint32_t* __restrict__ off, const uint32_t* __restrict__ adj,
     const uint32_t* __restrict__ roots, uint32_t n_roots, uint32_t chunk,
     unsigned long long* __restrict__ out, unsigned long long* __restrict__ work) {
-  __shared__ uint32_t s_keys[kWavesPerBlock][kWaveTable];
-  __shared__ uint32_t s_vals[kWavesPerBlock][kWaveTable];
-  __shared__ unsigned long long s_rows[kWavesPerBlock][kWave];
-  __shared__ uint32_t s_pre[kWavesPerBlock][kWave];
-  __shared__ uint32_t s_beg[kWavesPerBlock][kWave];
-  __shared__ uint32_t s_len[kWavesPerBlock][kWave];
-  __shared__ uint32_t s_sv[kWavesPerBlock][kWave];
+  __shared__ unsigned long long s_rows[kTierWaves][kWave];
+  __shared__ uint32_t s_pre[kTierWaves][kWave];
+  __shared__ uint32_t s_beg[kTierWaves][kWave];
+  __shared__ uint32_t s_len[kTierWaves][kWave];
+  __shared__ uint32_t s_sv[kTierWaves][kWave];
   const uint32_t lane = lane_id();
   const uint32_t w = threadIdx.x / kWave;
-  uint32_t* keys = s_keys[w];
-  uint32_t* vals = s_vals[w];
   unsigned long long* rows = s_rows[w];
   uint32_t* pre = s_pre[w];
   uint32_t* beg = s_beg[w];
   uint32_t* lens = s_len[w];
   uint32_t* svals = s_sv[w];
-  constexpr uint32_t hmask = kWaveTable - 1;
   uint64_t acc = 0, acc3 = 0, acc4 = 0;
   const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
   const uint64_t nwaves = (uint64_t)gridDim.x * blockDim.x / kWave;
@@ -136,46 +149,18 @@ __global__ __launch_bounds__(kBlock) void clique_wave_kernel(
       const uint32_t sb = uniform(off[u]), d = uniform(off[u + 1]) - sb;  // d <= 64 by tiering
       const bool act = lane < d;
       const uint32_t s = act ? adj[sb + lane] : kEmpty;
-      keys[lane] = kEmpty;
-      keys[lane + kWave] = kEmpty;
-      rows[lane] = 0ull;
-      __builtin_amdgcn_wave_barrier();
-      if (act) lds_hash_insert(keys, vals, hmask, s, lane);
       uint32_t b = 0, len = 0;
       if (act) {
         b = off[s];
         len = off[s + 1] - b;
       }
+      rows[lane] = 0ull;
       lens[lane] = len;
-      const bool probe = act && use_probe_wave(len, d);
-      const uint32_t incl = wave_incl_scan(probe ? 0u : len);
-      pre[lane] = incl;
       beg[lane] = b;
-      const uint32_t total = wave_bcast(incl, kWave - 1);
+      svals[lane] = s;
       __builtin_amdgcn_wave_barrier();
-      for (uint32_t t = 0; t < total; t += kWave) {
-        const uint32_t f = t + lane;
-        if (f < total) {
-          const uint32_t j = upper_index(pre, kWave, f);
-          const uint32_t excl = j ? pre[j - 1] : 0u;
-          const uint32_t x = adj[beg[j] + (f - excl)];
-          const int idx = lds_hash_find(keys, vals, hmask, x);
-          if (idx >= 0) atomicOr(&rows[j], 1ull << idx);
-        }
-      }
-      // Probed lists: the (probed row, element of S) pairs are dealt out
-      // over the lanes, so all binary searches of a root run side by side.
-      const uint64_t pm = wave_ballot(probe);
-      if (pm) {
-        svals[lane] = s;
-        __builtin_amdgcn_wave_barrier();
-        const uint32_t np = (uint32_t)__popcll(pm);
-        for (uint32_t f = lane; f < np * d; f += kWave) {
-          const uint32_t k = f / d, t = f - k * d;
-          const uint32_t i = select_bit(pm, k);
-          if (sorted_contains(adj + beg[i], lens[i], svals[t])) atomicOr(&rows[i], 1ull << t);
-        }
-      }
+      for (uint32_t f = 0; f < d * (d - 1) / 2; f += kWave)  // d >= 2 by tiering
+        pair_search(adj, beg, lens, svals, d, f, rows);
       __builtin_amdgcn_wave_barrier();
       const uint64_t row = act ? rows[lane] : 0ull;
       uint64_t c = 0;
@@ -249,17 +234,11 @@ __global__ __launch_bounds__(kBlock) void clique_wave_kernel(
     }
   }
   if (MODE == kAll) {
-    acc3 = wave_sum_u64(acc3);
-    acc4 = wave_sum_u64(acc4);
-    acc = wave_sum_u64(acc);
-    if (lane == 0) {
-      if (acc3) atomicAdd(out, (unsigned long long)acc3);
-      if (acc4) atomicAdd(out + 1, (unsigned long long)acc4);
-      if (acc) atomicAdd(out + 2, (unsigned long long)acc);
-    }
+    block_add(out, acc3);
+    block_add(out + 1, acc4);
+    block_add(out + 2, acc);
   } else if (MODE != kWork) {
-    acc = wave_sum_u64(acc);
-    if (lane == 0 && acc) atomicAdd(out, (unsigned long long)acc);
+    block_add(out, acc);
   }
 }
 
@@ -932,17 +911,11 @@ __global__ __launch_bounds__(BS, block_waves(K, MODE, LDS_ROWS, MAXW)) void cliq
     acc4 = s_tot[threadIdx.x / kWave][2];
   }
   if (MODE == kAll) {
-    acc3 = wave_sum_u64(acc3);
-    acc4 = wave_sum_u64(acc4);
-    acc = wave_sum_u64(acc);
-    if (lane_id() == 0) {
-      if (acc3) atomicAdd(out, (unsigned long long)acc3);
-      if (acc4) atomicAdd(out + 1, (unsigned long long)acc4);
-      if (acc) atomicAdd(out + 2, (unsigned long long)acc);
-    }
+    block_add(out, acc3);
+    block_add(out + 1, acc4);
+    block_add(out + 2, acc);
   } else if (MODE != kWork) {
-    acc = wave_sum_u64(acc);
-    if (lane_id() == 0 && acc) atomicAdd(out, (unsigned long long)acc);
+    block_add(out, acc);
   }
 }
 
@@ -1019,8 +992,8 @@ int launch_wave_tier(gpm_graph* g, hipStream_t stream, const RootTiers* t, unsig
   const uint64_t waves_wanted = (t->n_wave + chunk - 1) / chunk;
   const uint64_t waves = std::min<uint64_t>(waves_wanted, (uint64_t)cus * 32);
   const unsigned blocks =
-      (unsigned)std::max<uint64_t>(1, (waves + kWavesPerBlock - 1) / kWavesPerBlock);
-  hipLaunchKernelGGL((clique_wave_kernel<K, MODE>), dim3(blocks), dim3(kBlock), 0, stream,
+      (unsigned)std::max<uint64_t>(1, (waves + kTierWaves - 1) / kTierWaves);
+  hipLaunchKernelGGL((clique_wave_kernel<K, MODE>), dim3(blocks), dim3(kTierBlock), 0, stream,
                      g->toff, g->tadj, t->d_wave, t->n_wave, chunk, out, work);
   GPM_HIP(hipGetLastError());
   if ((MODE == kCount || MODE == kAll) && stream == g->stream) timing_mark(g, "clique_wave");

@@ -898,8 +898,7 @@ __global__ __launch_bounds__(kSquareBlock) void square_kernel(
       }
     }
   }
-  acc = wave_sum_u64(acc);
-  if (lane_id() == 0 && acc) atomicAdd(count, (unsigned long long)acc);
+  block_add(count, acc);
 }
 
 __global__ void zero_f32_kernel(float* a, uint64_t n) {

@@ -260,22 +260,6 @@ __global__ __launch_bounds__(kBlock) void pair_triangles_kernel(
   }
 }
 
-// Adds the threads' values to *out with one atomic per block of kBlock threads:
-// atomics to one address serialise (about 10 ns each), and four per wave of a
-// full launch took 1.5 ms.
-__device__ __forceinline__ void block_add(unsigned long long* out, uint64_t value) {
-  __shared__ unsigned long long s_part[kBlock / kWave];
-  value = wave_sum_u64(value);
-  __syncthreads();  // an earlier call's parts have been read
-  if (lane_id() == 0) s_part[threadIdx.x / kWave] = value;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned long long t = 0;
-    for (int i = 0; i < kBlock / kWave; ++i) t += s_part[i];
-    if (t) atomicAdd(out, t);
-  }
-}
-
 // Edge sums over the undirected edges {v, x} (each once: x > v), from the per-edge
 // triangle counts c and the degrees; one wave per v:
 //   out[0] += 2c                      (sum: 6T)
@@ -473,8 +457,7 @@ __global__ __launch_bounds__(kCycBlock) void cycles_kernel(
     }
     __syncthreads();
   }
-  acc = wave_sum_u64(acc);
-  if (lane_id() == 0 && acc) atomicAdd(out, (unsigned long long)acc);
+  block_add(out, acc);
 }
 
 // Block per root of fewer than kCycHeavy wedges (statically interleaved).
@@ -507,8 +490,7 @@ __global__ __launch_bounds__(kLightBlock) void light_cycles_kernel(
     });
     __syncthreads();
   }
-  acc = wave_sum_u64(acc);
-  if (lane_id() == 0 && acc) atomicAdd(out, (unsigned long long)acc);
+  block_add(out, acc);
 }
 
 // below[u] = neighbours of u of lower rank; wedges[u] = sum over them of their

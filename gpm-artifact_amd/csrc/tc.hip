@@ -309,8 +309,7 @@ __global__ __launch_bounds__(kBlock) void tc_vertex_block_kernel(
       __syncthreads();
     }
   }
-  cnt = wave_sum_u64(cnt);
-  if (lane_id() == 0 && cnt) atomicAdd(out, (unsigned long long)cnt);
+  block_add(out, cnt);
 }
 
 // The two kernels below read the DAG relabelled by total degree: every list

@@ -2,8 +2,12 @@
 wrong: out-degrees around the edges of a 16-position block, a 64-bit row word
 and a 128-position chunk, sparse and dense local graphs, hub ids inside and
 outside the id bitmap, and orders that are not by degree."""
+from math import comb
+
 import numpy as np
 import pytest
+
+import graphs
 
 pytestmark = pytest.mark.gpu
 
@@ -64,3 +68,25 @@ def test_degree_order_and_kahn_agree(gpm, orc):
         with gpm.DeviceGraph(dag, oriented=True) as dg:
             assert list(dg.clique_all()) == want
             assert dg.clique(5, policy=gpm.SCHED_DEGREE_SPLIT) == want[2]
+
+
+@pytest.mark.parametrize("n", [3, 4, 11, 12, 13, 24, 63, 64, 65, 66])
+def test_wave_tier_complete(gpm, n):
+    """Roots of 1 .. n - 1 later vertices: one and several windows of row searches."""
+    with gpm.DeviceGraph(gpm.orient(graphs.complete(n)), oriented=True) as dag:
+        for k in (3, 4, 5):
+            assert dag.clique(k) == comb(n, k)
+
+
+@pytest.mark.parametrize("met", [2, 3, 13, 40])
+def test_wave_tier_long_lists(gpm, met):
+    """500 vertices joined to `met` of a complete graph's 200 each: lists far longer
+    than the roots'."""
+    core, m = graphs.complete(200), 500
+    src = np.repeat(np.arange(200), 199)
+    outer = np.repeat(200 + np.arange(m), met)
+    inner = (np.arange(m)[:, None] * 7 + np.arange(met) * (200 // met)).reshape(-1) % 200
+    g = gpm.csr_from_edges(200 + m, np.concatenate([src, outer]), np.concatenate([core.adj, inner]))
+    with gpm.DeviceGraph(gpm.orient(g), oriented=True) as dag:
+        for k in (3, 4, 5):
+            assert dag.clique(k) == comb(200, k) + m * comb(met, k - 1)
