@@ -55,6 +55,9 @@ constexpr int kBlock = 256;
 constexpr int kWavesPerBlock = kBlock / kWave;
 constexpr int kMaxQ = 16;
 constexpr uint32_t kMaxGroup = 3;
+// Counters that a block of match_kernel adds its counts up in, so that a launch of
+// few queries adds to each of theirs once per block instead of once per task.
+constexpr uint32_t kBlockCounts = 64;
 
 struct QPlan {
   uint32_t n;               // query vertices
@@ -431,9 +434,22 @@ __host__ __device__ constexpr bool weighted_steps(int mode) {
   return mode == kModeTrial || mode == kModeLog;
 }
 
+// The task queue: kShards counters, a cache line each; counter i deals out the tasks
+// i, i + kShards, ...  A wave draws on its own and, once that is drained, on the next.
+// Additions to one address take about 10 ns each: the short tasks of triangle, diamond
+// and three-star queries on R-MAT scale 18 took 1.05 ms with one counter and an
+// addition to their count per task, 0.85 with eight counters (0.82 with 32), 0.52 with
+// the counts added up per block besides (kBlockCounts).
+constexpr uint32_t kShards = 8, kShardStride = 32;
+constexpr uint32_t kQueueWords = kShards * kShardStride;
+// Tasks of a counter.
+__device__ __forceinline__ uint32_t shard_tasks(uint32_t n_tasks, uint32_t shard) {
+  return n_tasks > shard ? (n_tasks - shard - 1) / kShards + 1 : 0u;
+}
+
 // Budget of a task in a budgeted count: the task stops once its steps reach
-// `limit` while the launch's queue holds no task for an idle wave; while
-// the queue still has tasks, the limit is raised by `quantum` instead (so
+// `limit` while the wave's counter of the queue holds no task for an idle wave;
+// while it still has tasks, the limit is raised by `quantum` instead (so
 // tasks stop only in the launch's tail, when idle waves could take their
 // parts in the next launch).
 struct TaskBudget {
@@ -645,22 +661,39 @@ __global__ __launch_bounds__(kBlock) void match_kernel(
     DevGraph g, const QPlan* __restrict__ plans, uint32_t nq, uint32_t n_tasks,
     const uint32_t* __restrict__ roots, const uint32_t* __restrict__ rlen,
     const HeavyTask* __restrict__ heavy, uint32_t n_heavy, uint32_t split_len,
-    unsigned int* __restrict__ queue, unsigned long long* __restrict__ counts,
+    unsigned int* __restrict__ queue, unsigned long long* __restrict__ counts, uint32_t n_counts,
     unsigned long long* __restrict__ work, uint64_t budget, unsigned int* __restrict__ aborted) {
   __shared__ WaveState s_state[kWavesPerBlock];
+  __shared__ unsigned long long s_count[kBlockCounts];
   WaveState& s = s_state[threadIdx.x / kWave];
   const uint32_t lane = lane_id();
+  const bool summed = n_counts <= kBlockCounts;
+  for (uint32_t i = threadIdx.x; i < kBlockCounts; i += kBlock) s_count[i] = 0ull;
+  __syncthreads();
   // Every lane writes the same values (no lane-dependent branch).
   for (int d = 0; d < kMaxQ; ++d) s.cut[d] = kNoCut;
+  uint32_t shard = blockIdx.x % kShards, drained = 0;
   while (true) {
+    // Other waves' counters are read before they are added to: at the end of a launch
+    // most are drained.
+    const uint32_t mine = shard_tasks(n_tasks, shard);
+    unsigned int* counter = queue + shard * kShardStride;
     uint32_t t = 0;
-    if (lane == 0) t = atomicAdd(queue, 1u);
+    if (lane == 0)
+      t = drained && __hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= mine
+              ? mine
+              : atomicAdd(counter, 1u);
     t = uniform(wave_bcast(t, 0));
-    if (t >= n_tasks) break;
+    if (t >= mine) {
+      shard = (shard + 1) % kShards;
+      if (++drained == kShards) break;
+      continue;
+    }
+    t = shard + t * kShards;
     uint64_t c = 0;
     uint32_t qid;
     uint64_t steps = 0;
-    TaskBudget tb{budget, budget, queue, n_tasks};
+    TaskBudget tb{budget, budget, counter, mine};
     if (t < n_heavy) {
       const HeavyTask h = heavy[t];
       const QPlan& p = plans[uniform(h.plan)];
@@ -694,7 +727,10 @@ __global__ __launch_bounds__(kBlock) void match_kernel(
     if (stopped) {
       if (lane == 0) aborted[1 + atomicAdd(aborted, 1u)] = t;
     } else if (lane == 0 && c) {
-      atomicAdd(&counts[qid], (unsigned long long)c);
+      if (summed)
+        atomicAdd(&s_count[qid], (unsigned long long)c);
+      else
+        atomicAdd(&counts[qid], (unsigned long long)c);
     }
     if (kMode == kModeLog && lane == 0) work[t] = steps;
     if (kMode == kModeTrial && lane == 0 && steps) {
@@ -710,6 +746,10 @@ __global__ __launch_bounds__(kBlock) void match_kernel(
     // log's stall).  tests/test_match_isa.py checks every mode's loop shape.
     __builtin_amdgcn_wave_barrier();
   }
+  if (!summed) return;
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < n_counts; i += kBlock)
+    if (s_count[i]) atomicAdd(&counts[i], s_count[i]);
 }
 
 // ------------------------------------------------------------------ squares
@@ -1317,14 +1357,19 @@ std::vector<uint32_t> batch_key(const gpm_query* queries, int n_queries, const g
   return k;
 }
 
+// Blocks of 64 threads that clear a batch's counters and its queue.
+unsigned zero_blocks(const MatchBatch* b) {
+  return (unsigned)std::max<int>(b->n_queries, (int)kQueueWords) / 64 + 1;
+}
+
 // Enqueues one enumeration launch over n_tasks tasks, the first n_heavy of
 // them heavy parts at d_heavy and the rest b's light chunks.  zero_counts:
 // clear the counters first (the first launch of a call).  budget > 0: a
 // budgeted count whose stopped tasks are listed in d_abort.
 int launch_tasks(gpm_graph* g, MatchBatch* b, const HeavyTask* d_heavy, uint32_t n_heavy,
                  uint32_t n_tasks, bool zero_counts, uint64_t budget, unsigned int* d_abort) {
-  hipLaunchKernelGGL(zero_kernel, dim3((b->n_queries + 64) / 64 + 1), dim3(64), 0, g->stream,
-                     b->d_counts, zero_counts ? b->n_queries : 0, b->d_queue, 4);
+  hipLaunchKernelGGL(zero_kernel, dim3(zero_blocks(b)), dim3(64), 0, g->stream,
+                     b->d_counts, zero_counts ? b->n_queries : 0, b->d_queue, (int)kQueueWords);
   if (budget)
     hipLaunchKernelGGL(zero_kernel, dim3(1), dim3(64), 0, g->stream, nullptr, 0, d_abort, 1);
   auto* kernel = budget ? (b->merge ? &match_kernel<kModeBudget, true>
@@ -1335,7 +1380,7 @@ int launch_tasks(gpm_graph* g, MatchBatch* b, const HeavyTask* d_heavy, uint32_t
                                          : &match_kernel<kModeCount, false>;
   hipLaunchKernelGGL(kernel, dim3(b->grid), dim3(kBlock), 0, g->stream, b->dg, b->d_plans, b->nq,
                      n_tasks, b->d_roots, b->d_rlen, d_heavy, n_heavy, b->split_len, b->d_queue,
-                     b->d_counts, b->d_work, budget, d_abort);
+                     b->d_counts, (uint32_t)b->n_queries, b->d_work, budget, d_abort);
   GPM_HIP(hipGetLastError());
   return GPM_OK;
 }
@@ -1513,11 +1558,11 @@ int run_passes(gpm_graph* g, MatchBatch* b) {
 // enumeration depending on the reset (no stream capture, no memset node).
 int build_graph(MatchBatch* b) {
   GPM_HIP(hipGraphCreate(&b->graph, 0));
-  int n_queries = b->n_queries, four = 4;
-  void* zargs[] = {&b->d_counts, &n_queries, &b->d_queue, &four};
+  int n_queries = b->n_queries, words = kQueueWords;
+  void* zargs[] = {&b->d_counts, &n_queries, &b->d_queue, &words};
   hipKernelNodeParams zp{};
   zp.func = reinterpret_cast<void*>(&zero_kernel);
-  zp.gridDim = dim3((b->n_queries + 64) / 64 + 1);
+  zp.gridDim = dim3(zero_blocks(b));
   zp.blockDim = dim3(64);
   zp.sharedMemBytes = 0;
   zp.kernelParams = zargs;
@@ -1526,10 +1571,11 @@ int build_graph(MatchBatch* b) {
   GPM_HIP(hipGraphAddKernelNode(&zn, b->graph, nullptr, 0, &zp));
   uint64_t no_budget = 0;
   unsigned int* no_abort = nullptr;
+  uint32_t n_counts = (uint32_t)b->n_queries;
   void* margs[] = {&b->dg,      &b->d_plans,   &b->nq,      &b->n_tasks,
                    &b->d_roots, &b->d_rlen,    &b->d_heavy, &b->n_heavy,
-                   &b->split_len, &b->d_queue, &b->d_counts, &b->d_work,
-                   &no_budget,  &no_abort};
+                   &b->split_len, &b->d_queue, &b->d_counts, &n_counts,
+                   &b->d_work,  &no_budget,    &no_abort};
   hipKernelNodeParams mp{};
   mp.func = b->merge ? reinterpret_cast<void*>(&match_kernel<kModeCount, true>)
                      : reinterpret_cast<void*>(&match_kernel<kModeCount, false>);
@@ -1810,7 +1856,7 @@ int build_batch(gpm_graph* g, std::vector<QPlan> plans, int n_counters, const gp
   const size_t root_bytes = align(std::max<uint64_t>(root_total, 1) * 4);
   const size_t count_bytes = align((size_t)(n_slots + 1) * 8);
   const size_t work_bytes = trial ? align((size_t)(3 * nq0 + 1) * 8) : 0;
-  const size_t small_bytes = align((size_t)(nq0 + 1 + 4) * 4);
+  const size_t small_bytes = align((size_t)(nq0 + 1) * 4) + align(kQueueWords * 4);
   const size_t lvoff_bytes = align(g->h_lvoff.size() * 4);
   const size_t total =
       plan_bytes + 2 * root_bytes + count_bytes + work_bytes + small_bytes + lvoff_bytes;
@@ -1830,7 +1876,7 @@ int build_batch(gpm_graph* g, std::vector<QPlan> plans, int n_counters, const gp
     mp += work_bytes;
   }
   b->d_rootcnt = reinterpret_cast<unsigned int*>(mp);
-  b->d_queue = b->d_rootcnt + nq0 + 1;
+  b->d_queue = reinterpret_cast<unsigned int*>(mp + align((size_t)(nq0 + 1) * 4));
   mp += small_bytes;
   uint32_t* d_lvoff = reinterpret_cast<uint32_t*>(mp);
   b->n_queries = n_slots;
