@@ -44,9 +44,7 @@ namespace {
 constexpr uint32_t kBlockCap = 512;
 // Threads per block of the block tiers.  Rows are shared by the whole block,
 // so wider blocks raise the waves per SIMD that hide latency without more LDS.
-// The k = 5 count keeps 128 registers and more: two blocks of the LDS tier fit
-// a CU (three of 256 threads were slower, 11.6 against 10.3 ms a launch on
-// R-MAT scale 20: too few waves for the row build), and one of the wide tier.
+// Three blocks of the LDS tier fit a CU, and one of the wide tier.
 constexpr int kLdsBlock = 512;
 constexpr int kWideBlock = 512;
 constexpr int kHbmBlock = 1024;
@@ -260,12 +258,8 @@ __device__ __forceinline__ uint32_t block_incl_scan(uint32_t v, uint32_t* s_wsum
 // block: rows are taken BS at a time, a block scan of their popcounts
 // gives each pair an owner row, and j is found by popcount over the words.
 //
-// MAXW > 0 (rows in LDS, W <= MAXW): rows are read MAXW words at a time
-// with no per-word branch, so all loads of a row are in flight together and
-// one wait covers them (words past W belong to the next row or to the tail
-// of the block's LDS, and are masked out by m[x] = 0 for x >= W).
-// MAXW == 0 is the generic path for rows in HBM.
-template <int K, int MAXW, int BS, bool ALL = false>
+// For rows in HBM.
+template <int K, int BS, bool ALL>
 __device__ __forceinline__ uint64_t count_pairs(const unsigned long long* rows, uint32_t d,
                                                 uint32_t W, uint32_t RS, uint32_t part,
                                                 uint32_t n_parts, uint32_t* s_pre,
@@ -278,15 +272,7 @@ __device__ __forceinline__ uint64_t count_pairs(const unsigned long long* rows, 
     uint32_t pc = 0;
     if (t0 < nr) {
       const unsigned long long* r0 = rows + (size_t)(part + t0 * n_parts) * RS;
-      if (MAXW > 0) {
-#pragma unroll
-        for (int w = 0; w < MAXW; ++w) {
-          const unsigned long long x = r0[w];
-          pc += w < (int)W ? (uint32_t)__popcll(x) : 0u;
-        }
-      } else {
-        for (uint32_t w = 0; w < W; ++w) pc += (uint32_t)__popcll(r0[w]);
-      }
+      for (uint32_t w = 0; w < W; ++w) pc += (uint32_t)__popcll(r0[w]);
     }
     if (ALL) c3 += pc;
     const uint32_t incl = block_incl_scan(pc, s_wsum);
@@ -296,90 +282,27 @@ __device__ __forceinline__ uint64_t count_pairs(const unsigned long long* rows, 
     for (uint32_t p = threadIdx.x; p < total; p += BS) {
       const uint32_t jj = upper_index(s_pre, BS, p);
       uint32_t kth = p - (jj ? s_pre[jj - 1] : 0u);
-      if (MAXW > 0) {
-        // LDS rows: row index < 1024 and stride < 32, so the 24-bit multiply
-        // (full rate; a 32-bit multiply issues at quarter rate) is exact.
-        const unsigned long long* ri = rows + __umul24(part + (c0 + jj) * n_parts, RS);
-        uint64_t wi[MAXW > 0 ? MAXW : 1];
-#pragma unroll
-        for (int x = 0; x < MAXW; ++x) wi[x] = x < (int)W ? ri[x] : 0ull;
-        // j = position of the kth set bit of row i.
-        uint32_t j = 0;
-        bool found = false;
-#pragma unroll
-        for (int x = 0; x < MAXW; ++x) {
-          const uint32_t pw = (uint32_t)__popcll(wi[x]);
-          if (!found && kth < pw) {
-            j = x * 64 + select_bit(wi[x], kth);
-            found = true;
-          } else if (!found) {
-            kth -= pw;
-          }
-        }
-        const unsigned long long* rj = rows + __umul24(j, RS);
-        uint64_t m[MAXW > 0 ? MAXW : 1];
-#pragma unroll
-        for (int x = 0; x < MAXW; ++x) m[x] = wi[x] & rj[x];
-        if (K == 4) {
-#pragma unroll
-          for (int x = 0; x < MAXW; ++x) c += __popcll(m[x]);
-        } else {
-          if (ALL)
-#pragma unroll
-            for (int x = 0; x < MAXW; ++x) c4 += __popcll(m[x]);
-#pragma unroll
-          for (int x = 0; x < MAXW; ++x) {
-            uint64_t mm = m[x];
-            while (mm) {
-              const uint32_t l = x * 64 + ctz64(mm);
-              mm &= mm - 1;
-              // Row l holds only positions > l (rows are upper triangular),
-              // so its words below x are zero and are not read.  Up to 8
-              // words, a word of row l is read only by lanes whose m word is
-              // non-zero (fewer LDS reads; 33.1 -> 29.5 ms per fused pass on
-              // R-MAT s20); the 16-word tier measured faster with every
-              // word read under one wait.
-              // One 32-bit sum per l (at most 16 x 64 bits), one 64-bit add.
-              const unsigned long long* rl = rows + __umul24(l, RS);
-              uint32_t cl = 0;
-              if (MAXW <= 8) {
-#pragma unroll
-                for (int y = x; y < MAXW; ++y)
-                  if (m[y]) cl += (uint32_t)__popcll(m[y] & rl[y]);
-              } else {
-                uint64_t a[MAXW > 0 ? MAXW : 1];
-#pragma unroll
-                for (int y = x; y < MAXW; ++y) a[y] = rl[y];
-#pragma unroll
-                for (int y = x; y < MAXW; ++y) cl += (uint32_t)__popcll(m[y] & a[y]);
-              }
-              c += cl;
-            }
-          }
-        }
+      const unsigned long long* ri = rows + (size_t)(part + (c0 + jj) * n_parts) * RS;
+      uint32_t w = 0;
+      while (true) {
+        const uint32_t pw = (uint32_t)__popcll(ri[w]);
+        if (kth < pw) break;
+        kth -= pw;
+        ++w;
+      }
+      const uint32_t j = w * 64 + select_bit(ri[w], kth);
+      const unsigned long long* rj = rows + (size_t)j * RS;
+      if (K == 4) {
+        for (uint32_t x = 0; x < W; ++x) c += __popcll(ri[x] & rj[x]);
       } else {
-        const unsigned long long* ri = rows + (size_t)(part + (c0 + jj) * n_parts) * RS;
-        uint32_t w = 0;
-        while (true) {
-          const uint32_t pw = (uint32_t)__popcll(ri[w]);
-          if (kth < pw) break;
-          kth -= pw;
-          ++w;
-        }
-        const uint32_t j = w * 64 + select_bit(ri[w], kth);
-        const unsigned long long* rj = rows + (size_t)j * RS;
-        if (K == 4) {
-          for (uint32_t x = 0; x < W; ++x) c += __popcll(ri[x] & rj[x]);
-        } else {
-          for (uint32_t x = 0; x < W; ++x) {
-            uint64_t mm = ri[x] & rj[x];
-            if (ALL) c4 += __popcll(mm);
-            while (mm) {
-              const uint32_t l = x * 64 + ctz64(mm);
-              mm &= mm - 1;
-              const unsigned long long* rl = rows + (size_t)l * RS;
-              for (uint32_t y = x; y < W; ++y) c += __popcll(ri[y] & rj[y] & rl[y]);
-            }
+        for (uint32_t x = 0; x < W; ++x) {
+          uint64_t mm = ri[x] & rj[x];
+          if (ALL) c4 += __popcll(mm);
+          while (mm) {
+            const uint32_t l = x * 64 + ctz64(mm);
+            mm &= mm - 1;
+            const unsigned long long* rl = rows + (size_t)l * RS;
+            for (uint32_t y = x; y < W; ++y) c += __popcll(ri[y] & rj[y] & rl[y]);
           }
         }
       }
@@ -639,12 +562,15 @@ __device__ __forceinline__ uint32_t count5_row(const uint32_t* rows32, uint32_t 
   for (int c = 0; c < NC; ++c) ri[c] = 4 * c + g < 2 * W ? row[4 * c + g] : 0u;
   float s = 0.f;
   const uint32_t nt = (ni + 15) / 16;
-  if (nt == 1) {
-    s = count5_blocks<NC, 1, ALL>(rows32, RS32, ri, list, nt, 0, c4);
-  } else if (nt == 2) {
-    s = count5_blocks<NC, 2, ALL>(rows32, RS32, ri, list, nt, 0, c4);
+  // One row block at a time keeps the registers of the 8-word tier low enough for three
+  // resident blocks, which also hide the row build's loads better (two of four or two
+  // row blocks at a time: 9.9 ms a fused launch on R-MAT scale 20, three of one 8.9);
+  // the wide tier's single block per CU gains from two (2.9 ms, 3.15 with one).
+  constexpr uint32_t J = NC <= 4 ? 1 : 2;
+  if (J == 1 || nt == 1) {
+    for (uint32_t jg = 0; jg < nt; ++jg)
+      s += count5_blocks<NC, 1, ALL>(rows32, RS32, ri, list, nt, jg, c4);
   } else {
-    constexpr int J = NC <= 2 ? 4 : NC <= 4 ? 2 : 2;
     for (uint32_t jg = 0; jg < nt; jg += J)
       s += count5_blocks<NC, J, ALL>(rows32, RS32, ri, list, nt, jg, c4);
   }
@@ -668,14 +594,59 @@ __device__ __forceinline__ uint32_t count5_rows(const unsigned long long* rows, 
   return c;
 }
 
+// The k = 4 count of a root, sum over j, l in row j, of |row_j & row_l|: the same
+// product as a row's k = 5 count (count5_row), of all rows unmasked.  The blocks
+// part, part + n_parts, ... of 16 rows go to the waves there and back, since their
+// costs fall with the index (two or four blocks at a time left waves without one).
+// list: 0 .. d - 1, then d.  Of a 4-clique launch on R-MAT scale 20 it leaves the row
+// build: LDS tier 5.1 -> 3.2 ms, of which 3.0 are the build, and wide tier 0.99 -> 0.32,
+// against AND + popcount over the set bits as for rows in HBM.
+template <int NC, int BS>
+__device__ __forceinline__ uint32_t count4_rows(const unsigned long long* rows, uint32_t d,
+                                                uint32_t W, uint32_t RS, uint32_t part,
+                                                uint32_t n_parts, const uint16_t* list) {
+  constexpr uint32_t kWaves = BS / kWave;
+  const uint32_t g = lane_id() >> 4, w = uniform(threadIdx.x / kWave);
+  uint32_t all[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) all[c] = 4 * c + g < 2 * W ? ~0u : 0u;
+  const uint32_t nt = (d + 15) / 16;
+  uint32_t c = 0, unused = 0;
+  for (uint32_t k = 0; part + k * kWaves * n_parts < nt; ++k) {
+    const uint32_t jg = part + (k * kWaves + (k & 1 ? kWaves - 1 - w : w)) * n_parts;
+    if (jg < nt)
+      c += (uint32_t)count5_blocks<NC, 1, false>(reinterpret_cast<const uint32_t*>(rows), 2 * RS,
+                                                 all, list, nt, jg, unused);
+  }
+  return c;
+}
+
 // Block per root.  LDS_ROWS: rows, S, lens, begins and the bitmap of S live in
 // dynamic LDS (|S| <= cap, W <= MAXW words per row).  Otherwise rows live in this block's
 // HBM region `grows` (cap*W words) and membership in S is a binary search.
 // Waves per SIMD the registers have to leave room for: as many as the LDS of
-// two resident blocks (k = 5, 8-word rows) needs.
+// three resident blocks (8-word rows) needs.
 constexpr int block_waves(int k, int mode, bool lds_rows, int maxw) {
-  return k == 5 && (mode == kCount || mode == kAll) && lds_rows && maxw == 8 ? 4 : 1;
+  return k >= 4 && (mode == kCount || mode == kAll) && lds_rows && maxw == 8 ? 6 : 1;
 }
+
+// into = GPM_ROWS(128-position chunks of this root's rows), among the tier's counts.
+#define GPM_BY_CHUNKS(into)                                                 \
+  if (MAXW == 8) {                                                          \
+    switch ((W + 1) / 2) {                                                  \
+      case 0: case 1: into = GPM_ROWS(1); break;                            \
+      case 2: into = GPM_ROWS(2); break;                                    \
+      case 3: into = GPM_ROWS(3); break;                                    \
+      default: into = GPM_ROWS(4); break;                                   \
+    }                                                                       \
+  } else {                                                                  \
+    switch ((W + 1) / 2) {                                                  \
+      case 0: case 1: case 2: case 3: case 4: case 5: into = GPM_ROWS(5); break; \
+      case 6: into = GPM_ROWS(6); break;                                    \
+      case 7: into = GPM_ROWS(7); break;                                    \
+      default: into = GPM_ROWS(8); break;                                   \
+    }                                                                       \
+  }
 
 template <int K, int MODE, bool LDS_ROWS, int MAXW, int BS>
 __global__ __launch_bounds__(BS, block_waves(K, MODE, LDS_ROWS, MAXW)) void clique_block_kernel(
@@ -720,6 +691,7 @@ __global__ __launch_bounds__(BS, block_waves(K, MODE, LDS_ROWS, MAXW)) void cliq
   }
   const uint32_t id_base = n > kIdBits ? n - kIdBits : 0u;
   constexpr bool kCount5 = LDS_ROWS && K == 5 && (MODE == kCount || MODE == kAll);
+  constexpr bool kCount4 = LDS_ROWS && K == 4 && MODE == kCount;
   uint64_t acc = 0, acc3 = 0, acc4 = 0;
   if (kCount5 && threadIdx.x < BS / kWave * 3) (&s_tot[0][0])[threadIdx.x] = 0ull;
   while (true) {
@@ -826,21 +798,7 @@ __global__ __launch_bounds__(BS, block_waves(K, MODE, LDS_ROWS, MAXW)) void cliq
       constexpr bool ALL = MODE == kAll;
       uint32_t r3 = 0, r4 = 0, c = 0;
 #define GPM_ROWS(NC) count5_rows<NC, ALL, BS>(rows, d, W, RS, part, n_parts, lists, r3, r4)
-      if (MAXW == 8) {
-        switch ((W + 1) / 2) {
-          case 0: case 1: c = GPM_ROWS(1); break;
-          case 2: c = GPM_ROWS(2); break;
-          case 3: c = GPM_ROWS(3); break;
-          default: c = GPM_ROWS(4); break;
-        }
-      } else {
-        switch ((W + 1) / 2) {
-          case 0: case 1: case 2: case 3: case 4: case 5: c = GPM_ROWS(5); break;
-          case 6: c = GPM_ROWS(6); break;
-          case 7: c = GPM_ROWS(7); break;
-          default: c = GPM_ROWS(8); break;
-        }
-      }
+      GPM_BY_CHUNKS(c)
 #undef GPM_ROWS
       // The totals stay in LDS: the count needs the registers.
       const uint64_t w5 = wave_sum_u64(c), w3 = ALL ? wave_sum_u64(r3) : 0,
@@ -853,41 +811,15 @@ __global__ __launch_bounds__(BS, block_waves(K, MODE, LDS_ROWS, MAXW)) void cliq
           t[2] += w4;
         }
       }
+    } else if constexpr (kCount4) {
+      uint16_t* list = reinterpret_cast<uint16_t*>(lens);
+      for (uint32_t i = threadIdx.x; i < d + kWave; i += BS) list[i] = (uint16_t)min(i, d);
+      __syncthreads();
+#define GPM_ROWS(NC) count4_rows<NC, BS>(rows, d, W, RS, part, n_parts, list)
+      GPM_BY_CHUNKS(c)
+#undef GPM_ROWS
     } else if ((MODE == kCount || MODE == kAll) && K >= 4) {
-      // Narrowest register width that holds this root's rows.
-      constexpr bool ALL = MODE == kAll;
-      // One instantiation per word count: the k = 5 loop reads MAXW words
-      // of every row it visits, so a narrower width saves LDS reads.
-#define GPM_PAIRS(NW)                                                                     \
-  count_pairs<K, (MAXW == 8 ? ((NW) <= 8 ? (NW) : 8) : (MAXW == 16 ? (NW) : MAXW)), BS, ALL>( \
-      rows, d, W, RS, part, n_parts, s_pre, s_wsum, acc3, acc4)
-      if (MAXW == 8) {
-        switch (W) {
-          case 0: case 1: case 2: c = GPM_PAIRS(2); break;
-          case 3: c = GPM_PAIRS(3); break;
-          case 4: c = GPM_PAIRS(4); break;
-          case 5: c = GPM_PAIRS(5); break;
-          case 6: c = GPM_PAIRS(6); break;
-          case 7: c = GPM_PAIRS(7); break;
-          default: c = GPM_PAIRS(8); break;
-        }
-      } else if (MAXW == 16) {
-        switch (W) {
-          case 0: case 1: case 2: case 3: case 4: case 5: case 6: case 7: case 8: case 9:
-            c = GPM_PAIRS(9); break;
-          case 10: c = GPM_PAIRS(10); break;
-          case 11: c = GPM_PAIRS(11); break;
-          case 12: c = GPM_PAIRS(12); break;
-          case 13: c = GPM_PAIRS(13); break;
-          case 14: c = GPM_PAIRS(14); break;
-          case 15: c = GPM_PAIRS(15); break;
-          default: c = GPM_PAIRS(16); break;
-        }
-      } else {
-        c = count_pairs<K, MAXW, BS, ALL>(rows, d, W, RS, part, n_parts, s_pre, s_wsum, acc3,
-                                          acc4);
-      }
-#undef GPM_PAIRS
+      c = count_pairs<K, BS, MODE == kAll>(rows, d, W, RS, part, n_parts, s_pre, s_wsum, acc3, acc4);
     } else {
       c = count_rows<K, MODE, BS>(rows, d, W, RS, part, n_parts, lens);
     }
@@ -1049,8 +981,8 @@ int launch_tiers(gpm_graph* g, const RootTiers* t, unsigned long long* out,
 template <int MODE>
 int launch_k(gpm_graph* g, int k, const RootTiers* t, unsigned long long* out,
              unsigned long long* work) {
-  if (MODE == kAll) return launch_tiers<5, MODE>(g, t, out, work);
-  switch (k) {
+  if constexpr (MODE == kAll) return launch_tiers<5, MODE>(g, t, out, work);
+  else switch (k) {
     case 3: return launch_tiers<3, MODE>(g, t, out, work);
     case 4: return launch_tiers<4, MODE>(g, t, out, work);
     default: return launch_tiers<5, MODE>(g, t, out, work);

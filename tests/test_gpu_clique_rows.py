@@ -90,3 +90,13 @@ def test_wave_tier_long_lists(gpm, met):
     with gpm.DeviceGraph(gpm.orient(g), oriented=True) as dag:
         for k in (3, 4, 5):
             assert dag.clique(k) == comb(200, k) + m * comb(met, k - 1)
+
+
+@pytest.mark.parametrize("degree", [65, 96, 97, 300, 512, 700, 1000])
+def test_k4_split(gpm, orc, degree):
+    """4-cliques of hubs cut into parts of row blocks, more of them than row blocks too."""
+    d = hub_dag(gpm, degree, 0.3, degree)
+    want = orc.clique(d.offsets, d.adj, 4)
+    with gpm.DeviceGraph(d, oriented=True) as dg:
+        assert dg.clique(4) == want
+        assert dg.clique(4, policy=gpm.SCHED_DEGREE_SPLIT) == want
