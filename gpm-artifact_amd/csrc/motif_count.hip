@@ -144,11 +144,11 @@ __global__ __launch_bounds__(kBlock) void stream_triangles_kernel(
       }
     }
     __syncthreads();
-    auto count = [&](uint32_t pos) {  // one triangle on entry `pos` of S
+    auto count = [&](uint32_t pos, uint32_t triangles) {  // on entry `pos` of S
       if (pos < kTriCounters)
-        atomicAdd(&s_cnt[pos], 1u);
+        atomicAdd(&s_cnt[pos], triangles);
       else
-        atomicAdd(&tri[sb + pos], 1u);
+        atomicAdd(&tri[sb + pos], triangles);
     };
     for (uint32_t c0 = begin; c0 < end; c0 += kBlock) {
       // Lane l holds the list of neighbour c0 + kWaves l + w.
@@ -187,6 +187,7 @@ __global__ __launch_bounds__(kBlock) void stream_triangles_kernel(
       while (more) {
         uint32_t y[kCycWindows];
         const uint32_t entry = vb + ci;  // of v's list: the neighbour being streamed
+        uint32_t hits = 0;  // of the wave: one addition to the streamed neighbour's count
         more = next();
         if (more) load(y);
 #pragma unroll
@@ -201,11 +202,10 @@ __global__ __launch_bounds__(kBlock) void stream_triangles_kernel(
             const uint32_t p = upper_index(S, nlow, x[k]);
             if (p > 0 && S[p - 1] == x[k]) pos = p - 1;
           }
-          if (pos != kEmpty) {
-            count(pos);
-            if (entry >= sb) count(entry - sb);
-          }
+          if (pos != kEmpty) count(pos, 1u);
+          hits += (uint32_t)__popcll(wave_ballot(pos != kEmpty));
         }
+        if (entry >= sb && hits && lane == 0) count(entry - sb, hits);
 #pragma unroll
         for (uint32_t k = 0; k < kCycWindows; ++k) x[k] = y[k];
       }
