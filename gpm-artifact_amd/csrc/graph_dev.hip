@@ -350,7 +350,7 @@ int adopt_device_csr(uint32_t n, uint64_t m, uint32_t* d_off, uint32_t* d_adj,
       st = fail(GPM_EHIP, "event creation failed");
       break;
     }
-    if (hipMalloc(&g->counters, 64 * sizeof(unsigned long long)) != hipSuccess) {
+    if (hipMalloc(&g->counters, kCounters * sizeof(unsigned long long)) != hipSuccess) {
       st = fail(GPM_ENOMEM, "device counters");
       break;
     }
@@ -421,7 +421,7 @@ int gpm_graph_create(const uint32_t* offsets, uint32_t n, const uint32_t* adj,
       }
       if (hipMalloc(&g->off, (size_t)(n + 1) * 4) != hipSuccess ||
           hipMalloc(&g->adj, std::max<uint64_t>(m, 1) * 4) != hipSuccess ||
-          hipMalloc(&g->counters, 64 * sizeof(unsigned long long)) != hipSuccess) {
+          hipMalloc(&g->counters, kCounters * sizeof(unsigned long long)) != hipSuccess) {
         st = fail(GPM_ENOMEM, "device CSR allocation (n=%u, m=%llu)", n, (unsigned long long)m);
         break;
       }
@@ -524,7 +524,7 @@ int gpm_graph_orient(gpm_graph* sym, gpm_graph** dag) {
     if (stream_take(g->device, &g->stream) != hipSuccess ||
         hipEventCreate(&g->ev0) != hipSuccess || hipEventCreate(&g->ev1) != hipSuccess)
       st = fail(GPM_EHIP, "stream/event creation failed");
-    else if (hipMalloc(&g->counters, 64 * sizeof(unsigned long long)) != hipSuccess)
+    else if (hipMalloc(&g->counters, kCounters * sizeof(unsigned long long)) != hipSuccess)
       st = fail(GPM_ENOMEM, "device counters");
     else
       st = timing_end(sym);

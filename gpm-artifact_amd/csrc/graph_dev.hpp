@@ -13,6 +13,11 @@
 
 constexpr uint32_t kSigLabels = 8;
 
+// A handle's counters: 64 for sums and queues, then the bit matrix patterns' queue,
+// whose counters have a cache line each.
+constexpr uint32_t kQueueShards = 8, kQueueStride = 16, kPatternQueue = 64;
+constexpr uint32_t kCounters = kPatternQueue + kQueueShards * kQueueStride;
+
 struct gpm_graph {
   int device = 0;
   uint32_t n = 0;
@@ -56,7 +61,7 @@ struct gpm_graph {
   const char* mark_name[kMaxMarks] = {};
   double mark_ms[kMaxMarks] = {};
   int n_marks = 0;
-  // Scratch: one growable device buffer plus a block of 64 counters.
+  // Scratch: one growable device buffer plus a block of kCounters counters.
   void* scratch = nullptr;
   size_t scratch_bytes = 0;
   unsigned long long* counters = nullptr;

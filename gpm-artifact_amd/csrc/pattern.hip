@@ -558,8 +558,9 @@ extern "C" int gpm_pattern(gpm_graph* g, int pattern_id, int formulation, uint64
         blk = BlockMask{g->bmask, g->bmask_shift};
       }
       if ((st = timing_begin(g)) != GPM_OK) return st;
-      if ((st = zero_counters(g, 16)) != GPM_OK) return st;
-      st = bits ? launch_pattern_bits(g, pattern_id, counting, g->counters + 8, g->counters)
+      if ((st = zero_counters(g, bits ? (int)kCounters : 16)) != GPM_OK) return st;
+      st = bits ? launch_pattern_bits(g, pattern_id, counting, g->counters + kPatternQueue,
+                                      g->counters)
            : counting ? launch_pid<GPM_FORM_PATTERN>(g, pattern_id, blk, g->counters)
                       : launch_pid<GPM_FORM_G2MINER>(g, pattern_id, blk, g->counters);
       if (st != GPM_OK) return st;

@@ -39,6 +39,7 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kWaves = kBlock / kWave;
 constexpr uint32_t kBitsMaxN = 16384;
+static_assert(kPatternQueue + kQueueShards * kQueueStride <= kCounters, "the queue is in the counters");
 // A segment: the 2048 ids whose bits are one word per lane.
 constexpr uint32_t kSegWords = kWave, kSegIds = 32 * kSegWords;
 // Entries of a list: a segment's ids, filled up with the empty row's index.
@@ -267,9 +268,12 @@ __device__ __forceinline__ uint64_t sum_products(const uint32_t* x, const uint32
 // their operands: 210 registers, 2 waves per SIMD; bounds that make it spill are
 // not safe, as matrix instructions read every lane's register); otherwise P1,
 // P4 and Motif4.  R-MAT, 16 edges a vertex, all of P1 - P8 and Motif4: n = 512
-// direct 362 ms on lists, 1.7 ms here; n = 2048 counting 982 ms, 13.8 ms, half
+// direct 362 ms on lists, 1.3 ms here; n = 2048 counting 982 ms, 13.5 ms, half
 // of it P3 (3.2 M blocks of 16 x 16 pairs, 16 chunks each): latency of the row
-// loads bounds it, at two waves per SIMD.
+// loads bounds it, at two waves per SIMD.  The chunks come from kQueueShards
+// counters, and a block adds its sums up: additions to one address take about
+// 10 ns each, and with one counter and a sum per wave they were most of the n = 512
+// launches (P1 - P8 and Motif4: 1.71 ms so, 1.26 now).
 template <bool PRODUCTS>
 __global__ __launch_bounds__(kBlock, PRODUCTS ? 2 : 4) void pattern_bits_kernel(
     const uint32_t* __restrict__ adj, const uint32_t* __restrict__ src, uint64_t m, Bits g,
@@ -285,12 +289,26 @@ __global__ __launch_bounds__(kBlock, PRODUCTS ? 2 : 4) void pattern_bits_kernel(
   const uint32_t segs = g.rw / kSegWords, words = (g.n + 31) / 32, chunks = (g.n + 127) / 128;
   const uint32_t none = g.n;
   uint64_t c[6] = {0, 0, 0, 0, 0, 0};
+  const uint32_t n_chunks = (uint32_t)((m + chunk - 1) / chunk);
+  uint32_t shard = blockIdx.x % kQueueShards, drained = 0;
   while (true) {
-    unsigned long long base = 0;
-    if (lane == 0) base = atomicAdd(queue, (unsigned long long)chunk);
-    base = __shfl(base, 0, kWave);
-    if (base >= m) break;
-    const uint64_t stop = min((unsigned long long)m, base + chunk);
+    // Each counter deals out every kQueueShards-th chunk; other blocks' are read before
+    // they are added to, since most are drained by then.
+    const uint32_t mine = n_chunks > shard ? (n_chunks - shard - 1) / kQueueShards + 1 : 0u;
+    unsigned long long* counter = queue + shard * kQueueStride;
+    uint32_t t = 0;
+    if (lane == 0)
+      t = drained && __hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= mine
+              ? mine
+              : (uint32_t)atomicAdd(counter, 1ull);
+    t = uniform(wave_bcast(t, 0));
+    if (t >= mine) {
+      shard = (shard + 1) % kQueueShards;
+      if (++drained == kQueueShards) break;
+      continue;
+    }
+    const uint64_t base = ((uint64_t)t * kQueueShards + shard) * chunk;
+    const uint64_t stop = min(m, base + chunk);
     for (uint64_t e = base; e < stop; ++e) {
       const uint32_t v0 = uniform(src[e]), v1 = uniform(adj[e]);
       if (v0 == v1 || (pid == 4 && v1 >= v0)) continue;
@@ -397,10 +415,7 @@ __global__ __launch_bounds__(kBlock, PRODUCTS ? 2 : 4) void pattern_bits_kernel(
     }
   }
 #pragma unroll
-  for (int i = 0; i < (PRODUCTS ? 3 : 6); ++i) {
-    c[i] = wave_sum_u64(c[i]);
-    if (lane == 0 && c[i]) atomicAdd(&out[i], (unsigned long long)c[i]);
-  }
+  for (int i = 0; i < (PRODUCTS ? 3 : 6); ++i) block_add(&out[i], c[i]);
 }
 
 unsigned grid_of(const gpm_graph* g, uint64_t threads) {
