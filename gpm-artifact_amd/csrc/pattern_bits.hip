@@ -42,6 +42,9 @@ constexpr uint32_t kBitsMaxN = 16384;
 static_assert(kPatternQueue + kQueueShards * kQueueStride <= kCounters, "the queue is in the counters");
 // A segment: the 2048 ids whose bits are one word per lane.
 constexpr uint32_t kSegWords = kWave, kSegIds = 32 * kSegWords;
+// Columns of a step of a product.
+constexpr uint32_t kStepIds = 512;
+static_assert(kSegIds % kStepIds == 0, "rows are whole steps");
 // Entries of a list: a segment's ids, filled up with the empty row's index.
 constexpr uint32_t kListLen = kSegIds + kWave;
 enum Matrix { kN, kNotN, kBelowNotN, kAboveNotN, kBelowN, kAboveN, kMatrices };
@@ -125,13 +128,16 @@ __device__ __forceinline__ uint32_t list_bits(uint32_t word, uint32_t seg, uint3
 struct Product {
   const uint32_t *x, *y;   // matrices of a's and b's rows
   const uint32_t *ca, *cb; // column sets of X[a] (with R2's ids for Q) and of Y[b], in LDS
-  uint32_t rw, chunks;
+  uint32_t rw, steps;      // words of a row; steps of kStepIds columns that hold ids
   bool in;                 // Q: b in X[a], or not
 };
 
 // Blocks ja .. ja + J - 1 of R1 (list a) against blocks lb .. lb + L - 1 of R2.
-// The sizes of all J x L tiles accumulate over the chunks; the adjacency of one
-// block of b at a time then masks its column of tiles.  A lane's sum stays
+// A step takes 512 columns: a lane loads four words of a row together (64 bytes of
+// every row, where a word each left the wave 16 bytes of 16 lines), and matrix
+// instruction k of the step multiplies word k of every lane, the same columns on both
+// sides.  The sizes of all J x L tiles accumulate over the steps; the adjacency of
+// one block of b at a time then masks its column of tiles.  A lane's sum stays
 // below 2^24: 4 J L sizes of at most kBitsMaxN.
 template <int J, int L>
 __device__ __forceinline__ uint32_t product_tiles(const Product& p, const uint16_t* a,
@@ -140,33 +146,37 @@ __device__ __forceinline__ uint32_t product_tiles(const Product& p, const uint16
   const uint32_t lane = lane_id(), r16 = lane & 15, g = lane >> 4;
   uint32_t ra[J], rb[L], ib[L];
 #pragma unroll
-  for (int q = 0; q < J; ++q) ra[q] = a[16 * (ja + q) + r16] * p.rw + g;
+  for (int q = 0; q < J; ++q) ra[q] = a[16 * (ja + q) + r16] * p.rw + 4 * g;
 #pragma unroll
   for (int q = 0; q < L; ++q) {
     ib[q] = b[16 * (lb + q) + r16];
-    rb[q] = ib[q] * p.rw + g;
+    rb[q] = ib[q] * p.rw + 4 * g;
   }
   floatx4 both[J][L];
 #pragma unroll
   for (int q = 0; q < J; ++q)
 #pragma unroll
     for (int t = 0; t < L; ++t) both[q][t] = floatx4{0.f, 0.f, 0.f, 0.f};
-  for (uint32_t c = 0; c < p.chunks; ++c) {
-    const uint32_t ca = p.ca[4 * c + g], cb = p.cb[4 * c + g];
-    if (wave_ballot(cb != 0u) == 0ull) continue;
-    uint32_t wa[J], wb[L];
+  auto four = [](const uint32_t* w) { return *reinterpret_cast<const uintx4*>(w); };
+  for (uint32_t c = 0; c < p.steps; ++c) {
+    const uintx4 ca = four(p.ca + 16 * c + 4 * g), cb = four(p.cb + 16 * c + 4 * g);
+    if (wave_ballot((cb.x | cb.y | cb.z | cb.w) != 0u) == 0ull) continue;
+    uintx4 wa[J], wb[L];
 #pragma unroll
-    for (int q = 0; q < J; ++q) wa[q] = p.x[ra[q] + 4 * c];
+    for (int q = 0; q < J; ++q) wa[q] = four(p.x + ra[q] + 16 * c);
 #pragma unroll
-    for (int t = 0; t < L; ++t) wb[t] = p.y[rb[t] + 4 * c];
-    intx4 fb[L];
+    for (int t = 0; t < L; ++t) wb[t] = four(p.y + rb[t] + 16 * c);
 #pragma unroll
-    for (int t = 0; t < L; ++t) fb[t] = fp4_in_place(wb[t] & cb);
+    for (int k = 0; k < 4; ++k) {
+      intx4 fb[L];
 #pragma unroll
-    for (int q = 0; q < J; ++q) {
-      const intx4 fa = fp4_reciprocal(wa[q] & ca);
+      for (int t = 0; t < L; ++t) fb[t] = fp4_in_place(wb[t][k] & cb[k]);
 #pragma unroll
-      for (int t = 0; t < L; ++t) both[q][t] = mfma_fp4(fa, fb[t], both[q][t]);
+      for (int q = 0; q < J; ++q) {
+        const intx4 fa = fp4_reciprocal(wa[q][k] & ca[k]);
+#pragma unroll
+        for (int t = 0; t < L; ++t) both[q][t] = mfma_fp4(fa, fb[t], both[q][t]);
+      }
     }
   }
   float sum = 0.f;
@@ -176,13 +186,22 @@ __device__ __forceinline__ uint32_t product_tiles(const Product& p, const uint16
 #pragma unroll
     for (int q = 0; q < J; ++q) adj[q] = floatx4{0.f, 0.f, 0.f, 0.f};
     // b's ascend, the empty row (index n) last: it has no column.
-    const uint32_t first = uniform(ib[t]) / 128;
-    const uint32_t last = min(__builtin_amdgcn_readlane(ib[t], 15) / 128, p.chunks - 1);
+    const uint32_t first = uniform(ib[t]) / kStepIds;
+    const uint32_t last = min(__builtin_amdgcn_readlane(ib[t], 15) / kStepIds, p.steps - 1);
+    const uint32_t word = ib[t] / 32 - 4 * g, bit = 1u << (ib[t] & 31);
     for (uint32_t c = first; c <= last; ++c) {
-      const uint32_t ca = p.ca[4 * c + g];
-      const intx4 e = fp4_in_place(ib[t] / 32 == 4 * c + g ? 1u << (ib[t] & 31) : 0u);
+      const uintx4 ca = four(p.ca + 16 * c + 4 * g);
+      uintx4 wa[J];
 #pragma unroll
-      for (int q = 0; q < J; ++q) adj[q] = mfma_fp4(fp4_reciprocal(p.x[ra[q] + 4 * c] & ca), e, adj[q]);
+      for (int q = 0; q < J; ++q) wa[q] = four(p.x + ra[q] + 16 * c);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t w = word == 16 * c + k ? bit : 0u;
+        if (wave_ballot(w != 0u) == 0ull) continue;
+        const intx4 e = fp4_in_place(w);
+#pragma unroll
+        for (int q = 0; q < J; ++q) adj[q] = mfma_fp4(fp4_reciprocal(wa[q][k] & ca[k]), e, adj[q]);
+      }
     }
 #pragma unroll
     for (int q = 0; q < J; ++q)
@@ -279,14 +298,14 @@ __global__ __launch_bounds__(kBlock, PRODUCTS ? 2 : 4) void pattern_bits_kernel(
     const uint32_t* __restrict__ adj, const uint32_t* __restrict__ src, uint64_t m, Bits g,
     int pid, bool counting, uint32_t chunk, unsigned long long* __restrict__ queue,
     unsigned long long* __restrict__ out) {
-  extern __shared__ uint32_t s_words[];
+  extern __shared__ __align__(16) uint32_t s_words[];
   const uint32_t lane = lane_id(), wave = threadIdx.x / kWave;
   const uint32_t per_wave = 2 * g.rw + kListLen;  // words: two sets, two lists of halves
   uint32_t* s0 = s_words + wave * per_wave;
   uint32_t* s1 = s0 + g.rw;
   uint16_t* l0 = reinterpret_cast<uint16_t*>(s1 + g.rw);
   uint16_t* l1 = l0 + kListLen;
-  const uint32_t segs = g.rw / kSegWords, words = (g.n + 31) / 32, chunks = (g.n + 127) / 128;
+  const uint32_t segs = g.rw / kSegWords, words = (g.n + 31) / 32, steps = (g.n + kStepIds - 1) / kStepIds;
   const uint32_t none = g.n;
   uint64_t c[6] = {0, 0, 0, 0, 0, 0};
   const uint32_t n_chunks = (uint32_t)((m + chunk - 1) / chunk);
@@ -383,7 +402,7 @@ __global__ __launch_bounds__(kBlock, PRODUCTS ? 2 : 4) void pattern_bits_kernel(
         p.ca = s0;
         p.cb = pairs ? s1 : s0;
         p.rw = g.rw;
-        p.chunks = chunks;
+        p.steps = steps;
         p.in = pairs || !counting;
         uint64_t t = 0;
         for (uint32_t k = 0; k < segs; ++k) {
