@@ -1072,10 +1072,8 @@ int gpm_clique(gpm_graph* g, int k, const gpm_sched* sched, uint64_t* out) {
     if ((st = timing_begin(g)) != GPM_OK) return st;
     if ((st = zero_counters(g, 1)) != GPM_OK) return st;
     if ((st = launch_k<kCount>(g, k, t, g->counters, nullptr)) != GPM_OK) return st;
-    if ((st = timing_end(g)) != GPM_OK) return st;
     unsigned long long h = 0;
-    GPM_HIP(hipMemcpyAsync(&h, g->counters, sizeof(h), hipMemcpyDeviceToHost, g->stream));
-    GPM_HIP(hipStreamSynchronize(g->stream));
+    if ((st = timing_end(g, &h, g->counters, sizeof(h))) != GPM_OK) return st;
     *out = h;
     return GPM_OK;
   });
@@ -1095,10 +1093,8 @@ int gpm_clique_all(gpm_graph* g, const gpm_sched* sched, uint64_t out[3]) {
     if ((st = timing_begin(g)) != GPM_OK) return st;
     if ((st = zero_counters(g, 3)) != GPM_OK) return st;
     if ((st = launch_k<kAll>(g, 5, t, g->counters, nullptr)) != GPM_OK) return st;
-    if ((st = timing_end(g)) != GPM_OK) return st;
     unsigned long long h[3] = {0, 0, 0};
-    GPM_HIP(hipMemcpyAsync(h, g->counters, sizeof(h), hipMemcpyDeviceToHost, g->stream));
-    GPM_HIP(hipStreamSynchronize(g->stream));
+    if ((st = timing_end(g, h, g->counters, sizeof(h))) != GPM_OK) return st;
     for (int i = 0; i < 3; ++i) out[i] = h[i];
     return GPM_OK;
   });

@@ -217,9 +217,10 @@ int timing_mark(gpm_graph* g, const char* name) {
   return GPM_OK;
 }
 
-int timing_end(gpm_graph* g) {
+int timing_end(gpm_graph* g, void* dst, const void* src, size_t bytes) {
   GPM_HIP(hipEventRecord(g->ev1, g->stream));
-  GPM_HIP(hipEventSynchronize(g->ev1));
+  if (bytes) GPM_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, g->stream));
+  GPM_HIP(hipStreamSynchronize(g->stream));
   float ms = 0.f;
   GPM_HIP(hipEventElapsedTime(&ms, g->ev0, g->ev1));
   g->last_ms = ms;

@@ -136,7 +136,8 @@ int zero_counters(gpm_graph* g, int count);
 int timing_begin(gpm_graph* g);
 // Records an event after the kernel just launched; `name` must be static.
 int timing_mark(gpm_graph* g, const char* name);
-int timing_end(gpm_graph* g);
+// The results at src go to dst behind the stop mark: one wait for both.
+int timing_end(gpm_graph* g, void* dst = nullptr, const void* src = nullptr, size_t bytes = 0);
 // Mean list length an adjacency entry meets, sum d^2 / sum d (kept on the handle).
 double mean_met_degree(gpm_graph* g);
 // Number of compute units of the handle's device.

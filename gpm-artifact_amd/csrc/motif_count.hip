@@ -758,11 +758,9 @@ int motif4_by_identities(gpm_graph* g, uint64_t out[6]) {
                        static_cast<const CycleTask*>(tk.light), tk.n_light, g->counters + 5);
   GPM_HIP(hipGetLastError());
   timing_mark(g, "motif_cycles");
-  if ((st = timing_end(g)) != GPM_OK) return st;
-  double ms_main = g->last_ms;
   unsigned long long h[6];
-  GPM_HIP(hipMemcpyAsync(h, g->counters, sizeof(h), hipMemcpyDeviceToHost, g->stream));
-  GPM_HIP(hipStreamSynchronize(g->stream));
+  if ((st = timing_end(g, h, g->counters, sizeof(h))) != GPM_OK) return st;
+  double ms_main = g->last_ms;
   uint64_t k4 = 0;
   if ((st = gpm_clique(g->dag, 4, nullptr, &k4)) != GPM_OK) return st;
   g->last_ms = ms_main + g->dag->last_ms;

@@ -564,10 +564,8 @@ extern "C" int gpm_pattern(gpm_graph* g, int pattern_id, int formulation, uint64
            : counting ? launch_pid<GPM_FORM_PATTERN>(g, pattern_id, blk, g->counters)
                       : launch_pid<GPM_FORM_G2MINER>(g, pattern_id, blk, g->counters);
       if (st != GPM_OK) return st;
-      if ((st = timing_end(g)) != GPM_OK) return st;
       unsigned long long hh[6];
-      GPM_HIP(hipMemcpyAsync(hh, g->counters, sizeof(hh), hipMemcpyDeviceToHost, g->stream));
-      GPM_HIP(hipStreamSynchronize(g->stream));
+      if ((st = timing_end(g, hh, g->counters, sizeof(hh))) != GPM_OK) return st;
       for (int i = 0; i < 6; ++i) h[i] = hh[i];
       if (counting) h[0] = h1_only ? h[1] : h[1] - h[2];  // modulo 2^64, exact when >= 0
     }

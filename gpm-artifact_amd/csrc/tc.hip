@@ -778,12 +778,10 @@ int tc_run(gpm_graph* g, int variant, int reps, uint64_t* out) {
     for (int r = 0; r < reps; ++r)
       if ((st = enqueue_tc(g, variant, r == 0)) != GPM_OK) return st;
   }
-  if ((st = timing_end(g)) != GPM_OK) return st;
-  g->last_ms /= graph ? (double)launches * kTcGraphReps : (double)reps;
   unsigned long long h[kTcGraphReps] = {};
   const int nread = graph ? kTcGraphReps : 1;
-  GPM_HIP(hipMemcpyAsync(h, g->counters, nread * sizeof(h[0]), hipMemcpyDeviceToHost, g->stream));
-  GPM_HIP(hipStreamSynchronize(g->stream));
+  if ((st = timing_end(g, h, g->counters, nread * sizeof(h[0]))) != GPM_OK) return st;
+  g->last_ms /= graph ? (double)launches * kTcGraphReps : (double)reps;
   for (int r = 1; r < nread; ++r)
     if (h[r] != h[0]) return fail(GPM_EHIP, "repeated triangle counts disagree");
   *out = h[0];
