@@ -873,6 +873,19 @@ __device__ __forceinline__ void square_walk(const DevGraph& g, const QPlan& p,
   }
 }
 
+// Pairs (a, b) the DFS would look at below every root, before its filters.
+__global__ __launch_bounds__(kBlock) void square_pairs_kernel(DevGraph g, QPlan p,
+                                                              const uint32_t* __restrict__ roots,
+                                                              uint32_t n_roots,
+                                                              unsigned long long* __restrict__ pairs) {
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n_roots; i += gridDim.x * blockDim.x) {
+    uint32_t begin, an, bn;
+    label_slice(g, roots[i], p.label[1], &begin, &an);
+    label_slice(g, roots[i], p.label[2], &begin, &bn);
+    pairs[i] = (unsigned long long)an * bn;
+  }
+}
+
 // The roots of one square plan, heaviest first, a block per root.  `classes`:
 // vertices of depth 3's label; band: counters in LDS.
 template <bool kWide>
@@ -1691,7 +1704,13 @@ bool square_plan(const QPlan& p, QPlan* sq) {
   std::swap(sq->nlf_n[2], sq->nlf_n[3]);
   std::swap(sq->nlf_label[2], sq->nlf_label[3]);
   std::swap(sq->nlf_count[2], sq->nlf_count[3]);
-  return true;
+  sq->bn[2] = 1u;
+  sq->bn[3] = 6u;
+  for (uint32_t d = 2; d < 4; ++d) {
+    sq->same[d] = 0;
+    for (uint32_t j = 0; j < d; ++j) sq->same[d] |= (sq->label[j] == sq->label[d] ? 1u : 0u) << j;
+  }
+  return true;  // the tail is depth 3 alone in either order
 }
 
 // Builds g->lpos and g->lloc if missing.
@@ -1721,51 +1740,71 @@ int ensure_label_positions(gpm_graph* g, const uint32_t* d_lvoff) {
 
 // Moves the roots of the square plans (which: their indexes in plans) that the
 // square kernel takes out of the batch's tasks: the lists in b->d_roots, b->d_rlen
-// and rlen are sorted by length and the plans keep the shorter end.  GPM_ENOMEM
-// changes nothing.
+// and rlen are sorted by weight and the plans keep the lighter end, in the square's
+// order (the DFS walks a light root's pairs there, not whole lists of its neighbours:
+// R-MAT scale 21 with 8 labels, 70 ms so, 2.1 in this order).  GPM_ENOMEM changes
+// nothing.
 int build_squares(gpm_graph* g, std::vector<QPlan>& plans, const std::vector<uint32_t>& which,
                   std::vector<uint32_t>& rlen, const uint32_t* d_lvoff, int n_counters,
                   MatchBatch* b) {
   if (which.empty()) return GPM_OK;
   int st = ensure_label_positions(g, d_lvoff);
   if (st != GPM_OK) return st;
-  std::vector<uint32_t> roots;
+  struct Laid {  // a plan's roots and lengths by weight, the first `take` for the kernel
+    std::vector<uint32_t> roots, lens;
+    uint32_t take = 0;
+    size_t valid_at = 0;
+    bool wide = false;
+  };
+  std::vector<Laid> laid(which.size());
   size_t valid_words = 0;
-  std::vector<size_t> root_at, valid_at;
-  std::vector<uint32_t> taken;
-  for (const uint32_t i : which) {
+  uint32_t most = 0;
+  for (const uint32_t i : which) most = std::max(most, plans[i].n_roots);
+  struct Pairs {
+    unsigned long long* d = nullptr;
+    ~Pairs() { (void)hipFree(d); }
+  } d_pairs;
+  if (hipMalloc(&d_pairs.d, (size_t)most * 8) != hipSuccess) {
+    d_pairs.d = nullptr;
+    (void)hipGetLastError();
+    return fail(GPM_ENOMEM, "square plans' weights");
+  }
+  for (size_t w = 0; w < which.size(); ++w) {
     QPlan p;
-    (void)square_plan(plans[i], &p);
+    (void)square_plan(plans[which[w]], &p);
     std::vector<uint32_t> mine(p.n_roots), order(p.n_roots);
+    std::vector<unsigned long long> pairs(p.n_roots);
+    hipLaunchKernelGGL(square_pairs_kernel, dim3(std::min((p.n_roots + kBlock - 1) / kBlock, 1024u)),
+                       dim3(kBlock), 0, g->stream, b->dg, p, b->d_roots + p.root_off, p.n_roots,
+                       d_pairs.d);
+    GPM_HIP(hipGetLastError());
     GPM_HIP(hipMemcpyAsync(mine.data(), b->d_roots + p.root_off, (size_t)p.n_roots * 4,
                            hipMemcpyDeviceToHost, g->stream));
+    GPM_HIP(hipMemcpyAsync(pairs.data(), d_pairs.d, (size_t)p.n_roots * 8, hipMemcpyDeviceToHost,
+                           g->stream));
     GPM_HIP(hipStreamSynchronize(g->stream));
     std::iota(order.begin(), order.end(), 0u);
     std::sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) {
-      const uint32_t lx = rlen[p.root_off + x], ly = rlen[p.root_off + y];
-      return lx > ly || (lx == ly && mine[x] < mine[y]);
+      return pairs[x] > pairs[y] || (pairs[x] == pairs[y] && mine[x] < mine[y]);
     });
-    root_at.push_back(roots.size());
-    const uint32_t classes = g->h_lvoff[p.label[3] + 1] - g->h_lvoff[p.label[3]];
-    // One band: every root with a depth-1 entry (4 labels, ER n=200k m=1M: 0.76 ms
-    // with all roots here, 0.91 with those of 16 entries and more, 0.87 all DFS).
+    Laid& l = laid[w];
+    const auto first = rlen.begin() + p.root_off;
+    l.wide = *std::max_element(first, first + p.n_roots) > 65535u;
+    // One band: every root with a pair (4 labels, ER n=200k m=1M: 0.76 ms with all
+    // roots here, 0.91 with those of 16 depth-1 entries and more, 0.87 all DFS).
     // More: a pair of the DFS costs a CU 0.29 us, a band 2.9 us on light roots
     // (no labels, same graph, 6 bands: 13.4 ms here, 20.5 from 16 entries on, 22.4
     // all DFS; R-MAT scale 18 ef 4, 8 bands: 17.6, 16.3, 1260), so from
-    // sqrt(10 bands) entries on.
-    const bool wide = rlen[p.root_off + order[0]] > 65535u;
-    const uint32_t bands = (classes + square_band(wide) - 1) / square_band(wide);
-    const uint32_t least = bands <= 1 ? 1u : (uint32_t)std::ceil(std::sqrt(10.0 * bands));
-    uint32_t take = 0;
-    std::vector<uint32_t> lens(p.n_roots);
-    for (uint32_t k = 0; k < p.n_roots; ++k) {
-      lens[k] = rlen[p.root_off + order[k]];
-      take += lens[k] >= least;
+    // 10 pairs a band on.
+    const uint32_t classes = g->h_lvoff[p.label[3] + 1] - g->h_lvoff[p.label[3]];
+    const uint64_t bands = (classes + square_band(l.wide) - 1) / square_band(l.wide);
+    const uint64_t least = bands <= 1 ? 1 : 10 * bands;
+    for (const uint32_t r : order) {
+      l.roots.push_back(mine[r]);
+      l.lens.push_back(first[r]);
+      l.take += pairs[r] >= least;
     }
-    std::copy(lens.begin(), lens.end(), rlen.begin() + p.root_off);
-    for (const uint32_t r : order) roots.push_back(mine[r]);
-    taken.push_back(take);
-    valid_at.push_back(valid_words);
+    l.valid_at = valid_words;
     valid_words += (classes + 31) / 32;
   }
   const size_t counts = ((size_t)n_counters + 1) * 2;  // words
@@ -1782,19 +1821,22 @@ int build_squares(gpm_graph* g, std::vector<QPlan>& plans, const std::vector<uin
     QPlan sq;
     (void)square_plan(plans[which[k]], &sq);
     QPlan& p = plans[which[k]];
-    if ((st = h2d(g, b->d_roots + p.root_off, roots.data() + root_at[k], (size_t)p.n_roots * 4)) != GPM_OK ||
-        (st = h2d(g, b->d_rlen + p.root_off, rlen.data() + p.root_off, (size_t)p.n_roots * 4)) != GPM_OK)
+    const Laid& l = laid[k];
+    std::copy(l.lens.begin(), l.lens.end(), rlen.begin() + p.root_off);
+    if ((st = h2d(g, b->d_roots + p.root_off, l.roots.data(), l.roots.size() * 4)) != GPM_OK ||
+        (st = h2d(g, b->d_rlen + p.root_off, l.lens.data(), l.lens.size() * 4)) != GPM_OK)
       return st;
     const uint32_t first = g->h_lvoff[sq.label[3]], count = g->h_lvoff[sq.label[3] + 1] - first;
     hipLaunchKernelGGL(square_valid_kernel,
                        dim3(std::max(1u, std::min((count + 32 * kBlock - 1) / (32 * kBlock), 1024u))),
                        dim3(kBlock), 0, g->stream, b->dg, sq, g->lverts + first, count,
-                       d_valid + valid_at[k]);
+                       d_valid + l.valid_at);
     GPM_HIP(hipGetLastError());
-    b->squares.push_back({sq, b->d_roots + p.root_off, d_valid + valid_at[k], taken[k], count,
-                          rlen[p.root_off] > 65535u});
-    p.root_off += taken[k];
-    p.n_roots -= taken[k];
+    b->squares.push_back(
+        {sq, b->d_roots + p.root_off, d_valid + l.valid_at, l.take, count, l.wide});
+    p = sq;
+    p.root_off += l.take;
+    p.n_roots -= l.take;
   }
   return GPM_OK;
 }

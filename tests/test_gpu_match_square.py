@@ -65,3 +65,19 @@ def test_hub(gpm):
         with gpm.DeviceGraph(g, oriented=False, labels=lab, n_labels=2) as dg:
             got = dg.match_batch([(4, SQUARE, [0, 1, 0, 1])]).tolist()
         assert got == [2 * m * (m - 1)]
+
+
+@pytest.mark.parametrize("kind", ["er", "rmat"])
+def test_bands_and_orders_agree_with_the_dfs(gpm, kind):
+    """Two labels of more vertices than a band, light roots left to the DFS, every order
+    of the cycle, against the DFS of all roots (a replayed graph keeps it)."""
+    g = gpm.er_graph(150000, 700000, 3) if kind == "er" else gpm.rmat_graph(17, 6, 3)
+    n = len(g.offsets) - 1
+    lab = gpm.gen_labels(n, 2, 7)
+    with gpm.DeviceGraph(g, oriented=False, labels=lab, n_labels=2) as dg:
+        for labels in ((0, 0, 0, 0), (0, 1, 0, 1), (0, 0, 1, 1), (0, 1, 1, 1)):
+            for edges in (SQUARE, PATH_FIRST):
+                q = [(4, edges, list(labels))]
+                want = dg.match_batch(q, autotune=0, chunk=8, use_graph=1).tolist()
+                assert dg.match_batch(q, policy=0).tolist() == want
+                assert dg.match_batch(q, policy=1).tolist() == want
