@@ -69,16 +69,16 @@ def measured_lds(kernel, scale):
     SQ_INSTS_LDS_STORE_BANDWIDTH, 64-byte units), "active": LDS-active share of
     CU cycles (SQ_LDS_IDX_ACTIVE / (GRBM_GUI_ACTIVE x CUs)), "conflict": bank-conflict
     share of LDS-active cycles, "valu_instr": VALU wave64 instructions issued
-    (SQ_INSTS_VALU), "valu_active": VALU-busy share of SIMD cycles} per launch."""
+    (SQ_INSTS_VALU - SQ_INSTS_MFMA), "valu_active": VALU-busy share of SIMD cycles} per launch."""
     return _profile_json(LDS_PROFILE, "lds_json", kernel, scale)
 
 
 def roofline(dom, dom_ms, alg_bytes, traffic, lds):
     """Roofline of the dominant k-clique kernel.  Its rows live in LDS and its
-    inner loops are row-word ANDs and popcounts; the PMC summary shows it
-    issuing VALU instructions at ~93 % of the chip's rate with LDS at ~15 % of
-    its bandwidth, so the bound is VALU issue: achieved = VALU wave64
-    instructions per launch (SQ_INSTS_VALU) / the launch's event-timed
+    inner loops expand row words to operands of the matrix cores; the PMC summary
+    shows it issuing VALU instructions at ~94 % of the chip's rate with the matrix
+    cores and LDS at ~16 % of theirs, so the bound is VALU issue: achieved = VALU
+    wave64 instructions per launch (SQ_INSTS_VALU - SQ_INSTS_MFMA) / the launch's event-timed
     duration, peak = 1024 SIMDs x 2.4 GHz / 4 cycles per wave64 instruction.
     LDS bandwidth and HBM traffic are reported beside it, and the canonical
     edge-rooted plan's bytes over the same time as a plain rate (the bitmap
