@@ -150,6 +150,10 @@ int try_topo(gpm_graph* g);
 // Orients the SYMMETRIC graph by (degree, id) (prep.hip): CSR in new device buffers
 // *d_off, *d_adj, the caller's, and the offsets on the host; lists keep their order.
 int orient_device(gpm_graph* sym, uint32_t** d_off, uint32_t** d_adj, std::vector<uint32_t>* h_off);
+// The vertices [first, first + count) by decreasing out-degree, equal ones by id, as
+// rank[v] where rank (a host array of all vertices) is given, to out (prep.hip).
+int degree_order_device(gpm_graph* g, uint32_t first, uint32_t count, const uint32_t* rank,
+                        uint32_t* out);
 // Relabels the ORIENTED graph g by (out-degree + in-degree, id) on the device
 // (prep.hip).  Where every edge goes up in that order -- gpm_graph_orient and
 // gpm_csr_orient give such graphs -- *ordered is set and *toff / *tadj /

@@ -143,6 +143,17 @@ __global__ void scatter_rank_kernel(const uint32_t* __restrict__ order, uint32_t
     new_id[order[r]] = r;
 }
 
+// Degree order of a range: sort keys max_deg - deg(v) and values rank[v] (or v).
+__global__ void order_keys_kernel(const uint32_t* __restrict__ off, uint32_t first, uint32_t count,
+                                  uint32_t max_deg, const uint32_t* __restrict__ rank,
+                                  uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += gridDim.x * blockDim.x) {
+    const uint32_t v = first + i;
+    keys[i] = max_deg - (off[v + 1] - off[v]);
+    vals[i] = rank ? rank[v] : v;
+  }
+}
+
 // Keys new_id[u] << 32 | new_id[x] for every entry (u, x); one wave per u.
 __global__ void relabel_keys_kernel(const uint32_t* __restrict__ off, const uint32_t* __restrict__ adj,
                                     const uint32_t* __restrict__ new_id, uint32_t n,
@@ -602,6 +613,36 @@ int orient_device(gpm_graph* sym, uint32_t** d_off, uint32_t** d_adj, std::vecto
   GPM_HIP(hipStreamSynchronize(sym->stream));
   b.release(*d_off);
   b.release(*d_adj);
+  return GPM_OK;
+}
+
+int degree_order_device(gpm_graph* g, uint32_t first, uint32_t count, const uint32_t* rank,
+                        uint32_t* out) {
+  if (!count) return GPM_OK;
+  struct Drain {  // the buffers below are freed only once the stream is done with them
+    hipStream_t s;
+    ~Drain() { (void)hipStreamSynchronize(s); }
+  };
+  Bufs b;
+  Drain drain{g->stream};
+  const unsigned bits = (unsigned)bits_for(g->max_deg);
+  size_t sort = 0;
+  uint32_t* none = nullptr;
+  GPM_HIP(rocprim::radix_sort_pairs(nullptr, sort, none, none, none, none, count, 0u, bits,
+                                    g->stream));
+  const uint64_t part = aligned((uint64_t)count * 4), rank_at = aligned(sort) + 3 * part;
+  char* temp = nullptr;
+  int st;
+  if ((st = b.alloc(&temp, rank_at + (rank ? (uint64_t)g->n * 4 : 0))) != GPM_OK) return st;
+  uint32_t* keys = reinterpret_cast<uint32_t*>(temp + aligned(sort));
+  uint32_t* sorted = reinterpret_cast<uint32_t*>(temp + aligned(sort) + part);
+  uint32_t* vals = reinterpret_cast<uint32_t*>(temp + aligned(sort) + 2 * part);
+  uint32_t* d_rank = rank ? reinterpret_cast<uint32_t*>(temp + rank_at) : nullptr;
+  if (rank && (st = h2d(g, d_rank, rank, (size_t)g->n * 4)) != GPM_OK) return st;
+  hipLaunchKernelGGL(order_keys_kernel, dim3(grid_for_items(count, device_cus(g))), dim3(kBlock), 0,
+                     g->stream, g->off, first, count, g->max_deg, d_rank, keys, vals);
+  GPM_HIP(hipGetLastError());
+  GPM_HIP(rocprim::radix_sort_pairs(temp, sort, keys, sorted, vals, out, count, 0u, bits, g->stream));
   return GPM_OK;
 }
 

@@ -1,4 +1,4 @@
-// Root tiers: the host-side split of root vertices into size classes that
+// Root tiers: the split of root vertices into size classes that
 // decides which kernel serves each root (one wave, one block with LDS rows,
 // one block with rows in HBM).  The plain degree scheduler orders each tier
 // by decreasing out-degree; the learned scheduler orders it by predicted cost
@@ -15,6 +15,7 @@ struct gpm_graph;
 namespace gpm {
 
 struct RootTiers {
+  uint32_t* d_all = nullptr;    // where set, the four lists below are parts of it
   uint32_t* d_wave = nullptr;   // roots served by one wave
   uint32_t n_wave = 0;
   uint32_t n_wave_above[2] = {0, 0};  // ... of out-degree above 8, above 16
