@@ -129,7 +129,7 @@ void stream_give(int device, hipStream_t stream);
 int ensure_scratch(gpm_graph* g, size_t bytes);
 // Builds g->src (COO sources) if missing.
 int ensure_src(gpm_graph* g);
-// Zeroes the 64-entry counter block with a kernel (no memset node, so the
+// Zeroes the first `count` counters with a kernel (no memset node, so the
 // sequence stays valid inside a captured graph).
 int zero_counters(gpm_graph* g, int count);
 // Starts / stops event timing around the kernels of one mining call.

@@ -24,7 +24,7 @@
 //    embeddings (on the reference's HPRD queries, the largest root needed
 //    1.8M serial steps without it and 60K with it).
 //  * Enumeration (device): one wave per task (a chunk of root candidates of
-//    one query), tasks pulled from one queue by a persistent grid.  The DFS
+//    one query), tasks pulled from a queue by a persistent grid.  The DFS
 //    keeps no candidate lists: at depth d it streams the label-l slice of the
 //    shortest backward neighbour's list 64 entries at a time, keeps a 64-bit
 //    ballot of the entries that pass (degree, injectivity, membership in the
@@ -643,7 +643,7 @@ struct HeavyTask {
   uint32_t cut[kCutLevels];
 };
 
-// Persistent enumeration: every wave pulls tasks from one queue until it is
+// Persistent enumeration: every wave pulls tasks from the queue until it is
 // drained.  Tasks [0, n_heavy) are parts of heavy roots (heaviest first);
 // the rest are chunks of a query's root list, which skip the heavy roots.
 // Counted per task: steps = windows + descents.  A plan trial (kTrial)

@@ -23,7 +23,7 @@
 // between them the size is 0 whatever Q says).  P1, P4 and the direct Motif4
 // have one inner loop: |C & X[a]| summed over a.
 //
-// A row has n / 128 chunks to multiply, whatever the lists' lengths, so this
+// A row has n / 512 steps to multiply, whatever the lists' lengths, so this
 // path is for graphs of at most kBitsMaxN vertices and not for sparse large
 // ones (bits_pay).
 #include <algorithm>
@@ -284,12 +284,12 @@ __device__ __forceinline__ uint64_t sum_products(const uint32_t* x, const uint32
 
 // One wave per directed edge, in chunks from a queue.  LDS per wave: two lists
 // and two sets of rw words.  PRODUCTS: P2, P3, P5 - P8 (16 tiles of sizes and
-// their operands: 210 registers, 2 waves per SIMD; bounds that make it spill are
+// their operands: 226 registers, 2 waves per SIMD; bounds that make it spill are
 // not safe, as matrix instructions read every lane's register); otherwise P1,
 // P4 and Motif4.  R-MAT, 16 edges a vertex, all of P1 - P8 and Motif4: n = 512
-// direct 362 ms on lists, 1.3 ms here; n = 2048 counting 982 ms, 13.5 ms, half
-// of it P3 (3.2 M blocks of 16 x 16 pairs, 16 chunks each): latency of the row
-// loads bounds it, at two waves per SIMD.  The chunks come from kQueueShards
+// direct 362 ms on lists, 1.0 ms here; n = 2048 counting 982 ms, 8.0 ms, a third
+// of it P3 (3.2 M blocks of 16 x 16 pairs, 4 steps each): latency of the row loads
+// bounds it, at two waves per SIMD (four with half the tiles: 9.3 ms).  The chunks come from kQueueShards
 // counters, and a block adds its sums up: additions to one address take about
 // 10 ns each, and with one counter and a sum per wave they were most of the n = 512
 // launches (P1 - P8 and Motif4: 1.71 ms so, 1.26 now).
@@ -443,13 +443,16 @@ unsigned grid_of(const gpm_graph* g, uint64_t threads) {
 }
 
 // Whether the matrix path is the faster one.  It costs every edge n / 2048
-// segments of set work and every 16 x 16 pairs n / 128 chunks; lists cost an edge
+// segments of set work and every 16 x 16 pairs n / 512 steps; lists cost an edge
 // the pairs of its sets, each at least a window and a search.  So it is taken
 // up to one segment, and beyond where the degree an edge meets, dw = sum d^2 /
 // sum d, is large.  P2, P3, P6, P8 (both formulations) and P4, ms in all, matrix
 // against lists: Erdos-Renyi n = 1500, dw = 17: 2.0 against 6.7; n = 4096, dw = 9:
 // 3.8, 3.7; dw = 17: 8.4, 13; n = 16384, dw = 17: 532, 44; R-MAT n = 1500, dw = 48:
-// 2.0, 143; n = 8192, dw = 63: 30, 881; n = 16384, dw = 83: 226, 2994.
+// 2.0, 143; n = 8192, dw = 63: 30, 881; n = 16384, dw = 83: 226, 2994.  (Since rows are
+// loaded 16 bytes a lane the matrix side takes 1.0, 1.5, 17 and 117 in the first and the
+// three R-MAT cases; the line leaves graphs of 4096 and more vertices that are near it
+// to the lists.)
 bool bits_pay(gpm_graph* g) {
   if (g->n > kBitsMaxN || !g->m) return false;
   if (g->n <= kSegIds) return true;
