@@ -493,20 +493,38 @@ __global__ __launch_bounds__(kLightBlock) void light_cycles_kernel(
   block_add(out, acc);
 }
 
-// below[u] = neighbours of u of lower rank; wedges[u] = sum over them of their
-// neighbours below u (zero on entry): the entry (v, u) of v's list adds its
-// position, as many entries as v has below u.  One wave per v.
+// below[u] = neighbours of u of lower rank.
+__global__ __launch_bounds__(kBlock) void lower_counts_kernel(const uint32_t* __restrict__ off,
+                                                              const uint32_t* __restrict__ adj,
+                                                              uint32_t n,
+                                                              uint32_t* __restrict__ below) {
+  for (uint32_t u = blockIdx.x * blockDim.x + threadIdx.x; u < n; u += gridDim.x * blockDim.x)
+    below[u] = count_below(adj + off[u], off[u + 1] - off[u], u);
+}
+
+// wedges[u] += for every entry (u, v), v < u, the entries below u of v's list (zero on
+// entry): exactly what for_wedges visits from u, whether or not v's list holds u, since
+// light_cycles_kernel's table relies on it.  One lane per entry, so that hubs' lists are
+// spread over the chip; a wave within one list adds up first.
 __global__ __launch_bounds__(kBlock) void wedge_totals_kernel(
-    const uint32_t* __restrict__ off, const uint32_t* __restrict__ adj, uint32_t n,
-    uint32_t* __restrict__ below, unsigned long long* __restrict__ wedges) {
+    const uint32_t* __restrict__ off, const uint32_t* __restrict__ adj, uint32_t n, uint64_t m,
+    unsigned long long* __restrict__ wedges) {
   const uint32_t lane = lane_id();
-  const uint32_t nw = gridDim.x * blockDim.x / kWave;
-  for (uint32_t v = (blockIdx.x * blockDim.x + threadIdx.x) / kWave; v < n; v += nw) {
-    const uint32_t b = off[v], len = off[v + 1] - b;
-    const uint32_t first = count_below(adj + b, len, v);
-    if (lane == 0) below[v] = first;
-    for (uint32_t p = first + lane; p < len; p += kWave)
-      if (p) atomicAdd(&wedges[adj[b + p]], (unsigned long long)p);
+  const uint64_t step = (uint64_t)gridDim.x * blockDim.x;
+  for (uint64_t e0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x - lane; e0 < m; e0 += step) {
+    const uint64_t e = e0 + lane;
+    uint32_t u = kEmpty, c = 0;
+    if (e < m) {
+      u = upper_index(off, n + 1, (uint32_t)e) - 1;  // the last vertex whose list is not past e
+      const uint32_t v = adj[e];
+      if (v < u) c = count_below(adj + off[v], off[v + 1] - off[v], u);
+    }
+    if (wave_ballot(u != uniform(u)) == 0ull) {
+      const uint64_t sum = wave_sum_u64(c);
+      if (lane == 0 && sum) atomicAdd(&wedges[u], (unsigned long long)sum);
+    } else if (c) {
+      atomicAdd(&wedges[u], (unsigned long long)c);
+    }
   }
 }
 
@@ -626,8 +644,10 @@ int ensure_motif_tasks(gpm_graph* g) {
   if (n) {
     hipLaunchKernelGGL(zero_u32_kernel, dim3(grid_of(g, 2ull * n)), dim3(256), 0, g->stream,
                        reinterpret_cast<unsigned int*>(d_wedges), 2ull * n);
-    hipLaunchKernelGGL(wedge_totals_kernel, dim3(grid_of(g, (uint64_t)n * kWave)), dim3(kBlock), 0,
-                       g->stream, g->rk_off, g->rk_adj, n, d_below, d_wedges);
+    hipLaunchKernelGGL(lower_counts_kernel, dim3(grid_of(g, n)), dim3(kBlock), 0, g->stream,
+                       g->rk_off, g->rk_adj, n, d_below);
+    hipLaunchKernelGGL(wedge_totals_kernel, dim3(grid_of(g, g->m)), dim3(kBlock), 0, g->stream,
+                       g->rk_off, g->rk_adj, n, g->m, d_wedges);
     GPM_HIP(hipGetLastError());
     GPM_HIP(hipMemcpyAsync(wedges.data(), d_wedges, (size_t)n * 8, hipMemcpyDeviceToHost,
                            g->stream));
