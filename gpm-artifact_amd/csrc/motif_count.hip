@@ -260,6 +260,48 @@ __global__ __launch_bounds__(kBlock) void pair_triangles_kernel(
   }
 }
 
+// The same counts where lists are one-sided, hold a vertex twice or itself: a wave per
+// entry (u, v) with v > u walks the shorter of both ends' upper lists and searches the
+// longer (last of equal entries).  Three atomics a triangle, so mirrored lists take the
+// kernels above.
+__global__ __launch_bounds__(kBlock) void entry_triangles_kernel(
+    const uint32_t* __restrict__ off, const uint32_t* __restrict__ adj,
+    const uint32_t* __restrict__ below, uint32_t n, uint64_t m, uint32_t* __restrict__ tri) {
+  const uint32_t lane = lane_id();
+  const uint64_t nw = (uint64_t)gridDim.x * kBlock / kWave;
+  auto upper = [&](uint32_t v, uint32_t* b, uint32_t* len) {  // entries above v
+    const uint32_t end = off[v + 1];
+    for (*b = off[v] + below[v]; *b < end && adj[*b] == v;) ++*b;
+    *len = end - *b;
+  };
+  for (uint64_t e = ((uint64_t)blockIdx.x * kBlock + threadIdx.x) / kWave; e < m; e += nw) {
+    const uint32_t u = upper_index(off, n + 1, (uint32_t)e) - 1, v = adj[e];
+    if (v <= u) continue;
+    uint32_t ab, na, bb, nb;
+    upper(u, &ab, &na);
+    upper(v, &bb, &nb);
+    if (na > nb) {
+      uint32_t t = ab;
+      ab = bb;
+      bb = t;
+      t = na;
+      na = nb;
+      nb = t;
+    }
+    uint32_t hits = 0;
+    for (uint32_t i = lane; i < na; i += kWave) {
+      const uint32_t w = adj[ab + i], p = upper_index(adj + bb, nb, w);
+      if (p > 0 && adj[bb + p - 1] == w) {
+        atomicAdd(&tri[ab + i], 1u);
+        atomicAdd(&tri[bb + p - 1], 1u);
+        ++hits;
+      }
+    }
+    hits = wave_sum_u32(hits);
+    if (lane == 0 && hits) atomicAdd(&tri[e], hits);
+  }
+}
+
 // Edge sums over the undirected edges {v, x} (each once: x > v), from the per-edge
 // triangle counts c and the degrees; one wave per v:
 //   out[0] += 2c                      (sum: 6T)
@@ -277,6 +319,7 @@ __global__ __launch_bounds__(kBlock) void edge_stats_kernel(
     const uint64_t da = end - b;
     for (uint32_t e = b + below[v] + lane_id(); e < end; e += kWave) {
       const uint32_t x = adj[e];
+      if (x == v) continue;
       const uint64_t c = tri[e], db = off[x + 1] - off[x];
       s6t += 2 * c;
       spaw += c ? c * (da + db - 4) : 0;
@@ -401,8 +444,9 @@ __device__ __forceinline__ void for_wedges(const uint32_t* __restrict__ off,
 // evenly without it.
 __global__ __launch_bounds__(kCycBlock) void cycles_kernel(
     const uint32_t* __restrict__ off, const uint32_t* __restrict__ adj, uint32_t n,
-    const CycleTask* __restrict__ tasks, uint32_t n_tasks, unsigned int* __restrict__ queue,
-    uint32_t* __restrict__ counters, unsigned long long* __restrict__ out) {
+    const CycleTask* __restrict__ tasks, uint32_t n_tasks, uint32_t narrow_below,
+    unsigned int* __restrict__ queue, uint32_t* __restrict__ counters,
+    unsigned long long* __restrict__ out) {
   __shared__ __align__(16) uint32_t s_cnt[kCycWords];
   __shared__ uint32_t s_task;
   uint64_t acc = 0;
@@ -419,7 +463,7 @@ __global__ __launch_bounds__(kCycBlock) void cycles_kernel(
     t.lo = uniform(t.lo);
     t.hi = uniform(t.hi);
     t.band = uniform(t.band);
-    const uint32_t half = t.n_below < 65536u ? 1u : 0u;  // counters of 16 bits
+    const uint32_t half = t.n_below < narrow_below ? 1u : 0u;  // counters of 16 bits
     const uint32_t words = (t.hi - t.band + half) >> half;
     uint32_t* cnt = counters + (uint64_t)blockIdx.x * n;
     if (t.lo == t.band) {
@@ -504,20 +548,27 @@ __global__ __launch_bounds__(kBlock) void lower_counts_kernel(const uint32_t* __
 
 // wedges[u] += for every entry (u, v), v < u, the entries below u of v's list (zero on
 // entry): exactly what for_wedges visits from u, whether or not v's list holds u, since
-// light_cycles_kernel's table relies on it.  One lane per entry, so that hubs' lists are
+// light_cycles_kernel's table relies on it.  *mirrored += those entries that v's list
+// answers and that u's holds once: half of all entries where every edge is in both lists
+// and none is twice in one or a loop.  One lane per entry, so that hubs' lists are
 // spread over the chip; a wave within one list adds up first.
 __global__ __launch_bounds__(kBlock) void wedge_totals_kernel(
     const uint32_t* __restrict__ off, const uint32_t* __restrict__ adj, uint32_t n, uint64_t m,
-    unsigned long long* __restrict__ wedges) {
+    unsigned long long* __restrict__ wedges, unsigned long long* __restrict__ mirrored) {
   const uint32_t lane = lane_id();
   const uint64_t step = (uint64_t)gridDim.x * blockDim.x;
+  uint64_t answered = 0;
   for (uint64_t e0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x - lane; e0 < m; e0 += step) {
     const uint64_t e = e0 + lane;
     uint32_t u = kEmpty, c = 0;
     if (e < m) {
       u = upper_index(off, n + 1, (uint32_t)e) - 1;  // the last vertex whose list is not past e
       const uint32_t v = adj[e];
-      if (v < u) c = count_below(adj + off[v], off[v + 1] - off[v], u);
+      if (v < u) {
+        const uint32_t b = off[v], len = off[v + 1] - b;
+        c = count_below(adj + b, len, u);
+        if (c < len && adj[b + c] == u && (e == off[u] || adj[e - 1] != v)) ++answered;
+      }
     }
     if (wave_ballot(u != uniform(u)) == 0ull) {
       const uint64_t sum = wave_sum_u64(c);
@@ -526,6 +577,7 @@ __global__ __launch_bounds__(kBlock) void wedge_totals_kernel(
       atomicAdd(&wedges[u], (unsigned long long)c);
     }
   }
+  block_add(mirrored, answered);
 }
 
 __global__ void zero_u32_kernel(unsigned int* p, uint64_t count) {
@@ -625,6 +677,9 @@ uint32_t rk_degree(const gpm_graph* g, uint32_t v) {
   return g->motif.h_off[v + 1] - g->motif.h_off[v];
 }
 
+// Roots of fewer lower neighbours have 16-bit counters (a repeated entry could pass them).
+uint32_t narrow_limit(const gpm_graph* g) { return g->motif.mirrored ? 65536u : 0u; }
+
 // The tasks of the motif counters (g->motif), built once per handle from every
 // vertex's lower neighbours and wedge total.
 int ensure_motif_tasks(gpm_graph* g) {
@@ -639,22 +694,25 @@ int ensure_motif_tasks(gpm_graph* g) {
     return fail(GPM_ENOMEM, "lower-neighbour counts (%u)", n);
   }
   uint32_t* d_below = g->motif.below;
-  std::vector<unsigned long long> wedges(n);
+  std::vector<unsigned long long> wedges(n + 1, 0ull);  // and the mirrored entries
   std::vector<uint32_t> below(n);
   if (n) {
-    hipLaunchKernelGGL(zero_u32_kernel, dim3(grid_of(g, 2ull * n)), dim3(256), 0, g->stream,
-                       reinterpret_cast<unsigned int*>(d_wedges), 2ull * n);
+    hipLaunchKernelGGL(zero_u32_kernel, dim3(grid_of(g, 2ull * n + 2)), dim3(256), 0, g->stream,
+                       reinterpret_cast<unsigned int*>(d_wedges), 2ull * n + 2);
     hipLaunchKernelGGL(lower_counts_kernel, dim3(grid_of(g, n)), dim3(kBlock), 0, g->stream,
                        g->rk_off, g->rk_adj, n, d_below);
-    hipLaunchKernelGGL(wedge_totals_kernel, dim3(grid_of(g, g->m)), dim3(kBlock), 0, g->stream,
-                       g->rk_off, g->rk_adj, n, g->m, d_wedges);
+    hipLaunchKernelGGL(wedge_totals_kernel, dim3(std::min(grid_of(g, g->m), 8u * device_cus(g))),
+                       dim3(kBlock), 0, g->stream, g->rk_off, g->rk_adj, n, g->m, d_wedges,
+                       d_wedges + n);
     GPM_HIP(hipGetLastError());
-    GPM_HIP(hipMemcpyAsync(wedges.data(), d_wedges, (size_t)n * 8, hipMemcpyDeviceToHost,
+    GPM_HIP(hipMemcpyAsync(wedges.data(), d_wedges, ((size_t)n + 1) * 8, hipMemcpyDeviceToHost,
                            g->stream));
     GPM_HIP(hipMemcpyAsync(below.data(), d_below, (size_t)n * 4, hipMemcpyDeviceToHost,
                            g->stream));
     GPM_HIP(hipStreamSynchronize(g->stream));
   }
+  g->motif.mirrored = 2 * wedges[n] == g->m;
+  const uint32_t narrow_below = narrow_limit(g);
   std::vector<uint32_t> roots;
   std::vector<CycleTask> heavy, light;
   for (uint32_t u = n; u-- > 0;) {
@@ -667,7 +725,7 @@ int ensure_motif_tasks(gpm_graph* g) {
                    [&](uint32_t a, uint32_t b) { return wedges[a] > wedges[b]; });
   bool hbm = false;
   for (const uint32_t u : roots) {
-    const uint32_t band = below[u] < 65536u ? 2 * kCycWords : kCycWords;
+    const uint32_t band = below[u] < narrow_below ? 2 * kCycWords : kCycWords;
     uint32_t hi = u;
     auto task_to = [&](uint32_t lo) {
       heavy.push_back({u, below[u], lo, hi, hi - lo > band ? hi - band : lo});
@@ -681,7 +739,7 @@ int ensure_motif_tasks(gpm_graph* g) {
   }
   // Triangle tasks, in decreasing degree (rank).
   std::vector<TriangleTask> tri;
-  for (uint32_t v = n; v-- > 0;) {
+  for (uint32_t v = g->motif.mirrored ? n : 0u; v-- > 0;) {
     const uint32_t deg = rk_degree(g, v), high = deg - below[v];
     if (deg <= kTriPairs) break;  // so have all vertices of lower rank
     if (!high) continue;
@@ -747,13 +805,17 @@ int motif4_by_identities(gpm_graph* g, uint64_t out[6]) {
   unsigned int* queue = reinterpret_cast<unsigned int*>(g->counters + 8);
   if (g->m) {
     hipLaunchKernelGGL(zero_u32_kernel, dim3(grid_of(g, g->m)), dim3(256), 0, g->stream, tri, g->m);
+    if (!tk.mirrored)
+      hipLaunchKernelGGL(entry_triangles_kernel, dim3(grid_of(g, g->m * kWave)), dim3(kBlock), 0,
+                         g->stream, g->rk_off, g->rk_adj, tk.below, g->n, g->m, tri);
     if (tk.n_triangles)
       hipLaunchKernelGGL(stream_triangles_kernel,
                          dim3((unsigned)std::min<uint64_t>(tk.n_triangles, (uint64_t)cus * 8)),
                          dim3(kBlock), 0, g->stream, g->rk_off, g->rk_adj, tk.below, g->n,
                          static_cast<const TriangleTask*>(tk.triangles), tk.n_triangles, tri);
-    hipLaunchKernelGGL(pair_triangles_kernel, dim3(grid_of(g, (uint64_t)g->n * kTriPairs)),
-                       dim3(kBlock), 0, g->stream, g->rk_off, g->rk_adj, tk.below, g->n, tri);
+    if (tk.mirrored)
+      hipLaunchKernelGGL(pair_triangles_kernel, dim3(grid_of(g, (uint64_t)g->n * kTriPairs)),
+                         dim3(kBlock), 0, g->stream, g->rk_off, g->rk_adj, tk.below, g->n, tri);
     hipLaunchKernelGGL(edge_stats_kernel, dim3(sum_grid((uint64_t)g->n * kWave)), dim3(kBlock), 0,
                        g->stream, g->rk_off, g->rk_adj, tk.below, tri, g->n, g->counters);
     GPM_HIP(hipGetLastError());
@@ -769,8 +831,8 @@ int motif4_by_identities(gpm_graph* g, uint64_t out[6]) {
                        ccnt, cyc_bytes / 4);
   if (tk.n_heavy)
     hipLaunchKernelGGL(cycles_kernel, dim3(blocks_c), dim3(kCycBlock), 0, g->stream, g->rk_off,
-                       g->rk_adj, g->n, static_cast<const CycleTask*>(tk.heavy), tk.n_heavy, queue,
-                       ccnt, g->counters + 5);
+                       g->rk_adj, g->n, static_cast<const CycleTask*>(tk.heavy), tk.n_heavy,
+                       narrow_limit(g), queue, ccnt, g->counters + 5);
   if (tk.n_light)
     hipLaunchKernelGGL(light_cycles_kernel,
                        dim3((unsigned)std::min<uint64_t>(tk.n_light, (uint64_t)cus * 5)),

@@ -98,3 +98,18 @@ def test_ends_past_the_lists_that_point_back(gpm, orc, mids, ends, pool):
     dst += [np.array([0, 0])]
     g = directed(gpm, sink + extra, np.concatenate(src), np.concatenate(dst))
     assert motif4(gpm, g) == recount(gpm, orc, g)
+
+
+@pytest.mark.parametrize("n,m,mutual,loops", [(40, 300, 0.0, 0), (300, 6000, 0.3, 0), (300, 6000, 0.999, 0),
+                                              (120, 3000, 1.0, 1), (1500, 30000, 0.5, 20)])
+def test_triangles_of_one_sided_lists(gpm, orc, n, m, mutual, loops):
+    """A random digraph with some, nearly all and all edges in both lists, and loops."""
+    rng = np.random.default_rng(n + m)
+    src, dst = rng.integers(0, n, m), (rng.random(m) ** 2 * n).astype(np.int64)
+    both = rng.random(m) < mutual
+    own = rng.permutation(n)[:loops]
+    keep = src != dst
+    g = gpm.csr_from_edges(n, np.concatenate([src[keep], dst[keep & both], own]).astype(np.uint32),
+                           np.concatenate([dst[keep], src[keep & both], own]).astype(np.uint32),
+                           gpm.CSR_SORT | gpm.CSR_DEDUP)
+    assert motif4(gpm, g) == recount(gpm, orc, g)
