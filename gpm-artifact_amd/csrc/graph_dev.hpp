@@ -109,9 +109,10 @@ struct gpm_graph {
   unsigned long long* bmask = nullptr;
   uint32_t bmask_shift = 0;
   // SYMMETRIC graphs: adjacency bit matrices of the fixed patterns
-  // (pattern_bits.hip), built on first use; nbits_off: they cannot be built.
+  // (pattern_bits.hip), built on first use; nbits_off: they cannot be built,
+  // nbits_mirrored: every edge is in both its lists.
   uint32_t* nbits = nullptr;
-  bool nbits_off = false;
+  bool nbits_off = false, nbits_mirrored = false;
 };
 
 namespace gpm {
@@ -178,8 +179,9 @@ constexpr size_t kMlpWeights = 4 + 4 + 64 * 4 + 64 + 64 * 64 + 64 + 64 + 1;
 int mlp_forward(const float* d_feat, uint32_t n, const float* d_packed, float* d_out, int cus,
                 hipStream_t stream);
 // Fixed patterns on adjacency bit matrices (pattern_bits.hip).  *ok: the graph's
-// patterns are counted that way; the matrices are there.
-int prepare_pattern_bits(gpm_graph* g, bool* ok);
+// patterns are counted that way; the matrices are there.  pairs: the counting form's
+// pair counts (P4 - P6).
+int prepare_pattern_bits(gpm_graph* g, bool pairs, bool* ok);
 // Enqueues the count of pattern `pid` (the direct formulation's h[0 .. 5], or the
 // counting one's h[1], h[2]) into the zeroed out[6]; *queue is zero on entry.
 int launch_pattern_bits(gpm_graph* g, int pid, bool counting, unsigned long long* queue,

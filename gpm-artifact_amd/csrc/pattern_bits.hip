@@ -85,12 +85,13 @@ __global__ __launch_bounds__(kBlock) void zero_words_kernel(uint32_t* p, uint64_
     p[i] = 0u;
 }
 
-// The other matrices from N, and the number of bits of N.
+// The other matrices from N; total[0] += the bits of N, total[1] += those whose mirror
+// is set.
 __global__ __launch_bounds__(kBlock) void derived_bits_kernel(uint32_t* __restrict__ base,
                                                               uint32_t n, uint32_t rw,
                                                               unsigned long long* __restrict__ total) {
   const uint64_t words = (uint64_t)(n + 1) * rw;
-  uint64_t set = 0;
+  uint64_t set = 0, mirrored = 0;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < words;
        i += (uint64_t)gridDim.x * blockDim.x) {
     const uint32_t v = (uint32_t)(i / rw), w = (uint32_t)(i % rw);
@@ -103,9 +104,11 @@ __global__ __launch_bounds__(kBlock) void derived_bits_kernel(uint32_t* __restri
     base[kBelowN * words + i] = m & lo;
     base[kAboveN * words + i] = m & hi;
     set += (uint32_t)__popc(m);
+    for (uint32_t b = m; b; b &= b - 1)
+      mirrored += (base[(32 * w + (uint32_t)__builtin_ctz(b)) * (uint64_t)rw + v / 32] >> (v & 31)) & 1u;
   }
-  set = wave_sum_u64(set);
-  if (lane_id() == 0 && set) atomicAdd(total, (unsigned long long)set);
+  block_add(&total[0], set);
+  block_add(&total[1], mirrored);
 }
 
 // ---------------------------------------------------------------- the count
@@ -472,8 +475,8 @@ int ensure_bits(gpm_graph* g, bool* ok) {
     g->nbits_off = true;
     return GPM_OK;
   }
-  unsigned long long set = 0;
-  int st = zero_counters(g, 1);
+  unsigned long long set[2] = {0, 0};
+  int st = zero_counters(g, 2);
   if (st == GPM_OK) {
     hipLaunchKernelGGL(zero_words_kernel, dim3(grid_of(g, words)), dim3(kBlock), 0, g->stream, bits,
                        words);
@@ -482,18 +485,19 @@ int ensure_bits(gpm_graph* g, bool* ok) {
     hipLaunchKernelGGL(derived_bits_kernel, dim3(grid_of(g, words)), dim3(kBlock), 0, g->stream,
                        bits, g->n, rw, g->counters);
     if (hipGetLastError() != hipSuccess ||
-        hipMemcpyAsync(&set, g->counters, sizeof(set), hipMemcpyDeviceToHost, g->stream) !=
+        hipMemcpyAsync(set, g->counters, sizeof(set), hipMemcpyDeviceToHost, g->stream) !=
             hipSuccess ||
         hipStreamSynchronize(g->stream) != hipSuccess)
       st = fail(GPM_EHIP, "adjacency bit matrices");
   }
-  if (st != GPM_OK || set != g->m) {
+  if (st != GPM_OK || set[0] != g->m) {
     (void)hipStreamSynchronize(g->stream);
     (void)hipFree(bits);
     g->nbits_off = st == GPM_OK;
     return st;
   }
   g->nbits = bits;
+  g->nbits_mirrored = set[1] == set[0];
   *ok = true;
   return GPM_OK;
 }
@@ -502,10 +506,13 @@ int ensure_bits(gpm_graph* g, bool* ok) {
 
 namespace gpm {
 
-int prepare_pattern_bits(gpm_graph* g, bool* ok) {
+int prepare_pattern_bits(gpm_graph* g, bool pairs, bool* ok) {
   *ok = false;
   if (!bits_pay(g)) return GPM_OK;
   const int st = ensure_bits(g, ok);
+  // The lists take a pair's adjacency from the end of the shorter list, the matrices from
+  // one side: the same only where every edge is in both its lists.
+  if (pairs && !g->nbits_mirrored) *ok = false;
   return st != GPM_OK || !*ok ? st : ensure_src(g);
 }
 
