@@ -51,6 +51,9 @@ struct gpm_graph {
   std::vector<double> h_lpair;
   std::vector<uint32_t> h_off;
   double met_degree = -1.0;  // see mean_met_degree
+  // 1: every edge is once in both its lists and there are no loops, 0: not so (an
+  // unsymmetrised edge file), -1: not known yet.
+  int mirrored = -1;
   std::vector<uint32_t> h_labels;
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -78,14 +81,13 @@ struct gpm_graph {
   gpm_graph* dag = nullptr;
   // Motif counters (motif_count.hip), built on first use: host offsets and
   // lower-neighbour counts of rk_off / rk_adj, and the task lists of the 4-cycle
-  // kernels (hbm: some heavy task counts in HBM) and the triangle kernel.  mirrored:
-  // every edge is once in both its lists, and there are no loops.
+  // kernels (hbm: some heavy task counts in HBM) and the triangle kernel.
   struct {
     std::vector<uint32_t> h_off;
     uint32_t* below = nullptr;
     void *heavy = nullptr, *light = nullptr, *triangles = nullptr;
     uint32_t n_heavy = 0, n_light = 0, n_triangles = 0;
-    bool hbm = false, mirrored = false, built = false;
+    bool hbm = false, built = false;
   } motif;
   // Last prepared matching batch (match.hip), replayed on identical calls.
   void* match_cache = nullptr;

@@ -1713,6 +1713,40 @@ bool square_plan(const QPlan& p, QPlan* sq) {
   return true;  // the tail is depth 3 alone in either order
 }
 
+// *out += the entries (u, x), x < u, that x's list answers and that u's holds once.
+__global__ __launch_bounds__(kBlock) void mirrored_entries_kernel(
+    DevGraph g, const uint32_t* __restrict__ labels, uint32_t n, uint64_t m,
+    unsigned long long* __restrict__ out) {
+  uint64_t answered = 0;
+  for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < m;
+       e += (uint64_t)gridDim.x * blockDim.x) {
+    const uint32_t u = upper_index(g.off, n + 1, (uint32_t)e) - 1, x = g.ladj[e];
+    if (x >= u || (e > g.off[u] && g.ladj[e - 1] == x)) continue;
+    uint32_t lo, len;
+    label_slice(g, x, labels[u], &lo, &len);
+    if (sorted_contains(g.ladj + lo, len, u)) ++answered;
+  }
+  block_add(out, answered);
+}
+
+// Sets g->mirrored if it is not known: one pass over the entries per handle (device-built
+// graphs know it).
+int ensure_mirrored(gpm_graph* g, const DevGraph& dg) {
+  if (g->mirrored >= 0) return GPM_OK;
+  int st = zero_counters(g, 1);
+  if (st != GPM_OK) return st;
+  const unsigned blocks = (unsigned)std::max<uint64_t>(
+      1, std::min<uint64_t>((g->m + kBlock - 1) / kBlock, (uint64_t)device_cus(g) * 8));
+  hipLaunchKernelGGL(mirrored_entries_kernel, dim3(blocks), dim3(kBlock), 0, g->stream, dg,
+                     g->labels, g->n, g->m, g->counters);
+  GPM_HIP(hipGetLastError());
+  unsigned long long answered = 0;
+  GPM_HIP(hipMemcpyAsync(&answered, g->counters, sizeof(answered), hipMemcpyDeviceToHost, g->stream));
+  GPM_HIP(hipStreamSynchronize(g->stream));
+  g->mirrored = 2 * answered == g->m ? 1 : 0;
+  return GPM_OK;
+}
+
 // Builds g->lpos and g->lloc if missing.
 int ensure_label_positions(gpm_graph* g, const uint32_t* d_lvoff) {
   if (g->lloc) return GPM_OK;
@@ -2033,12 +2067,16 @@ int build_batch(gpm_graph* g, std::vector<QPlan> plans, int n_counters, const gp
     }
   }
   // Square plans leave the tasks.  (A model sizes tasks by predicted root costs,
-  // and a hipGraph replays one launch: both keep the DFS.)
+  // and a hipGraph replays one launch: both keep the DFS.  So do lists that are not
+  // mirrored: the DFS reads an edge off the list of its plan's order, and leaves out
+  // loops, which the square's counters do not.)
   if (squares && !learned && !tun.use_graph) {
     std::vector<uint32_t> which;
     QPlan sq;
     for (uint32_t i = 0; i < nq; ++i)
       if (plans[i].n_roots && square_plan(plans[i], &sq)) which.push_back(i);
+    if (!which.empty() && (st = ensure_mirrored(g, b->dg)) != GPM_OK) return st;
+    if (g->mirrored != 1) which.clear();
     st = build_squares(g, plans, which, rlen, d_lvoff, n_counters, b);
     if (st == GPM_ENOMEM)
       clear_error();  // the DFS takes them

@@ -678,7 +678,7 @@ uint32_t rk_degree(const gpm_graph* g, uint32_t v) {
 }
 
 // Roots of fewer lower neighbours have 16-bit counters (a repeated entry could pass them).
-uint32_t narrow_limit(const gpm_graph* g) { return g->motif.mirrored ? 65536u : 0u; }
+uint32_t narrow_limit(const gpm_graph* g) { return g->mirrored == 1 ? 65536u : 0u; }
 
 // The tasks of the motif counters (g->motif), built once per handle from every
 // vertex's lower neighbours and wedge total.
@@ -711,7 +711,7 @@ int ensure_motif_tasks(gpm_graph* g) {
                            g->stream));
     GPM_HIP(hipStreamSynchronize(g->stream));
   }
-  g->motif.mirrored = 2 * wedges[n] == g->m;
+  g->mirrored = 2 * wedges[n] == g->m ? 1 : 0;
   const uint32_t narrow_below = narrow_limit(g);
   std::vector<uint32_t> roots;
   std::vector<CycleTask> heavy, light;
@@ -739,7 +739,7 @@ int ensure_motif_tasks(gpm_graph* g) {
   }
   // Triangle tasks, in decreasing degree (rank).
   std::vector<TriangleTask> tri;
-  for (uint32_t v = g->motif.mirrored ? n : 0u; v-- > 0;) {
+  for (uint32_t v = g->mirrored == 1 ? n : 0u; v-- > 0;) {
     const uint32_t deg = rk_degree(g, v), high = deg - below[v];
     if (deg <= kTriPairs) break;  // so have all vertices of lower rank
     if (!high) continue;
@@ -805,7 +805,7 @@ int motif4_by_identities(gpm_graph* g, uint64_t out[6]) {
   unsigned int* queue = reinterpret_cast<unsigned int*>(g->counters + 8);
   if (g->m) {
     hipLaunchKernelGGL(zero_u32_kernel, dim3(grid_of(g, g->m)), dim3(256), 0, g->stream, tri, g->m);
-    if (!tk.mirrored)
+    if (g->mirrored != 1)
       hipLaunchKernelGGL(entry_triangles_kernel, dim3(grid_of(g, g->m * kWave)), dim3(kBlock), 0,
                          g->stream, g->rk_off, g->rk_adj, tk.below, g->n, g->m, tri);
     if (tk.n_triangles)
@@ -813,7 +813,7 @@ int motif4_by_identities(gpm_graph* g, uint64_t out[6]) {
                          dim3((unsigned)std::min<uint64_t>(tk.n_triangles, (uint64_t)cus * 8)),
                          dim3(kBlock), 0, g->stream, g->rk_off, g->rk_adj, tk.below, g->n,
                          static_cast<const TriangleTask*>(tk.triangles), tk.n_triangles, tri);
-    if (tk.mirrored)
+    if (g->mirrored == 1)
       hipLaunchKernelGGL(pair_triangles_kernel, dim3(grid_of(g, (uint64_t)g->n * kTriPairs)),
                          dim3(kBlock), 0, g->stream, g->rk_off, g->rk_adj, tk.below, g->n, tri);
     hipLaunchKernelGGL(edge_stats_kernel, dim3(sum_grid((uint64_t)g->n * kWave)), dim3(kBlock), 0,

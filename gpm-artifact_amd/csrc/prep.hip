@@ -468,8 +468,10 @@ int build(uint32_t n, const uint32_t* src, const uint32_t* dst, uint64_t n_edges
   b.release(d_adj);
   hipStream_t s = stream;
   stream = nullptr;  // the handle owns it now
-  return adopt_device_csr(n, m, d_off, d_adj, std::move(h_off), h_adj.data(), labels, n_labels,
-                          graph_flags, s, out);
+  st = adopt_device_csr(n, m, d_off, d_adj, std::move(h_off), h_adj.data(), labels, n_labels,
+                        graph_flags, s, out);
+  if (st == GPM_OK && sym && dedup && drop_self) (*out)->mirrored = 1;
+  return st;
 }
 
 int relabel(gpm_graph* g, gpm_graph** out, uint32_t** perm) {
@@ -554,6 +556,7 @@ int relabel(gpm_graph* g, gpm_graph** out, uint32_t** perm) {
     std::free(p);
     return st;
   }
+  (*out)->mirrored = g->mirrored;
   *perm = p;
   return GPM_OK;
 }
