@@ -442,11 +442,12 @@ __device__ __forceinline__ void for_wedges(const uint32_t* __restrict__ off,
 // bounds are some 20 dependent loads, and 16 waves share the CU.  Cutting the
 // heaviest roots into narrower bands lost (7.3 - 9.4 ms): the queue's order ends
 // evenly without it.
+// kMirrored: no list holds a vertex twice, which could pass a counter of 16 bits.
+template <bool kMirrored>
 __global__ __launch_bounds__(kCycBlock) void cycles_kernel(
     const uint32_t* __restrict__ off, const uint32_t* __restrict__ adj, uint32_t n,
-    const CycleTask* __restrict__ tasks, uint32_t n_tasks, uint32_t narrow_below,
-    unsigned int* __restrict__ queue, uint32_t* __restrict__ counters,
-    unsigned long long* __restrict__ out) {
+    const CycleTask* __restrict__ tasks, uint32_t n_tasks, unsigned int* __restrict__ queue,
+    uint32_t* __restrict__ counters, unsigned long long* __restrict__ out) {
   __shared__ __align__(16) uint32_t s_cnt[kCycWords];
   __shared__ uint32_t s_task;
   uint64_t acc = 0;
@@ -463,7 +464,7 @@ __global__ __launch_bounds__(kCycBlock) void cycles_kernel(
     t.lo = uniform(t.lo);
     t.hi = uniform(t.hi);
     t.band = uniform(t.band);
-    const uint32_t half = t.n_below < narrow_below ? 1u : 0u;  // counters of 16 bits
+    const uint32_t half = kMirrored && t.n_below < 65536u ? 1u : 0u;  // counters of 16 bits
     const uint32_t words = (t.hi - t.band + half) >> half;
     uint32_t* cnt = counters + (uint64_t)blockIdx.x * n;
     if (t.lo == t.band) {
@@ -677,9 +678,6 @@ uint32_t rk_degree(const gpm_graph* g, uint32_t v) {
   return g->motif.h_off[v + 1] - g->motif.h_off[v];
 }
 
-// Roots of fewer lower neighbours have 16-bit counters (a repeated entry could pass them).
-uint32_t narrow_limit(const gpm_graph* g) { return g->mirrored == 1 ? 65536u : 0u; }
-
 // The tasks of the motif counters (g->motif), built once per handle from every
 // vertex's lower neighbours and wedge total.
 int ensure_motif_tasks(gpm_graph* g) {
@@ -712,7 +710,6 @@ int ensure_motif_tasks(gpm_graph* g) {
     GPM_HIP(hipStreamSynchronize(g->stream));
   }
   g->mirrored = 2 * wedges[n] == g->m ? 1 : 0;
-  const uint32_t narrow_below = narrow_limit(g);
   std::vector<uint32_t> roots;
   std::vector<CycleTask> heavy, light;
   for (uint32_t u = n; u-- > 0;) {
@@ -725,7 +722,7 @@ int ensure_motif_tasks(gpm_graph* g) {
                    [&](uint32_t a, uint32_t b) { return wedges[a] > wedges[b]; });
   bool hbm = false;
   for (const uint32_t u : roots) {
-    const uint32_t band = below[u] < narrow_below ? 2 * kCycWords : kCycWords;
+    const uint32_t band = g->mirrored == 1 && below[u] < 65536u ? 2 * kCycWords : kCycWords;
     uint32_t hi = u;
     auto task_to = [&](uint32_t lo) {
       heavy.push_back({u, below[u], lo, hi, hi - lo > band ? hi - band : lo});
@@ -830,9 +827,10 @@ int motif4_by_identities(gpm_graph* g, uint64_t out[6]) {
     hipLaunchKernelGGL(zero_u32_kernel, dim3(grid_of(g, cyc_bytes / 4)), dim3(256), 0, g->stream,
                        ccnt, cyc_bytes / 4);
   if (tk.n_heavy)
-    hipLaunchKernelGGL(cycles_kernel, dim3(blocks_c), dim3(kCycBlock), 0, g->stream, g->rk_off,
-                       g->rk_adj, g->n, static_cast<const CycleTask*>(tk.heavy), tk.n_heavy,
-                       narrow_limit(g), queue, ccnt, g->counters + 5);
+    hipLaunchKernelGGL(g->mirrored == 1 ? cycles_kernel<true> : cycles_kernel<false>,
+                       dim3(blocks_c), dim3(kCycBlock), 0, g->stream, g->rk_off, g->rk_adj, g->n,
+                       static_cast<const CycleTask*>(tk.heavy), tk.n_heavy, queue, ccnt,
+                       g->counters + 5);
   if (tk.n_light)
     hipLaunchKernelGGL(light_cycles_kernel,
                        dim3((unsigned)std::min<uint64_t>(tk.n_light, (uint64_t)cus * 5)),
