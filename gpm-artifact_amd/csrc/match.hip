@@ -41,6 +41,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <memory>
 #include <numeric>
 #include <queue>
 #include <vector>
@@ -2387,18 +2388,24 @@ int plan_queries(gpm_graph* g, const gpm_query* queries, int n_queries, const gp
     }
     return GPM_OK;
   }
-  MatchBatch* t = new MatchBatch();
+  const std::unique_ptr<MatchBatch, void (*)(void*)> t(new MatchBatch(), free_batch);
   std::vector<double> scale;
-  int st = build_batch(g, trial_plans, 0, tun, t, &scale);
+  int st = build_batch(g, trial_plans, 0, tun, t.get(), &scale);
+  if (st == GPM_ENOMEM) {  // untried: the plans of the label statistics
+    (void)hipGetLastError();
+    clear_error();
+    return GPM_OK;
+  }
+  if (st != GPM_OK) return st;
   std::vector<unsigned long long> work(3 * (size_t)t->n_queries, 0ull);
-  if (st == GPM_OK && t->n_tasks) {
+  if (t->n_tasks) {
     hipLaunchKernelGGL(zero_kernel, dim3((3 * t->n_queries + 64) / 64 + 1), dim3(64), 0,
                        g->stream, t->d_work, 3 * t->n_queries, nullptr, 0);
-    st = launch_batch(g, t);
-    if (st == GPM_OK && (hipMemcpyAsync(work.data(), t->d_work, work.size() * 8,
-                                        hipMemcpyDeviceToHost, g->stream) != hipSuccess ||
-                         hipStreamSynchronize(g->stream) != hipSuccess))
-      st = fail(GPM_EHIP, "plan trial");
+    if ((st = launch_batch(g, t.get())) != GPM_OK) return st;
+    if (hipMemcpyAsync(work.data(), t->d_work, work.size() * 8, hipMemcpyDeviceToHost, g->stream) !=
+            hipSuccess ||
+        hipStreamSynchronize(g->stream) != hipSuccess)
+      return fail(GPM_EHIP, "plan trial");
   }
   // Estimated cost of a plan: its total weighted steps (sampled x scale).
   // Heavy roots are dealt out in parts and short batches are cut further at
