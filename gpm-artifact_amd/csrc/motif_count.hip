@@ -745,6 +745,8 @@ int ensure_motif_tasks(gpm_graph* g) {
     for (uint32_t c = 0; c < end; c += kTriLists) tri.push_back({v, c, std::min(end, c + kTriLists)});
   }
   auto put = [&](const auto& list, void** d) -> int {
+    (void)hipFree(*d);  // of an attempt that did not get to the end
+    *d = nullptr;
     if (list.empty()) return GPM_OK;
     if (hipMalloc(d, list.size() * sizeof(list[0])) != hipSuccess) {
       *d = nullptr;
