@@ -446,10 +446,11 @@ extern "C" int gpm_setops(int op, int variant, uint32_t n_pairs, const uint64_t*
                           uint32_t* out_ab, uint32_t* out_b) {
   return ::gpm::guarded([&]() -> int {
     clear_error();
-    void* workspace = nullptr;
-    const int st = run_setops(op, variant, n_pairs, a_off, a, b_off, b, ub, counts, out_a, out_ab,
-                              out_b, &workspace);
-    (void)hipFree(workspace);
-    return st;
+    struct Workspace {
+      void* p = nullptr;
+      ~Workspace() { (void)hipFree(p); }
+    } workspace;
+    return run_setops(op, variant, n_pairs, a_off, a, b_off, b, ub, counts, out_a, out_ab, out_b,
+                      &workspace.p);
   });
 }
