@@ -2614,12 +2614,10 @@ extern "C" int gpm_match_batch(gpm_graph* g, const gpm_query* queries, int n_que
     MatchBatch* b = static_cast<MatchBatch*>(g->match_cache);
     if (!b || b->key != key) {
       free_match_cache(g);
-      b = new MatchBatch();
-      int st = prepare_batch(g, queries, n_queries, tun, b);
-      if (st != GPM_OK) {
-        free_batch(b);
-        return st;
-      }
+      std::unique_ptr<MatchBatch, void (*)(void*)> made(new MatchBatch(), free_batch);
+      int st = prepare_batch(g, queries, n_queries, tun, made.get());
+      if (st != GPM_OK) return st;
+      b = made.release();
       b->key.swap(key);
       g->match_cache = b;
     }
