@@ -112,6 +112,7 @@ int get_tiers(gpm_graph* g, const TierRequest& req, const RootTiers** out) {
     if (st == GPM_OK) return keep(g, std::move(key), t, out);
     release(t);
     if (st != GPM_ENOMEM) return st;
+    (void)hipGetLastError();  // or the next launch's check reports it
     clear_error();
   }
   std::vector<uint32_t> candidates;
