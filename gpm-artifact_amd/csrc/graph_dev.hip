@@ -74,7 +74,10 @@ std::vector<std::pair<int, hipStream_t>>& idle_streams() {
 }
 }  // namespace
 
-hipError_t stream_take(int device, hipStream_t* stream) {
+hipError_t stream_take(hipStream_t* stream) {
+  int device = 0;
+  const hipError_t e = hipGetDevice(&device);
+  if (e != hipSuccess) return e;
   {
     std::lock_guard<std::mutex> lock(idle_mutex);
     auto& idle = idle_streams();
@@ -88,9 +91,11 @@ hipError_t stream_take(int device, hipStream_t* stream) {
   return hipStreamCreateWithFlags(stream, hipStreamNonBlocking);
 }
 
-void stream_give(int device, hipStream_t stream) {
+void stream_give(hipStream_t stream) {
   if (!stream) return;
-  if (hipStreamSynchronize(stream) == hipSuccess) {
+  hipDevice_t device = 0;
+  if (hipStreamSynchronize(stream) == hipSuccess &&
+      hipStreamGetDevice(stream, &device) == hipSuccess) {
     std::lock_guard<std::mutex> lock(idle_mutex);
     if (idle_streams().size() < kIdleStreams) {
       idle_streams().emplace_back(device, stream);
@@ -269,7 +274,7 @@ void release(gpm_graph* g) {
     if (e) (void)hipEventDestroy(e);
   if (g->ev0) hipEventDestroy(g->ev0);
   if (g->ev1) hipEventDestroy(g->ev1);
-  stream_give(g->device, g->stream);
+  stream_give(g->stream);
   delete g;
 }
 
@@ -415,7 +420,7 @@ int gpm_graph_create(const uint32_t* offsets, uint32_t n, const uint32_t* adj,
     if (labels) g->h_labels.assign(labels, labels + n);
     int st = GPM_OK;
     do {
-      if (stream_take(g->device, &g->stream) != hipSuccess ||
+      if (stream_take(&g->stream) != hipSuccess ||
           hipEventCreate(&g->ev0) != hipSuccess || hipEventCreate(&g->ev1) != hipSuccess) {
         st = fail(GPM_EHIP, "stream/event creation failed");
         break;
@@ -522,7 +527,7 @@ int gpm_graph_orient(gpm_graph* sym, gpm_graph** dag) {
     g->adj = adj;
     for (uint32_t v = 0; v < g->n; ++v) g->max_deg = std::max(g->max_deg, h_off[v + 1] - h_off[v]);
     g->h_off = std::move(h_off);
-    if (stream_take(g->device, &g->stream) != hipSuccess ||
+    if (stream_take(&g->stream) != hipSuccess ||
         hipEventCreate(&g->ev0) != hipSuccess || hipEventCreate(&g->ev1) != hipSuccess)
       st = fail(GPM_EHIP, "stream/event creation failed");
     else if (hipMalloc(&g->counters, kCounters * sizeof(unsigned long long)) != hipSuccess)

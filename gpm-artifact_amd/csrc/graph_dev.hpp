@@ -125,10 +125,10 @@ namespace gpm {
 // source's DMA lands: a kernel launched next on the handle's stream could
 // read the old contents.)
 int h2d(gpm_graph* g, void* dst, const void* src, size_t bytes);
-// A non-blocking stream of the device, its caller's until stream_give, which waits for
-// its work.
-hipError_t stream_take(int device, hipStream_t* stream);
-void stream_give(int device, hipStream_t stream);
+// A non-blocking stream of the current device (a call for a handle of another device
+// gets one too), its caller's until stream_give, which waits for its work.
+hipError_t stream_take(hipStream_t* stream);
+void stream_give(hipStream_t stream);
 // Grows g->scratch to at least `bytes`; returns status.
 int ensure_scratch(gpm_graph* g, size_t bytes);
 // Builds g->src (COO sources) if missing.

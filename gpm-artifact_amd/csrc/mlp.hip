@@ -259,7 +259,7 @@ int gpm_mlp_predict(const float* feat, uint32_t n, const float* norm_mean, const
     GPM_HIP(hipGetDevice(&dev));
     float *d_w = nullptr, *d_feat = nullptr, *d_out = nullptr;
     hipStream_t stream = nullptr;
-    hipError_t e = stream_take(dev, &stream);
+    hipError_t e = stream_take(&stream);
     if (e == hipSuccess) e = hipMalloc(&d_w, (wcount + 1) * 4);  // and the check's word
     if (e == hipSuccess) e = hipMalloc(&d_feat, (size_t)std::max(n, 1u) * 16);
     if (e == hipSuccess) e = hipMalloc(&d_out, (size_t)std::max(n, 1u) * 4);
@@ -285,7 +285,7 @@ int gpm_mlp_predict(const float* feat, uint32_t n, const float* norm_mean, const
     (void)hipFree(d_w);
     (void)hipFree(d_feat);
     (void)hipFree(d_out);
-    stream_give(dev, stream);
+    stream_give(stream);
     if (e == hipSuccess && bad) return fail(GPM_EINVAL, "features must be finite and > -1");
     if (e != hipSuccess) return fail(GPM_EHIP, "mlp predict: %s", hipGetErrorString(e));
     return GPM_OK;

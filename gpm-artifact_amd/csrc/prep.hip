@@ -361,14 +361,11 @@ int build(uint32_t n, const uint32_t* src, const uint32_t* dst, uint64_t n_edges
   GPM_HIP(hipGetDevice(&dev));
   GPM_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   hipStream_t stream = nullptr;
-  GPM_HIP(stream_take(dev, &stream));
+  GPM_HIP(stream_take(&stream));
   struct StreamGuard {
-    int device;
     hipStream_t* s;
-    ~StreamGuard() {
-      stream_give(device, *s);
-    }
-  } guard{dev, &stream};
+    ~StreamGuard() { stream_give(*s); }
+  } guard{&stream};
   Bufs b;
   int st;
   // One workspace: the records as emitted (later the unique keys), the sorted
@@ -480,14 +477,11 @@ int relabel(gpm_graph* g, gpm_graph** out, uint32_t** perm) {
   const uint64_t m = g->m;
   int cus = device_cus(g);
   hipStream_t stream = nullptr;
-  GPM_HIP(stream_take(g->device, &stream));
+  GPM_HIP(stream_take(&stream));
   struct StreamGuard {
-    int device;
     hipStream_t* s;
-    ~StreamGuard() {
-      stream_give(device, *s);
-    }
-  } guard{g->device, &stream};
+    ~StreamGuard() { stream_give(*s); }
+  } guard{&stream};
   // The source graph's pending work must be done before this stream reads it.
   GPM_HIP(hipStreamSynchronize(g->stream));
   Bufs b;
