@@ -1067,6 +1067,7 @@ int gpm_clique(gpm_graph* g, int k, const gpm_sched* sched, uint64_t* out) {
     std::vector<float> deg_cost;
     int st = prepare_request(g, sched, (uint32_t)(k - 1), &req, &deg_cost);
     if (st != GPM_OK) return st;
+    if (k == 4) req.min_part_rows = 16;  // count4_rows deals whole blocks of 16 rows
     const RootTiers* t = nullptr;
     if ((st = get_tiers(g, req, &t)) != GPM_OK) return st;
     if ((st = timing_begin(g)) != GPM_OK) return st;

@@ -17,10 +17,10 @@ namespace {
 TierKey key_of(const TierRequest& r, uint32_t n) {
   TierKey k;
   char buf[256];
-  std::snprintf(buf, sizeof(buf), "%u/%u/%u/%u/%u/%u/%d/%u/%a/%u/%u/%u/%d", r.min_deg,
+  std::snprintf(buf, sizeof(buf), "%u/%u/%u/%u/%u/%u/%d/%u/%a/%u/%u/%u/%u/%d", r.min_deg,
                 r.wave_cap, r.block_cap, r.block2_cap, r.root_begin, r.root_end, r.policy, r.chunk,
                 (double)r.heavy_cost, r.resident_block, r.resident_block2, r.resident_big,
-                r.rank != nullptr);
+                r.min_part_rows, r.rank != nullptr);
   k.params = buf;
   if (r.policy == GPM_SCHED_LEARNED && r.cost) k.cost.assign(r.cost, r.cost + n);
   if (r.n_root_list) k.roots.assign(r.root_list, r.root_list + r.n_root_list);
@@ -189,7 +189,7 @@ int get_tiers(gpm_graph* g, const TierRequest& req, const RootTiers** out) {
         const double c = std::max(0.f, req.cost[v]);
         if (target > 0.0 && c > target)
           np = (uint32_t)std::min<double>(kMaxParts, std::ceil(c / target));
-        np = std::max(1u, std::min(np, d / kMinRowsPerPart));
+        np = std::max(1u, std::min(np, d / req.min_part_rows));
         if (np > 1) {
           any = true;
           ++n_split;

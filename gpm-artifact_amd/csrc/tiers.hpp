@@ -62,14 +62,14 @@ struct TierRequest {
   // root predicted to cost more than a quarter of a block's fair share of
   // its tier is split into parts (0 = never split).
   uint32_t resident_block = 0, resident_block2 = 0, resident_big = 0;
+  uint32_t min_part_rows = 8;  // fewest rows a part is given: every part builds all rows
   // When set, the uploaded root lists hold rank[v] instead of v (kernels
   // that read the topologically relabelled DAG).
   const uint32_t* rank = nullptr;
 };
 
-// Most parts a root is split into, and fewest rows a part is given.
+// Most parts a root is split into.
 constexpr uint32_t kMaxParts = 64;
-constexpr uint32_t kMinRowsPerPart = 8;
 
 // Returns cached tiers for (graph, request); builds and uploads on a miss.
 int get_tiers(gpm_graph* g, const TierRequest& req, const RootTiers** out);
