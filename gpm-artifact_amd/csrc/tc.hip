@@ -10,7 +10,7 @@
 //                partial sums that a one-block kernel adds up.
 //  GPM_TC_VERTEX (v_centric, TCSolver.cuh:64-113, tc_hi_warp_vertex.cuh):
 //                on the DAG relabelled by total degree (gpm_graph's
-//                toff/tadj): one wave per root u with |N+(u)| <= 64 searches
+//                toff/tadj): 8 or 16 lanes per root u with |N+(u)| <= 16 search
 //                the pairs of N+(u) in each other's lists; one 256-thread block
 //                per larger root streams the lists N+(v), v in N+(u), past an
 //                LDS bitmap of N+(u).  Graphs of near-uniform degrees, and
@@ -621,14 +621,14 @@ int enqueue_tc(gpm_graph* g, int variant, bool mark) {
       GPM_HIP(hipGetLastError());
       if (mark) timing_mark(g, "tc_vertex_block");
     }
-    // The roots are in decreasing degree: those above 16, above 8 and the rest.
-    const uint32_t cuts[] = {0, t->n_wave_above[1], t->n_wave_above[0], t->n_wave};
-    for (int c = 0; c < 3; ++c) {
+    // The roots are in decreasing degree: those above 8 and the rest.
+    const uint32_t cuts[] = {0, t->n_wave_above8, t->n_wave};
+    for (int c = 0; c < 2; ++c) {
       const uint32_t count = cuts[c + 1] - cuts[c];
       if (!count) continue;
-      const int G = c == 0 ? 32 : c == 1 ? 16 : 8;
+      const int G = c == 0 ? 16 : 8;
       const uint64_t blocks = ((uint64_t)count * G + kBlock - 1) / kBlock;
-      auto kern = c == 0 ? tc_pairs_kernel<32> : c == 1 ? tc_pairs_kernel<16> : tc_pairs_kernel<8>;
+      auto kern = c == 0 ? tc_pairs_kernel<16> : tc_pairs_kernel<8>;
       hipLaunchKernelGGL(kern, dim3((unsigned)std::min<uint64_t>(blocks, (uint64_t)cus * 8)),
                          dim3(kBlock), 0, g->stream, g->toff, g->tadj, t->d_wave + cuts[c], count,
                          g->counters);

@@ -65,8 +65,7 @@ int device_tiers(gpm_graph* g, const TierRequest& req, uint32_t rb, uint32_t re,
     if (d < req.min_deg) continue;
     if (d <= req.wave_cap) {
       ++t->n_wave;
-      t->n_wave_above[0] += d > 8;
-      t->n_wave_above[1] += d > 16;
+      t->n_wave_above8 += d > 8;
     } else if (d <= req.block_cap) {
       ++t->n_block;
       t->max_block_deg = std::max(t->max_block_deg, d);
@@ -211,11 +210,7 @@ int get_tiers(gpm_graph* g, const TierRequest& req, const RootTiers** out) {
   }
   RootTiers t;
   t.n_wave = (uint32_t)wave.size();
-  for (const uint32_t v : wave) {
-    const uint32_t d = g->h_off[v + 1] - g->h_off[v];
-    t.n_wave_above[0] += d > 8;
-    t.n_wave_above[1] += d > 16;
-  }
+  for (const uint32_t v : wave) t.n_wave_above8 += g->h_off[v + 1] - g->h_off[v] > 8;
   t.n_block = (uint32_t)block.size();
   t.n_big = (uint32_t)big.size();
   t.max_block_deg = maxb;

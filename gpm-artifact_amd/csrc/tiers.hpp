@@ -18,7 +18,7 @@ struct RootTiers {
   uint32_t* d_all = nullptr;    // where set, the four lists below are parts of it
   uint32_t* d_wave = nullptr;   // roots served by one wave
   uint32_t n_wave = 0;
-  uint32_t n_wave_above[2] = {0, 0};  // ... of out-degree above 8, above 16
+  uint32_t n_wave_above8 = 0;   // ... of out-degree above 8
   uint32_t* d_block = nullptr;  // roots served by one block, rows in LDS
   uint32_t n_block = 0;
   uint32_t max_block_deg = 0;
