@@ -113,16 +113,27 @@ __global__ __launch_bounds__(kBlock) void derived_bits_kernel(uint32_t* __restri
 
 // ---------------------------------------------------------------- the count
 
-// The set bits of a segment (one word per lane) as ascending ids into list,
-// filled up with `none` to a multiple of 64; returns how many there are.
-__device__ __forceinline__ uint32_t list_bits(uint32_t word, uint32_t seg, uint32_t none,
-                                              uint16_t* list) {
-  const uint32_t incl = wave_incl_scan((uint32_t)__popc(word));
-  const uint32_t total = uniform(wave_bcast(incl, kWave - 1));
-  uint32_t at = incl - (uint32_t)__popc(word);
-  const uint32_t id0 = seg * kSegIds + 32 * lane_id();
+// The set bits of as many segments from *seg on (word(w): word w of the set) as fit the
+// list, as ascending ids, filled up with `none` to a multiple of 64; returns how
+// many there are and moves *seg on.  (A list per segment padded every segment's few ids
+// to a block: Erdos-Renyi n = 16384, degree 46, 64 pairs of blocks an edge for the 9 that
+// hold its ids, 374 ms for the direct P2, 28.5 now; lists 441.)
+template <typename F>
+__device__ __forceinline__ uint32_t list_bits(F&& set_word, uint32_t* seg, uint32_t segs,
+                                              uint32_t none, uint16_t* list) {
+  uint32_t total = 0;
   __builtin_amdgcn_wave_barrier();
-  for (; word; word &= word - 1) list[at++] = (uint16_t)(id0 + __builtin_ctz(word));
+  for (uint32_t s = uniform(*seg); s < segs; ++s) {
+    uint32_t word = set_word(s * kSegWords + lane_id());
+    const uint32_t incl = wave_incl_scan((uint32_t)__popc(word));
+    const uint32_t here = uniform(wave_bcast(incl, kWave - 1));
+    if (total + here > kSegIds) break;  // the next list's
+    uint32_t at = total + incl - (uint32_t)__popc(word);
+    const uint32_t id0 = s * kSegIds + 32 * lane_id();
+    for (; word; word &= word - 1) list[at++] = (uint16_t)(id0 + __builtin_ctz(word));
+    total += here;
+    *seg = s + 1;
+  }
   list[total + lane_id()] = (uint16_t)none;
   __builtin_amdgcn_wave_barrier();
   return total;
@@ -193,6 +204,8 @@ __device__ __forceinline__ uint32_t product_tiles(const Product& p, const uint16
     const uint32_t last = min(__builtin_amdgcn_readlane(ib[t], 15) / kStepIds, p.steps - 1);
     const uint32_t word = ib[t] / 32 - 4 * g, bit = 1u << (ib[t] & 31);
     for (uint32_t c = first; c <= last; ++c) {
+      // Ids of several segments may leave steps out.
+      if (p.steps > kSegIds / kStepIds && wave_ballot(ib[t] / kStepIds == c) == 0ull) continue;
       const uintx4 ca = four(p.ca + 16 * c + 4 * g);
       uintx4 wa[J];
 #pragma unroll
@@ -286,7 +299,7 @@ __device__ __forceinline__ uint64_t sum_products(const uint32_t* x, const uint32
 }
 
 // One wave per directed edge, in chunks from a queue.  LDS per wave: two lists
-// and two sets of rw words.  PRODUCTS: P2, P3, P5 - P8 (16 tiles of sizes and
+// and two sets of rw words.  ONE: the graph has one segment.  PRODUCTS: P2, P3, P5 - P8 (16 tiles of sizes and
 // their operands: 226 registers, 2 waves per SIMD; bounds that make it spill are
 // not safe, as matrix instructions read every lane's register); otherwise P1,
 // P4 and Motif4.  R-MAT, 16 edges a vertex, all of P1 - P8 and Motif4: n = 512
@@ -296,7 +309,7 @@ __device__ __forceinline__ uint64_t sum_products(const uint32_t* x, const uint32
 // counters, and a block adds its sums up: additions to one address take about
 // 10 ns each, and with one counter and a sum per wave they were most of the n = 512
 // launches (P1 - P8 and Motif4: 1.71 ms so, 1.26 now).
-template <bool PRODUCTS>
+template <bool PRODUCTS, bool ONE>
 __global__ __launch_bounds__(kBlock, PRODUCTS ? 2 : 4) void pattern_bits_kernel(
     const uint32_t* __restrict__ adj, const uint32_t* __restrict__ src, uint64_t m, Bits g,
     int pid, bool counting, uint32_t chunk, unsigned long long* __restrict__ queue,
@@ -308,7 +321,7 @@ __global__ __launch_bounds__(kBlock, PRODUCTS ? 2 : 4) void pattern_bits_kernel(
   uint32_t* s1 = s0 + g.rw;
   uint16_t* l0 = reinterpret_cast<uint16_t*>(s1 + g.rw);
   uint16_t* l1 = l0 + kListLen;
-  const uint32_t segs = g.rw / kSegWords, words = (g.n + 31) / 32, steps = (g.n + kStepIds - 1) / kStepIds;
+  const uint32_t segs = ONE ? 1u : g.rw / kSegWords, words = (g.n + 31) / 32, steps = (g.n + kStepIds - 1) / kStepIds;
   const uint32_t none = g.n;
   uint64_t c[6] = {0, 0, 0, 0, 0, 0};
   const uint32_t n_chunks = (uint32_t)((m + chunk - 1) / chunk);
@@ -347,8 +360,8 @@ __global__ __launch_bounds__(kBlock, PRODUCTS ? 2 : 4) void pattern_bits_kernel(
       // sum over a in R of |set & X[a]|
       auto sums = [&](auto r, int x, const uint32_t* set) {
         uint64_t t = 0;
-        for (uint32_t k = 0; k < segs; ++k) {
-          const uint32_t na = list_bits(r(k * kSegWords + lane), k, none, l0);
+        for (uint32_t k = 0; k < segs;) {
+          const uint32_t na = list_bits(r, &k, segs, none, l0);
           t += sum_rows(g.row(x, 0), set, g.rw, words, l0, na);
         }
         return t;
@@ -408,12 +421,14 @@ __global__ __launch_bounds__(kBlock, PRODUCTS ? 2 : 4) void pattern_bits_kernel(
         p.steps = steps;
         p.in = pairs || !counting;
         uint64_t t = 0;
-        for (uint32_t k = 0; k < segs; ++k) {
-          const uint32_t na = list_bits(r1(k * kSegWords + lane), k, none, l0);
+        for (uint32_t k = 0; k < segs;) {
+          const uint32_t first = k, na = list_bits(r1, &k, segs, none, l0);
           if (!na) continue;
-          for (uint32_t k2 = 0; k2 < (wedge ? k + 1 : segs); ++k2) {
-            const uint32_t nb = list_bits(r2(k2 * kSegWords + lane), k2, none, l1);
-            if (nb) t += product(p, l0, na, l1, nb, wedge && k2 == k);
+          // One set's lists are cut at the same segments.
+          for (uint32_t k2 = 0; k2 < (wedge ? k : segs);) {
+            const bool same = wedge && k2 == first;
+            const uint32_t nb = list_bits(r2, &k2, segs, none, l1);
+            if (nb) t += product(p, l0, na, l1, nb, same);
           }
         }
         if (!counting) {
@@ -428,8 +443,8 @@ __global__ __launch_bounds__(kBlock, PRODUCTS ? 2 : 4) void pattern_bits_kernel(
           if (!wedge) fill(s1, d10);
           const uint32_t* x = g.row(wedge ? kAboveNotN : kNotN, 0);
           const uint32_t* y = g.row(pid == 8 ? kBelowN : kBelowNotN, 0);
-          for (uint32_t k = 0; k < segs; ++k) {
-            const uint32_t nb = list_bits(r2(k * kSegWords + lane), k, none, l1);
+          for (uint32_t k = 0; k < segs;) {
+            const uint32_t nb = list_bits(r2, &k, segs, none, l1);
             c[1] += sum_products(x, wedge ? s0 : s1, y, s0, g.rw, words, l1, nb);
           }
         }
@@ -528,8 +543,12 @@ int launch_pattern_bits(gpm_graph* g, int pid, bool counting, unsigned long long
   const unsigned blocks = (unsigned)std::min<uint64_t>(
       (g->m + (uint64_t)chunk * kWaves - 1) / (chunk * kWaves), (uint64_t)device_cus(g) * per_cu);
   const bool products = pid != GPM_P1 && pid != GPM_P4 && pid != GPM_MOTIF4;
-  hipLaunchKernelGGL(products ? pattern_bits_kernel<true> : pattern_bits_kernel<false>, dim3(blocks), dim3(kBlock), lds, g->stream, g->adj,
-                     g->src, g->m, b, pid, counting, chunk, queue, out);
+  const bool one = g->n <= kSegIds;
+  auto kern = products ? (one ? pattern_bits_kernel<true, true> : pattern_bits_kernel<true, false>)
+              : one    ? pattern_bits_kernel<false, true>
+                       : pattern_bits_kernel<false, false>;
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(kBlock), lds, g->stream, g->adj, g->src, g->m, b,
+                     pid, counting, chunk, queue, out);
   GPM_HIP(hipGetLastError());
   timing_mark(g, counting ? "pattern_counting" : "pattern_direct");
   return GPM_OK;
