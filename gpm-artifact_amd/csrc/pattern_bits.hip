@@ -228,6 +228,28 @@ __device__ __forceinline__ uint32_t product_tiles(const Product& p, const uint16
   return (uint32_t)sum;
 }
 
+// The pairs of two short lists one by one, each lane some of the columns: where a row has
+// many steps, a tile of mostly empty rows takes longer.  Erdos-Renyi n = 16384, degree
+// 80, P6 (0.4 common neighbours an edge): 6.8 ms in tiles, 4.5 so.
+constexpr uint32_t kFewPairs = 4;
+__device__ __forceinline__ uint64_t few_pairs(const Product& p, const uint16_t* a, uint32_t na,
+                                              const uint16_t* b, uint32_t nb) {
+  uint32_t sum = 0;
+  for (uint32_t i = 0; i < na; ++i) {
+    const uint32_t* x = p.x + uniform(a[i]) * p.rw;
+    for (uint32_t j = 0; j < nb; ++j) {
+      const uint32_t ib = uniform(b[j]);
+      const uint32_t* y = p.y + ib * p.rw;
+      const bool in = ((x[ib / 32] & p.ca[ib / 32]) >> (ib & 31)) & 1u;
+      uint32_t c = 0;
+      for (uint32_t w = lane_id(); w < 16 * p.steps; w += kWave)
+        c += (uint32_t)__popc(x[w] & p.ca[w] & y[w] & p.cb[w]);
+      if (in == p.in) sum += c;
+    }
+  }
+  return sum;
+}
+
 // Every pair of the lists a (na entries) and b (nb); triangular: only pairs with
 // b's block up to a's count (lists of one set, X or Y leave nothing beyond).
 __device__ __forceinline__ uint64_t product(const Product& p, const uint16_t* a, uint32_t na,
@@ -299,7 +321,9 @@ __device__ __forceinline__ uint64_t sum_products(const uint32_t* x, const uint32
 }
 
 // One wave per directed edge, in chunks from a queue.  LDS per wave: two lists
-// and two sets of rw words.  ONE: the graph has one segment.  PRODUCTS: P2, P3, P5 - P8 (16 tiles of sizes and
+// and two sets of rw words.  ONE: the graph has one segment.  SUMS: the
+// frequency sums too (the counting P2, P3, P7, P8), which spilled scalars slow down, so
+// several segments have an instance without them.  PRODUCTS: P2, P3, P5 - P8 (16 tiles of sizes and
 // their operands: 226 registers, 2 waves per SIMD; bounds that make it spill are
 // not safe, as matrix instructions read every lane's register); otherwise P1,
 // P4 and Motif4.  R-MAT, 16 edges a vertex, all of P1 - P8 and Motif4: n = 512
@@ -309,7 +333,7 @@ __device__ __forceinline__ uint64_t sum_products(const uint32_t* x, const uint32
 // counters, and a block adds its sums up: additions to one address take about
 // 10 ns each, and with one counter and a sum per wave they were most of the n = 512
 // launches (P1 - P8 and Motif4: 1.71 ms so, 1.26 now).
-template <bool PRODUCTS, bool ONE>
+template <bool PRODUCTS, bool ONE, bool SUMS>
 __global__ __launch_bounds__(kBlock, PRODUCTS ? 2 : 4) void pattern_bits_kernel(
     const uint32_t* __restrict__ adj, const uint32_t* __restrict__ src, uint64_t m, Bits g,
     int pid, bool counting, uint32_t chunk, unsigned long long* __restrict__ queue,
@@ -396,20 +420,27 @@ __global__ __launch_bounds__(kBlock, PRODUCTS ? 2 : 4) void pattern_bits_kernel(
         auto r1 = [&](uint32_t w) { return i1 ? both(w) : wedge ? d01(w) : d10(w); };
         auto r2 = [&](uint32_t w) { return i2 ? both(w) : d01(w); };
         // Edges without a common neighbour, or whose ends share all of them,
-        // often have nothing to count.
-        uint32_t any1 = 0, any2 = 0;
+        // often have nothing to count: R1 and R2 need an entry each, R2 two in P2 and P8
+        // (b and one of its columns) and three in P3 and P7 (and an a).
+        const uint32_t least = wedge ? 3u : pairs ? 1u : 2u;
+        uint32_t any1 = 0, in2 = 0;
         for (uint32_t w = lane; w < g.rw; w += kWave) {
           any1 |= r1(w);
-          any2 |= r2(w);
+          in2 += (uint32_t)__popc(r2(w));
         }
-        if (wave_ballot(any2 != 0u) == 0ull) continue;
-        if (wave_ballot(any1 != 0u) == 0ull && (!counting || pairs)) continue;
-        if (pairs) {
-          fill(s0, [&](uint32_t w) { return r2(w) | d10(w); });
-          fill(s1, d10);
-        } else {
-          fill(s0, r2);
+        if (wave_ballot(any1 != 0u) == 0ull) continue;
+        const uint32_t lanes = (uint32_t)__popcll(wave_ballot(in2 != 0u));
+        if (lanes < least && (lanes == 0u || uniform(wave_sum_u32(in2)) < least)) continue;
+        __builtin_amdgcn_wave_barrier();
+        for (uint32_t w = lane; w < g.rw; w += kWave) {
+          const uint32_t r = r2(w), d = pairs ? d10(w) : 0u;
+          s0[w] = r | d;
+          if (pairs) s1[w] = d;
         }
+        __builtin_amdgcn_wave_barrier();
+        // R2, and R1 where it is the same set, off the words in LDS.
+        auto set2 = [&](uint32_t w) { return pairs ? s0[w] & ~s1[w] : s0[w]; };
+        auto set1 = [&](uint32_t w) { return wedge || pid == 6 ? set2(w) : r1(w); };
         Product p;
         p.x = g.row(wedge ? kBelowNotN : kNotN, 0);
         p.y = g.row(pairs ? kNotN
@@ -422,20 +453,23 @@ __global__ __launch_bounds__(kBlock, PRODUCTS ? 2 : 4) void pattern_bits_kernel(
         p.in = pairs || !counting;
         uint64_t t = 0;
         for (uint32_t k = 0; k < segs;) {
-          const uint32_t first = k, na = list_bits(r1, &k, segs, none, l0);
+          const uint32_t first = k, na = list_bits(set1, &k, segs, none, l0);
           if (!na) continue;
           // One set's lists are cut at the same segments.
           for (uint32_t k2 = 0; k2 < (wedge ? k : segs);) {
             const bool same = wedge && k2 == first;
-            const uint32_t nb = list_bits(r2, &k2, segs, none, l1);
-            if (nb) t += product(p, l0, na, l1, nb, same);
+            const uint32_t nb = list_bits(set2, &k2, segs, none, l1);
+            if (!ONE && !SUMS && na * nb <= kFewPairs)
+              t += few_pairs(p, l0, na, l1, nb);
+            else if (nb)
+              t += product(p, l0, na, l1, nb, same);
           }
         }
         if (!counting) {
           c[0] += t;
         } else if (pairs) {
           c[1] += t;
-        } else {
+        } else if (SUMS) {
           c[2] += t;
           // Frequency times count per v in R2 (s0): P2, P8: non-neighbours in
           // D10 times the entries of R2 below v; P3, P7: non-neighbours in R2
@@ -444,7 +478,7 @@ __global__ __launch_bounds__(kBlock, PRODUCTS ? 2 : 4) void pattern_bits_kernel(
           const uint32_t* x = g.row(wedge ? kAboveNotN : kNotN, 0);
           const uint32_t* y = g.row(pid == 8 ? kBelowN : kBelowNotN, 0);
           for (uint32_t k = 0; k < segs;) {
-            const uint32_t nb = list_bits(r2, &k, segs, none, l1);
+            const uint32_t nb = list_bits(set2, &k, segs, none, l1);
             c[1] += sum_products(x, wedge ? s0 : s1, y, s0, g.rw, words, l1, nb);
           }
         }
@@ -543,10 +577,12 @@ int launch_pattern_bits(gpm_graph* g, int pid, bool counting, unsigned long long
   const unsigned blocks = (unsigned)std::min<uint64_t>(
       (g->m + (uint64_t)chunk * kWaves - 1) / (chunk * kWaves), (uint64_t)device_cus(g) * per_cu);
   const bool products = pid != GPM_P1 && pid != GPM_P4 && pid != GPM_MOTIF4;
-  const bool one = g->n <= kSegIds;
-  auto kern = products ? (one ? pattern_bits_kernel<true, true> : pattern_bits_kernel<true, false>)
-              : one    ? pattern_bits_kernel<false, true>
-                       : pattern_bits_kernel<false, false>;
+  const bool one = g->n <= kSegIds, sums = counting && pid != GPM_P5 && pid != GPM_P6;
+  auto kern = !products ? (one ? pattern_bits_kernel<false, true, false>
+                               : pattern_bits_kernel<false, false, false>)
+              : one  ? pattern_bits_kernel<true, true, true>
+              : sums ? pattern_bits_kernel<true, false, true>
+                     : pattern_bits_kernel<true, false, false>;
   hipLaunchKernelGGL(kern, dim3(blocks), dim3(kBlock), lds, g->stream, g->adj, g->src, g->m, b,
                      pid, counting, chunk, queue, out);
   GPM_HIP(hipGetLastError());
