@@ -52,12 +52,14 @@ int device_cus(const gpm_graph* g) {
 
 double mean_met_degree(gpm_graph* g) {
   if (g->met_degree < 0.0) {
-    double d2 = 0.0;
+    double d2 = 0.0, d3 = 0.0;
     for (uint32_t v = 0; v < g->n; ++v) {
       const double d = g->h_off[v + 1] - g->h_off[v];
       d2 += d * d;
+      d3 += d * d * d;
     }
     g->met_degree = g->m ? d2 / (double)g->m : 0.0;
+    if (g->m) g->met_skew = d3 * (double)g->m / (d2 * d2);
   }
   return g->met_degree;
 }

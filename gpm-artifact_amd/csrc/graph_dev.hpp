@@ -50,7 +50,7 @@ struct gpm_graph {
   // when L > 1024.  Feeds the matcher's cost estimates.
   std::vector<double> h_lpair;
   std::vector<uint32_t> h_off;
-  double met_degree = -1.0;  // see mean_met_degree
+  double met_degree = -1.0, met_skew = 1.0;  // see mean_met_degree
   // 1: every edge is once in both its lists and there are no loops, 0: not so (an
   // unsymmetrised edge file), -1: not known yet.
   int mirrored = -1;
@@ -142,7 +142,9 @@ int timing_begin(gpm_graph* g);
 int timing_mark(gpm_graph* g, const char* name);
 // The results at src go to dst behind the stop mark: one wait for both.
 int timing_end(gpm_graph* g, void* dst = nullptr, const void* src = nullptr, size_t bytes = 0);
-// Mean list length an adjacency entry meets, sum d^2 / sum d (kept on the handle).
+// Mean list length an adjacency entry meets, dw = sum d^2 / sum d, and (g->met_skew) the
+// mean square over its square, sum d^3 / (dw^2 sum d): 1 where all lists have one
+// length.  Kept on the handle.
 double mean_met_degree(gpm_graph* g);
 // Number of compute units of the handle's device.
 int device_cus(const gpm_graph* g);
@@ -180,10 +182,9 @@ constexpr size_t kMlpWeights = 4 + 4 + 64 * 4 + 64 + 64 * 64 + 64 + 64 + 1;
 // `stream` (mlp.hip).
 int mlp_forward(const float* d_feat, uint32_t n, const float* d_packed, float* d_out, int cus,
                 hipStream_t stream);
-// Fixed patterns on adjacency bit matrices (pattern_bits.hip).  *ok: the graph's
-// patterns are counted that way; the matrices are there.  pairs: the counting form's
-// pair counts (P4 - P6).
-int prepare_pattern_bits(gpm_graph* g, bool pairs, bool* ok);
+// Fixed patterns on adjacency bit matrices (pattern_bits.hip).  *ok: pattern `pid` in
+// this form is counted that way; the matrices are there.
+int prepare_pattern_bits(gpm_graph* g, int pid, bool counting, bool* ok);
 // Enqueues the count of pattern `pid` (the direct formulation's h[0 .. 5], or the
 // counting one's h[1], h[2]) into the zeroed out[6]; *queue is zero on entry.
 int launch_pattern_bits(gpm_graph* g, int pid, bool counting, unsigned long long* queue,

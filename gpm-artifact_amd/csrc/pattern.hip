@@ -551,7 +551,7 @@ extern "C" int gpm_pattern(gpm_graph* g, int pattern_id, int formulation, uint64
       // The matrix path counts the same pairs whether a block mask would have
       // ruled them out or not.
       bool bits = false;
-      if ((st = prepare_pattern_bits(g, counting && h1_only, &bits)) != GPM_OK) return st;
+      if ((st = prepare_pattern_bits(g, pattern_id, counting, &bits)) != GPM_OK) return st;
       BlockMask blk{nullptr, 0};
       if (prefilter && !bits) {
         if ((st = ensure_block_mask(g)) != GPM_OK) return st;

@@ -494,21 +494,33 @@ unsigned grid_of(const gpm_graph* g, uint64_t threads) {
       1, std::min<uint64_t>((threads + kBlock - 1) / kBlock, (uint64_t)device_cus(g) * 16));
 }
 
-// Whether the matrix path is the faster one.  It costs every edge n / 2048
-// segments of set work and every 16 x 16 pairs n / 512 steps; lists cost an edge
-// the pairs of its sets, each at least a window and a search.  So it is taken
-// up to one segment, and beyond where the degree an edge meets, dw = sum d^2 /
-// sum d, is large.  P2, P3, P6, P8 (both formulations) and P4, ms in all, matrix
-// against lists: Erdos-Renyi n = 1500, dw = 17: 2.0 against 6.7; n = 4096, dw = 9:
-// 3.8, 3.7; dw = 17: 8.4, 13; n = 16384, dw = 17: 532, 44; R-MAT n = 1500, dw = 48:
-// 2.0, 143; n = 8192, dw = 63: 30, 881; n = 16384, dw = 83: 226, 2994.  (Since rows are
-// loaded 16 bytes a lane the matrix side takes 1.0, 1.5, 17 and 117 in the first and the
-// three R-MAT cases; the line leaves graphs of 4096 and more vertices that are near it
-// to the lists.)
-bool bits_pay(gpm_graph* g) {
+// Whether the matrix path is the faster one for the pattern.  Up to one segment it is
+// everywhere (a half of the lists' time on sparse graphs, a hundredth on dense or skewed
+// ones).  Beyond, an edge costs it n / 2048 segments of set work and a block pair n / 512
+// steps, and lists the pairs of its sets, so the lists get longer with the graph: dw =
+// sum d^2 / sum d >= 16 sqrt(n / 2048).  On skewed lists the hubs' edges, one wave's
+// work each, bound the list kernels: matrix / list ms on R-MAT n = 16384, 31762
+// entries, P2 1.8 / 480, counting 3.7 / 20; counting P3 5.3 / 43.  On lists of
+// about one length the patterns that are cheap on lists cross later, measured on
+// Erdos-Renyi graphs:
+//   counting P3 (its sums read whole rows):  n = 8192: dw = 32 8.9 / 6.5, 65 34 / 41;
+//                                            n = 16384: 81 215 / 168, 129 569 / 661
+//   counting P2:  n = 16384: dw = 47 71 / 58, 81 264 / 373;  n = 8192: 32 9.6 / 12.5
+//   P1:           n = 16384: dw = 47 6.3 / 5.5, 81 16 / 20;  Motif4: 47 17 / 13, 57 23 / 21
+// Vertices of few common neighbours leave the matrices up to 1.3 times the lists' time in
+// P5 - P7 (n = 16384, dw = 101, P6 7.1 / 5.5); where there are some they take a fifth
+// (groups of 200 in n = 16000: P6 19 / 86), which the degrees do not tell.
+bool bits_pay(gpm_graph* g, int pid, bool counting) {
   if (g->n > kBitsMaxN || !g->m) return false;
   if (g->n <= kSegIds) return true;
-  return mean_met_degree(g) >= 16.0 * std::sqrt((double)g->n / kSegIds);
+  const double segs = (double)g->n / kSegIds, dw = mean_met_degree(g);
+  if (dw < 16.0 * std::sqrt(segs)) return false;
+  if (segs <= 2.0) return true;
+  if (pid == GPM_P1) return dw >= 8.0 * segs || g->met_skew >= 1.5;
+  if (pid == GPM_MOTIF4) return dw >= 7.0 * segs || g->met_skew >= 1.5;
+  if (counting && pid == GPM_P2) return dw >= 8.0 * segs || g->met_skew >= 2.5;
+  if (counting && pid == GPM_P3) return dw >= 14.0 * segs || g->met_skew >= 2.5;
+  return true;
 }
 
 // Builds g->nbits if missing; *ok is false where the lists hold an entry twice
@@ -555,9 +567,10 @@ int ensure_bits(gpm_graph* g, bool* ok) {
 
 namespace gpm {
 
-int prepare_pattern_bits(gpm_graph* g, bool pairs, bool* ok) {
+int prepare_pattern_bits(gpm_graph* g, int pid, bool counting, bool* ok) {
   *ok = false;
-  if (!bits_pay(g)) return GPM_OK;
+  if (!bits_pay(g, pid, counting)) return GPM_OK;
+  const bool pairs = counting && (pid == GPM_P4 || pid == GPM_P5 || pid == GPM_P6);
   const int st = ensure_bits(g, ok);
   // The lists take a pair's adjacency from the end of the shorter list, the matrices from
   // one side: the same only where every edge is in both its lists.
