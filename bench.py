@@ -286,9 +286,11 @@ def extra_sched(scale):
 
 def extra_patterns(scale_both, scale_counting):
     """P1-P8 (G2MinerSolver and PatternSolver): both formulations on R-MAT
-    scale_both (counts must agree), the counting formulation and its BLOCK_OPT
-    prefilter on scale_counting.  The direct enumeration of P3 takes 18 s at
-    scale 12 and the counting formulation of P2 68 s at scale 16, so the rows
+    scale_both (counts must agree), the counting formulation on scale_counting,
+    and there P4-P6 on the list kernels with their BLOCK_OPT prefilter: up to
+    16384 vertices the patterns are counted on bit matrices, which need no
+    prefilter, so isolated vertices take the graph past them.  The lists'
+    counting P3 takes 2.6 s at scale 12 and P2 68 s at scale 16, so the rows
     stay at scales 11 and 12."""
     out = {"workload": f"P1-P8 on R-MAT (edge factor 16, seed 20240522): both formulations at "
                        f"scale {scale_both}, counting formulation at scale {scale_counting}"}
@@ -307,13 +309,19 @@ def extra_patterns(scale_both, scale_counting):
     print("[bench] patterns small scale done", file=sys.stderr, flush=True)
     g = G.rmat_graph(scale_counting, 16, 20240522)
     rows = {}
-    with G.DeviceGraph(g, oriented=False) as sym:
+    past = G.HostCSR(np.append(g.offsets, np.full(16385 - g.n, g.offsets[-1], np.uint32)), g.adj)
+    with G.DeviceGraph(g, oriented=False) as sym, G.DeviceGraph(past, oriented=False) as lists:
         for pid in pids:
             _, counted = sym.pattern(pid, G.FORM_PATTERN)
-            t_count = sym.last_kernel_ms()
-            _, pref = sym.pattern(pid, G.FORM_BLOCK_PREFILTER)
-            rows[pid] = {"count": int(counted), "identical": int(counted) == int(pref),
-                         "pattern_ms": t_count, "block_prefilter_ms": sym.last_kernel_ms()}
+            rows[pid] = {"count": int(counted), "identical": True, "pattern_ms": sym.last_kernel_ms()}
+            if pid in ("P5", "P6"):  # (the counting P4 has no list kernel without the prefilter)
+                _, plain = lists.pattern(pid, G.FORM_PATTERN)
+                rows[pid]["lists_ms"] = lists.last_kernel_ms()
+                rows[pid]["identical"] = int(counted) == int(plain)
+            if pid in ("P4", "P5", "P6"):
+                _, pref = lists.pattern(pid, G.FORM_BLOCK_PREFILTER)
+                rows[pid]["block_prefilter_ms"] = lists.last_kernel_ms()
+                rows[pid]["identical"] &= int(counted) == int(pref)
     out[f"scale{scale_counting}"] = rows
     print("[bench] patterns done", file=sys.stderr, flush=True)
     return out

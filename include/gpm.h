@@ -331,7 +331,10 @@ enum gpm_formulation {
   GPM_FORM_PATTERN = 1, /* frequency x count - correction (PatternSolver)   */
   GPM_FORM_BLOCK_PREFILTER = 2, /* PatternSolver with the BLOCK_OPT block-
                                    mask prefilter for P4, P5, P6
-                                   (PatternSolver.cuh:109-151)              */
+                                   (PatternSolver.cuh:109-151).  Graphs whose
+                                   pattern is counted on adjacency bit
+                                   matrices (at most 16384 vertices) need no
+                                   mask: the same counts without it          */
 };
 
 /*
@@ -465,8 +468,6 @@ int gpm_match_batch(gpm_graph* g, const gpm_query* queries, int n_queries,
  * root candidate v, 0 for other vertices (n entries); feat[4v .. 4v+3] = the
  * model's features of root candidate v (degree, depth-1 label-slice length,
  * degrees summed over that slice, query size), zeros elsewhere (4n).
- * Both currently return GPM_EUNSUPPORTED: the root log stopped responding
- * once on the device and stays switched off until the cause is found.
  */
 int gpm_match_root_work(gpm_graph* g, const gpm_query* query, int policy, uint64_t* work);
 int gpm_match_root_features(gpm_graph* g, const gpm_query* query, int policy, float* feat);
