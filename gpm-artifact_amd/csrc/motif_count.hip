@@ -56,6 +56,7 @@ constexpr uint32_t kLightSlots = 4096;
 static_assert(kLightSlots >= 2 * kCycHeavy, "load factor at most 1/2");
 // 64-entry windows of a list in flight per wave.
 constexpr uint32_t kCycWindows = 4;
+constexpr uint32_t kCycShort = 2;  // lists of so many entries are the lanes' own
 
 // The wedges u - v - x with lo <= x < hi (hi <= u), v one of the n_below first
 // neighbours of u.  Ranks from band on have their counters in LDS.
@@ -378,7 +379,12 @@ __device__ __forceinline__ void count_below2(const uint32_t* __restrict__ a, uin
 // over the block's waves one by one (whole groups of 64 left most waves idle on
 // roots of a few hundred): the lanes find the bounds of their lists' parts, then
 // the wave streams one part after another, 64 consecutive entries a load and the
-// next windows loaded before the last are handled.
+// next windows loaded before the last are handled.  Parts of up to kCycShort entries
+// are left to the lanes that found them: a hub over 200000 vertices of two neighbours
+// is one block's, which loaded them for one lane's work at a time (K(2, 200000): 4.8 ms
+// in windows alone, 1.2 ms; R-MAT scale 19: 6.9 and 6.6 ms).  With 4 or 8 entries
+// R-MAT scale 19 gains more (6.5, 6.3 ms), but graphs of even degrees lose (100000
+// vertices of degree 16: 0.44 ms with 0 - 2, 0.46 and 0.51 ms).
 template <int BS, typename F>
 __device__ __forceinline__ void for_wedges(const uint32_t* __restrict__ off,
                                            const uint32_t* __restrict__ adj, const CycleTask& t,
@@ -396,7 +402,9 @@ __device__ __forceinline__ void for_wedges(const uint32_t* __restrict__ off,
       b += first;
       len = end - first;
     }
-    uint64_t todo = wave_ballot(len != 0u);
+    for (uint32_t i = 0; i < kCycShort; ++i)
+      if (len <= kCycShort && i < len) f(adj[b + i]);
+    uint64_t todo = wave_ballot(len > kCycShort);
     uint32_t cb = 0, cn = 0, ct = 0, x[kCycWindows];
     auto next = [&]() {  // moves on to the next batch of windows; false after the last
       ct += kCycWindows * kWave;
@@ -436,7 +444,7 @@ __device__ __forceinline__ void for_wedges(const uint32_t* __restrict__ off,
 // clears them on the way.  Lower ranks count in HBM (the block's n counters at
 // `counters`): the increments' previous values sum to C(count, 2) there, and a
 // second walk clears them.  R-MAT scale 19 (2.2e9 wedges, 98 % of them below 7100
-// roots): 7.0 ms with the light roots, against 42.7 ms for one 256-thread block
+// roots): 6.6 ms with the light roots, against 42.7 ms for one 256-thread block
 // per CU that searched the owner of every wedge, kept 40000 32-bit counters in
 // LDS and listed the touched ones.  What is left is latency: a group's list
 // bounds are some 20 dependent loads, and 16 waves share the CU.  Cutting the
