@@ -1,8 +1,8 @@
 // Fixed-pattern counting on a symmetric graph (replaces G2MinerSolver and
 // PatternSolver, src/G2MinerSolver.cuh and src/PatternSolver.cuh).
 //
-// The kernels here work on sorted lists.  Graphs of up to 16384 vertices whose
-// lists are not short are counted on adjacency bit matrices instead
+// The kernels here work on sorted lists.  Graphs of up to 16384 vertices are
+// counted on adjacency bit matrices instead where those are faster, by pattern
 // (pattern_bits.hip), with the same results.
 //
 // Direct formulation (GPM_FORM_G2MINER): one wave per directed edge
@@ -40,7 +40,8 @@
 //    new_edge_warp.cuh:647-679): P4, P5 and P6 first test a pair against a
 //    64-bit block mask per vertex (bit b set when the vertex has a neighbour
 //    in id block b, blocks of 2^shift ids, 64 blocks cover all ids) and
-//    binary-search only pairs the mask cannot rule out.
+//    binary-search only pairs the mask cannot rule out.  Bit matrices have no
+//    searches to save, and no part of the mask.
 #include <algorithm>
 #include <vector>
 

@@ -284,7 +284,7 @@ __global__ __launch_bounds__(kBlock) void setops_kernel(
 // First entry of x that is not above the one before it within its list (off[0 ..
 // n_lists]: where the lists begin and end), to *first (preset to the largest value)
 // per array; blockIdx.y is the array.  Bound by the one read of the entries.  4096
-// pairs (25 MB): the call took 4.1 ms with this on the host, 2.85 with it here and
+// pairs (25 MB): the call took 3.7 - 4.0 ms with this on the host, 2.6 with it here and
 // short results packed.
 struct Lists {
   const uint32_t* x[2];
